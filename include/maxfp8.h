@@ -476,6 +476,18 @@ int maxfp8_fused_silu(
     int64_t out_row_stride, int64_t scales_ld, int in_dtype, int quantize, void* stream);
 
 /*
+ * silu(gate) * up and the quantisation of the result for the matmul behind it, in one pass: the bytes and scales of
+ * maxfp8_fused_silu with quantize == 0 (round_activation != 0: == 2) followed by maxfp8_quantize_dynamic_scaled_fp8 on its
+ * bf16 result, without that tensor being written and read back.  group_size 128: out_scales[k / 128, m] (row stride scales_ld);
+ * group_size == inter: one scale per row, out_scales[m], inter at most 32768.  The other operands as in maxfp8_fused_silu.
+ */
+int maxfp8_silu_quantize_dynamic_scaled_fp8(
+    void* out_fp8, void* out_scales, const void* in, const uint32_t* row_offsets,
+    int64_t num_offsets, int64_t max_rows, int64_t inter, int64_t in_row_stride,
+    int64_t out_row_stride, int64_t group_size, int64_t scales_ld, int in_dtype,
+    int round_activation, float scale_ub, void* stream);
+
+/*
  * Elementwise f32 -> e4m3fn (clamp to +-448, round to nearest even), the cast
  * inside fp8_quantize (max/kernels/src/internal_utils/fp8_utils.mojo:96-143).
  * Exposed so the hardware convert can be checked exhaustively.

@@ -43,6 +43,7 @@ EXPORTS = (
     "maxfp8_quantize_tensor_dynamic_scaled_fp8",
     "maxfp8_moe_create_indices",
     "maxfp8_fused_silu",
+    "maxfp8_silu_quantize_dynamic_scaled_fp8",
     "maxfp8_cast_f32_to_e4m3fn",
     "maxfp8_cast_e4m3fn_to_f32",
     "maxfp8_cast_f32_to_bf16",
@@ -115,6 +116,8 @@ def lib() -> ctypes.CDLL:
     L.maxfp8_moe_create_indices.argtypes = [vp] * 6 + [i64, i64, vp]
     L.maxfp8_fused_silu.restype = ci
     L.maxfp8_fused_silu.argtypes = [vp] * 4 + [i64] * 6 + [ci, ci, vp]
+    L.maxfp8_silu_quantize_dynamic_scaled_fp8.restype = ci
+    L.maxfp8_silu_quantize_dynamic_scaled_fp8.argtypes = [vp] * 4 + [i64] * 7 + [ci, ci, cf, vp]
     L.maxfp8_cast_f32_to_e4m3fn.restype = ci
     L.maxfp8_cast_f32_to_e4m3fn.argtypes = [vp, vp, i64, vp]
     L.maxfp8_cast_f32_to_bf16.restype = ci

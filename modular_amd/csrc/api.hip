@@ -37,8 +37,8 @@ int rmsnorm_quantize_dispatch(void*, void*, const void*, const void*, int64_t, i
 int quantize_static_dispatch(void*, const void*, int64_t, int64_t, int64_t, int64_t, int, float, hipStream_t);
 int quantize_tensor_dispatch(void*, void*, const void*, int64_t, int64_t, int64_t, int64_t, int, int, float, hipStream_t);
 int moe_create_indices_dispatch(uint32_t*, uint32_t*, uint32_t*, int32_t*, uint32_t*, const int32_t*, int64_t, int64_t, hipStream_t);
-int fused_silu_dispatch(void*, float*, const void*, const uint32_t*, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int,
-                        hipStream_t);
+int fused_silu_dispatch(void*, float*, const void*, const uint32_t*, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, bool,
+                        float, hipStream_t);
 int cast_f32_to_e4m3fn_dispatch(void*, const float*, int64_t, hipStream_t);
 int cast_e4m3fn_to_f32_dispatch(float*, const void*, int64_t, hipStream_t);
 int cast_f32_to_bf16_dispatch(void*, const float*, int64_t, hipStream_t);
@@ -339,23 +339,41 @@ int maxfp8_moe_create_indices(uint32_t* token_expert_order, uint32_t* expert_sta
                                      expert_usage_stats, (const int32_t*)topk_ids, n, num_experts, (hipStream_t)stream);
 }
 
-int maxfp8_fused_silu(void* out, void* out_scales, const void* in, const uint32_t* row_offsets, int64_t num_offsets,
-                      int64_t max_rows, int64_t inter, int64_t in_row_stride, int64_t out_row_stride, int64_t scales_ld,
-                      int in_dtype, int quantize, void* stream) {
+static int fused_silu_common(void* out, void* out_scales, const void* in, const uint32_t* row_offsets, int64_t num_offsets,
+                             int64_t max_rows, int64_t inter, int64_t in_row_stride, int64_t out_row_stride, int64_t scales_ld,
+                             int in_dtype, int mode, bool row_scales, float scale_ub, void* stream) {
   if (in_dtype != MAXFP8_BF16) MAXFP8_FAIL(MAXFP8_ERR_DTYPE, "fused_silu: input dtype %d is not bf16", in_dtype);
   if (max_rows < 0 || inter < 0 || num_offsets < 1) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused_silu: bad sizes");
   if (max_rows == 0 || inter == 0) return MAXFP8_OK;
+  if (max_rows >= ((int64_t)1 << 31) || inter >= ((int64_t)1 << 30)) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused_silu: sizes must fit 31 bits");
   if (inter % 128 != 0)
     MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused_silu: the output width %lld must be a multiple of 128", (long long)inter);
-  if (quantize < 0 || quantize > 2) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused_silu: quantize = %d is not 0, 1 or 2", quantize);
-  const bool quant = quantize == 1;
-  if (in_row_stride < 2 * inter || out_row_stride < inter || (quant && scales_ld < max_rows))
+  const bool quant = mode != 0 && mode != 2;
+  if (in_row_stride < 2 * inter || out_row_stride < inter || (quant && !row_scales && scales_ld < max_rows))
     MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused_silu: strides smaller than the extents");
   if (!out || !in || !row_offsets || (quant && !out_scales)) MAXFP8_FAIL(MAXFP8_ERR_NULL, "fused_silu: null pointer");
   if (!is_aligned(in, 16) || in_row_stride % 8 != 0 || !is_aligned(out, 16) || out_row_stride % 8 != 0)
     MAXFP8_FAIL(MAXFP8_ERR_ALIGN, "fused_silu: rows must be 16-byte aligned");
   return fused_silu_dispatch(out, (float*)out_scales, in, row_offsets, num_offsets, max_rows, inter, in_row_stride,
-                             out_row_stride, scales_ld, quantize, (hipStream_t)stream);
+                             out_row_stride, scales_ld, mode, row_scales, scale_ub, (hipStream_t)stream);
+}
+
+int maxfp8_fused_silu(void* out, void* out_scales, const void* in, const uint32_t* row_offsets, int64_t num_offsets,
+                      int64_t max_rows, int64_t inter, int64_t in_row_stride, int64_t out_row_stride, int64_t scales_ld,
+                      int in_dtype, int quantize, void* stream) {
+  if (quantize < 0 || quantize > 2) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused_silu: quantize = %d is not 0, 1 or 2", quantize);
+  return fused_silu_common(out, out_scales, in, row_offsets, num_offsets, max_rows, inter, in_row_stride, out_row_stride, scales_ld,
+                           in_dtype, quantize, false, 0.0f, stream);
+}
+
+int maxfp8_silu_quantize_dynamic_scaled_fp8(void* out_fp8, void* out_scales, const void* in, const uint32_t* row_offsets,
+                                            int64_t num_offsets, int64_t max_rows, int64_t inter, int64_t in_row_stride,
+                                            int64_t out_row_stride, int64_t group_size, int64_t scales_ld, int in_dtype,
+                                            int round_activation, float scale_ub, void* stream) {
+  if (group_size != 128 && group_size != inter)
+    MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "silu_quantize: group size %lld is not 128 or the row's %lld outputs", (long long)group_size, (long long)inter);
+  return fused_silu_common(out_fp8, out_scales, in, row_offsets, num_offsets, max_rows, inter, in_row_stride, out_row_stride, scales_ld,
+                           in_dtype, round_activation ? 4 : 3, group_size != 128, scale_ub, stream);
 }
 
 size_t maxfp8_matmul_workspace_bytes(int64_t M, int64_t N, int64_t K) {

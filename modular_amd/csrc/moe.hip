@@ -245,14 +245,45 @@ __device__ __forceinline__ void silu_mul8(const float (&gate)[8], const float (&
   for (int j = 0; j < 8; ++j) f[j] = sig[j] * up[j];
 }
 
+// What the silu kernel does with its eight products.
+enum SiluOut {
+  kSiluBf16,       // stores them as bf16
+  kSiluQuant,      // quantises the f32 products with the op's own recipe: max(amax, 1e-4) / 448, value / scale
+  kSiluBf16Quant,  // rounds them to bf16 and quantises that like quantize_dynamic_scaled_fp8 with groups of 128: the bytes
+                   // and scales of kSiluBf16 followed by the quantiser, without the bf16 tensor between them
+};
+
+__device__ __forceinline__ uint2 pack_e4m3fn8(const float (&q)[8]) {
+  int lo = 0, hi = 0;
+  lo = cvt_pk_e4m3fn(q[0], q[1], lo, false);
+  lo = cvt_pk_e4m3fn(q[2], q[3], lo, true);
+  hi = cvt_pk_e4m3fn(q[4], q[5], hi, false);
+  hi = cvt_pk_e4m3fn(q[6], q[7], hi, true);
+  return make_uint2((uint32_t)lo, (uint32_t)hi);
+}
+__device__ __forceinline__ void unpack_bf16x8(const uint4& v, float (&f)[8]) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    f[2 * j] = __uint_as_float(w[j] << 16);
+    f[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
+  }
+}
+__device__ __forceinline__ uint4 pack_bf16x8(const float (&f)[8]) {
+  return make_uint4(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7]));
+}
+
 // 16 lanes own 128 consecutive outputs of one row (8 each): one 16-byte load of gate and of up
-// per lane; QUANT: amax over the 16 lanes by DPP, 8-byte packed fp8 store, lane 0 writes the scale.
-template <bool QUANT, bool ROUND_ACT = false>
+// per lane; quantised: amax over the 16 lanes by DPP, 8-byte packed fp8 store, lane 0 writes the scale.
+// Bound by the bytes (5 per output where the result is quantised) with the exponential and the division close behind.  Graph
+// timing, operands cold: 2048 x 14336 as kSiluBf16 and the quantiser behind it 46.7 us, as kSiluBf16Quant 35.9 (147 MB:
+// 4.1 TB/s); 32768 x 2048 104.6 and 80; 16 x 14336 6.5 and 3.7.
+template <SiluOut OUT, bool ROUND_ACT>
 __global__ __launch_bounds__(256) void fused_silu_bf16_kernel(void* __restrict__ out, float* __restrict__ scales,
                                                               const uint16_t* __restrict__ in,
                                                               const uint32_t* __restrict__ row_offsets, int num_offsets,
                                                               int64_t max_rows, int inter, int64_t in_stride,
-                                                              int64_t out_stride, int64_t scales_ld) {
+                                                              int64_t out_stride, int64_t scales_ld, float scale_ub) {
   // (the buffers hold max_rows rows: an offset beyond that -- a stale or damaged routing tensor -- must not
   // turn into accesses outside them)
   const uint32_t rows_dev = row_offsets[num_offsets - 1];
@@ -260,69 +291,144 @@ __global__ __launch_bounds__(256) void fused_silu_bf16_kernel(void* __restrict__
   const int groups = inter >> 7;
   const int tid = threadIdx.x, sub = tid & 15;
   const int64_t total = rows * groups;
+  const bool narrow = total < ((int64_t)1 << 31);
   for (int64_t item = (int64_t)blockIdx.x * 16 + (tid >> 4); item < total; item += (int64_t)gridDim.x * 16) {
-    const int64_t m = item / groups;
+    // (a 64-bit division is half as many instructions as the item's arithmetic)
+    const int64_t m = narrow ? (int64_t)((uint32_t)item / (uint32_t)groups) : item / groups;
     const int g = (int)(item - m * groups);
     const uint16_t* src = in + m * in_stride + g * 128 + sub * 8;
+    float gate[8], up[8], f[8];
     const uint4 gv = *reinterpret_cast<const uint4*>(src);
     const uint4 uv = *reinterpret_cast<const uint4*>(src + inter);
-    const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w}, uw[4] = {uv.x, uv.y, uv.z, uv.w};
-    float gate[8], up[8], f[8];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      gate[2 * j] = __uint_as_float(gw[j] << 16);
-      gate[2 * j + 1] = __uint_as_float(gw[j] & 0xffff0000u);
-      up[2 * j] = __uint_as_float(uw[j] << 16);
-      up[2 * j + 1] = __uint_as_float(uw[j] & 0xffff0000u);
-    }
+    unpack_bf16x8(gv, gate);
+    unpack_bf16x8(uv, up);
     silu_mul8<ROUND_ACT>(gate, up, f);
-    if constexpr (!QUANT) {
-      uint32_t w[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = pack_bf16x2(f[2 * j], f[2 * j + 1]);
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out) + m * out_stride + g * 128 + sub * 8) =
-          make_uint4(w[0], w[1], w[2], w[3]);
+    if constexpr (OUT == kSiluBf16) {
+      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out) + m * out_stride + g * 128 + sub * 8) = pack_bf16x8(f);
     } else {
+      if constexpr (OUT == kSiluBf16Quant) unpack_bf16x8(pack_bf16x8(f), f);
       float amax = 0.0f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(f[j]));
       amax = row16_max(amax);
-      const float scale = fmaxf(amax, 1e-4f) / 448.0f;
-      const float divisor[8] = {scale, scale, scale, scale, scale, scale, scale, scale};
-      float q[8];
-      exact_div8<true>(f, divisor, q);   // (one reciprocal and one test of the divisor for the lane's eight quotients)
+      float scale, q[8];
+      if constexpr (OUT == kSiluQuant) {
+        scale = fmaxf(amax, 1e-4f) / 448.0f;
+        const float divisor[8] = {scale, scale, scale, scale, scale, scale, scale, scale};
+        exact_div8<true>(f, divisor, q);   // (one reciprocal and one test of the divisor for the lane's eight quotients)
+      } else {
+        float recip;
+        dynamic_scale_f32(amax, scale_ub, scale, recip);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = f[j] * recip;
+      }
 #pragma unroll
       for (int j = 0; j < 8; ++j) q[j] = clamp448(q[j]);
-      int lo = 0, hi = 0;
-      lo = cvt_pk_e4m3fn(q[0], q[1], lo, false);
-      lo = cvt_pk_e4m3fn(q[2], q[3], lo, true);
-      hi = cvt_pk_e4m3fn(q[4], q[5], hi, false);
-      hi = cvt_pk_e4m3fn(q[6], q[7], hi, true);
-      *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(out) + m * out_stride + g * 128 + sub * 8) =
-          make_uint2((uint32_t)lo, (uint32_t)hi);
+      *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(out) + m * out_stride + g * 128 + sub * 8) = pack_e4m3fn8(q);
       if (sub == 0) scales[(int64_t)g * scales_ld + m] = scale;
     }
   }
 }
 
+// The same with one scale per row (per-token quantisation of the bf16 product): one block per row, NV 16-byte vectors of
+// bf16 products per thread stay in registers between the amax and the convert pass; inter <= THREADS * 8 * NV.
+// 2048 x 14336: 45.6 us as two kernels, 38.0 as one; 32768 x 2048 (256 threads: every one has its vector) 105 and 79.
+template <int THREADS, int NV, bool ROUND_ACT>
+__global__ __launch_bounds__(THREADS) void fused_silu_row_quant_kernel(uint8_t* __restrict__ out, float* __restrict__ scales,
+                                                                               const uint16_t* __restrict__ in,
+                                                                               const uint32_t* __restrict__ row_offsets, int num_offsets,
+                                                                               int64_t max_rows, int inter, int64_t in_stride,
+                                                                               int64_t out_stride, float scale_ub) {
+  __shared__ float red[THREADS / 64];
+  const uint32_t rows_dev = row_offsets[num_offsets - 1];
+  const int64_t rows = (int64_t)rows_dev < max_rows ? (int64_t)rows_dev : max_rows;
+  const int64_t m = blockIdx.x;
+  if (m >= rows) return;
+  const int tid = threadIdx.x, nvec = inter >> 3;
+  const uint4* gate_row = reinterpret_cast<const uint4*>(in + m * in_stride);
+  const uint4* up_row = reinterpret_cast<const uint4*>(in + m * in_stride + inter);
+  uint4 h[NV];
+  float amax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int idx = tid + i * THREADS;
+    h[i] = make_uint4(0, 0, 0, 0);
+    if (idx < nvec) {
+      float gate[8], up[8], f[8];
+      unpack_bf16x8(gate_row[idx], gate);
+      unpack_bf16x8(up_row[idx], up);
+      silu_mul8<ROUND_ACT>(gate, up, f);
+      h[i] = pack_bf16x8(f);
+      unpack_bf16x8(h[i], f);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(f[j]));
+    }
+  }
+  amax = wave_max(amax);
+  if ((tid & 63) == 0) red[tid >> 6] = amax;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < THREADS / 64; ++w) amax = fmaxf(amax, red[w]);
+  float scale, recip;
+  dynamic_scale_f32(amax, scale_ub, scale, recip);
+  if (tid == 0) scales[m] = scale;
+  uint2* dst = reinterpret_cast<uint2*>(out + m * out_stride);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int idx = tid + i * THREADS;
+    if (idx < nvec) {
+      float f[8];
+      unpack_bf16x8(h[i], f);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = clamp448(f[j] * recip);
+      dst[idx] = pack_e4m3fn8(f);
+    }
+  }
+}
+
+template <bool ROUND_ACT>
+static bool launch_silu_row(void* out, float* scales, const void* in, const uint32_t* row_offsets, int64_t num_offsets, int64_t max_rows,
+                            int64_t inter, int64_t in_stride, int64_t out_stride, float scale_ub, hipStream_t stream) {
+  auto launch = [&](auto kern, int threads) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)max_rows), dim3(threads), 0, stream, (uint8_t*)out, scales, (const uint16_t*)in,
+                       row_offsets, (int)num_offsets, max_rows, (int)inter, in_stride, out_stride, scale_ub);
+    return true;
+  };
+  if (inter <= 2048) return launch(fused_silu_row_quant_kernel<256, 1, ROUND_ACT>, 256);
+  if (inter <= 4096) return launch(fused_silu_row_quant_kernel<512, 1, ROUND_ACT>, 512);
+  if (inter <= 8192) return launch(fused_silu_row_quant_kernel<512, 2, ROUND_ACT>, 512);
+  if (inter <= 16384) return launch(fused_silu_row_quant_kernel<1024, 2, ROUND_ACT>, 1024);
+  if (inter <= 32768) return launch(fused_silu_row_quant_kernel<1024, 4, ROUND_ACT>, 1024);
+  return false;
+}
+
+// mode: the ABI's `quantize`
 int fused_silu_dispatch(void* out, float* scales, const void* in, const uint32_t* row_offsets, int64_t num_offsets,
                         int64_t max_rows, int64_t inter, int64_t in_stride, int64_t out_stride, int64_t scales_ld,
-                        int mode, hipStream_t stream) {
-  const bool quant = mode == 1;
+                        int mode, bool row_scales, float scale_ub, hipStream_t stream) {
+  if (row_scales) {
+    const bool ok = mode == 4
+                        ? launch_silu_row<true>(out, scales, in, row_offsets, num_offsets, max_rows, inter, in_stride, out_stride, scale_ub, stream)
+                        : launch_silu_row<false>(out, scales, in, row_offsets, num_offsets, max_rows, inter, in_stride, out_stride, scale_ub, stream);
+    if (!ok) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused_silu: one scale per row takes rows of at most 32768 outputs");
+    return launch_status("fused_silu_quantized (row)");
+  }
   // the number of rows in use is only known on the device: the grid is sized for max_rows and
   // walks the items in strides
   const int64_t items = max_rows * (inter / 128);
   const unsigned blocks = (unsigned)(ceil_div(items, 16) < 8192 ? ceil_div(items, 16) : 8192);
-  if (quant)
-    hipLaunchKernelGGL(fused_silu_bf16_kernel<true>, dim3(blocks), dim3(256), 0, stream, out, scales, (const uint16_t*)in,
-                       row_offsets, (int)num_offsets, max_rows, (int)inter, in_stride, out_stride, scales_ld);
-  else if (mode == 2)
-    hipLaunchKernelGGL((fused_silu_bf16_kernel<false, true>), dim3(blocks), dim3(256), 0, stream, out, scales, (const uint16_t*)in,
-                       row_offsets, (int)num_offsets, max_rows, (int)inter, in_stride, out_stride, scales_ld);
-  else
-    hipLaunchKernelGGL(fused_silu_bf16_kernel<false>, dim3(blocks), dim3(256), 0, stream, out, scales, (const uint16_t*)in,
-                       row_offsets, (int)num_offsets, max_rows, (int)inter, in_stride, out_stride, scales_ld);
-  return launch_status(quant ? "fused_silu_quantized" : "fused_silu");
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, stream, out, scales, (const uint16_t*)in, row_offsets, (int)num_offsets, max_rows,
+                       (int)inter, in_stride, out_stride, scales_ld, scale_ub);
+  };
+  switch (mode) {
+    case 1: launch(fused_silu_bf16_kernel<kSiluQuant, false>); break;
+    case 2: launch(fused_silu_bf16_kernel<kSiluBf16, true>); break;
+    case 3: launch(fused_silu_bf16_kernel<kSiluBf16Quant, false>); break;
+    case 4: launch(fused_silu_bf16_kernel<kSiluBf16Quant, true>); break;
+    default: launch(fused_silu_bf16_kernel<kSiluBf16, false>); break;
+  }
+  return launch_status(mode == 0 || mode == 2 ? "fused_silu" : "fused_silu_quantized");
 }
 
 }  // namespace maxfp8

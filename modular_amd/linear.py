@@ -83,11 +83,11 @@ class MLP(torch.nn.Module):
     views of its halves), so nothing is concatenated per call.  With SiLU and no bias the activation
     and the product with `up` are one kernel (`fused_silu` with the activation rounded to bf16 before
     the product, as the reference's two bf16 operations `ops.silu(gate) * up` round it, linear.py:1072)
-    whose bf16 result `down_proj` quantises like any other input: five launches for the whole block.
+    whose bf16 result `down_proj` quantises like any other input -- with dynamic block or per-token scales inside the
+    same kernel (`silu_quantize`: the bytes of the two kernels), four launches for the whole block, otherwise five.
 
-    `fuse_activation_quant=True` (dynamic block scaling only) also folds the quantisation for
-    `down_proj` into that kernel (`fused_silu_quantized`: four launches, no bf16 intermediate).
-    That kernel is the expert-parallel MoE quantiser (ep_comm.mojo:4505-4624), whose recipe is not
+    `fuse_activation_quant=True` (dynamic block scaling only) quantises the f32 product instead of its bf16
+    rounding (`fused_silu_quantized`).  That kernel is the expert-parallel MoE quantiser (ep_comm.mojo:4505-4624), whose recipe is not
     the one `down_proj` applies -- scale = max(amax, 1e-4) / 448 without the upper bound of 1200,
     a division instead of a multiplication by the reciprocal, the f32 product instead of its bf16
     rounding -- so the fp8 codes it hands to the second matmul can differ by a step from the
@@ -173,7 +173,7 @@ class MLP(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         from .kernels import dynamic_scaled_matmul, quantize_dynamic_scaled_float8
-        from .moe_kernels import fused_silu, fused_silu_quantized
+        from .moe_kernels import fused_silu, fused_silu_quantized, silu_quantize, silu_quantize_group
 
         cfg = self.quant_config
         lead = x.shape[:-1]
@@ -189,7 +189,14 @@ class MLP(torch.nn.Module):
             return y.reshape(*lead, self.hidden_dim)
         if self._silu_kernel():
             both = quantized_matmul(x2, self.gate_up_weight, self.gate_up_weight_scale, None, cfg)
-            hidden = fused_silu(both, self._all_rows(x2.shape[0], x2.device), round_activation=True)
+            rows_used = self._all_rows(x2.shape[0], x2.device)
+            group = silu_quantize_group(cfg, x2.shape[0], self.feed_forward_length)
+            if group is not None and self.down_proj.weight_scale.dtype == torch.float32:
+                hq, hs = silu_quantize(both, rows_used, group, round_activation=True)
+                y = dynamic_scaled_matmul(hq, self.down_proj.weight, hs, self.down_proj.weight_scale, cfg.input_scale,
+                                          cfg.weight_scale, out_type=torch.bfloat16)
+                return y.reshape(*lead, self.hidden_dim)
+            hidden = fused_silu(both, rows_used, round_activation=True)
             return self.down_proj(hidden).reshape(*lead, self.hidden_dim)
         act = self._ACTIVATIONS[self.activation_function]
         if self._one_matmul and self.gate_proj.bias is None:

@@ -7,9 +7,10 @@
     its top_k rows; other dtypes: row_index=..., the
     gather rides on the quantiser's loads)
     gate_up = grouped matmul                             grouped_dynamic_scaled_fp8_matmul
-    silu(gate) * up on the rows in use                   fused_silu
-    quantise 1 x 128, down = grouped matmul that stores  grouped_dynamic_scaled_fp8_matmul(out_row_index=...)
-    its rows back in (token, k) order
+    silu(gate) * up on the rows in use, rounded to bf16  silu_quantize
+    and quantised 1 x 128
+    down = grouped matmul that stores its rows back in   grouped_dynamic_scaled_fp8_matmul(out_row_index=...)
+    (token, k) order
 
 Every step is one of this package's HIP kernels; the two row permutations cost no pass of their own."""
 from __future__ import annotations
@@ -17,7 +18,7 @@ from __future__ import annotations
 import torch
 
 from .kernels import grouped_dynamic_scaled_fp8_matmul, quantize_dynamic_scaled_float8
-from .moe_kernels import fused_silu, fused_silu_quantized, moe_create_indices
+from .moe_kernels import fused_silu, fused_silu_quantized, moe_create_indices, silu_quantize, silu_quantize_group
 from .quant_config import QuantConfig
 
 
@@ -101,11 +102,10 @@ def expert_matmuls_fp8(
     bounds (every row on one expert, every expert active) stand in and nothing waits for the GPU:
     same result, and the whole function can be captured in a HIP graph.
 
-    `fuse_activation_quant=True` runs silu(gate) * up and the quantisation for the down projection as one kernel
-    (`fused_silu_quantized`, the form the reference's expert-parallel path uses, ep_kernels.py:1168-1290) instead of
-    `fused_silu` followed by the quantiser: one pass over gate_up instead of three passes over it and its
-    activation; the product is quantised from f32 instead of from its bf16 rounding, so the fp8 codes can differ
-    by one step from the two-kernel form."""
+    By default silu(gate) * up is rounded to bf16 and quantised for the down projection like any bf16 tensor
+    (`silu_quantize`: the values of `fused_silu` followed by the quantiser, in one kernel).
+    `fuse_activation_quant=True` quantises the f32 product (`fused_silu_quantized`, the form the reference's
+    expert-parallel path uses, ep_kernels.py:1168-1290), so the fp8 codes can differ by one step from the default."""
     if x.dim() != 2 or router_idx.dim() != 2 or router_idx.shape[0] != x.shape[0]:
         raise ValueError("expected x [seq, hidden] and router_idx [seq, k]")
     if not (quant_config.input_scale.is_block and quant_config.weight_scale.is_block):
@@ -133,6 +133,8 @@ def expert_matmuls_fp8(
     gate_up = strategy.grouped_matmul(gate_up_proj, gate_up_scales, expert_inputs=expert_inputs)
     if fuse_activation_quant:
         gate_up_quant, gate_up_act_scales = strategy.fused_silu_quantize(gate_up, expert_inputs=expert_inputs)
+    elif group == silu_quantize_group(quant_config, gate_up.shape[0], gate_up.shape[1] // 2):
+        gate_up_quant, gate_up_act_scales = silu_quantize(gate_up, expert_start, group)
     else:
         gate_up_quant, gate_up_act_scales = strategy.quantize(fused_silu(gate_up, expert_start), group)
     down_inputs = (gate_up_quant, gate_up_act_scales) + expert_inputs[2:]

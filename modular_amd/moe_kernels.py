@@ -83,3 +83,36 @@ def fused_silu_quantized(input: torch.Tensor, row_offsets: torch.Tensor, quant_c
                                       _stream(input))
     _lib.check(st)
     return out, scales
+
+
+def silu_quantize(input: torch.Tensor, row_offsets: torch.Tensor, group_size: int, *, round_activation: bool = False,
+                  scale_ub: float = 1200.0) -> tuple[torch.Tensor, torch.Tensor]:
+    """`quantize_dynamic_scaled_float8(fused_silu(input, row_offsets, round_activation=...))` with float32 scales in one kernel:
+    the same bytes and scales without the bf16 tensor between the two.  group_size 128: scales transposed, [I / 128, M_pad]
+    (M_pad rounds the rows up to 16 bytes of scales); group_size I: one scale per row, [1, rows]."""
+    _check_silu_input(input, row_offsets)
+    input = input.contiguous()
+    rows, two_i = input.shape
+    inter = two_i // 2
+    ld = -(-rows // 4) * 4 if group_size == 128 else rows
+    out = torch.empty((rows, inter), dtype=_FP8, device=input.device)
+    scales = torch.empty((inter // 128 if group_size == 128 else 1, ld), dtype=torch.float32, device=input.device)
+    st = _lib.lib().maxfp8_silu_quantize_dynamic_scaled_fp8(
+        out.data_ptr(), scales.data_ptr(), input.data_ptr(), row_offsets.data_ptr(), row_offsets.shape[0], rows, inter, two_i, inter,
+        group_size, ld, _DT[input.dtype], int(round_activation), float(scale_ub), _stream(input))
+    _lib.check(st)
+    return out, scales
+
+
+def silu_quantize_group(quant_config: QuantConfig, rows: int, inter: int) -> int | None:
+    """The group size `silu_quantize` uses for the quantisation the config asks for, or None where it takes two kernels
+    (static or per-tensor scales, other blocks, scales of another dtype, rows that are too long).
+
+    Per-token scales keep a row on one CU, which computes its exponentials alone: a few long rows are quicker as two
+    kernels (16 x 28672: 7.8 against 11.3 us; 16 x 14336: level; 128 x 28672: 14.0 against 12.2)."""
+    i, w = quant_config.input_scale, quant_config.weight_scale
+    if not i.origin.is_dynamic or w.dtype != torch.float32 or inter % 128 != 0:
+        return None
+    if i.is_block and w.is_block and tuple(i.block_size) == (1, 128):
+        return 128
+    return inter if i.is_colwise and w.is_rowwise and 128 < inter <= (32768 if rows >= 128 else 14336) else None
