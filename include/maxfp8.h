@@ -268,8 +268,10 @@ int maxfp8_batched_matmul_dynamic_scaled_fp8(
 int maxfp8_matmul_describe(int64_t M, int64_t N, int64_t K, int block_scaling, int with_workspace,
                            char* buf, size_t len);
 
-/* Bytes of workspace that lets AUTO use every kernel for this shape. */
+/* Bytes of workspace that lets the tiled kernels use every plan for this shape. */
 size_t maxfp8_matmul_workspace_bytes(int64_t M, int64_t N, int64_t K);
+/* The same for MAXFP8_ALGO_AUTO: 0 where it picks a kernel that needs none. */
+size_t maxfp8_matmul_auto_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /*
  * Diagnostic with no counterpart in the reference.  Two kernels hand f32 sums from block to block inside one launch

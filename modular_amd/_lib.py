@@ -35,6 +35,7 @@ EXPORTS = (
     "maxfp8_matmul_noalloc_max_scratch_bytes",
     "maxfp8_batched_matmul_dynamic_scaled_fp8",
     "maxfp8_matmul_workspace_bytes",
+    "maxfp8_matmul_auto_workspace_bytes",
     "maxfp8_matmul_describe",
     "maxfp8_grouped_matmul_dynamic_scaled_fp8",
     "maxfp8_grouped_matmul_rowwise_dynamic_scaled_fp8",
@@ -102,6 +103,8 @@ def lib() -> ctypes.CDLL:
     L.maxfp8_matmul_describe.argtypes = [i64, i64, i64, ci, ci, ctypes.c_char_p, ctypes.c_size_t]
     L.maxfp8_matmul_workspace_bytes.restype = ctypes.c_size_t
     L.maxfp8_matmul_workspace_bytes.argtypes = [i64, i64, i64]
+    L.maxfp8_matmul_auto_workspace_bytes.restype = ctypes.c_size_t
+    L.maxfp8_matmul_auto_workspace_bytes.argtypes = [i64, i64, i64]
     L.maxfp8_grouped_matmul_dynamic_scaled_fp8.restype = ci
     L.maxfp8_grouped_matmul_dynamic_scaled_fp8.argtypes = [vp] * 7 + [i64] * 7 + [ci, ci, ci, vp]
     L.maxfp8_grouped_matmul_rowwise_dynamic_scaled_fp8.restype = ci

@@ -59,6 +59,12 @@ int gemm_skinny_dispatch(const GemmArgs&, bool, int64_t, hipStream_t);
 int gemm_skinny_max_m();
 bool gemm_short_k_ok(const GemmArgs&, bool, int64_t);
 int gemm_short_k_dispatch(const GemmArgs&, int64_t, hipStream_t);
+int gemm_mid_dispatch(const GemmArgs&, bool, hipStream_t);
+bool gemm_mid_ok(int64_t M, int64_t N, int64_t K);
+int gemm_mid_shape(int64_t M, int64_t N, int64_t K, float* us);
+float gemm_skinny_cost(int64_t M, int64_t N, int64_t K);
+float gemm_tiled_small_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
+float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
 bool gemm_skinny_preferred(int64_t M, int64_t N, int64_t K);
 int gemm_skinny_read_probe(const void* b, int64_t M, int64_t N, int64_t K, int64_t ldb, hipStream_t stream);
 int gemm_persist_probe(const GemmArgs&, bool, int, hipStream_t);
@@ -153,6 +159,7 @@ static const Tuning* read_tuning(unsigned generation) {
   t->grouped_w4_hot_rest = num("MAXFP8_GROUPED_W4_HOT_REST", 32);
   t->grouped_w4_cold_rows = num("MAXFP8_GROUPED_W4_COLD_ROWS", 128);
   t->skinny = num("MAXFP8_SKINNY", 0);
+  t->mid = num("MAXFP8_MID", -1);
   t->short_k = num("MAXFP8_SHORT_K", 1) != 0;
   t->generation = generation;
   return t;
@@ -188,6 +195,83 @@ const char* maxfp8_version(void) { return "maxfp8 0.2 (gfx950)"; }
 void maxfp8_tuning_reload(void) { tuning_reload(); }
 
 }  // extern "C"
+
+namespace maxfp8 {
+// The kernel for tens to a few hundred tokens (gemm_mid.hip), beside the ABI's algo values.
+constexpr int kAlgoMid = 100;
+
+// Which kernel MAXFP8_ALGO_AUTO gives a fast-layout matmul whose caller brings all the workspace it is asked for.  At most
+// 16 rows: the decode kernel.  Up to 64 rows: the decode kernel's own rule between itself and the tiles, the tiles also where
+// they are estimated 8 per cent quicker (the estimates' own error); up to 320 the tiles.  Against either the kernel in between,
+// by the same 8 per cent (up to 32 rows, where wide matrices miss their estimate by more, 15; against unsplit tiles, whose
+// estimate is the roughest, 25: 36 x 17632 x 3328 19 against 24 us, 140 x 1728 x 768 7.6 against 5.5).  Where the tiles' plan is none of the small ones (no estimate) they keep what they get.  Forced
+// shapes keep the other kernels out.
+static int choose_uncached(int64_t M, int64_t N, int64_t K) {
+  const Tuning& t = tuning();
+  const int plain = gemm_skinny_preferred(M, N, K) ? MAXFP8_ALGO_SKINNY : MAXFP8_ALGO_TILED;
+  if (t.mid > 0) return gemm_mid_ok(M, N, K) ? kAlgoMid : plain;
+  if (M <= 16 || M > 320 || t.mid == 0 || t.tile || t.splitk || t.one_region || t.w4 >= 0 || t.w4_split == 1 || t.skinny) return plain;
+  const float tiles = gemm_tiled_small_cost(M, N, K, true);
+  int algo = plain;
+  float us = tiles;
+  if (M <= 64) {
+    const float decode = gemm_skinny_cost(M, N, K);
+    if (plain == MAXFP8_ALGO_SKINNY) {
+      us = decode;
+      // (unsplit tiles in the decode kernel's range only for the shortest K, where four waves have no K to split: 48 x 32768 x 512
+      // 17.2 against 7.8 us; 49 x 20272 x 640 with row scales 10.9 against 13.0)
+      const bool splits = gemm_tiled_plan_workspace_bytes(M, N, K, true) > 0;
+      if (tiles > 0.f && tiles < 0.92f * decode && (splits || K <= 512)) {
+        us = tiles;
+        algo = MAXFP8_ALGO_TILED;
+      }
+    }
+  }
+  if (us == 0.f || !gemm_mid_ok(M, N, K)) return algo;
+  float mid;
+  gemm_mid_shape(M, N, K, &mid);
+  const float margin = algo == MAXFP8_ALGO_TILED && gemm_tiled_plan_workspace_bytes(M, N, K, true) == 0 ? 0.75f : M <= 32 ? 0.85f : 0.92f;
+  return mid < margin * us ? kAlgoMid : algo;
+}
+// (asked on every call: the answers are kept, keyed by the shape and the generation of the tuning switches)
+static int choose_kernel(int64_t M, int64_t N, int64_t K) {
+  if (M <= 16) return tuning().mid > 0 ? choose_uncached(M, N, K) : MAXFP8_ALGO_SKINNY;
+  if (M > 320) return MAXFP8_ALGO_TILED;
+  struct Entry { int64_t M, N, K; unsigned generation; int algo; };
+  static Entry table[128];  // (algo 0: empty)
+  static std::mutex mu;
+  const unsigned generation = tuning().generation;
+  const uint64_t h = ((uint64_t)M * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)N * 0xc2b2ae3d27d4eb4full) ^ ((uint64_t)K * 0x165667b19e3779f9ull);
+  Entry& e = table[(h >> 32) % 128];
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (e.algo && e.M == M && e.N == N && e.K == K && e.generation == generation) return e.algo;
+  }
+  const int algo = choose_uncached(M, N, K);
+  std::lock_guard<std::mutex> lock(mu);
+  e = Entry{M, N, K, generation, algo};
+  return algo;
+}
+
+// The same for the fused QKV matmul, whose tiles never split K: decode kernel (at most 64 rows), the kernel in between (at
+// most 320) or the tiles.
+static int choose_qkv(int64_t T, int64_t N, int64_t K) {
+  const Tuning& t = tuning();
+  const int plain = T <= gemm_skinny_max_m() ? MAXFP8_ALGO_SKINNY : MAXFP8_ALGO_TILED;
+  if (t.mid > 0) return gemm_mid_ok(T, N, K) ? kAlgoMid : plain;
+  if (T <= 16 || !gemm_mid_ok(T, N, K) || t.mid == 0 || t.tile || t.skinny) return plain;
+  float mid;
+  gemm_mid_shape(T, N, K, &mid);
+  const float tiles = gemm_tiled_qkv_cost(T, N, K, true);
+  float us = tiles;
+  int algo = MAXFP8_ALGO_TILED;
+  if (T <= gemm_skinny_max_m()) {
+    const float decode = gemm_skinny_cost(T, N, K);
+    if (decode < us) { us = decode; algo = MAXFP8_ALGO_SKINNY; }
+  }
+  return mid < 0.92f * us ? kAlgoMid : algo;
+}
+}  // namespace maxfp8
 
 static int quantize_common(void* out_fp8, void* out_scales, const void* in, const uint32_t* row_index, uint32_t index_div,
                            int64_t M, int64_t K, int64_t in_row_stride, int64_t out_row_stride, int64_t group_size,
@@ -380,14 +464,27 @@ int maxfp8_silu_quantize_dynamic_scaled_fp8(void* out_fp8, void* out_scales, con
 }
 
 size_t maxfp8_matmul_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0 || K <= 0 || gemm_skinny_preferred(M, N, K)) return 0;
+  if (M <= 0 || N <= 0 || K <= 0 || (gemm_skinny_preferred(M, N, K) && choose_kernel(M, N, K) != MAXFP8_ALGO_TILED)) return 0;
   return gemm_tiled_workspace_bytes(M, N, K);  // split-K partial sums; 0 when no split would be used
+}
+
+size_t maxfp8_matmul_auto_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0 || choose_kernel(M, N, K) != MAXFP8_ALGO_TILED) return 0;
+  return gemm_tiled_workspace_bytes(M, N, K);
 }
 
 }  // extern "C"
 
 namespace maxfp8 {
 struct BatchStrides { int64_t n, a, b, c, a_scales, b_scales; };  // n batches; steps in elements
+
+// 17 to 64 rows whose tiles would split K, without the workspace for it
+static int without_workspace(int64_t M, int64_t N, int64_t K) {
+  float mid;
+  if (M <= 16 || tuning().mid == 0 || tuning().skinny || !gemm_mid_ok(M, N, K)) return MAXFP8_ALGO_SKINNY;
+  gemm_mid_shape(M, N, K, &mid);
+  return mid < 0.92f * gemm_skinny_cost(M, N, K) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
+}
 
 static int matmul_common(void* c, const void* a, const void* b, const void* a_scales, const void* b_scales, int64_t M,
                          int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int input_granularity,
@@ -427,6 +524,7 @@ static int matmul_common(void* c, const void* a, const void* b, const void* a_sc
   const bool automatic = algo == MAXFP8_ALGO_AUTO;
   if (automatic) {
     if (!fast_layout) algo = MAXFP8_ALGO_NAIVE;
+    else if (bt.n == 1) algo = choose_kernel(M, N, K);
     // (a batch of short K and more than 32 rows: the tiles -- 128 heads x 48 x 512 x 128: 6.6 us against the decode kernel's 31,
     // 48 x 128 x 512: 6.6 against 14.5; 16 heads: 4.1 against 5.2 and 6.1 against 5.5)
     else if (gemm_skinny_preferred(M, N, K) && !(bt.n > 1 && M > 32 && K <= 512)) algo = MAXFP8_ALGO_SKINNY;
@@ -436,7 +534,7 @@ static int matmul_common(void* c, const void* a, const void* b, const void* a_sc
     // worst case over all tile shapes: a plan that does not split runs the same with and without a workspace.)
     if (algo == MAXFP8_ALGO_TILED && M <= gemm_skinny_max_m() && bt.n == 1 &&
         gemm_tiled_plan_workspace_bytes(M, N, K, block) > (workspace ? workspace_bytes : 0))
-      algo = MAXFP8_ALGO_SKINNY;
+      algo = without_workspace(M, N, K);
   }
   if (algo == MAXFP8_ALGO_NAIVE) {
     if (block)
@@ -446,7 +544,8 @@ static int matmul_common(void* c, const void* a, const void* b, const void* a_sc
     return naive_rowwise_dispatch(c, a, b, a_scales, b_scales, M, N, K, lda, ldb, ldc, tensor ? 0 : 1,
                                   tensor ? 0 : b_scales_ld, c_dtype, scales_dtype, st);
   }
-  if (algo != MAXFP8_ALGO_TILED && algo != MAXFP8_ALGO_SKINNY) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "matmul: unknown algo %d", algo);
+  if (algo != MAXFP8_ALGO_TILED && algo != MAXFP8_ALGO_SKINNY && !(automatic && algo == kAlgoMid))
+    MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "matmul: unknown algo %d", algo);
   if (!fast_layout)
     MAXFP8_FAIL(MAXFP8_ERR_ALIGN,
                 "matmul: the MFMA kernels need 16-byte aligned rows, K %% 16 == 0, (1,128,128) blocks and "
@@ -475,6 +574,7 @@ static int matmul_common(void* c, const void* a, const void* b, const void* a_sc
   }
   p.a_batch = bt.a; p.b_batch = bt.b; p.c_batch = bt.c;
   p.a_scales_batch = bt.a_scales; p.b_scales_batch = bt.b_scales;
+  if (algo == kAlgoMid) return gemm_mid_dispatch(p, block, st);
   if (automatic && gemm_short_k_ok(p, block, bt.n)) return gemm_short_k_dispatch(p, bt.n, st);
   if (algo == MAXFP8_ALGO_SKINNY) return gemm_skinny_dispatch(p, block, bt.n, st);
   if (workspace && !is_aligned(workspace, 16)) MAXFP8_FAIL(MAXFP8_ERR_ALIGN, "matmul: workspace must be 16-byte aligned");
@@ -488,9 +588,17 @@ extern "C" {
 int maxfp8_matmul_describe(int64_t M, int64_t N, int64_t K, int block_scaling, int with_workspace, char* buf, size_t len) {
   if (!buf || len == 0) return 0;
   if (M <= 0 || N <= 0 || K <= 0) return snprintf(buf, len, "nothing to do");
-  if (gemm_skinny_preferred(M, N, K)) return snprintf(buf, len, "skinny");
-  if (M <= gemm_skinny_max_m() && !with_workspace && gemm_tiled_plan_workspace_bytes(M, N, K, block_scaling != 0) > 0)
-    return snprintf(buf, len, "skinny");
+  // ("skinny" names the launches whose blocks split K among their waves: up to 64 rows both kernels that do, beyond that
+  // the one there is with its tiles)
+  int algo = choose_kernel(M, N, K);
+  if (algo == MAXFP8_ALGO_TILED && M <= gemm_skinny_max_m() && !with_workspace && gemm_tiled_plan_workspace_bytes(M, N, K, block_scaling != 0) > 0)
+    algo = without_workspace(M, N, K);
+  if (algo == MAXFP8_ALGO_SKINNY || (algo == kAlgoMid && M <= gemm_skinny_max_m())) return snprintf(buf, len, "skinny");
+  if (algo == kAlgoMid) {
+    float us;
+    const int sel = tuning().mid > 0 ? tuning().mid : gemm_mid_shape(M, N, K, &us), bm = 16 * (sel / 10), bn = 16 * (sel % 10);
+    return snprintf(buf, len, "%dx%d x%lld, K split over the block's waves", bm, bn, (long long)(ceil_div(M, bm) * ceil_div(N, bn)));
+  }
   return gemm_tiled_describe(M, N, K, block_scaling != 0, with_workspace != 0, buf, len);
 }
 
@@ -517,7 +625,8 @@ int maxfp8_matmul_dynamic_scaled_fp8_noalloc(void* c, const void* a, const void*
   // entry points add the same partial sums in the same order.
   const bool block = input_granularity == MAXFP8_GRAN_BLOCK && weight_granularity == MAXFP8_GRAN_BLOCK;
   size_t need = 0;
-  if (M > 0 && N > 0 && K > 0 && maxfp8_matmul_workspace_bytes(M, N, K) > 0) need = gemm_tiled_plan_workspace_bytes(M, N, K, block);
+  const size_t useful = algo == MAXFP8_ALGO_AUTO ? maxfp8_matmul_auto_workspace_bytes(M, N, K) : maxfp8_matmul_workspace_bytes(M, N, K);
+  if (M > 0 && N > 0 && K > 0 && useful > 0) need = gemm_tiled_plan_workspace_bytes(M, N, K, block);
   if (need > kScratchBytes)
     MAXFP8_FAIL(MAXFP8_ERR_WORKSPACE,
                 "matmul (no-alloc): the split of %lld x %lld x %lld uses %zu bytes of scratch, the library's static buffer holds "
@@ -626,7 +735,9 @@ int maxfp8_fused_qkv_matmul_ragged_paged_scale(void* output, const void* input, 
   p.kv.batch = (int)batch_size;
   p.kv.bf16_scaling = block ? 0 : 1;
   hipStream_t st = (hipStream_t)stream;
-  if (algo == MAXFP8_ALGO_AUTO) algo = T <= gemm_skinny_max_m() ? MAXFP8_ALGO_SKINNY : MAXFP8_ALGO_TILED;
+  const bool automatic = algo == MAXFP8_ALGO_AUTO;
+  if (automatic) algo = choose_qkv(T, N, K);
+  if (automatic && algo == kAlgoMid) return gemm_mid_dispatch(p, block, st);
   if (algo == MAXFP8_ALGO_SKINNY) return gemm_skinny_dispatch(p, block, 1, st);
   if (algo != MAXFP8_ALGO_TILED) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused qkv matmul: algo %d is not available", algo);
   return gemm_tiled_dispatch(p, block, 0, 1, st);

@@ -2142,6 +2142,31 @@ static TiledPlan cached_plan(int64_t M, int64_t N, int64_t K, bool blockscale, b
   return plan;
 }
 
+// Estimated microseconds of this shape's plan with all the workspace it asks for, where the plan is one of those that small
+// matmuls get: a K split, every tile cut, one round of three-stage 128 x 128 tiles (fitted like gemm_mid_shape's estimates:
+// within 7, 5 and 20 per cent for nine launches in ten); 0 for every other plan.
+float gemm_tiled_small_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
+  const TiledPlan plan = cached_plan(M, N, K, blockscale, true, ~(size_t)0, 1, false);
+  const float slabs = (float)ceil_div(K, 128), stream = (float)N * (float)K / 6e6f;
+  if (plan.w4) {
+    if (!plan.w4_split || ceil_div(M, 32 * plan.w4) * ceil_div(N, 256) * 2 > compute_units()) return 0.f;
+    const int unit = gemm_w4_split(M, N, K, plan.w4).unit;
+    return 10.5f + 0.646f * (float)unit + 0.886f * (float)ceil_div((int64_t)slabs, unit) + 0.659f * stream;
+  }
+  if (plan.two.axis || plan.streamk) return 0.f;
+  if (plan.splits > 1)
+    return 8.2f + 0.33f * (float)ceil_div((int64_t)slabs, plan.splits) * (kShapes[plan.variant - 1].bm == 128 ? 1.f : 1.25f) +
+           1.024f * (float)plan.splits * (float)M * (float)N * 8.0f / 4.0e6f + 0.63f * stream;
+  if (plan.variant == 4) return 4.9f + 0.559f * slabs * (float)ceil_div(ceil_div(M, 128) * ceil_div(N, 128), 256) + 0.36f * stream;
+  return 0.f;
+}
+
+// The same for a fused QKV matmul (whole tiles of the two shapes its epilogue exists in)
+float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
+  const TiledPlan plan = cached_plan(M, N, K, blockscale, false, 0, 1, true);
+  return region_cost(M, N, (int)ceil_div(K, 128), kShapes[plan.variant - 1], blockscale);
+}
+
 // "256x256 x896" / "256x256 x448, K split 2" / "256x256 x768 + columns from 24576: 256x128 x256"
 int gemm_tiled_describe(int64_t M, int64_t N, int64_t K, bool blockscale, bool has_workspace, char* buf, size_t len) {
   const TiledPlan plan = make_plan(M, N, K, blockscale, has_workspace, has_workspace ? gemm_tiled_workspace_bytes(M, N, K) : 0, 1, false);

@@ -383,7 +383,9 @@ def dynamic_scaled_matmul(
     a_ld = a_scales.stride(0) if a_scales.shape[0] > 1 else a_scales.shape[1]
     b_ld = b_scales.stride(0) if b_scales.shape[0] > 1 else b_scales.shape[1]
     # split-K scratch for problems whose tiles would cover only part of the chip (0 bytes otherwise)
-    ws_bytes = _lib.lib().maxfp8_matmul_workspace_bytes(M, N, K) if algo in ("auto", "tiled") else 0
+    lib = _lib.lib()
+    ws_bytes = (lib.maxfp8_matmul_auto_workspace_bytes(M, N, K) if algo == "auto" else
+                lib.maxfp8_matmul_workspace_bytes(M, N, K) if algo == "tiled" else 0)
     ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=a.device) if ws_bytes else None
     st = _lib.lib().maxfp8_matmul_dynamic_scaled_fp8(
         c.data_ptr(), a.data_ptr(), b.data_ptr(), a_scales.data_ptr(), b_scales.data_ptr(), M, N, K,
