@@ -274,6 +274,36 @@ size_t maxfp8_matmul_workspace_bytes(int64_t M, int64_t N, int64_t K);
 size_t maxfp8_matmul_auto_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /*
+ * A whole FP8 linear: y[M, N] (bf16) = quantise(x[M, K] bf16) . w[N, K]^T, the two ops above with nothing in between for the
+ * caller to hold.  Not ops of the reference; what its `quantized_matmul` (max/python/max/nn/quant_ops.py:336-592) computes.
+ *   _dynamic_  weight_granularity BLOCK (1 x 128 activation groups, 128 x 128 weight blocks, w_scales[ceil(N/128), K/128]) or
+ *              ROWWISE (per token x per channel, w_scales[N, 1]); f32 scales, scale_ub as in the quantiser.
+ *   _static_   per-tensor scales known on the host: quantise(x, input_scale), result times input_scale * weight_scale.
+ * Either one launch -- a few tokens: the decode kernel quantises what it needs itself -- or the quantiser and
+ * MAXFP8_ALGO_AUTO's matmul through the workspace, of maxfp8_linear_workspace_bytes bytes (0 for the one launch, which
+ * takes 16-byte aligned rows; weight_granularity TENSOR for the static form).  Same results as the ops one by one.
+ * The _qkv_ form is maxfp8_fused_qkv_matmul_ragged_paged_scale behind the same quantisation.
+ */
+size_t maxfp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int weight_granularity);
+int maxfp8_linear_dynamic_scaled_fp8(
+    void* y, const void* x, const void* w, const void* w_scales,
+    int64_t M, int64_t N, int64_t K, int64_t x_row_stride, int64_t ldw, int64_t ldy,
+    int weight_granularity, int64_t w_scales_ld, float scale_ub,
+    void* workspace, size_t workspace_bytes, void* stream);
+int maxfp8_linear_static_scaled_fp8(
+    void* y, const void* x, const void* w, int64_t M, int64_t N, int64_t K,
+    int64_t x_row_stride, int64_t ldw, int64_t ldy, float input_scale, float weight_scale,
+    void* workspace, size_t workspace_bytes, void* stream);
+size_t maxfp8_linear_qkv_workspace_bytes(int64_t T, int64_t N, int64_t K, int weight_granularity);
+int maxfp8_linear_qkv_ragged_paged_scale(
+    void* output, const void* x, int64_t x_row_stride, const uint32_t* input_row_offsets,
+    const void* wqkv, const void* weight_scale, void* kv_blocks, const uint32_t* cache_lengths,
+    const uint32_t* lookup_table, const void* bias, int64_t T, int64_t N, int64_t K, int64_t q_dim,
+    int64_t batch_size, int64_t num_blocks, int64_t kv_dim, int64_t num_layers, int64_t layer_idx,
+    int64_t page_size, int64_t num_kv_heads, int64_t head_dim, int64_t lut_ld, int weight_granularity,
+    int64_t weight_scale_ld, float scale_ub, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Diagnostic with no counterpart in the reference.  Two kernels hand f32 sums from block to block inside one launch
  * (the four-wave kernel that computes its last round of tiles in pieces; the eight-wave kernel's work split along K,
  * MAXFP8_STREAMK).  A block that waits for such a hand-over does so for a bounded time (seconds: a GPU that stopped in

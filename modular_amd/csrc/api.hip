@@ -35,6 +35,7 @@ int quantize_scatter_dispatch(void*, void*, const void*, int64_t, int64_t, int64
 int rmsnorm_quantize_dispatch(void*, void*, const void*, const void*, int64_t, int64_t, int64_t, int64_t, int, int, float,
                               float, float, hipStream_t);
 int quantize_static_dispatch(void*, const void*, int64_t, int64_t, int64_t, int64_t, int, float, hipStream_t);
+int quantize_static_for_matmul_dispatch(void*, float*, const void*, int64_t, int64_t, int64_t, int, float, float, hipStream_t);
 int quantize_tensor_dispatch(void*, void*, const void*, int64_t, int64_t, int64_t, int64_t, int, int, float, hipStream_t);
 int moe_create_indices_dispatch(uint32_t*, uint32_t*, uint32_t*, int32_t*, uint32_t*, const int32_t*, int64_t, int64_t, hipStream_t);
 int fused_silu_dispatch(void*, float*, const void*, const uint32_t*, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, bool,
@@ -56,6 +57,8 @@ size_t gemm_tiled_plan_workspace_bytes(int64_t, int64_t, int64_t, bool);
 int gemm_tiled_describe(int64_t, int64_t, int64_t, bool, bool, char*, size_t);
 int gemm_grouped_dispatch(const GemmArgs&, bool, int64_t, int64_t, hipStream_t);
 int gemm_skinny_dispatch(const GemmArgs&, bool, int64_t, hipStream_t);
+bool gemm_skinny_quant_ok(int64_t M, int64_t N, int64_t K, bool blockscale);
+int gemm_skinny_quant_dispatch(const GemmArgs&, bool, hipStream_t);
 int gemm_skinny_max_m();
 bool gemm_short_k_ok(const GemmArgs&, bool, int64_t);
 int gemm_short_k_dispatch(const GemmArgs&, int64_t, hipStream_t);
@@ -149,6 +152,7 @@ static const Tuning* read_tuning(unsigned generation) {
   t->w4 = (w4 == 0 || w4 == 4 || w4 == 5 || w4 == 6) ? w4 : -1;
   const int w4_split = num("MAXFP8_W4_SPLIT", -1);
   t->w4_split = (w4_split == 0 || w4_split == 1) ? w4_split : -1;
+  t->skinny_quant = num("MAXFP8_SKINNY_QUANT", 1) != 0;
   t->skinny_alds = num("MAXFP8_SKINNY_ALDS", 1) != 0;
   const char* sb = getenv("MAXFP8_GROUPED_SHARE");
   t->grouped_share = sb ? (float)atof(sb) : 0.5f;
@@ -644,6 +648,103 @@ int maxfp8_matmul_dynamic_scaled_fp8_noalloc(void* c, const void* a, const void*
                        gk, a_scales_ld, b_scales_ld, c_dtype, scales_dtype, algo, ws, ws ? need : 0, one, stream);
 }
 
+// ---- a whole linear: quantise bf16 activations, then the scaled matmul --------------------------------------------
+// What the two launches of a linear keep in the caller's workspace: fp8 activations, their scales, the matmul's partial sums.
+}  // extern "C"
+namespace maxfp8 {
+struct LinearLayout { size_t scales, partial, partial_bytes, total; int64_t scales_ld; };
+static LinearLayout linear_layout(int64_t M, int64_t N, int64_t K, bool block, bool fixed) {
+  auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
+  LinearLayout l;
+  l.scales_ld = block ? ceil_div(M, 4) * 4 : M;
+  l.scales = up((size_t)M * (size_t)K);
+  l.partial = l.scales + up((fixed ? 2 : block ? (size_t)(K / 128) * l.scales_ld : (size_t)M) * 4);
+  l.partial_bytes = maxfp8_matmul_auto_workspace_bytes(M, N, K);
+  l.total = l.partial + l.partial_bytes;
+  return l;
+}
+// does the decode kernel quantise by itself? (the layout as far as it is the operands': see linear_common)
+static bool linear_in_one(int64_t M, int64_t N, int64_t K, bool block) {
+  return M > 0 && N > 0 && K > 0 && choose_kernel(M, N, K) == MAXFP8_ALGO_SKINNY && gemm_skinny_quant_ok(M, N, K, block);
+}
+
+static int linear_common(void* y, const void* x, const void* w, const void* w_scales, int64_t M, int64_t N, int64_t K, int64_t ldx,
+                         int64_t ldw, int64_t ldy, bool block, int64_t w_scales_ld, bool fixed, float input_scale, float weight_scale,
+                         float scale_ub, void* workspace, size_t workspace_bytes, void* stream) {
+  if (M < 0 || N < 0 || K < 0) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "linear: negative size");
+  if (M == 0 || N == 0) return MAXFP8_OK;
+  if (M >= ((int64_t)1 << 31) || N >= ((int64_t)1 << 31) || K >= ((int64_t)1 << 31)) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "linear: sizes must fit 31 bits");
+  if (ldx < K || ldw < K || ldy < N) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "linear: row strides smaller than the rows");
+  if (K <= 0 || K % (block ? 128 : 4) != 0)
+    MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "linear: K = %lld is not a positive multiple of %d", (long long)K, block ? 128 : 4);
+  if (block && w_scales_ld < K / 128) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "linear: scale leading dimension too small");
+  if (!y || !x || !w || (!fixed && !w_scales)) MAXFP8_FAIL(MAXFP8_ERR_NULL, "linear: null pointer");
+  hipStream_t st = (hipStream_t)stream;
+  if (linear_in_one(M, N, K, block) && is_aligned(x, 16) && ldx % 8 == 0 && is_aligned(w, 16) && ldw % 16 == 0 && K % 16 == 0 &&
+      offsets_fit(K, ldw, ldw, 0, false) && 32 * ldx < ((int64_t)1 << 31)) {
+    GemmArgs p;
+    memset(&p, 0, sizeof(p));
+    p.b = (const uint8_t*)w;
+    p.c = y;
+    p.b_scales = (const float*)w_scales;
+    p.M = (int)M; p.N = (int)N; p.K = (int)K;
+    p.ldb = ldw; p.ldc = ldy;
+    p.b_scales_ld = w_scales_ld;
+    p.b_scale_stride = w_scales_ld;
+    p.c_dtype = MAXFP8_BF16;
+    p.scales_dtype = MAXFP8_F32;
+    p.c_vec_ok = (ldy % 4 == 0) && is_aligned(y, 8);
+    p.x = (const uint16_t*)x;
+    p.ldx = ldx;
+    p.x_static = fixed ? 1 : 0;
+    p.x_scale_ub = scale_ub;
+    p.x_recip = fixed ? 1.0f / input_scale : 0.f;
+    p.x_scale = input_scale * weight_scale;
+    return gemm_skinny_quant_dispatch(p, block, st);
+  }
+  const LinearLayout l = linear_layout(M, N, K, block, fixed);
+  if (!workspace || workspace_bytes < l.total)
+    MAXFP8_FAIL(MAXFP8_ERR_WORKSPACE, "linear: %lld x %lld x %lld needs %zu bytes of workspace (maxfp8_linear_workspace_bytes), got %zu", (long long)M,
+                (long long)N, (long long)K, l.total, workspace ? workspace_bytes : (size_t)0);
+  if (!is_aligned(workspace, 16)) MAXFP8_FAIL(MAXFP8_ERR_ALIGN, "linear: workspace must be 16-byte aligned");
+  uint8_t* q = (uint8_t*)workspace;
+  float* scales = (float*)(q + l.scales);
+  int rc;
+  if (fixed) rc = quantize_static_for_matmul_dispatch(q, scales, x, M, K, ldx, MAXFP8_BF16, input_scale, weight_scale, st);
+  else rc = quantize_dispatch(q, scales, x, M, K, ldx, K, block ? 128 : K, l.scales_ld, MAXFP8_BF16, MAXFP8_F32, scale_ub, 1, 0, 0, 0, nullptr, 1, st);
+  if (rc != MAXFP8_OK) return rc;
+  const int gran_in = fixed ? MAXFP8_GRAN_TENSOR : block ? MAXFP8_GRAN_BLOCK : MAXFP8_GRAN_COLWISE;
+  const int gran_w = fixed ? MAXFP8_GRAN_TENSOR : block ? MAXFP8_GRAN_BLOCK : MAXFP8_GRAN_ROWWISE;
+  const BatchStrides one = {1, 0, 0, 0, 0, 0};
+  return matmul_common(y, q, w, scales, fixed ? scales + 1 : w_scales, M, N, K, K, ldw, ldy, gran_in, gran_w, block ? 1 : -1, block ? 128 : -1,
+                       block ? 128 : -1, l.scales_ld, fixed ? 1 : w_scales_ld, MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO,
+                       l.partial_bytes ? q + l.partial : nullptr, l.partial_bytes, one, st);
+}
+}  // namespace maxfp8
+extern "C" {
+
+size_t maxfp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int weight_granularity) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const bool block = weight_granularity == MAXFP8_GRAN_BLOCK;
+  return linear_in_one(M, N, K, block) ? 0 : linear_layout(M, N, K, block, weight_granularity == MAXFP8_GRAN_TENSOR).total;
+}
+
+int maxfp8_linear_dynamic_scaled_fp8(void* y, const void* x, const void* w, const void* w_scales, int64_t M, int64_t N, int64_t K,
+                                     int64_t x_row_stride, int64_t ldw, int64_t ldy, int weight_granularity, int64_t w_scales_ld,
+                                     float scale_ub, void* workspace, size_t workspace_bytes, void* stream) {
+  if (weight_granularity != MAXFP8_GRAN_BLOCK && weight_granularity != MAXFP8_GRAN_ROWWISE)
+    MAXFP8_FAIL(MAXFP8_ERR_GRANULARITY, "linear: weight granularity %d is not block or rowwise", weight_granularity);
+  return linear_common(y, x, w, w_scales, M, N, K, x_row_stride, ldw, ldy, weight_granularity == MAXFP8_GRAN_BLOCK, w_scales_ld, false, 1.f, 1.f,
+                       scale_ub, workspace, workspace_bytes, stream);
+}
+
+int maxfp8_linear_static_scaled_fp8(void* y, const void* x, const void* w, int64_t M, int64_t N, int64_t K, int64_t x_row_stride,
+                                    int64_t ldw, int64_t ldy, float input_scale, float weight_scale, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
+  return linear_common(y, x, w, nullptr, M, N, K, x_row_stride, ldw, ldy, false, 1, true, input_scale, weight_scale, 0.f, workspace,
+                       workspace_bytes, stream);
+}
+
 int maxfp8_batched_matmul_dynamic_scaled_fp8(void* c, const void* a, const void* b, const void* a_scales,
                                              const void* b_scales, int64_t B, int64_t M, int64_t N, int64_t K,
                                              int64_t a_batch_stride, int64_t lda, int64_t b_batch_stride, int64_t ldb,
@@ -659,7 +760,10 @@ int maxfp8_batched_matmul_dynamic_scaled_fp8(void* c, const void* a, const void*
                        a_scales_ld, b_scales_ld, c_dtype, scales_dtype, algo, nullptr, 0, bt, stream);
 }
 
-int maxfp8_fused_qkv_matmul_ragged_paged_scale(void* output, const void* input, const uint32_t* input_row_offsets,
+}  // extern "C"
+
+// x != nullptr: the decode kernel quantises x (bf16 rows of ldx elements) by itself; input and input_scale are not used
+static int qkv_common(void* output, const void* input, const void* x, int64_t ldx, float scale_ub, const uint32_t* input_row_offsets,
                                                const void* wqkv, const void* input_scale, const void* weight_scale,
                                                void* kv_blocks, const uint32_t* cache_lengths, const uint32_t* lookup_table,
                                                const void* bias, int64_t T, int64_t N, int64_t K, int64_t q_dim,
@@ -680,7 +784,7 @@ int maxfp8_fused_qkv_matmul_ragged_paged_scale(void* output, const void* input, 
   if (rest != k_dim && !(rest == 2 * k_dim && kv_dim == 2))
     MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused qkv matmul: N = %lld is not q_dim %lld plus one or two times kv_heads * head_dim = %lld",
                 (long long)N, (long long)q_dim, (long long)k_dim);
-  if (!input || !wqkv || !input_scale || !weight_scale || !kv_blocks || !cache_lengths || !lookup_table || !input_row_offsets ||
+  if ((!x && (!input || !input_scale)) || !wqkv || !weight_scale || !kv_blocks || !cache_lengths || !lookup_table || !input_row_offsets ||
       (q_dim > 0 && !output))
     MAXFP8_FAIL(MAXFP8_ERR_NULL, "fused qkv matmul: null pointer");
   if (scales_dtype != MAXFP8_F32) MAXFP8_FAIL(MAXFP8_ERR_DTYPE, "fused qkv matmul: scales must be float32");
@@ -689,7 +793,7 @@ int maxfp8_fused_qkv_matmul_ragged_paged_scale(void* output, const void* input, 
   const bool block = !per_tensor && !per_channel;
   if (block && !(gm == 1 && gn == 128 && gk == 128))
     MAXFP8_FAIL(MAXFP8_ERR_GRANULARITY, "fused qkv matmul: block scaling needs the (1, 128, 128) granularity");
-  if (block && (input_scale_ld < T || weight_scale_ld < ceil_div(K, 128)))
+  if (block && ((!x && input_scale_ld < T) || weight_scale_ld < ceil_div(K, 128)))
     MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused qkv matmul: scale leading dimensions too small");
   // the MFMA kernels' layout, and 8-element chunks that stay inside one of Q / K / V and one cache row
   if (!is_aligned(input, 16) || !is_aligned(wqkv, 16) || K % 16 != 0 || K <= 0)
@@ -735,12 +839,76 @@ int maxfp8_fused_qkv_matmul_ragged_paged_scale(void* output, const void* input, 
   p.kv.batch = (int)batch_size;
   p.kv.bf16_scaling = block ? 0 : 1;
   hipStream_t st = (hipStream_t)stream;
+  if (x) {
+    p.a = nullptr;
+    p.x = (const uint16_t*)x;
+    p.ldx = ldx;
+    p.x_scale_ub = scale_ub;
+    return gemm_skinny_quant_dispatch(p, block, st);
+  }
   const bool automatic = algo == MAXFP8_ALGO_AUTO;
   if (automatic) algo = choose_qkv(T, N, K);
   if (automatic && algo == kAlgoMid) return gemm_mid_dispatch(p, block, st);
   if (algo == MAXFP8_ALGO_SKINNY) return gemm_skinny_dispatch(p, block, 1, st);
   if (algo != MAXFP8_ALGO_TILED) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused qkv matmul: algo %d is not available", algo);
   return gemm_tiled_dispatch(p, block, 0, 1, st);
+}
+
+extern "C" {
+
+int maxfp8_fused_qkv_matmul_ragged_paged_scale(void* output, const void* input, const uint32_t* input_row_offsets,
+                                               const void* wqkv, const void* input_scale, const void* weight_scale,
+                                               void* kv_blocks, const uint32_t* cache_lengths, const uint32_t* lookup_table,
+                                               const void* bias, int64_t T, int64_t N, int64_t K, int64_t q_dim,
+                                               int64_t batch_size, int64_t num_blocks, int64_t kv_dim, int64_t num_layers,
+                                               int64_t layer_idx, int64_t page_size, int64_t num_kv_heads, int64_t head_dim,
+                                               int64_t lut_ld, int64_t gm, int64_t gn, int64_t gk, int64_t input_scale_ld,
+                                               int64_t weight_scale_ld, int scales_dtype, int algo, void* stream) {
+  return qkv_common(output, input, nullptr, 0, 0.f, input_row_offsets, wqkv, input_scale, weight_scale, kv_blocks, cache_lengths, lookup_table,
+                    bias, T, N, K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads, head_dim, lut_ld, gm,
+                    gn, gk, input_scale_ld, weight_scale_ld, scales_dtype, algo, stream);
+}
+
+static bool qkv_in_one(int64_t T, int64_t N, int64_t K, bool block) {
+  return T > 0 && N > 0 && K > 0 && choose_qkv(T, N, K) == MAXFP8_ALGO_SKINNY && gemm_skinny_quant_ok(T, N, K, block);
+}
+
+size_t maxfp8_linear_qkv_workspace_bytes(int64_t T, int64_t N, int64_t K, int weight_granularity) {
+  if (T <= 0 || N <= 0 || K <= 0) return 0;
+  const bool block = weight_granularity == MAXFP8_GRAN_BLOCK;
+  return qkv_in_one(T, N, K, block) ? 0 : linear_layout(T, N, K, block, false).partial;
+}
+
+int maxfp8_linear_qkv_ragged_paged_scale(void* output, const void* x, int64_t x_row_stride, const uint32_t* input_row_offsets,
+                                         const void* wqkv, const void* weight_scale, void* kv_blocks, const uint32_t* cache_lengths,
+                                         const uint32_t* lookup_table, const void* bias, int64_t T, int64_t N, int64_t K, int64_t q_dim,
+                                         int64_t batch_size, int64_t num_blocks, int64_t kv_dim, int64_t num_layers, int64_t layer_idx,
+                                         int64_t page_size, int64_t num_kv_heads, int64_t head_dim, int64_t lut_ld, int weight_granularity,
+                                         int64_t weight_scale_ld, float scale_ub, void* workspace, size_t workspace_bytes, void* stream) {
+  if (weight_granularity != MAXFP8_GRAN_BLOCK && weight_granularity != MAXFP8_GRAN_ROWWISE)
+    MAXFP8_FAIL(MAXFP8_ERR_GRANULARITY, "qkv linear: weight granularity %d is not block or rowwise", weight_granularity);
+  const bool block = weight_granularity == MAXFP8_GRAN_BLOCK;
+  const int64_t gm = 1, gn = block ? 128 : 1, gk = block ? 128 : -1;
+  if (T < 0 || N < 0 || K < 0) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "qkv linear: negative size");
+  if (batch_size == 0 || T == 0 || N == 0) return MAXFP8_OK;
+  if (!x) MAXFP8_FAIL(MAXFP8_ERR_NULL, "qkv linear: null pointer");
+  if (x_row_stride < K || K <= 0 || K % (block ? 128 : 16) != 0) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "qkv linear: K = %lld does not suit the scaling", (long long)K);
+  if (qkv_in_one(T, N, K, block) && is_aligned(x, 16) && x_row_stride % 8 == 0 && 32 * x_row_stride < ((int64_t)1 << 31))
+    return qkv_common(output, nullptr, x, x_row_stride, scale_ub, input_row_offsets, wqkv, nullptr, weight_scale, kv_blocks, cache_lengths,
+                      lookup_table, bias, T, N, K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads,
+                      head_dim, lut_ld, gm, gn, gk, 0, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_SKINNY, stream);
+  const LinearLayout l = linear_layout(T, N, K, block, false);
+  if (!workspace || workspace_bytes < l.partial)
+    MAXFP8_FAIL(MAXFP8_ERR_WORKSPACE, "qkv linear: needs %zu bytes of workspace, got %zu", l.partial, workspace ? workspace_bytes : (size_t)0);
+  if (!is_aligned(workspace, 16)) MAXFP8_FAIL(MAXFP8_ERR_ALIGN, "qkv linear: workspace must be 16-byte aligned");
+  uint8_t* q = (uint8_t*)workspace;
+  float* scales = (float*)(q + l.scales);
+  const int rc = quantize_dispatch(q, scales, x, T, K, x_row_stride, K, block ? 128 : K, l.scales_ld, MAXFP8_BF16, MAXFP8_F32, scale_ub, 1, 0, 0, 0,
+                                   nullptr, 1, (hipStream_t)stream);
+  if (rc != MAXFP8_OK) return rc;
+  return qkv_common(output, q, nullptr, 0, 0.f, input_row_offsets, wqkv, scales, weight_scale, kv_blocks, cache_lengths, lookup_table, bias, T, N,
+                    K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads, head_dim, lut_ld, gm, gn, gk,
+                    block ? l.scales_ld : T, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_AUTO, stream);
 }
 
 }  // extern "C"

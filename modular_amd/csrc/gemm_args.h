@@ -64,6 +64,13 @@ struct GemmArgs {
   // four-wave kernel only: slabs per block of the tail (the tiles beyond the last whole round of the chip, cut evenly along
   // K among the blocks; 0: every tile is computed whole by one block)
   int tail_units;           // the four-wave kernel: slabs of a run of its cut tail (0: whole tiles only)
+  // decode kernel with the quantisation inside (a is not used then): the bf16 activations, their row stride in elements, and
+  // how they are quantised -- dynamically (scales bounded by x_scale_ub) or by a fixed scale (x_static; x_recip its reciprocal,
+  // x_scale what the result is multiplied by in place of a_scales and b_scales)
+  const uint16_t* x;
+  int64_t ldx;
+  int x_static;
+  float x_scale_ub, x_recip, x_scale;
   // fused QKV only
   int kv_on;
   KvStore kv;

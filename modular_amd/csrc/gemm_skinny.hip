@@ -56,12 +56,16 @@ __device__ __forceinline__ uint32_t sk_clamp_u32(int64_t v) {
 // wave), instead of two loads per slab and 16-token group: on a launch that is a single round of blocks those loads
 // are half of the loop's vector-memory instructions and cost 8 % of the kernel, whatever they fetch.
 constexpr int kSkinnyALdsBytes = 8192;
-template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, bool ALDS = false>
+// How the activations reach the loop: loaded per slab, copied to LDS before it, or (any larger value) quantised into LDS
+// before it from the bf16 activations by the block itself, that many 16-byte loads per lane.
+enum SkinnyActs { kActsPerSlab = 0, kActsLds = 1 };
+template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, int ACTS = kActsPerSlab>
 struct SkinnyCfg {
+  static constexpr bool ALDS = ACTS != kActsPerSlab, QUANT = ACTS > kActsLds;
   static constexpr int WAVES = NWAVES;
   static constexpr int SLOT = NTW * 2048;                    // one slab of the block's rows
   // VMEM instructions a wave issues per slab, in this order: activations, scales, weight DMA
-  static constexpr int PER = (ALDS ? 0 : 2 * MT) + (BLOCKSCALE ? MT + 1 : 0) + 2 * NTW;
+  static constexpr int PER = (ALDS ? 0 : 2 * MT) + (BLOCKSCALE ? (QUANT ? 1 : MT + 1) : 0) + 2 * NTW;
   // slabs in flight per wave: RING_KB of weights, limited by the 6-bit vmcnt counter and by the
   // registers the activation fragments of the in-flight slabs take (96)
   static constexpr int D_BYTES = RING_KB * 1024 / SLOT, D_CNT = 63 / PER + 1, D_REGS = 96 / (MT * 8);
@@ -73,10 +77,27 @@ struct SkinnyCfg {
   static constexpr int SMEM = RINGS;  // (ALDS: plus WAVES * M * the share's bytes, added at the launch)
 };
 
-template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, bool ALDS = false>
+// LDS of the activations a wave keeps for its share of K (per_wave slabs), beside the rings: M rows, one after the other
+template <int ACTS>
+__host__ __device__ constexpr uint32_t skinny_acts_row(uint32_t per_wave) {
+  // (quantised in place: rows 16 bytes apart in the bank order, so that 16 tokens read without conflicts; copied: whole
+  // 1024-byte copies)
+  return ACTS > kActsLds ? per_wave * 128u + 16u : (per_wave * 128u + 1023u) & ~1023u;
+}
+// ... and the scales that the quantisation leaves there: one per token and slab (block scaling), or the waves' largest values
+// and the scale per token
+template <int ACTS, bool BLOCKSCALE>
+__host__ __device__ constexpr uint32_t skinny_acts_bytes(uint32_t M, uint32_t per_wave) {
+  if (ACTS == kActsPerSlab) return 0;
+  const uint32_t rows = M * skinny_acts_row<ACTS>(per_wave);
+  return ACTS > kActsLds ? rows + (BLOCKSCALE ? (M * per_wave * 4u + 15u) & ~15u : 128u) : rows;
+}
+
+template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, int ACTS = kActsPerSlab>
 __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in) {
   const GemmArgs p = gridDim.y == 1 ? p_in : batch_view(p_in, blockIdx.y);
-  using Cfg = SkinnyCfg<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ALDS>;
+  using Cfg = SkinnyCfg<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ACTS>;
+  constexpr bool ALDS = Cfg::ALDS, QUANT = Cfg::QUANT;
   static_assert(!ALDS || MT == 1, "activations in LDS: one 16-token group");
   constexpr int WAVES = Cfg::WAVES, DEPTH = Cfg::DEPTH, SLOT = Cfg::SLOT, PER = Cfg::PER;
   static_assert((DEPTH - 1) * PER < 64, "vmcnt is a 6-bit counter");
@@ -116,10 +137,30 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in)
   uint8_t* ring = smem + wave * Cfg::RING;
   // ALDS: token t's bytes of this wave's share of K sit at a_lds + t * a_tok; lane (lm, lq) reads token min(lm, M - 1)
   // (the columns of C past M are never stored, so what their lanes multiply does not matter)
-  [[maybe_unused]] const uint32_t a_tok = ((uint32_t)per_wave * 128u + 1023u) & ~1023u;  // (whole copies: 1024 bytes each)
-  [[maybe_unused]] uint8_t* a_lds = smem + Cfg::RINGS + wave * ((uint32_t)p.M * a_tok);
+  [[maybe_unused]] const uint32_t a_tok = skinny_acts_row<ACTS>((uint32_t)per_wave);
+  [[maybe_unused]] uint8_t* a_lds = smem + Cfg::RINGS + wave * skinny_acts_bytes<ACTS, BLOCKSCALE>((uint32_t)p.M, (uint32_t)per_wave);
+  [[maybe_unused]] float* a_sc = reinterpret_cast<float*>(a_lds + (uint32_t)p.M * a_tok);  // QUANT
   [[maybe_unused]] const uint32_t a_rd = (uint32_t)(lm < p.M ? lm : p.M - 1) * a_tok + lq * 16;
-  if constexpr (ALDS) {
+  // QUANT: this lane's bf16 activations, load i = 512 consecutive elements of the share of token i / pieces (zeros past it).
+  // They go out before the first weight copies, so that waiting for them is not waiting for those.
+  constexpr int NLOADS = QUANT ? ACTS : 1;
+  [[maybe_unused]] v4i xv[NLOADS];
+  [[maybe_unused]] const int pieces = (per_wave + 3) / 4, n_loads = p.M * pieces;
+  if constexpr (QUANT) {
+    const __amdgpu_buffer_rsrc_t x_rsrc = sk_rsrc(p.x, sk_clamp_u32(((int64_t)(p.M - 1) * p.ldx + p.K) * 2));
+    const uint32_t share_end = (uint32_t)(s_end > s_begin ? s_end : s_begin) * 128u;
+    const uint32_t k_end = share_end < (uint32_t)p.K ? share_end : (uint32_t)p.K;
+    int t = 0, piece = 0;
+#pragma unroll
+    for (int i = 0; i < NLOADS; ++i) {
+      if (i < n_loads) {
+        const uint32_t k = (uint32_t)s_begin * 128u + (uint32_t)piece * 512u + (uint32_t)lane * 8u;
+        xv[i] = sk_load16(x_rsrc, k < k_end ? k * 2u : 0x80000000u, (uint32_t)t * (uint32_t)p.ldx * 2u);
+        if (++piece == pieces) { piece = 0; ++t; }
+      }
+    }
+  }
+  if constexpr (ALDS && !QUANT) {
     // one instruction moves 1024 consecutive bytes of a token; bytes past K or past the share are not fetched (zeros)
     const uint32_t share_begin = (uint32_t)s_begin * 128u, share_end = (uint32_t)(s_end > s_begin ? s_end : s_begin) * 128u;
     const uint32_t k_end = share_end < (uint32_t)p.K ? share_end : (uint32_t)p.K;
@@ -133,15 +174,16 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in)
 
   __amdgpu_buffer_rsrc_t as_rsrc = sk_rsrc(nullptr, 0), bs_rsrc = sk_rsrc(nullptr, 0);
   uint32_t as_voff[MT];
-  if constexpr (BLOCKSCALE) {
+  if constexpr (BLOCKSCALE && !QUANT) {
     as_rsrc = sk_rsrc(p.a_scales, sk_clamp_u32(((int64_t)(nslab - 1) * p.a_scales_ld + p.M) * 4));
-    bs_rsrc = sk_rsrc(p.b_scales + (int64_t)(n0 / 128) * p.b_scales_ld, (uint32_t)nslab * 4u);
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       const int m = t * 16 + lm;
       as_voff[t] = (uint32_t)(m < p.M ? m : p.M - 1) * 4u;
     }
   }
+
+  if constexpr (BLOCKSCALE) bs_rsrc = sk_rsrc(p.b_scales + (int64_t)(n0 / 128) * p.b_scales_ld, (uint32_t)nslab * 4u);
 
   v4f acc[MT][NTW];
 #pragma unroll
@@ -178,9 +220,11 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in)
       }
     }
     if constexpr (BLOCKSCALE) {
+      if constexpr (!QUANT) {
 #pragma unroll
-      for (int t = 0; t < MT; ++t)
-        as_v[d][t] = sk_load_f32(as_rsrc, as_voff[t], (uint32_t)sl * (uint32_t)p.a_scales_ld * 4u);
+        for (int t = 0; t < MT; ++t)
+          as_v[d][t] = sk_load_f32(as_rsrc, as_voff[t], (uint32_t)sl * (uint32_t)p.a_scales_ld * 4u);
+      }
       bs_v[d] = sk_load_f32(bs_rsrc, 0, (uint32_t)sl * 4u);
     }
     uint8_t* slot = ring + d * SLOT;
@@ -203,6 +247,7 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in)
       const v4i lo = *reinterpret_cast<const v4i*>(a_lds + a_rd + at);
       const v4i hi = *reinterpret_cast<const v4i*>(a_lds + a_rd + at + 64);
       af[d][0] = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      if constexpr (QUANT && BLOCKSCALE) as_v[d][0] = a_sc[(lm < p.M ? lm : p.M - 1) * per_wave + (slab < s_end ? slab - s_begin : 0)];
     }
 #pragma unroll
     for (int nt = 0; nt < NTW; ++nt) {
@@ -229,6 +274,93 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in)
   };
 
   for_each_slot([&](auto d_c) { issue(s_begin + decltype(d_c)::value, d_c); });
+  if constexpr (QUANT) {
+    // While the first weight slabs are on their way: the arithmetic of quantize_dynamic_scaled_fp8 (quant.hip), so that the
+    // codes and scales are those that kernel would have left in memory.
+    auto unpack = [](const v4i& w, float (&f)[8]) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        f[2 * j] = __uint_as_float((uint32_t)w[j] << 16);
+        f[2 * j + 1] = __uint_as_float((uint32_t)w[j] & 0xffff0000u);
+      }
+    };
+    auto store = [&](const float (&f)[8], float recip, int t, int piece) {
+      int lo = 0, hi = 0;
+      lo = cvt_pk_e4m3fn(clamp448(f[0] * recip), clamp448(f[1] * recip), lo, false);
+      lo = cvt_pk_e4m3fn(clamp448(f[2] * recip), clamp448(f[3] * recip), lo, true);
+      hi = cvt_pk_e4m3fn(clamp448(f[4] * recip), clamp448(f[5] * recip), hi, false);
+      hi = cvt_pk_e4m3fn(clamp448(f[6] * recip), clamp448(f[7] * recip), hi, true);
+      const uint32_t at = (uint32_t)piece * 512u + (uint32_t)lane * 8u;
+      if (at < (uint32_t)per_wave * 128u)
+        *reinterpret_cast<uint2*>(a_lds + (uint32_t)t * a_tok + at) = make_uint2((uint32_t)lo, (uint32_t)hi);
+    };
+    auto amax8 = [](const float (&f)[8]) {
+      float m = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(f[j]));
+      return m;
+    };
+    int t = 0, piece = 0;
+    if constexpr (BLOCKSCALE) {
+#pragma unroll
+      for (int i = 0; i < NLOADS; ++i) {
+        if (i < n_loads) {
+          float f[8], scale, recip;
+          unpack(xv[i], f);
+          dynamic_scale_f32(row16_max(amax8(f)), p.x_scale_ub, scale, recip);
+          store(f, recip, t, piece);
+          const int slab = piece * 4 + lq;
+          if (lm == 0 && slab < per_wave) a_sc[t * per_wave + slab] = scale;
+          if (++piece == pieces) { piece = 0; ++t; }
+        }
+      }
+    } else {
+      // one scale per token: the waves' shares meet in LDS (word 16 * wave + t of the first wave's scale area)
+      float* meet = reinterpret_cast<float*>(smem + Cfg::RINGS + (uint32_t)p.M * a_tok);
+      constexpr uint32_t kWaveStep = 16;  // (each wave's area holds 32 words: 16 for the waves' values of ITS tokens, 16 scales)
+      const uint32_t area = skinny_acts_bytes<ACTS, BLOCKSCALE>((uint32_t)p.M, (uint32_t)per_wave) / 4u;
+      if (!p.x_static) {
+        float m = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NLOADS; ++i) {
+          if (i < n_loads) {
+            float f[8];
+            unpack(xv[i], f);
+            m = fmaxf(m, amax8(f));
+            if (++piece == pieces) {
+              m = wave_max(m);
+              if (lane == 0) meet[wave * area + t] = m;
+              m = 0.0f;
+              piece = 0;
+              ++t;
+            }
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+      }
+      t = piece = 0;
+      float scale = 0.f, recip = p.x_recip;
+#pragma unroll
+      for (int i = 0; i < NLOADS; ++i) {
+        if (i < n_loads) {
+          if (piece == 0 && !p.x_static) {
+            float m = meet[t];
+#pragma unroll
+            for (int w = 1; w < WAVES; ++w) m = fmaxf(m, meet[w * area + t]);
+            dynamic_scale_f32(m, p.x_scale_ub, scale, recip);
+            if (lane == 0) a_sc[kWaveStep + t] = scale;
+          }
+          float f[8];
+          unpack(xv[i], f);
+          store(f, recip, t, piece);
+          if (++piece == pieces) { piece = 0; ++t; }
+        }
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
   for (int base = s_begin; base < s_end; base += DEPTH) {
     for_each_slot([&](auto d_c) {
       constexpr int d = decltype(d_c)::value;
@@ -270,7 +402,7 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in)
       // fused QKV: the reference's bf16 roundings, then C or the row's K / V page (see tile_body)
       const int64_t row_off = kv_row_offset(p.kv, m);
       float a_s = 1.f;
-      if constexpr (!BLOCKSCALE) a_s = p.a_scales[(int64_t)m * p.a_scale_stride];
+      if constexpr (!BLOCKSCALE) a_s = QUANT ? a_sc[16 + m] : p.a_scales[(int64_t)m * p.a_scale_stride];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int nn = (n + i < p.N) ? n + i : p.N - 1;
@@ -295,8 +427,11 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in)
       }
       continue;
     }
-    if constexpr (!BLOCKSCALE) {
-      const float a_s = scale_at(p.a_scales, (int64_t)m * p.a_scale_stride, p.scales_dtype);
+    if (!BLOCKSCALE && QUANT && p.x_static) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] *= p.x_scale;
+    } else if constexpr (!BLOCKSCALE) {
+      const float a_s = QUANT ? a_sc[16 + m] : scale_at(p.a_scales, (int64_t)m * p.a_scale_stride, p.scales_dtype);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int nn = (n + i < p.N) ? n + i : p.N - 1;
@@ -325,9 +460,9 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in)
 }
 
 int compute_units();
-template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, bool ALDS = false>
+template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, int ACTS = kActsPerSlab>
 static int launch_skinny_r(const GemmArgs& p, int64_t batch, hipStream_t stream) {
-  if constexpr (MT == 1 && !ALDS) {
+  if constexpr (MT == 1 && ACTS == kActsPerSlab) {
     // few tokens, a share of K per wave that fits, and a weight matrix small enough that the launch is about one round of
     // blocks: the activations go to LDS once (84 MB, M = 1: 17.8 -> 17.0 us; on a 470 MB matrix, where blocks come and
     // go, the per-slab loads cost nothing and this form measured 1 % slower).  Not for the fused QKV epilogue's build, a
@@ -338,27 +473,24 @@ static int launch_skinny_r(const GemmArgs& p, int64_t batch, hipStream_t stream)
     const int64_t per_wave = ceil_div(ceil_div(p.K, 128), NWAVES);
     const int64_t a_bytes = (int64_t)p.M * ((per_wave * 128 + 1023) / 1024 * 1024);  // per wave
     const int64_t blocks_per_cu = ceil_div(ceil_div((int64_t)p.N, 16 * NTW) * batch, (int64_t)compute_units());
-    using Plain = SkinnyCfg<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, false>;
+    using Plain = SkinnyCfg<NTW, MT, BLOCKSCALE, RING_KB, NWAVES>;
     if (tuning().skinny_alds && !p.kv_on && (int64_t)p.N * p.K < ((int64_t)1 << 27) && a_bytes <= kSkinnyALdsBytes &&
         blocks_per_cu * (Plain::SMEM + NWAVES * a_bytes) <= 160 * 1024)
-      return launch_skinny_r<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, true>(p, batch, stream);
+      return launch_skinny_r<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, kActsLds>(p, batch, stream);
   }
-  using Cfg = SkinnyCfg<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ALDS>;
-  auto kern = gemm_skinny_kernel<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ALDS>;
+  using Cfg = SkinnyCfg<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ACTS>;
+  auto kern = gemm_skinny_kernel<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ACTS>;
   static PerDeviceFlag attr;
   bool& attr_done = attr.here();
-  constexpr int smem_all = Cfg::SMEM + (ALDS ? NWAVES * kSkinnyALdsBytes : 0);
+  constexpr int smem_all = Cfg::QUANT ? 160 * 1024 : Cfg::SMEM + (Cfg::ALDS ? NWAVES * kSkinnyALdsBytes : 0);
   constexpr int smem_max = smem_all < 160 * 1024 ? smem_all : 160 * 1024;  // (what a launch asks for was checked against the CU's LDS)
   if (!attr_done) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem_max);
     if (e != hipSuccess) MAXFP8_FAIL(MAXFP8_ERR_LAUNCH, "gemm_skinny: cannot reserve %d bytes of LDS: %s", smem_max, hipGetErrorString(e));
     attr_done = true;
   }
-  int smem = Cfg::SMEM;
-  if constexpr (ALDS) {
-    const int64_t per_wave = ceil_div(ceil_div(p.K, 128), NWAVES);
-    smem += NWAVES * (int)(p.M * ((per_wave * 128 + 1023) / 1024 * 1024));
-  }
+  const uint32_t per_wave = (uint32_t)ceil_div(ceil_div(p.K, 128), NWAVES);
+  const int smem = Cfg::SMEM + NWAVES * (int)skinny_acts_bytes<ACTS, BLOCKSCALE>((uint32_t)p.M, per_wave);
   const int64_t blocks = ceil_div(p.N, 16 * NTW);
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)batch), dim3(NWAVES * 64), smem, stream, p);
   return launch_status("gemm_skinny");
@@ -408,6 +540,56 @@ static int pick_ntw(const GemmArgs& p, int64_t batch, hipStream_t stream) {
     case 4432: return launch_skinny_r<4, MT, BLOCKSCALE, 32, 4>(p, batch, stream);
     default: MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "skinny matmul: unknown shape selector %d", sel);
   }
+}
+
+// ---- with the quantisation inside -------------------------------------------------------------------------------
+// A block quantises the activations of its waves' shares of K itself, from bf16, while its first weight slabs are on their
+// way: no quantisation launch in front and no fp8 activations in memory.  Linear of one token, graph timing, against the
+// quantiser and the plain kernel behind it: 4096 x 4096 8.5 -> 6.2 us, 28672 x 4096 24.1 -> 20.0, 10240 x 8192 19.7 -> 15.6 (block
+// scaling; row scaling 7.9 -> 6.2, 23.6 -> 20.4, 18.8 -> 15.8).
+// Every block repeats the work, a third of a microsecond per 512 elements of a wave (its conversions come one after the
+// other, one wave per SIMD): with eight loads per wave the two ways are level (4 tokens of 4096: 9.1 and 8.6 us; 8 tokens 9.5
+// and 11.7).  With row scales every token costs a meeting of the waves on top, once per block of a CU: at most four tokens,
+// and together with the blocks a CU works on at most eight of them (4 tokens on 28672 x 4096: 24.9 and 26.3 us).
+constexpr int kQuantLoads = 8;
+static int skinny_quant_loads(int64_t M, int64_t K) {
+  return (int)(M * ceil_div(ceil_div(ceil_div(K, 128), 4), 4));
+}
+template <int NTW, bool BLOCKSCALE, int RING_KB>
+static bool skinny_quant_fits(int64_t M, int64_t N, int64_t K) {
+  const int64_t per_cu = ceil_div(ceil_div(N, 16 * NTW), (int64_t)compute_units());
+  if (skinny_quant_loads(M, K) > kQuantLoads || (!BLOCKSCALE && M > 1 && (M > 4 || M * per_cu > 8))) return false;
+  // (the quantised activations of the blocks that are on a CU together -- three keep the weight stream full -- fit its LDS)
+  const uint32_t per_wave = (uint32_t)ceil_div(ceil_div(K, 128), 4);
+  const int64_t smem = SkinnyCfg<NTW, 1, BLOCKSCALE, RING_KB, 4, kQuantLoads>::SMEM +
+                       4 * (int64_t)skinny_acts_bytes<kQuantLoads, BLOCKSCALE>((uint32_t)M, per_wave);
+  return (per_cu < 3 ? per_cu : 3) * smem <= 160 * 1024;
+}
+static int skinny_quant_shape(int64_t M, int64_t N, int64_t K) {
+  const int sel = tuning().skinny ? tuning().skinny : skinny_shape(M, N, K);
+  return sel == 1408 || sel == 2408 || sel == 4432 ? sel : 0;
+}
+bool gemm_skinny_quant_ok(int64_t M, int64_t N, int64_t K, bool blockscale) {
+  if (M < 1 || M > 16 || !tuning().skinny_quant || K % (blockscale ? 128 : 16) != 0) return false;
+  switch (skinny_quant_shape(M, N, K)) {
+    case 1408: return blockscale ? skinny_quant_fits<1, true, 8>(M, N, K) : skinny_quant_fits<1, false, 8>(M, N, K);
+    case 2408: return blockscale ? skinny_quant_fits<2, true, 8>(M, N, K) : skinny_quant_fits<2, false, 8>(M, N, K);
+    case 4432: return blockscale ? skinny_quant_fits<4, true, 32>(M, N, K) : skinny_quant_fits<4, false, 32>(M, N, K);
+    default: return false;
+  }
+}
+template <bool BLOCKSCALE>
+static int pick_quant(const GemmArgs& p, hipStream_t stream) {
+  switch (skinny_quant_shape(p.M, p.N, p.K)) {
+    case 1408: return launch_skinny_r<1, 1, BLOCKSCALE, 8, 4, kQuantLoads>(p, 1, stream);
+    case 2408: return launch_skinny_r<2, 1, BLOCKSCALE, 8, 4, kQuantLoads>(p, 1, stream);
+    default: return launch_skinny_r<4, 1, BLOCKSCALE, 32, 4, kQuantLoads>(p, 1, stream);
+  }
+}
+int gemm_skinny_quant_dispatch(const GemmArgs& p, bool blockscale, hipStream_t stream) {
+  if (skinny_quant_loads(p.M, p.K) > kQuantLoads)
+    MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "decode matmul with the quantisation inside: M = %d, K = %d do not fit", p.M, p.K);
+  return blockscale ? pick_quant<true>(p, stream) : pick_quant<false>(p, stream);
 }
 
 // ---- read-only probe ---------------------------------------------------------------------------

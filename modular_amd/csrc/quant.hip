@@ -411,11 +411,13 @@ __global__ __launch_bounds__(256) void rmsnorm_quant_generic_kernel(
 __global__ __launch_bounds__(256) void quant_static_bf16_kernel(uint8_t* __restrict__ out, const uint16_t* __restrict__ in,
                                                                 int64_t rows, int kvec, int64_t in_stride,
                                                                 int64_t out_stride, float recip, const void* scale_ptr,
-                                                                int scales_dtype) {
+                                                                int scales_dtype, float* leave_at, float leave0, float leave1) {
+  if (leave_at && blockIdx.x == 0 && threadIdx.x < 2) leave_at[threadIdx.x] = threadIdx.x ? leave1 : leave0;
   if (scale_ptr) recip = guarded_recip(load_elem(scale_ptr, scales_dtype, 0));
   const int64_t total = rows * kvec;
+  const bool narrow = total < ((int64_t)1 << 31);  // (a 64-bit division is more instructions than the eight conversions)
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-    const int64_t r = i / kvec;
+    const int64_t r = narrow ? (int64_t)((uint32_t)i / (uint32_t)kvec) : i / kvec;
     const int c = (int)(i - r * kvec);
     const uint4 v = reinterpret_cast<const uint4*>(in + r * in_stride)[c];
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -437,7 +439,9 @@ __global__ __launch_bounds__(256) void quant_static_bf16_kernel(uint8_t* __restr
 __global__ __launch_bounds__(256) void quant_static_generic_kernel(uint8_t* __restrict__ out, const void* __restrict__ in,
                                                                    int64_t rows, int64_t K, int64_t in_stride,
                                                                    int64_t out_stride, int in_dtype, float recip,
-                                                                   const void* scale_ptr, int scales_dtype) {
+                                                                   const void* scale_ptr, int scales_dtype, float* leave_at,
+                                                                   float leave0, float leave1) {
+  if (leave_at && blockIdx.x == 0 && threadIdx.x < 2) leave_at[threadIdx.x] = threadIdx.x ? leave1 : leave0;
   if (scale_ptr) recip = guarded_recip(load_elem(scale_ptr, scales_dtype, 0));
   const int64_t total = rows * K;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
@@ -637,9 +641,10 @@ int rmsnorm_quantize_dispatch(void* out_fp8, void* out_scales, const void* in, c
 }
 
 // scale_ptr == nullptr: quantise with the host value `scale`; otherwise with element 0 of scale_ptr
+// (leave, with `leave_at`: two floats the quantiser's first block puts there for the matmul behind it)
 static int quantize_by_scale(void* out_fp8, const void* in, int64_t rows, int64_t K, int64_t in_row_stride,
                              int64_t out_row_stride, int in_dtype, float scale, const void* scale_ptr, int scales_dtype,
-                             hipStream_t stream) {
+                             hipStream_t stream, float* leave_at = nullptr, float leave0 = 0.f, float leave1 = 0.f) {
   const float recip = 1.0f / scale;
   const bool fast = in_dtype == MAXFP8_BF16 && aligned16(in) && (in_row_stride % 8 == 0) && (K % 8 == 0) &&
                     (reinterpret_cast<uintptr_t>(out_fp8) % 8 == 0) && (out_row_stride % 8 == 0);
@@ -647,16 +652,23 @@ static int quantize_by_scale(void* out_fp8, const void* in, int64_t rows, int64_
   const unsigned blocks = (unsigned)(ceil_div(items, 256) < 16384 ? ceil_div(items, 256) : 16384);
   if (fast)
     hipLaunchKernelGGL(quant_static_bf16_kernel, dim3(blocks), dim3(256), 0, stream, (uint8_t*)out_fp8, (const uint16_t*)in,
-                       rows, (int)(K / 8), in_row_stride, out_row_stride, recip, scale_ptr, scales_dtype);
+                       rows, (int)(K / 8), in_row_stride, out_row_stride, recip, scale_ptr, scales_dtype, leave_at, leave0, leave1);
   else
     hipLaunchKernelGGL(quant_static_generic_kernel, dim3(blocks), dim3(256), 0, stream, (uint8_t*)out_fp8, in, rows, K,
-                       in_row_stride, out_row_stride, in_dtype, recip, scale_ptr, scales_dtype);
+                       in_row_stride, out_row_stride, in_dtype, recip, scale_ptr, scales_dtype, leave_at, leave0, leave1);
   return launch_status("quantize_static");
 }
 
 int quantize_static_dispatch(void* out_fp8, const void* in, int64_t rows, int64_t K, int64_t in_row_stride,
                              int64_t out_row_stride, int in_dtype, float scale, hipStream_t stream) {
   return quantize_by_scale(out_fp8, in, rows, K, in_row_stride, out_row_stride, in_dtype, scale, nullptr, MAXFP8_F32, stream);
+}
+
+// the same for a matmul behind it that takes the product of the two per-tensor scales, and 1, from `scales` on the device
+int quantize_static_for_matmul_dispatch(void* out_fp8, float* scales, const void* in, int64_t rows, int64_t K, int64_t in_row_stride,
+                                        int in_dtype, float input_scale, float weight_scale, hipStream_t stream) {
+  return quantize_by_scale(out_fp8, in, rows, K, in_row_stride, K, in_dtype, input_scale, nullptr, MAXFP8_F32, stream, scales,
+                           input_scale * weight_scale, 1.0f);
 }
 
 int quantize_tensor_dispatch(void* out_fp8, void* out_scales, const void* in, int64_t rows, int64_t K, int64_t in_row_stride,

@@ -17,6 +17,7 @@
 //   MAXFP8_GROUPED_OVERLAP=0   grouped, two launches: in line on the caller's stream
 //   MAXFP8_GROUPED_SHARE=x     grouped: scales the estimate of how much of the chip the small tiles need (0.5)
 //   MAXFP8_SKINNY_ALDS=0       decode kernel: activations loaded per slab even where a wave's share of them fits LDS
+//   MAXFP8_SKINNY_QUANT=0      linears: always the quantiser's launch in front of the decode kernel
 //   MAXFP8_SKINNY=<ntw>4<KB>   force a shape of the weight-streaming kernel (e.g. 1408, 2416)
 //   MAXFP8_MID=0 / <MT><NT>    the kernel for tens to a few hundred tokens: never / always, in 16 MT x 16 NT tiles (e.g. 43)
 //   MAXFP8_SHORT_K=0           batches of short K: the decode and tile kernels only
@@ -47,6 +48,7 @@ struct Tuning {
   int grouped_w4_hot_rest = 32, grouped_w4_cold_rows = 128;
   int skinny = 0;
   bool skinny_alds = true;
+  bool skinny_quant = true;
   bool short_k = true;
   int mid = -1;              // -1: the estimates decide
   unsigned generation = 0;  // counts the reloads: part of the key of every cache that depends on the switches
