@@ -36,6 +36,11 @@ EXPORTS = (
     "maxfp8_batched_matmul_dynamic_scaled_fp8",
     "maxfp8_matmul_workspace_bytes",
     "maxfp8_matmul_auto_workspace_bytes",
+    "maxfp8_linear_workspace_bytes",
+    "maxfp8_linear_dynamic_scaled_fp8",
+    "maxfp8_linear_static_scaled_fp8",
+    "maxfp8_linear_qkv_workspace_bytes",
+    "maxfp8_linear_qkv_ragged_paged_scale",
     "maxfp8_matmul_describe",
     "maxfp8_grouped_matmul_dynamic_scaled_fp8",
     "maxfp8_grouped_matmul_rowwise_dynamic_scaled_fp8",
@@ -103,6 +108,16 @@ def lib() -> ctypes.CDLL:
     L.maxfp8_matmul_describe.argtypes = [i64, i64, i64, ci, ci, ctypes.c_char_p, ctypes.c_size_t]
     L.maxfp8_matmul_workspace_bytes.restype = ctypes.c_size_t
     L.maxfp8_matmul_workspace_bytes.argtypes = [i64, i64, i64]
+    L.maxfp8_linear_workspace_bytes.restype = ctypes.c_size_t
+    L.maxfp8_linear_workspace_bytes.argtypes = [i64, i64, i64, ci]
+    L.maxfp8_linear_dynamic_scaled_fp8.restype = ci
+    L.maxfp8_linear_dynamic_scaled_fp8.argtypes = [vp] * 4 + [i64] * 6 + [ci, i64, cf, vp, ctypes.c_size_t, vp]
+    L.maxfp8_linear_static_scaled_fp8.restype = ci
+    L.maxfp8_linear_static_scaled_fp8.argtypes = [vp] * 3 + [i64] * 6 + [cf, cf, vp, ctypes.c_size_t, vp]
+    L.maxfp8_linear_qkv_workspace_bytes.restype = ctypes.c_size_t
+    L.maxfp8_linear_qkv_workspace_bytes.argtypes = [i64, i64, i64, ci]
+    L.maxfp8_linear_qkv_ragged_paged_scale.restype = ci
+    L.maxfp8_linear_qkv_ragged_paged_scale.argtypes = [vp, vp, i64] + [vp] * 7 + [i64] * 13 + [ci, i64, cf, vp, ctypes.c_size_t, vp]
     L.maxfp8_matmul_auto_workspace_bytes.restype = ctypes.c_size_t
     L.maxfp8_matmul_auto_workspace_bytes.argtypes = [i64, i64, i64]
     L.maxfp8_grouped_matmul_dynamic_scaled_fp8.restype = ci
@@ -137,6 +152,28 @@ def lib() -> ctypes.CDLL:
     L.maxfp8_mfma_issue_probe.argtypes = [ci, ci, ci, i64, vp, vp, vp, vp, vp, vp, vp]
     _lib = L
     return L
+
+
+NATIVE_PATH = os.path.join(_HERE, "lib", "_native.so")
+_native = None
+
+
+def native():
+    """The CPython module of the hot operators (csrc/bindings.cpp): each of its functions returns None for what it leaves to
+    the Python wrapper."""
+    global _native
+    if _native is None:
+        lib()
+        if not os.path.exists(NATIVE_PATH):
+            raise LibraryMissing(f"{NATIVE_PATH} not found: build it with `python -m modular_amd.build`")
+        import importlib.machinery
+        import importlib.util
+
+        loader = importlib.machinery.ExtensionFileLoader("modular_amd._native", NATIVE_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("modular_amd._native", loader))
+        loader.exec_module(module)
+        _native = module
+    return _native
 
 
 def last_error() -> str:

@@ -1,4 +1,5 @@
-"""Builds libmaxfp8.so (hand-written gfx950 HIP kernels + the C ABI) with hipcc.
+"""Builds libmaxfp8.so (hand-written gfx950 HIP kernels + the C ABI) with hipcc, and the CPython module of the hot
+operators on top of it (lib/_native.so) with g++.
 
     python -m modular_amd.build
 
@@ -47,6 +48,26 @@ def _compile(src: str, objdir: str, extra: list[str]) -> str:
     return obj
 
 
+def build_bindings() -> str:
+    """The CPython module of the hot operators (csrc/bindings.cpp), linked against the library beside it."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    out = os.path.join(LIBDIR, "_native.so")
+    libdir = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-I{d}" for d in cpp_extension.include_paths()], f"-I{sysconfig.get_paths()['include']}",
+           os.path.join(CSRC, "bindings.cpp"), "-o", out + ".tmp", f"-L{LIBDIR}", "-lmaxfp8", f"-L{libdir}", "-ltorch_python", "-ltorch",
+           "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{libdir}"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on bindings.cpp:\n{r.stderr[-4000:]}")
+    os.replace(out + ".tmp", out)
+    return out
+
+
 def build_library(extra: list[str] | None = None, verbose: bool = True) -> str:
     """Compile every HIP source for gfx950 and link the shared library."""
     extra = list(extra or [])
@@ -60,6 +81,7 @@ def build_library(extra: list[str] | None = None, verbose: bool = True) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr[-4000:]}")
     os.replace(LIB + ".tmp", LIB)
+    build_bindings()
     if verbose:
         print(f"built {LIB} ({os.path.getsize(LIB) // 1024} KiB)")
     return LIB

@@ -36,6 +36,18 @@ def _stream(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
+_BLOCK, _COLWISE, _ROWWISE = ScaleGranularity.BLOCK, ScaleGranularity.COLWISE, ScaleGranularity.ROWWISE
+
+
+def native_granularity(input_scale_spec: InputScaleSpec, weight_scale_spec: WeightScaleSpec) -> int:
+    """The weight granularity (as the C ABI counts) of the scalings the native operators take: 1 x 128 groups against 128 x
+    128 blocks, per token x per channel; -1 for every other."""
+    gi, gw = input_scale_spec.granularity, weight_scale_spec.granularity
+    if gi is _BLOCK and gw is _BLOCK:
+        return _lib.GRAN_BLOCK if input_scale_spec.block_size == (1, 128) and weight_scale_spec.block_size == (128, 128) else -1
+    return _lib.GRAN_ROWWISE if gi is _COLWISE and gw is _ROWWISE else -1
+
+
 def _require_gpu(*tensors: torch.Tensor) -> None:
     for t in tensors:
         if not t.is_cuda:
@@ -95,6 +107,14 @@ def quantize_dynamic_scaled_float8(
     (`scatter_index=restore_token_order`), without quantising a token top_k times.  bfloat16
     input, float32 scales and groups of 128 only.
     """
+    if (scales_type is torch.float32 and row_index is None and scatter_index is None and group_size_or_per_token == -1 and
+            out_type is _FP8):
+        kind = native_granularity(input_scale_spec, weight_scale_spec)
+        if kind >= 0:
+            block = kind == _lib.GRAN_BLOCK
+            done = _lib.native().quantize(input, 128 if block else -1, block, scale_ub)
+            if done is not None:
+                return done
     if input.dim() != 2:
         raise ValueError("input must be rank 2 tensor")
     if out_type != _FP8:
@@ -264,6 +284,10 @@ def rms_norm_fused_quantize_dynamic_scaled_fp8(
     (builtin_kernels/quantization.mojo:112-237).
 
     Returns (quantized, same shape as input, e4m3fn; scales [1, rows] with rows = input.numel() / K)."""
+    if out_type is _FP8 and scales_type is torch.float32:
+        done = _lib.native().rms_norm_quantize(input, gamma, epsilon, weight_offset, scale_ub)
+        if done is not None:
+            return done
     if input.dim() < 1:
         raise ValueError("input must have at least one axis")
     if gamma.dim() != 1:
@@ -308,6 +332,12 @@ def dynamic_scaled_matmul(
     algo: str = "auto",
 ) -> torch.Tensor:
     """C = A . B^T with scaling factors; `b` is [N, K] (already "transposed")."""
+    if algo == "auto" and out_type is torch.bfloat16:
+        kind = native_granularity(input_scale_spec, weight_scale_spec)
+        if kind >= 0:
+            done = _lib.native().matmul(a, b, a_scales, b_scales, kind)
+            if done is not None:
+                return done
     if a.dim() != 2 or b.dim() != 2 or a_scales.dim() != 2 or b_scales.dim() != 2:
         raise ValueError("All arguments must be rank 2 tensors")
     if a.shape[1] != b.shape[1]:
@@ -410,6 +440,10 @@ def batched_quantize_dynamic_scaled_fp8(
     Returns (quantized [B, M, K] e4m3fn, scales [B, K / group, M_pad]); M_pad rounds
     M up to 16 bytes of scales, the shape batched_dynamic_scaled_fp8_matmul expects.
     """
+    if scales_type is torch.float32 and group_size_or_per_token > 0:
+        done = _lib.native().batched_quantize(input, group_size_or_per_token, scale_ub)
+        if done is not None:
+            return done
     if input.dim() != 3:
         raise ValueError("input must be rank 3 tensor")
     if scales_type not in (torch.float32, torch.bfloat16):
@@ -452,6 +486,11 @@ def batched_dynamic_scaled_fp8_matmul(
     a_scales [B, ceil(K/128), M_pad], b_scales [B, ceil(N/128), ceil(K/128)].
     `out`, if given, is a [B, M, N] view with a contiguous last axis that receives the
     result in place (e.g. the [M, B, N] buffer the MLA graph writes, transposed)."""
+    if (out is None and algo == "auto" and out_type is torch.bfloat16 and
+            native_granularity(input_scale_spec, weight_scale_spec) == _lib.GRAN_BLOCK):
+        done = _lib.native().batched_matmul(a, b, a_scales, b_scales)
+        if done is not None:
+            return done
     if a.dtype != b.dtype:
         raise TypeError(f"a and b dtypes must match, but got {a.dtype}, {b.dtype}")
     if a_scales.dtype != b_scales.dtype or a_scales.dtype != torch.float32:

@@ -6,6 +6,9 @@ from __future__ import annotations
 
 import torch
 
+from . import _lib
+from .kernels import dynamic_scaled_matmul, native_granularity, quantize_dynamic_scaled_float8
+from .moe_kernels import fused_silu, fused_silu_quantized, silu_quantize, silu_quantize_group
 from .quant_config import QuantConfig, ScaleGranularity, ScaleOrigin
 from .quant_ops import quantized_matmul
 
@@ -65,12 +68,11 @@ class Linear(torch.nn.Module):
         return out
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, x.shape[-1])
+        x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
         y = quantized_matmul(x2, self.weight, self.weight_scale, self.input_scale, self.quant_config)
         if self.bias is not None:
             y = y + self.bias.to(y.dtype)
-        return y.reshape(*lead, self.out_dim)
+        return y if x.dim() == 2 else y.reshape(*x.shape[:-1], self.out_dim)
 
 
 class MLP(torch.nn.Module):
@@ -172,9 +174,6 @@ class MLP(torch.nn.Module):
         return t
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        from .kernels import dynamic_scaled_matmul, quantize_dynamic_scaled_float8
-        from .moe_kernels import fused_silu, fused_silu_quantized, silu_quantize, silu_quantize_group
-
         cfg = self.quant_config
         lead = x.shape[:-1]
         x2 = x.reshape(-1, x.shape[-1])
@@ -188,8 +187,14 @@ class MLP(torch.nn.Module):
                                       cfg.weight_scale, out_type=torch.bfloat16)
             return y.reshape(*lead, self.hidden_dim)
         if self._silu_kernel():
-            both = quantized_matmul(x2, self.gate_up_weight, self.gate_up_weight_scale, None, cfg)
             rows_used = self._all_rows(x2.shape[0], x2.device)
+            kind = native_granularity(cfg.input_scale, cfg.weight_scale)
+            if kind >= 0:
+                y = _lib.native().mlp(x2, self.gate_up_weight, self.gate_up_weight_scale, self.down_proj.weight,
+                                      self.down_proj.weight_scale, kind, rows_used, 1200.0)
+                if y is not None:
+                    return y if x.dim() == 2 else y.reshape(*lead, self.hidden_dim)
+            both = quantized_matmul(x2, self.gate_up_weight, self.gate_up_weight_scale, None, cfg)
             group = silu_quantize_group(cfg, x2.shape[0], self.feed_forward_length)
             if group is not None and self.down_proj.weight_scale.dtype == torch.float32:
                 hq, hs = silu_quantize(both, rows_used, group, round_activation=True)

@@ -17,7 +17,8 @@ from __future__ import annotations
 
 import torch
 
-from .kernels import grouped_dynamic_scaled_fp8_matmul, quantize_dynamic_scaled_float8
+from . import _lib
+from .kernels import grouped_dynamic_scaled_fp8_matmul, native_granularity, quantize_dynamic_scaled_float8
 from .moe_kernels import fused_silu, fused_silu_quantized, moe_create_indices, silu_quantize, silu_quantize_group
 from .quant_config import QuantConfig
 
@@ -98,9 +99,10 @@ def expert_matmuls_fp8(
     The grouped matmul op takes two host scalars (most tokens on one expert, active experts), which
     the reference copies from the device between the grouping and the first matmul
     (max/python/max/nn/moe/quant_strategy.py:175).  This package's kernels read the offsets on the
-    device and use the scalars only as upper bounds for their grids, so with `host_sync=False` the
-    bounds (every row on one expert, every expert active) stand in and nothing waits for the GPU:
-    same result, and the whole function can be captured in a HIP graph.
+    device and use the scalars only as upper bounds for their grids, so the bounds themselves (every row
+    on one expert, every expert active) stand in: same result, nothing waits for the GPU, and the
+    whole function can be captured in a HIP graph.  With `host_sync=True` the step-by-step route (an operand that
+    the native operator leaves to it, or `fuse_activation_quant`) still copies them, once.
 
     By default silu(gate) * up is rounded to bf16 and quantised for the down projection like any bf16 tensor
     (`silu_quantize`: the values of `fused_silu` followed by the quantiser, in one kernel).
@@ -110,6 +112,11 @@ def expert_matmuls_fp8(
         raise ValueError("expected x [seq, hidden] and router_idx [seq, k]")
     if not (quant_config.input_scale.is_block and quant_config.weight_scale.is_block):
         raise ValueError("the FP8 MoE path of this package is the block-scaled one")
+    if not fuse_activation_quant and native_granularity(quant_config.input_scale, quant_config.weight_scale) == _lib.GRAN_BLOCK:
+        ids = router_idx if router_idx.dtype == torch.int32 else router_idx.to(torch.int32)
+        done = _lib.native().moe_experts(x, ids, gate_up_proj, gate_up_proj_scales, down_proj, down_proj_scales, 1200.0)
+        if done is not None:
+            return done
     strategy = Fp8Strategy(quant_config, gate_up_proj.dtype)
     group = quant_config.input_scale.block_size[1]
     seq_len, top_k = router_idx.shape
@@ -119,6 +126,7 @@ def expert_matmuls_fp8(
     if not host_sync:
         # the bounds that need no look at the GPU: every row on one expert, every expert active
         usage_stats = torch.tensor([seq_len * top_k, num_experts], dtype=torch.int64).to(torch.uint32)
+    usage_stats = usage_stats.cpu()
 
     # sorted row r is assignment token_order[r] = token * top_k + slot: it reads token token_order[r] // top_k.  Seen
     # from the token: it is quantised once and stored to its top_k sorted rows restore_order[token * top_k + slot] --

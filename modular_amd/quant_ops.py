@@ -10,7 +10,8 @@ import weakref
 
 import torch
 
-from .kernels import (dynamic_scaled_matmul, fused_qkv_ragged_matmul_scaled_float8,
+from . import _lib
+from .kernels import (native_granularity, dynamic_scaled_matmul, fused_qkv_ragged_matmul_scaled_float8,
                       grouped_dynamic_scaled_fp8_matmul, grouped_matmul_rowwise_dynamic_scaled_fp8,
                       matmul_static_scaled_float8, quantize_dynamic_scaled_float8, quantize_static_scaled_float8,
                       quantize_tensor_dynamic_scaled_float8)
@@ -28,6 +29,9 @@ def matmul_float8(
     """x @ weight.T with float8 quantisation; x [M, K] bf16, weight [N, K] e4m3fn."""
     if input_scale is not None:
         # Static quantisation: the input scale was computed offline (quant_ops.py:384-417).
+        done = _lib.native().linear_static(x, weight, input_scale, weight_scale)
+        if done is not None:
+            return done
         xq = quantize_static_scaled_float8(x, input_scale, out_type=weight.dtype)
         if quant_config.weight_scale.is_tensor and weight_scale.dim() >= 2:
             # fused QKV: per-projection weight scales broadcast to rowwise [N, 1]; the scalar
@@ -53,7 +57,12 @@ def matmul_float8(
         return dynamic_scaled_matmul(xq, weight, x_scales, weight_scale, in_spec, w_spec,
                                      out_type=torch.bfloat16)
 
-    # dynamic per-row / block scaling (quant_ops.py:462-481)
+    # dynamic per-row / block scaling (quant_ops.py:462-481): in one step where the native operator takes it
+    kind = native_granularity(quant_config.input_scale, quant_config.weight_scale)
+    if kind >= 0:
+        done = _lib.native().linear(x, weight, weight_scale, kind, 1200.0)
+        if done is not None:
+            return done
     xq, x_scale = quantize_dynamic_scaled_float8(
         x, quant_config.input_scale, quant_config.weight_scale,
         scales_type=weight_scale.dtype, out_type=weight.dtype)
@@ -97,6 +106,16 @@ def quantized_fused_qkv_matmul(
     paged cache.  (Scales in bfloat16 are widened to float32 for the kernel, which is exact.)"""
     if quant_config.format not in (QuantFormat.COMPRESSED_TENSORS_FP8, QuantFormat.FBGEMM_FP8, QuantFormat.BLOCKSCALED_FP8):
         raise NotImplementedError(f"{quant_config.format} is not an FP8 format of this package")
+    blocks = kv_collection.kv_blocks
+    if (input_scale is None and quant_config.is_dynamic and kv_params.dtype is torch.bfloat16 and
+            blocks.shape[1:] == kv_params.blocks_shape(0)[1:]):
+        kind = native_granularity(quant_config.input_scale, quant_config.weight_scale)
+        if kind >= 0:
+            done = _lib.native().qkv_linear(x, wqkv, weight_scale, kind, 1200.0, input_row_offsets, blocks, kv_collection.cache_lengths,
+                                            kv_collection.lookup_table, bias, layer_idx,
+                                            _output_dim if _output_dim is not None else n_heads * kv_params.head_dim)
+            if done is not None:
+                return done
     common = dict(input_row_offsets=input_row_offsets, wqkv=wqkv, kv_collection=kv_collection, layer_idx=layer_idx,
                   n_heads=n_heads, bias=bias, _output_dim=_output_dim)
     if quant_config.is_static:
