@@ -67,7 +67,8 @@ bool gemm_mid_ok(int64_t M, int64_t N, int64_t K);
 int gemm_mid_shape(int64_t M, int64_t N, int64_t K, float* us);
 float gemm_skinny_cost(int64_t M, int64_t N, int64_t K);
 float gemm_tiled_small_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
-float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
+float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool has_workspace);
+size_t gemm_tiled_qkv_workspace_bytes(int64_t M, int64_t N, int64_t K, bool blockscale);
 bool gemm_skinny_preferred(int64_t M, int64_t N, int64_t K);
 int gemm_skinny_read_probe(const void* b, int64_t M, int64_t N, int64_t K, int64_t ldb, hipStream_t stream);
 int gemm_persist_probe(const GemmArgs&, bool, int, hipStream_t);
@@ -257,16 +258,16 @@ static int choose_kernel(int64_t M, int64_t N, int64_t K) {
   return algo;
 }
 
-// The same for the fused QKV matmul, whose tiles never split K: decode kernel (at most 64 rows), the kernel in between (at
-// most 320) or the tiles.
-static int choose_qkv(int64_t T, int64_t N, int64_t K) {
+// The same for the fused QKV matmul: decode kernel (at most 64 rows), the kernel in between (at most 320) or the tiles, whose
+// plan may cut them along K where the caller brings a workspace.
+static int choose_qkv(int64_t T, int64_t N, int64_t K, bool has_workspace) {
   const Tuning& t = tuning();
   const int plain = T <= gemm_skinny_max_m() ? MAXFP8_ALGO_SKINNY : MAXFP8_ALGO_TILED;
   if (t.mid > 0) return gemm_mid_ok(T, N, K) ? kAlgoMid : plain;
   if (T <= 16 || !gemm_mid_ok(T, N, K) || t.mid == 0 || t.tile || t.skinny) return plain;
   float mid;
   gemm_mid_shape(T, N, K, &mid);
-  const float tiles = gemm_tiled_qkv_cost(T, N, K, true);
+  const float tiles = gemm_tiled_qkv_cost(T, N, K, true, has_workspace);
   float us = tiles;
   int algo = MAXFP8_ALGO_TILED;
   if (T <= gemm_skinny_max_m()) {
@@ -770,7 +771,8 @@ static int qkv_common(void* output, const void* input, const void* x, int64_t ld
                                                int64_t batch_size, int64_t num_blocks, int64_t kv_dim, int64_t num_layers,
                                                int64_t layer_idx, int64_t page_size, int64_t num_kv_heads, int64_t head_dim,
                                                int64_t lut_ld, int64_t gm, int64_t gn, int64_t gk, int64_t input_scale_ld,
-                                               int64_t weight_scale_ld, int scales_dtype, int algo, void* stream) {
+                                               int64_t weight_scale_ld, int scales_dtype, int algo, void* workspace, size_t workspace_bytes,
+                                               void* stream) {
   if (T < 0 || N < 0 || K < 0 || q_dim < 0 || batch_size < 0) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused qkv matmul: negative size");
   if (batch_size == 0 || T == 0 || N == 0) return MAXFP8_OK;  // kv_cache_ragged.mojo:1193-1194
   if (T >= ((int64_t)1 << 31) || N >= ((int64_t)1 << 31) || K >= ((int64_t)1 << 31) || batch_size >= ((int64_t)1 << 31))
@@ -847,11 +849,12 @@ static int qkv_common(void* output, const void* input, const void* x, int64_t ld
     return gemm_skinny_quant_dispatch(p, block, st);
   }
   const bool automatic = algo == MAXFP8_ALGO_AUTO;
-  if (automatic) algo = choose_qkv(T, N, K);
+  if (automatic) algo = choose_qkv(T, N, K, workspace != nullptr);
   if (automatic && algo == kAlgoMid) return gemm_mid_dispatch(p, block, st);
   if (algo == MAXFP8_ALGO_SKINNY) return gemm_skinny_dispatch(p, block, 1, st);
   if (algo != MAXFP8_ALGO_TILED) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused qkv matmul: algo %d is not available", algo);
-  return gemm_tiled_dispatch(p, block, 0, 1, st);
+  p.workspace = (float*)workspace;
+  return gemm_tiled_dispatch(p, block, workspace_bytes, 1, st);
 }
 
 extern "C" {
@@ -866,17 +869,21 @@ int maxfp8_fused_qkv_matmul_ragged_paged_scale(void* output, const void* input, 
                                                int64_t weight_scale_ld, int scales_dtype, int algo, void* stream) {
   return qkv_common(output, input, nullptr, 0, 0.f, input_row_offsets, wqkv, input_scale, weight_scale, kv_blocks, cache_lengths, lookup_table,
                     bias, T, N, K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads, head_dim, lut_ld, gm,
-                    gn, gk, input_scale_ld, weight_scale_ld, scales_dtype, algo, stream);
+                    gn, gk, input_scale_ld, weight_scale_ld, scales_dtype, algo, nullptr, 0, stream);
 }
 
 static bool qkv_in_one(int64_t T, int64_t N, int64_t K, bool block) {
-  return T > 0 && N > 0 && K > 0 && choose_qkv(T, N, K) == MAXFP8_ALGO_SKINNY && gemm_skinny_quant_ok(T, N, K, block);
+  return T > 0 && N > 0 && K > 0 && choose_qkv(T, N, K, true) == MAXFP8_ALGO_SKINNY && gemm_skinny_quant_ok(T, N, K, block);
+}
+// what follows the quantised activations and their scales: the sums of cut tiles
+static size_t qkv_partial_bytes(int64_t T, int64_t N, int64_t K, bool block) {
+  return choose_qkv(T, N, K, true) == MAXFP8_ALGO_TILED ? gemm_tiled_qkv_workspace_bytes(T, N, K, block) : 0;
 }
 
 size_t maxfp8_linear_qkv_workspace_bytes(int64_t T, int64_t N, int64_t K, int weight_granularity) {
   if (T <= 0 || N <= 0 || K <= 0) return 0;
   const bool block = weight_granularity == MAXFP8_GRAN_BLOCK;
-  return qkv_in_one(T, N, K, block) ? 0 : linear_layout(T, N, K, block, false).partial;
+  return qkv_in_one(T, N, K, block) ? 0 : linear_layout(T, N, K, block, false).partial + qkv_partial_bytes(T, N, K, block);
 }
 
 int maxfp8_linear_qkv_ragged_paged_scale(void* output, const void* x, int64_t x_row_stride, const uint32_t* input_row_offsets,
@@ -896,10 +903,11 @@ int maxfp8_linear_qkv_ragged_paged_scale(void* output, const void* x, int64_t x_
   if (qkv_in_one(T, N, K, block) && is_aligned(x, 16) && x_row_stride % 8 == 0 && 32 * x_row_stride < ((int64_t)1 << 31))
     return qkv_common(output, nullptr, x, x_row_stride, scale_ub, input_row_offsets, wqkv, nullptr, weight_scale, kv_blocks, cache_lengths,
                       lookup_table, bias, T, N, K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads,
-                      head_dim, lut_ld, gm, gn, gk, 0, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_SKINNY, stream);
+                      head_dim, lut_ld, gm, gn, gk, 0, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_SKINNY, nullptr, 0, stream);
   const LinearLayout l = linear_layout(T, N, K, block, false);
-  if (!workspace || workspace_bytes < l.partial)
-    MAXFP8_FAIL(MAXFP8_ERR_WORKSPACE, "qkv linear: needs %zu bytes of workspace, got %zu", l.partial, workspace ? workspace_bytes : (size_t)0);
+  const size_t partial = qkv_partial_bytes(T, N, K, block), total = l.partial + partial;
+  if (!workspace || workspace_bytes < total)
+    MAXFP8_FAIL(MAXFP8_ERR_WORKSPACE, "qkv linear: needs %zu bytes of workspace, got %zu", total, workspace ? workspace_bytes : (size_t)0);
   if (!is_aligned(workspace, 16)) MAXFP8_FAIL(MAXFP8_ERR_ALIGN, "qkv linear: workspace must be 16-byte aligned");
   uint8_t* q = (uint8_t*)workspace;
   float* scales = (float*)(q + l.scales);
@@ -908,7 +916,7 @@ int maxfp8_linear_qkv_ragged_paged_scale(void* output, const void* x, int64_t x_
   if (rc != MAXFP8_OK) return rc;
   return qkv_common(output, q, nullptr, 0, 0.f, input_row_offsets, wqkv, scales, weight_scale, kv_blocks, cache_lengths, lookup_table, bias, T, N,
                     K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads, head_dim, lut_ld, gm, gn, gk,
-                    block ? l.scales_ld : T, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_AUTO, stream);
+                    block ? l.scales_ld : T, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_AUTO, q + l.partial, partial, stream);
 }
 
 }  // extern "C"

@@ -1870,12 +1870,12 @@ static int pick_splits(int64_t tiles, int slots, int nslab) {
 // The per-tile overhead of shape i on an M x N region: the persistent kernel (whole 256 x 256 tiles, no K split)
 // hides 3.5 of the 11.4 microseconds between two tiles (measured: 3.2 per round on q_b, 4.4 on kv_b).
 static bool persist_shape(int64_t M, int64_t N, int variant);
-static float tile_overhead(int64_t M, int64_t N, int i, int splits) {
-  return kShapes[i].t_tile - ((splits == 1 && persist_shape(M, N, i + 1)) ? 3.5f : 0.f);
+static float tile_overhead(int64_t M, int64_t N, int i, int splits, bool kv_on = false) {
+  return kShapes[i].t_tile - ((splits == 1 && !kv_on && persist_shape(M, N, i + 1)) ? 3.5f : 0.f);
 }
 
 // cost of a shape (microseconds) = rounds of resident blocks * time of one tile
-static int pick_shape(int64_t M, int64_t N, int nslab, bool blockscale, bool can_split, int64_t batch = 1) {
+static int pick_shape(int64_t M, int64_t N, int nslab, bool blockscale, bool can_split, int64_t batch = 1, bool kv_on = false) {
   int best = 0;
   float best_cost = 0.f;
   for (int i = 0; i < 4; ++i) {
@@ -1883,7 +1883,7 @@ static int pick_shape(int64_t M, int64_t N, int nslab, bool blockscale, bool can
     const int64_t tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn) * batch;
     const int sp = can_split ? pick_splits(tiles, t.slots, nslab) : 1;
     float cost = (float)ceil_div(tiles * sp, t.slots) *
-                 ((float)ceil_div(nslab, sp) * (blockscale ? t.t_slab_block : t.t_slab_row) + tile_overhead(M, N, i, sp));
+                 ((float)ceil_div(nslab, sp) * (blockscale ? t.t_slab_block : t.t_slab_row) + tile_overhead(M, N, i, sp, kv_on));
     // a split pays a second launch and one write + one read of sp * M * N f32 partial sums (~4 TB/s)
     if (sp > 1) cost += 5.0f + (float)sp * (float)M * (float)N * 8.0f / 4.0e6f;
     if (i == 0 || cost < best_cost) { best = i; best_cost = cost; }
@@ -1938,10 +1938,10 @@ static size_t workspace_bytes_uncached(int64_t M, int64_t N, int64_t K) {
 }
 
 // cost (microseconds) of an unsplit M x N region in tiles of shape t
-static float region_cost(int64_t M, int64_t N, int nslab, const TileShape& t, bool blockscale) {
+static float region_cost(int64_t M, int64_t N, int nslab, const TileShape& t, bool blockscale, bool kv_on = false) {
   const int64_t tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn);
   return (float)ceil_div(tiles, t.slots) *
-         ((float)nslab * (blockscale ? t.t_slab_block : t.t_slab_row) + tile_overhead(M, N, (int)(&t - kShapes), 1));
+         ((float)nslab * (blockscale ? t.t_slab_block : t.t_slab_row) + tile_overhead(M, N, (int)(&t - kShapes), 1, kv_on));
 }
 
 // A matmul whose tiles fill the chip a whole number of times plus a small rest wastes most of its
@@ -2060,8 +2060,7 @@ static TiledPlan make_plan(int64_t M, int64_t N, int64_t K, bool blockscale, boo
   const int nslab = (int)ceil_div(K, 128);
   plan.variant = tile_override();
   const bool free_choice = plan.variant == 0;
-  if (!plan.variant) plan.variant = pick_shape(M, N, nslab, blockscale, has_workspace && batch == 1, batch);
-  if (kv_on && plan.variant != 1) plan.variant = 3;  // the fused QKV kernels exist in the 256 x 256 and 128 x 128 shapes
+  if (!plan.variant) plan.variant = pick_shape(M, N, nslab, blockscale, has_workspace && batch == 1 && !kv_on, batch, kv_on);
   const TileShape& t = kShapes[plan.variant - 1];
   const int64_t tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn);
   // (wants_split: the shape calls for a K split, whether or not this workspace holds its partial sums -- what the
@@ -2090,12 +2089,20 @@ static TiledPlan make_plan(int64_t M, int64_t N, int64_t K, bool blockscale, boo
     plan.streamk = tuning().streamk == 2 || cost < 0.9f * other;
   }
   // the four-wave kernel against whatever the eight-wave shapes make of the matmul (one launch; a forced tile shape other
-  // than 256 x 256, a K split, a batch or the fused QKV epilogue keep it out)
-  if (batch == 1 && !kv_on && !plan.streamk && (free_choice || plan.variant == 1)) {
-    float other = plan.two.axis ? plan.two.cost : region_cost(M, N, nslab, t, blockscale);
-    if (!plan.two.axis && persist_shape(M, N, plan.variant))
+  // than 256 x 256, a K split or a batch keep it out).  The fused QKV projection has neither a K split of two launches nor
+  // two regions nor the persistent eight-wave kernel: where the plain matmul would split K, every tile is cut inside one
+  // launch by the same rule, and else the whole tiles are compared.  (Its tiles may have all four shapes: three stages instead of two
+  // on 128 x 128, 330 x 6144 x 4096 row 37.3 -> 27.7 us; 256 x 128 instead of 128 x 128, 512 x 10240 x 8192 row 65.0 -> 57.9.)
+  if (batch == 1 && !plan.streamk && (free_choice || plan.variant == 1)) {
+    float other = plan.two.axis ? plan.two.cost : region_cost(M, N, nslab, t, blockscale, kv_on);
+    if (!kv_on && !plan.two.axis && persist_shape(M, N, plan.variant))
       other = persistent_cost(tiles, t.slots, (float)nslab * (blockscale ? t.t_slab_block : t.t_slab_row) + tile_overhead(M, N, plan.variant - 1, 1));
-    plan.w4 = pick_w4(M, N, K, blockscale, other, wants_split, has_workspace ? workspace_bytes : 0, &plan.w4_split);
+    if (kv_on && has_workspace && free_choice) {
+      const TileShape& u = kShapes[pick_shape(M, N, nslab, blockscale, true) - 1];
+      if (pick_splits(ceil_div(M, u.bm) * ceil_div(N, u.bn), u.slots, nslab) > 1)
+        plan.w4 = pick_w4(M, N, K, blockscale, other, true, workspace_bytes, &plan.w4_split);
+    }
+    if (!plan.w4) plan.w4 = pick_w4(M, N, K, blockscale, other, wants_split, has_workspace ? workspace_bytes : 0, &plan.w4_split);
     if (plan.w4) plan.splits = 1;
   }
   return plan;
@@ -2161,10 +2168,27 @@ float gemm_tiled_small_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
   return 0.f;
 }
 
-// The same for a fused QKV matmul (whole tiles of the two shapes its epilogue exists in)
-float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
-  const TiledPlan plan = cached_plan(M, N, K, blockscale, false, 0, 1, true);
-  return region_cost(M, N, (int)ceil_div(K, 128), kShapes[plan.variant - 1], blockscale);
+// The same for a fused QKV matmul, of any plan (with the workspace it asks for, or without any)
+float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool has_workspace) {
+  const TiledPlan plan = cached_plan(M, N, K, blockscale, has_workspace, has_workspace ? ~(size_t)0 : 0, 1, true);
+  const int64_t slabs = ceil_div(K, 128), slots = compute_units();
+  const float stream = (float)N * (float)K / 6e6f;
+  if (plan.w4) {
+    const int64_t tiles = ceil_div(M, 32 * plan.w4) * ceil_div(N, 256);
+    if (plan.w4_split && tiles * 2 <= slots) {
+      const int unit = gemm_w4_split(M, N, K, plan.w4).unit;
+      return 10.5f + 0.646f * (float)unit + 0.886f * (float)ceil_div(slabs, unit) + 0.659f * stream;
+    }
+    return persistent_cost(tiles, (int)slots, (float)slabs * (blockscale ? kW4SlabBlock : kW4SlabRow)[plan.w4 - 4] + kW4Tile);
+  }
+  if (plan.variant == 4) return 4.9f + 0.559f * (float)slabs * (float)ceil_div(ceil_div(M, 128) * ceil_div(N, 128), 256) + 0.36f * stream;
+  return region_cost(M, N, (int)slabs, kShapes[plan.variant - 1], blockscale, true);
+}
+
+// The workspace of a fused QKV matmul's plan (its cut tiles' sums; 0: none are cut)
+size_t gemm_tiled_qkv_workspace_bytes(int64_t M, int64_t N, int64_t K, bool blockscale) {
+  const TiledPlan plan = cached_plan(M, N, K, blockscale, true, ~(size_t)0, 1, true);
+  return plan.w4 && plan.w4_split ? gemm_w4_split(M, N, K, plan.w4).bytes : 0;
 }
 
 // "256x256 x896" / "256x256 x448, K split 2" / "256x256 x768 + columns from 24576: 256x128 x256"
@@ -2267,12 +2291,16 @@ int gemm_tiled_dispatch(const GemmArgs& p_in, bool blockscale, size_t workspace_
 }
 
 static int gemm_tiled_launch(const GemmArgs& p, bool blockscale, int variant, dim3 grid, hipStream_t stream) {
-  if (p.kv_on) {  // fused QKV: the two larger shapes
+  if (p.kv_on) {
     if (blockscale) {
       if (variant == 1) return launch_tiled<256, 256, 2, 4, 2, true, true>(p, grid, stream, "gemm_qkv_block_256x256");
+      if (variant == 2) return launch_tiled<256, 128, 4, 2, 3, true, true>(p, grid, stream, "gemm_qkv_block_256x128");
+      if (variant == 4) return launch_tiled<128, 128, 2, 2, 3, true, true>(p, grid, stream, "gemm_qkv_block_128x128x3");
       return launch_tiled<128, 128, 2, 2, 2, true, true>(p, grid, stream, "gemm_qkv_block_128x128");
     }
     if (variant == 1) return launch_tiled<256, 256, 2, 4, 2, false, true>(p, grid, stream, "gemm_qkv_row_256x256");
+    if (variant == 2) return launch_tiled<256, 128, 4, 2, 3, false, true>(p, grid, stream, "gemm_qkv_row_256x128");
+    if (variant == 4) return launch_tiled<128, 128, 2, 2, 3, false, true>(p, grid, stream, "gemm_qkv_row_128x128x3");
     return launch_tiled<128, 128, 2, 2, 2, false, true>(p, grid, stream, "gemm_qkv_row_128x128");
   }
   if (variant == 1 && persist_ok(p, blockscale, grid))

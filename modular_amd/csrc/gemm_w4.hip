@@ -62,6 +62,11 @@ __device__ __forceinline__ float scalar_load_f32(const float* ptr) {
   return *(const_ptr_t)(uintptr_t)ptr;
 }
 
+__device__ __forceinline__ uint32_t scalar_load_u32(const uint32_t* ptr) {
+  typedef __attribute__((address_space(4))) const uint32_t* const_ptr_t;
+  return *(const_ptr_t)(uintptr_t)ptr;
+}
+
 // A fragment belongs in the accumulation registers: the load writes them, the MFMA reads them, nothing else touches it.
 // (Without the hint the allocator fills the ordinary registers with fragments first and then spills accumulators.)
 __device__ __forceinline__ v8i in_agprs(v8i f) {
@@ -117,7 +122,16 @@ constexpr int kW4GroupedTableBytes = (16 + 4 * kW4GroupedSlots + 8) * 4 + 4 * 96
 // rows are copied into LDS by two more copy instructions per wave, issued behind the stores of the tile before (in front
 // of the first tile: in the prologue) -- not loaded into registers in the epilogue, where waiting for such a load would
 // mean waiting for every weight copy in flight, in-order completion being what the copy waits rely on.
-template <int TM, int TN, bool BLOCKSCALE, int PROBE, int GROUPED = 0>
+//
+// KV: the fused QKV projection -- the reference's bf16 roundings in the epilogue, columns from q_dim on go to the rows' pages of
+// the cache.  Where a row's page lies is looked up by each wave for its own rows before the tile's slab loop and parked in
+// LDS: for the usual tile, whose rows belong to one sequence, with scalar loads alone, which wait for none of the copies in
+// flight.  The stores to Q are issued for every column (out of range, i.e. nothing, beyond q_dim), so the counts of the waits
+// hold; those to the pages come on top of them, which only makes a wait stricter.
+// Bound like the plain kernel, by the matrix pipe; the projection ran on the one-tile-per-block kernels before (quantiser
+// included, block scaling): 777 x 10240 x 8192 102.7 -> 72.5 us, 2011 x 10240 x 8192 207 -> 157, 3000 x 6144 x 4096 101 -> 80,
+// 4096 x 10240 x 8192 381 -> 299, 200 x 10240 x 8192 (every tile cut) 66 -> 38; the plain linear of those sizes: 64, 149, 72, 287, 35.
+template <int TM, int TN, bool BLOCKSCALE, int PROBE, int GROUPED = 0, bool KV = false>
 __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
   constexpr int WM = TM * 16, WN = TN * 16, BM = 2 * WM, BN = 2 * WN;
   constexpr int IA = BM / 32, IB = BN / 32;                  // copy instructions per wave and slab (8 rows each)
@@ -139,6 +153,7 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
   static_assert(IB % 2 == 0, "the weight copies go out in two halves");
 
   static_assert(!GROUPED || PROBE == 0, "the probe runs the dense form");
+  static_assert(!KV || (PROBE == 0 && !GROUPED), "the fused QKV projection is the dense form");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
@@ -391,7 +406,7 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
   // ---- where C goes: through a 2 KB side buffer per wave, 16 rows x 64 columns at a time, so that a store instruction
   // writes 8 rows x one whole 128-byte line
   uint8_t* wbuf = smem + SIDE_BASE + wave * SIDE_BYTES;
-  const __amdgpu_buffer_rsrc_t c_rsrc = t2_rsrc(p.c, t2_clamp_u32(((int64_t)(p.M - 1) * p.ldc + p.N) * 2));
+  const __amdgpu_buffer_rsrc_t c_rsrc = t2_rsrc(p.c, t2_clamp_u32(((int64_t)(p.M - 1) * p.ldc + (KV ? p.kv.q_dim : p.N)) * 2));
   const uint32_t c_row_bytes = (uint32_t)p.ldc * 2u;
 
   // Where tile number t lies.  Grouped: the tiles are numbered slot by slot, in a slot column by column, in a column
@@ -438,6 +453,54 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
       // (under the execution mask: a lane whose offset is merely out of range would still write a zero, into the next
       // wave's entries)
       if (l < 32) __builtin_amdgcn_raw_ptr_buffer_load_lds(i_rsrc, (lds_ptr_t)(idx_lds + 64), 4, (uint32_t)l * 4u, at + 256u, 0, 0);
+    }
+  };
+  // KV: row_tab[r] = the offset of the cache row of row row0 + r (the wave's part of the tile), -1: none
+  [[maybe_unused]] int64_t* const row_tab = reinterpret_cast<int64_t*>(smem + SIDE_BASE + 4 * SIDE_BYTES) + wave * WM;
+  [[maybe_unused]] auto look_up_rows = [&](int row0) {
+    const KvStore& kv = p.kv;
+    const int l = lane_here();
+    const int last = min(row0 + WM, p.M) - 1;
+    auto sequence_of = [&](int m) {  // the last sequence whose first row is <= m
+      int low = 0, high = kv.batch;
+      while (high - low > 1) {
+        const int mid = (low + high) >> 1;
+        if ((int64_t)m >= (int64_t)scalar_load_u32(kv.row_offsets + mid)) low = mid; else high = mid;
+      }
+      return low;
+    };
+    const int b = row0 <= last ? sequence_of(row0) : 0;
+    if (row0 > last || (kv.page_size >= WM && sequence_of(last) == b)) {
+      uint32_t slot0 = 0, blk[2] = {0xffffffffu, 0xffffffffu};
+      if (row0 <= last) {
+        const uint32_t token = (uint32_t)row0 - scalar_load_u32(kv.row_offsets + b) + scalar_load_u32(kv.cache_lengths + b);
+        const uint32_t page = token / (uint32_t)kv.page_size;
+        slot0 = token - page * (uint32_t)kv.page_size;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          if ((int64_t)page + i < kv.lut_ld) blk[i] = scalar_load_u32(kv.lookup_table + (int64_t)b * kv.lut_ld + page + i);
+      }
+#pragma unroll
+      for (int j = 0; j < (WM + 63) / 64; ++j) {
+        const int r = j * 64 + l;
+        const bool second = slot0 + (uint32_t)r >= (uint32_t)kv.page_size;
+        const uint32_t slot_r = slot0 + (uint32_t)r - (second ? (uint32_t)kv.page_size : 0u);
+        const int64_t block = second ? blk[1] : blk[0];
+        if (r < WM) row_tab[r] = row0 + r <= last && block < kv.num_blocks ? block * kv.block_stride + (int64_t)slot_r * kv.row_elems : -1;
+      }
+    } else {
+      constexpr int R = (WM + 63) / 64;
+      int64_t rows[R], off[R];
+      bool live[R];
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        rows[j] = row0 + j * 64 + l;
+        live[j] = j * 64 + l < WM && rows[j] <= last;
+      }
+      kv_row_offsets<R>(kv, rows, live, off);
+#pragma unroll
+      for (int j = 0; j < R; ++j)
+        if (j * 64 + l < WM) row_tab[j * 64 + l] = off[j];
     }
   };
   // ---- prologue: slabs 0 and 1 of the first tile
@@ -524,6 +587,9 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
     const SlabAt next0 = slab_at(next_at, next_job.s0, has_next ? 0u : 0x80000000u);
     const uint32_t next_bs0 = next_at.bs0 + (uint32_t)(bs_block(tn2) * p.b_scales_ld + next_job.s0);
     const int job_end = job.s1;
+    if constexpr (KV) {
+      if (tn * BN + wn * WN + WN > p.kv.q_dim && tn * BN + wn * WN < p.N) look_up_rows(cur_at.row0 + wm * WM);
+    }
 
     v4f acc[TM][TN];
 #pragma unroll
@@ -724,6 +790,18 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
     // (row scaling: every scale of the tile is loaded before the first store, so that no later wait for a load also
     // waits for the stores in front of it)
     float b_s[TN / 2][8], a_s_all[TM];
+    [[maybe_unused]] uint32_t bias[TN / 2][4];  // (two bf16 a word)
+    if constexpr (KV) {
+      if (p.kv.bias) {
+#pragma unroll
+        for (int q = 0; q < TN / 2; ++q)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int n = min(tn * BN + wn * WN + q * 32 + lq * 8 + 2 * i, p.N - 2);
+            bias[q][i] = (uint32_t)p.kv.bias[n] | ((uint32_t)p.kv.bias[n + 1] << 16);
+          }
+      }
+    }
     if constexpr (!BLOCKSCALE) {
 #pragma unroll
       for (int q = 0; q < TN / 2; ++q)
@@ -737,6 +815,14 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
         if (m >= p.M) m = p.M - 1;
         a_s_all[mt] = scale_at(p.a_scales, m * p.a_scale_stride, p.scales_dtype);
       }
+      if constexpr (KV) {  // (this op's scales are rounded to bf16)
+#pragma unroll
+        for (int q = 0; q < TN / 2; ++q)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) b_s[q][i] = bf16_round(b_s[q][i]);
+#pragma unroll
+        for (int mt = 0; mt < TM; ++mt) a_s_all[mt] = bf16_round(a_s_all[mt]);
+      }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     const uint32_t c_tile = ((uint32_t)(cur_at.row0 + wm * WM) * (uint32_t)p.ldc + (uint32_t)(tn * BN + wn * WN)) * 2u;
@@ -749,7 +835,7 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
     // the descriptor's range, i.e. nothing -- every store is still issued, so the counts of the waits stay exact)
     uint32_t c_lane_h[TN / 4];
 #pragma unroll
-    for (int h = 0; h < TN / 4; ++h) c_lane_h[h] = tn * BN + wn * WN + h * 64 + cc * 8 < p.N ? c_lane : 0x80000000u;
+    for (int h = 0; h < TN / 4; ++h) c_lane_h[h] = tn * BN + wn * WN + h * 64 + cc * 8 < (KV ? p.kv.q_dim : p.N) ? c_lane : 0x80000000u;
     // one step = 16 rows x 64 columns of the wave's part: two pairs of fragments converted and written to the side buffer ...
     auto stage = [&](int mt, int h) {
       float a_s = 1.f;
@@ -758,6 +844,25 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
       for (int qq = 0; qq < 2; ++qq) {
         const int q = 2 * h + qq;
         v4f lo = acc[mt][2 * q], hi = acc[mt][2 * q + 1];
+        if constexpr (KV) {
+          // the sum to bf16, the scales' product to bf16, their product to bf16, then the bias in bf16 (see tile_body)
+          const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+          uint32_t w[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            w[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
+            if constexpr (!BLOCKSCALE) {
+              const uint32_t sc = pack_bf16x2(a_s * b_s[q][2 * i], a_s * b_s[q][2 * i + 1]);
+              w[i] = pack_bf16x2(__uint_as_float(w[i] << 16) * __uint_as_float(sc << 16),
+                                 __uint_as_float(w[i] & 0xffff0000u) * __uint_as_float(sc & 0xffff0000u));
+            }
+            if (p.kv.bias)
+              w[i] = pack_bf16x2(__uint_as_float(w[i] << 16) + __uint_as_float(bias[q][i] << 16),
+                                 __uint_as_float(w[i] & 0xffff0000u) + __uint_as_float(bias[q][i] & 0xffff0000u));
+          }
+          *reinterpret_cast<v4u_t*>(wbuf + lm_e * 128 + (((qq * 4 + lq_e) ^ (lm_e & 7)) * 16)) = v4u_t{w[0], w[1], w[2], w[3]};
+          continue;
+        }
         if constexpr (!BLOCKSCALE) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
@@ -800,6 +905,16 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
           buffer_store_b128_guarded<2>(v[i], c_rsrc, dst[i] | (c_lane_h[h] & 0x80000000u), (uint32_t)(tn * BN + wn * WN) * 2u + (uint32_t)h * 128u);
         else
           buffer_store_b128_guarded<2>(v[i], c_rsrc_tile, c_lane_h[h], c_tile + (uint32_t)(mt * 16 + i * 8) * c_row_bytes + (uint32_t)h * 128u);
+      }
+      if constexpr (KV) {
+        if (tn * BN + wn * WN + h * 64 + 64 > p.kv.q_dim) {
+          const int n = tn * BN + wn * WN + h * 64 + cc * 8;
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const int64_t off = row_tab[mt * 16 + i * 8 + rr];
+            if (n >= p.kv.q_dim && n < p.N && off >= 0) *reinterpret_cast<v4u_t*>(kv_dst(p.kv, nullptr, 0, 0, off, n)) = v[i];
+          }
+        }
       }
     };
     if (GROUPED || job.kind == WHOLE) {
@@ -851,6 +966,12 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   w4_body<TM, TN, BLOCKSCALE, PROBE>(p, smem);
 }
 
+template <int TM, int TN, bool BLOCKSCALE>
+__global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_w4_qkv_kernel(GemmArgs p) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  w4_body<TM, TN, BLOCKSCALE, 0, 0, true>(p, smem);
+}
+
 template <int TM, int TN, bool BLOCKSCALE, bool SCATTER>
 __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_w4_grouped_kernel(GemmArgs p) {
   static_assert(BLOCKSCALE || !SCATTER, "the row index on C is the block-scaled MoE layer's");
@@ -868,7 +989,7 @@ constexpr int w4_lds_bytes() {
 bool gemm_w4_ok(const GemmArgs& p, bool blockscale) {
   if (p.M <= 0 || p.N <= 0 || p.N % 8 != 0 || p.K < 512 || p.K % 256 != 0) return false;
   const int64_t nslab = p.K / 128;
-  if (p.kv_on || p.splits > 1) return false;
+  if (p.splits > 1) return false;
   if (p.c_dtype != MAXFP8_BF16 || !p.c_vec8_ok) return false;
   const int64_t lim = 0x7ff00000ll;
   const int64_t rows = ceil_div(p.M, 192) * 192 + 192;
@@ -878,12 +999,14 @@ bool gemm_w4_ok(const GemmArgs& p, bool blockscale) {
   return true;
 }
 
-template <int TM, bool BLOCKSCALE, int PROBE>
+template <int TM, bool BLOCKSCALE, int PROBE, bool KV = false>
 static int launch_w4(const GemmArgs& p, unsigned blocks, hipStream_t stream, const char* name) {
   static PerDeviceFlag attr_done;
-  constexpr int lds = w4_lds_bytes<TM, 8, BLOCKSCALE>();
+  constexpr int lds = w4_lds_bytes<TM, 8, BLOCKSCALE>() + (KV ? 4 * TM * 16 * 8 : 0);  // (the cache rows of each wave's rows)
   static_assert(lds <= 160 * 1024, "one block's LDS");
-  auto kern = gemm_w4_kernel<TM, 8, BLOCKSCALE, PROBE>;
+  void (*kern)(GemmArgs);
+  if constexpr (KV) kern = gemm_w4_qkv_kernel<TM, 8, BLOCKSCALE>;
+  else kern = gemm_w4_kernel<TM, 8, BLOCKSCALE, PROBE>;
   bool& done = attr_done.here();
   if (!done) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -950,6 +1073,11 @@ int gemm_w4_launch(const GemmArgs& p_in, bool blockscale, int tm, bool split, hi
       p.streamk_slot = status == hipStreamCaptureStatusNone ? (int)(issued.fetch_add(1, std::memory_order_relaxed) % (kW4FlagSets / 2))
                                                             : kW4FlagSets / 2 + (int)(recorded.fetch_add(1, std::memory_order_relaxed) % (kW4FlagSets / 2));
     }
+  }
+  if (p.kv_on) {
+    if (tm == 4) return blockscale ? launch_w4<4, true, 0, true>(p, blocks, stream, "gemm_w4_qkv_block_128x256") : launch_w4<4, false, 0, true>(p, blocks, stream, "gemm_w4_qkv_row_128x256");
+    if (tm == 5) return blockscale ? launch_w4<5, true, 0, true>(p, blocks, stream, "gemm_w4_qkv_block_160x256") : launch_w4<5, false, 0, true>(p, blocks, stream, "gemm_w4_qkv_row_160x256");
+    return blockscale ? launch_w4<6, true, 0, true>(p, blocks, stream, "gemm_w4_qkv_block_192x256") : launch_w4<6, false, 0, true>(p, blocks, stream, "gemm_w4_qkv_row_192x256");
   }
   if (tm == 4)
     return blockscale ? launch_w4<4, true, 0>(p, blocks, stream, "gemm_w4_block_128x256") : launch_w4<4, false, 0>(p, blocks, stream, "gemm_w4_row_128x256");
