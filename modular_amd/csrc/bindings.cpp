@@ -75,13 +75,17 @@ bool linear_ok(const at::Tensor& x, const at::Tensor& w, const at::Tensor& s, in
     PyErr_Format(PyExc_TypeError, "%s takes %d arguments, got %zd", __func__, (n), nargs);  \
     return nullptr;                                                                         \
   }
-#define GUARDED(...)                                    \
-  try {                                                 \
-    __VA_ARGS__                                         \
-  } catch (const std::exception& e) {                   \
-    PyErr_SetString(PyExc_RuntimeError, e.what());      \
-    return nullptr;                                     \
+// a C++ exception (a tensor without memory of its own is asked for its pointer, an allocation fails) becomes Python's RuntimeError
+using Function = PyObject*(PyObject*, PyObject* const*, Py_ssize_t);
+template <Function* F>
+PyObject* guarded(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  try {
+    return F(self, args, nargs);
+  } catch (const std::exception& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
   }
+}
 
 // linear(x, w, w_scales, granularity, scale_ub) -> y
 PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -93,12 +97,10 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!x || !w || !s || !linear_ok(*x, *w, *s, granularity)) Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
-  GUARDED(
-    int status;
-    at::Tensor y = linear_of(*x, *w, *s, granularity, ub, stream, &status);
-    if (status != MAXFP8_OK) return raise(status);
-    return THPVariable_Wrap(std::move(y));
-  )
+  int status;
+  at::Tensor y = linear_of(*x, *w, *s, granularity, ub, stream, &status);
+  if (status != MAXFP8_OK) return raise(status);
+  return THPVariable_Wrap(std::move(y));
 }
 
 // linear_static(x, w, input_scale, weight_scale) -> y; the scales are tensors of one float on the CPU
@@ -110,18 +112,16 @@ PyObject* linear_static(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
-  GUARDED(
-    const int64_t M = x->size(0), K = x->size(1), N = w->size(0);
-    at::Tensor y = at::empty({M, N}, x->options());
-    const size_t need = maxfp8_linear_workspace_bytes(M, N, K, MAXFP8_GRAN_TENSOR);
-    at::Tensor ws;
-    if (need) ws = bytes_on(*x, need);
-    const int status = maxfp8_linear_static_scaled_fp8(y.data_ptr(), x->data_ptr(), w->data_ptr(), M, N, K, row_stride(*x), row_stride(*w), N,
-                                                       *static_cast<const float*>(si->data_ptr()), *static_cast<const float*>(sw->data_ptr()),
-                                                       need ? ws.data_ptr() : nullptr, need, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    return THPVariable_Wrap(std::move(y));
-  )
+  const int64_t M = x->size(0), K = x->size(1), N = w->size(0);
+  at::Tensor y = at::empty({M, N}, x->options());
+  const size_t need = maxfp8_linear_workspace_bytes(M, N, K, MAXFP8_GRAN_TENSOR);
+  at::Tensor ws;
+  if (need) ws = bytes_on(*x, need);
+  const int status = maxfp8_linear_static_scaled_fp8(y.data_ptr(), x->data_ptr(), w->data_ptr(), M, N, K, row_stride(*x), row_stride(*w), N,
+                                                     *static_cast<const float*>(si->data_ptr()), *static_cast<const float*>(sw->data_ptr()),
+                                                     need ? ws.data_ptr() : nullptr, need, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  return THPVariable_Wrap(std::move(y));
 }
 
 PyObject* pair(at::Tensor a, at::Tensor b) {
@@ -146,14 +146,12 @@ PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (group <= 0 || x->size(1) % group != 0) Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
-  GUARDED(
-    const int64_t M = x->size(0), K = x->size(1), ld = padded ? (M + 3) / 4 * 4 : M;
-    at::Tensor q = at::empty({M, K}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({K / group, ld}, x->options().dtype(at::kFloat));
-    const int status = maxfp8_quantize_dynamic_scaled_fp8(q.data_ptr(), s.data_ptr(), x->data_ptr(), M, K, row_stride(*x), K, group, ld, MAXFP8_BF16,
-                                                          MAXFP8_F32, ub, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    return pair(std::move(q), std::move(s));
-  )
+  const int64_t M = x->size(0), K = x->size(1), ld = padded ? (M + 3) / 4 * 4 : M;
+  at::Tensor q = at::empty({M, K}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({K / group, ld}, x->options().dtype(at::kFloat));
+  const int status = maxfp8_quantize_dynamic_scaled_fp8(q.data_ptr(), s.data_ptr(), x->data_ptr(), M, K, row_stride(*x), K, group, ld, MAXFP8_BF16,
+                                                        MAXFP8_F32, ub, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  return pair(std::move(q), std::move(s));
 }
 
 // rms_norm_quantize(x, gamma, epsilon, weight_offset, scale_ub) -> (q, scales [1, rows])
@@ -166,14 +164,12 @@ PyObject* rms_norm_quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
-  GUARDED(
-    const int64_t M = x->size(0), K = x->size(1);
-    at::Tensor q = at::empty({M, K}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({1, M}, x->options().dtype(at::kFloat));
-    const int status = maxfp8_rms_norm_fused_quantize_dynamic_scaled_fp8(q.data_ptr(), s.data_ptr(), x->data_ptr(), g->data_ptr(), M, K, row_stride(*x),
-                                                                         K, MAXFP8_BF16, MAXFP8_F32, eps, offset, ub, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    return pair(std::move(q), std::move(s));
-  )
+  const int64_t M = x->size(0), K = x->size(1);
+  at::Tensor q = at::empty({M, K}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({1, M}, x->options().dtype(at::kFloat));
+  const int status = maxfp8_rms_norm_fused_quantize_dynamic_scaled_fp8(q.data_ptr(), s.data_ptr(), x->data_ptr(), g->data_ptr(), M, K, row_stride(*x),
+                                                                       K, MAXFP8_BF16, MAXFP8_F32, eps, offset, ub, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  return pair(std::move(q), std::move(s));
 }
 
 // matmul(a, b, a_scales, b_scales, granularity of b) -> c [M, N] bf16; float32 block or per-token x per-channel scales
@@ -190,19 +186,17 @@ PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (sa->size(0) != (block ? a->size(1) / 128 : 1)) Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*a, &stream)) return nullptr;
-  GUARDED(
-    const int64_t M = a->size(0), K = a->size(1), N = b->size(0);
-    at::Tensor c = at::empty({M, N}, a->options().dtype(at::kBFloat16));
-    const size_t need = maxfp8_matmul_auto_workspace_bytes(M, N, K);
-    at::Tensor ws;
-    if (need) ws = bytes_on(*a, need);
-    const int status = maxfp8_matmul_dynamic_scaled_fp8(
-        c.data_ptr(), a->data_ptr(), b->data_ptr(), sa->data_ptr(), sb->data_ptr(), M, N, K, row_stride(*a), row_stride(*b), N,
-        block ? MAXFP8_GRAN_BLOCK : MAXFP8_GRAN_COLWISE, granularity, block ? 1 : -1, block ? 128 : -1, block ? 128 : -1, row_stride(*sa), sb->size(1),
-        MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO, need ? ws.data_ptr() : nullptr, need, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    return THPVariable_Wrap(std::move(c));
-  )
+  const int64_t M = a->size(0), K = a->size(1), N = b->size(0);
+  at::Tensor c = at::empty({M, N}, a->options().dtype(at::kBFloat16));
+  const size_t need = maxfp8_matmul_auto_workspace_bytes(M, N, K);
+  at::Tensor ws;
+  if (need) ws = bytes_on(*a, need);
+  const int status = maxfp8_matmul_dynamic_scaled_fp8(
+      c.data_ptr(), a->data_ptr(), b->data_ptr(), sa->data_ptr(), sb->data_ptr(), M, N, K, row_stride(*a), row_stride(*b), N,
+      block ? MAXFP8_GRAN_BLOCK : MAXFP8_GRAN_COLWISE, granularity, block ? 1 : -1, block ? 128 : -1, block ? 128 : -1, row_stride(*sa), sb->size(1),
+      MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO, need ? ws.data_ptr() : nullptr, need, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  return THPVariable_Wrap(std::move(c));
 }
 
 // batched_quantize(x [B, M, K] with contiguous channels, group, scale_ub) -> (q [B, M, K], scales [B, K / group, M_pad])
@@ -217,15 +211,13 @@ PyObject* batched_quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
-  GUARDED(
-    const int64_t B = x->size(0), M = x->size(1), K = x->size(2), ld = (M + 3) / 4 * 4;
-    at::Tensor q = at::empty({B, M, K}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({B, K / group, ld}, x->options().dtype(at::kFloat));
-    const int status = maxfp8_batched_quantize_dynamic_scaled_fp8(
-        q.data_ptr(), s.data_ptr(), x->data_ptr(), B, M, K, B > 1 ? x->stride(0) : M * K, M > 1 ? x->stride(1) : K, M * K, K, group, (K / group) * ld, ld,
-        MAXFP8_BF16, MAXFP8_F32, ub, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    return pair(std::move(q), std::move(s));
-  )
+  const int64_t B = x->size(0), M = x->size(1), K = x->size(2), ld = (M + 3) / 4 * 4;
+  at::Tensor q = at::empty({B, M, K}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({B, K / group, ld}, x->options().dtype(at::kFloat));
+  const int status = maxfp8_batched_quantize_dynamic_scaled_fp8(
+      q.data_ptr(), s.data_ptr(), x->data_ptr(), B, M, K, B > 1 ? x->stride(0) : M * K, M > 1 ? x->stride(1) : K, M * K, K, group, (K / group) * ld, ld,
+      MAXFP8_BF16, MAXFP8_F32, ub, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  return pair(std::move(q), std::move(s));
 }
 
 // batched_matmul(a, b, a_scales, b_scales) -> c [B, M, N] bf16; contiguous operands, block scaling
@@ -240,15 +232,13 @@ PyObject* batched_matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*a, &stream)) return nullptr;
-  GUARDED(
-    at::Tensor c = at::empty({B, M, N}, a->options().dtype(at::kBFloat16));
-    const int64_t ld = sa->size(2);
-    const int status = maxfp8_batched_matmul_dynamic_scaled_fp8(
-        c.data_ptr(), a->data_ptr(), b->data_ptr(), sa->data_ptr(), sb->data_ptr(), B, M, N, K, M * K, K, N * K, K, M * N, N, 1, 128, 128, kb * ld, ld,
-        nb * kb, kb, MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    return THPVariable_Wrap(std::move(c));
-  )
+  at::Tensor c = at::empty({B, M, N}, a->options().dtype(at::kBFloat16));
+  const int64_t ld = sa->size(2);
+  const int status = maxfp8_batched_matmul_dynamic_scaled_fp8(
+      c.data_ptr(), a->data_ptr(), b->data_ptr(), sa->data_ptr(), sb->data_ptr(), B, M, N, K, M * K, K, N * K, K, M * N, N, 1, 128, 128, kb * ld, ld,
+      nb * kb, kb, MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  return THPVariable_Wrap(std::move(c));
 }
 
 // silu(gate) * up of every row, rounded twice to bf16, and the down linear: see MLP
@@ -270,29 +260,27 @@ PyObject* mlp(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
-  GUARDED(
-    const int64_t M = x->size(0), F = d->size(1), H = d->size(0);
-    int status;
-    at::Tensor both = linear_of(*x, *gu, *sgu, granularity, ub, stream, &status);
-    if (status != MAXFP8_OK) return raise(status);
-    const bool block = granularity == MAXFP8_GRAN_BLOCK;
-    const int64_t group = block ? 128 : F, ld = block ? (M + 3) / 4 * 4 : M;
-    // one buffer: the quantised product, its scales, the down matmul's partial sums
-    const size_t at_scales = ((size_t)M * (size_t)F + 255) / 256 * 256, at_partial = at_scales + ((size_t)(F / group) * (size_t)ld * 4 + 255) / 256 * 256;
-    const size_t partial = maxfp8_matmul_auto_workspace_bytes(M, H, F);
-    at::Tensor ws = bytes_on(*x, at_partial + partial);
-    uint8_t* q = static_cast<uint8_t*>(ws.data_ptr());
-    status = maxfp8_silu_quantize_dynamic_scaled_fp8(q, q + at_scales, both.data_ptr(), static_cast<const uint32_t*>(rows->data_ptr()), 2, M, F, 2 * F, F,
-                                                     group, ld, MAXFP8_BF16, 1, ub, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    at::Tensor y = at::empty({M, H}, x->options());
-    status = maxfp8_matmul_dynamic_scaled_fp8(y.data_ptr(), q, d->data_ptr(), q + at_scales, sd->data_ptr(), M, H, F, F, row_stride(*d), H,
-                                              block ? MAXFP8_GRAN_BLOCK : MAXFP8_GRAN_COLWISE, granularity, block ? 1 : -1, block ? 128 : -1,
-                                              block ? 128 : -1, ld, sd->size(1), MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO,
-                                              partial ? q + at_partial : nullptr, partial, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    return THPVariable_Wrap(std::move(y));
-  )
+  const int64_t M = x->size(0), F = d->size(1), H = d->size(0);
+  int status;
+  at::Tensor both = linear_of(*x, *gu, *sgu, granularity, ub, stream, &status);
+  if (status != MAXFP8_OK) return raise(status);
+  const bool block = granularity == MAXFP8_GRAN_BLOCK;
+  const int64_t group = block ? 128 : F, ld = block ? (M + 3) / 4 * 4 : M;
+  // one buffer: the quantised product, its scales, the down matmul's partial sums
+  const size_t at_scales = ((size_t)M * (size_t)F + 255) / 256 * 256, at_partial = at_scales + ((size_t)(F / group) * (size_t)ld * 4 + 255) / 256 * 256;
+  const size_t partial = maxfp8_matmul_auto_workspace_bytes(M, H, F);
+  at::Tensor ws = bytes_on(*x, at_partial + partial);
+  uint8_t* q = static_cast<uint8_t*>(ws.data_ptr());
+  status = maxfp8_silu_quantize_dynamic_scaled_fp8(q, q + at_scales, both.data_ptr(), static_cast<const uint32_t*>(rows->data_ptr()), 2, M, F, 2 * F, F,
+                                                   group, ld, MAXFP8_BF16, 1, ub, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  at::Tensor y = at::empty({M, H}, x->options());
+  status = maxfp8_matmul_dynamic_scaled_fp8(y.data_ptr(), q, d->data_ptr(), q + at_scales, sd->data_ptr(), M, H, F, F, row_stride(*d), H,
+                                            block ? MAXFP8_GRAN_BLOCK : MAXFP8_GRAN_COLWISE, granularity, block ? 1 : -1, block ? 128 : -1,
+                                            block ? 128 : -1, ld, sd->size(1), MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO,
+                                            partial ? q + at_partial : nullptr, partial, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  return THPVariable_Wrap(std::move(y));
 }
 
 // qkv_linear(x, wqkv, w_scales, granularity, scale_ub, row_offsets, kv_blocks, cache_lengths, lookup_table, bias or None, layer, q_dim) -> q
@@ -316,19 +304,17 @@ PyObject* qkv_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
-  GUARDED(
-    at::Tensor q = at::empty({T, q_dim}, x->options());
-    const size_t need = maxfp8_linear_qkv_workspace_bytes(T, N, K, granularity);
-    at::Tensor ws;
-    if (need) ws = bytes_on(*x, need);
-    const int status = maxfp8_linear_qkv_ragged_paged_scale(
-        q.data_ptr(), x->data_ptr(), row_stride(*x), static_cast<const uint32_t*>(offsets->data_ptr()), w->data_ptr(), s->data_ptr(), blocks->data_ptr(),
-        static_cast<const uint32_t*>(lengths->data_ptr()), static_cast<const uint32_t*>(table->data_ptr()), bias ? bias->data_ptr() : nullptr, T, N, K,
-        q_dim, batch, blocks->size(0), blocks->size(1), blocks->size(2), layer, blocks->size(3), blocks->size(4), blocks->size(5), table->size(1),
-        granularity, s->size(1), ub, need ? ws.data_ptr() : nullptr, need, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    return THPVariable_Wrap(std::move(q));
-  )
+  at::Tensor q = at::empty({T, q_dim}, x->options());
+  const size_t need = maxfp8_linear_qkv_workspace_bytes(T, N, K, granularity);
+  at::Tensor ws;
+  if (need) ws = bytes_on(*x, need);
+  const int status = maxfp8_linear_qkv_ragged_paged_scale(
+      q.data_ptr(), x->data_ptr(), row_stride(*x), static_cast<const uint32_t*>(offsets->data_ptr()), w->data_ptr(), s->data_ptr(), blocks->data_ptr(),
+      static_cast<const uint32_t*>(lengths->data_ptr()), static_cast<const uint32_t*>(table->data_ptr()), bias ? bias->data_ptr() : nullptr, T, N, K,
+      q_dim, batch, blocks->size(0), blocks->size(1), blocks->size(2), layer, blocks->size(3), blocks->size(4), blocks->size(5), table->size(1),
+      granularity, s->size(1), ub, need ? ws.data_ptr() : nullptr, need, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  return THPVariable_Wrap(std::move(q));
 }
 
 // moe_experts(x, router [seq, k] int32, gate_up [E, 2I, H], its scales, down [E, H, I], its scales, scale_ub) -> [seq, k, H]
@@ -348,38 +334,36 @@ PyObject* moe_experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
-  GUARDED(
-    // the grouping: order [T], restore [T], starts [E + 1], expert ids [E], usage [2]
-    at::Tensor idx = at::empty({2 * T + 2 * E + 8}, x->options().dtype(at::kInt));
-    uint32_t* order = static_cast<uint32_t*>(idx.data_ptr());
-    uint32_t *restore = order + T, *start = restore + T, *ids = start + E + 1, *usage = ids + E;
-    int status = maxfp8_moe_create_indices(order, start, restore, reinterpret_cast<int32_t*>(ids), usage, r->data_ptr(), T, E, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    // every token quantised once and stored to its k rows of the grouped order
-    at::Tensor q = at::empty({T, H}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({H / 128, ld}, x->options().dtype(at::kFloat));
-    status = maxfp8_quantize_dynamic_scaled_fp8_scatter(q.data_ptr(), s.data_ptr(), x->data_ptr(), restore, k, seq, H, T, row_stride(*x), H, 128, ld,
-                                                        MAXFP8_BF16, MAXFP8_F32, ub, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    // (the bounds of the two host scalars: every row on one expert, every expert in use)
-    at::Tensor both = at::empty({T, 2 * F}, x->options());
-    status = maxfp8_grouped_matmul_dynamic_scaled_fp8(both.data_ptr(), q.data_ptr(), gu->data_ptr(), s.data_ptr(), sgu->data_ptr(), start,
-                                                      reinterpret_cast<const int32_t*>(ids), T, 2 * F, H, E, T, E, ld, MAXFP8_BF16, MAXFP8_F32,
-                                                      MAXFP8_ALGO_AUTO, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    at::Tensor hq = at::empty({T, F}, x->options().dtype(at::kFloat8_e4m3fn)), hs = at::empty({F / 128, ld}, x->options().dtype(at::kFloat));
-    status = maxfp8_silu_quantize_dynamic_scaled_fp8(hq.data_ptr(), hs.data_ptr(), both.data_ptr(), start, E + 1, T, F, 2 * F, F, 128, ld, MAXFP8_BF16, 0,
-                                                     ub, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    at::Tensor y = at::empty({seq, k, H}, x->options());
-    status = maxfp8_grouped_matmul_dynamic_scaled_fp8_scatter(y.data_ptr(), order, hq.data_ptr(), d->data_ptr(), hs.data_ptr(), sd->data_ptr(), start,
-                                                              reinterpret_cast<const int32_t*>(ids), T, H, F, E, T, E, ld, MAXFP8_BF16, MAXFP8_F32,
-                                                              MAXFP8_ALGO_AUTO, stream);
-    if (status != MAXFP8_OK) return raise(status);
-    return THPVariable_Wrap(std::move(y));
-  )
+  // the grouping: order [T], restore [T], starts [E + 1], expert ids [E], usage [2]
+  at::Tensor idx = at::empty({2 * T + 2 * E + 8}, x->options().dtype(at::kInt));
+  uint32_t* order = static_cast<uint32_t*>(idx.data_ptr());
+  uint32_t *restore = order + T, *start = restore + T, *ids = start + E + 1, *usage = ids + E;
+  int status = maxfp8_moe_create_indices(order, start, restore, reinterpret_cast<int32_t*>(ids), usage, r->data_ptr(), T, E, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  // every token quantised once and stored to its k rows of the grouped order
+  at::Tensor q = at::empty({T, H}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({H / 128, ld}, x->options().dtype(at::kFloat));
+  status = maxfp8_quantize_dynamic_scaled_fp8_scatter(q.data_ptr(), s.data_ptr(), x->data_ptr(), restore, k, seq, H, T, row_stride(*x), H, 128, ld,
+                                                      MAXFP8_BF16, MAXFP8_F32, ub, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  // (the bounds of the two host scalars: every row on one expert, every expert in use)
+  at::Tensor both = at::empty({T, 2 * F}, x->options());
+  status = maxfp8_grouped_matmul_dynamic_scaled_fp8(both.data_ptr(), q.data_ptr(), gu->data_ptr(), s.data_ptr(), sgu->data_ptr(), start,
+                                                    reinterpret_cast<const int32_t*>(ids), T, 2 * F, H, E, T, E, ld, MAXFP8_BF16, MAXFP8_F32,
+                                                    MAXFP8_ALGO_AUTO, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  at::Tensor hq = at::empty({T, F}, x->options().dtype(at::kFloat8_e4m3fn)), hs = at::empty({F / 128, ld}, x->options().dtype(at::kFloat));
+  status = maxfp8_silu_quantize_dynamic_scaled_fp8(hq.data_ptr(), hs.data_ptr(), both.data_ptr(), start, E + 1, T, F, 2 * F, F, 128, ld, MAXFP8_BF16, 0,
+                                                   ub, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  at::Tensor y = at::empty({seq, k, H}, x->options());
+  status = maxfp8_grouped_matmul_dynamic_scaled_fp8_scatter(y.data_ptr(), order, hq.data_ptr(), d->data_ptr(), hs.data_ptr(), sd->data_ptr(), start,
+                                                            reinterpret_cast<const int32_t*>(ids), T, H, F, E, T, E, ld, MAXFP8_BF16, MAXFP8_F32,
+                                                            MAXFP8_ALGO_AUTO, stream);
+  if (status != MAXFP8_OK) return raise(status);
+  return THPVariable_Wrap(std::move(y));
 }
 
-#define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(name)), METH_FASTCALL, nullptr}
+#define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&guarded<name>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {METHOD(linear), METHOD(linear_static), METHOD(quantize), METHOD(rms_norm_quantize), METHOD(matmul),
                          METHOD(batched_quantize), METHOD(batched_matmul), METHOD(mlp), METHOD(qkv_linear), METHOD(moe_experts),
                          {nullptr, nullptr, 0, nullptr}};
