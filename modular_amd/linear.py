@@ -161,6 +161,13 @@ class MLP(torch.nn.Module):
                 and cfg.input_scale.block_size == (1, 128) and self.down_proj.bias is None
                 and self.feed_forward_length % 128 == 0)
 
+    def _down_is_plain(self) -> bool:
+        """Whether `down_proj` is what the steps without a call of it compute: a program may have given the block another
+        module in its place, a bias, a static scale, another config or hooks."""
+        down = self.down_proj
+        return (type(down) is Linear and down.bias is None and down.input_scale is None
+                and (down.quant_config is self.quant_config or down.quant_config == self.quant_config) and not (down._forward_hooks or down._forward_pre_hooks or "forward" in down.__dict__))
+
     def _all_rows(self, rows: int, device: torch.device) -> torch.Tensor:
         """The row_offsets operand of the silu kernels for a dense block: [0, rows] (uint32, on the device).  Kept
         per row count, so that a call neither copies from the host nor breaks a HIP graph capture."""
@@ -188,14 +195,15 @@ class MLP(torch.nn.Module):
             return y.reshape(*lead, self.hidden_dim)
         if self._silu_kernel():
             rows_used = self._all_rows(x2.shape[0], x2.device)
-            kind = native_granularity(cfg.input_scale, cfg.weight_scale)
+            plain = self._down_is_plain()
+            kind = native_granularity(cfg.input_scale, cfg.weight_scale) if plain else -1
             if kind >= 0:
                 y = _lib.native().mlp(x2, self.gate_up_weight, self.gate_up_weight_scale, self.down_proj.weight,
                                       self.down_proj.weight_scale, kind, rows_used, 1200.0)
                 if y is not None:
                     return y if x.dim() == 2 else y.reshape(*lead, self.hidden_dim)
             both = quantized_matmul(x2, self.gate_up_weight, self.gate_up_weight_scale, None, cfg)
-            group = silu_quantize_group(cfg, x2.shape[0], self.feed_forward_length)
+            group = silu_quantize_group(cfg, x2.shape[0], self.feed_forward_length) if plain else None
             if group is not None and self.down_proj.weight_scale.dtype == torch.float32:
                 hq, hs = silu_quantize(both, rows_used, group, round_activation=True)
                 y = dynamic_scaled_matmul(hq, self.down_proj.weight, hs, self.down_proj.weight_scale, cfg.input_scale,
