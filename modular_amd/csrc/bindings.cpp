@@ -55,6 +55,18 @@ bool weight_scales_ok(const at::Tensor& s, const at::Tensor& w, int granularity)
 }
 at::Tensor bytes_on(const at::Tensor& like, size_t n) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
 
+// One call of the C ABI without the interpreter lock, as ctypes makes it: a launch waits where the queue is full, and other
+// threads go on meanwhile.  (The lock is back before an exception of the call's arguments leaves.)
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+template <class Call>
+int unlocked(Call call) {
+  const Unlocked released;
+  return call();
+}
+
 // y = quantise(x) . w^T: [M, N] bf16.  Null with *status set where the library refuses.
 at::Tensor linear_of(const at::Tensor& x, const at::Tensor& w, const at::Tensor& s, int granularity, float scale_ub, void* stream, int* status) {
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
@@ -62,8 +74,10 @@ at::Tensor linear_of(const at::Tensor& x, const at::Tensor& w, const at::Tensor&
   const size_t need = maxfp8_linear_workspace_bytes(M, N, K, granularity);
   at::Tensor ws;
   if (need) ws = bytes_on(x, need);
-  *status = maxfp8_linear_dynamic_scaled_fp8(y.data_ptr(), x.data_ptr(), w.data_ptr(), s.data_ptr(), M, N, K, row_stride(x), row_stride(w), N,
-                                             granularity, s.size(1), scale_ub, need ? ws.data_ptr() : nullptr, need, stream);
+  *status = unlocked([&] {
+    return maxfp8_linear_dynamic_scaled_fp8(y.data_ptr(), x.data_ptr(), w.data_ptr(), s.data_ptr(), M, N, K, row_stride(x), row_stride(w), N,
+        granularity, s.size(1), scale_ub, need ? ws.data_ptr() : nullptr, need, stream);
+  });
   return y;
 }
 bool linear_ok(const at::Tensor& x, const at::Tensor& w, const at::Tensor& s, int granularity) {
@@ -117,9 +131,11 @@ PyObject* linear_static(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const size_t need = maxfp8_linear_workspace_bytes(M, N, K, MAXFP8_GRAN_TENSOR);
   at::Tensor ws;
   if (need) ws = bytes_on(*x, need);
-  const int status = maxfp8_linear_static_scaled_fp8(y.data_ptr(), x->data_ptr(), w->data_ptr(), M, N, K, row_stride(*x), row_stride(*w), N,
-                                                     *static_cast<const float*>(si->data_ptr()), *static_cast<const float*>(sw->data_ptr()),
-                                                     need ? ws.data_ptr() : nullptr, need, stream);
+  const int status = unlocked([&] {
+    return maxfp8_linear_static_scaled_fp8(y.data_ptr(), x->data_ptr(), w->data_ptr(), M, N, K, row_stride(*x), row_stride(*w), N,
+        *static_cast<const float*>(si->data_ptr()), *static_cast<const float*>(sw->data_ptr()),
+        need ? ws.data_ptr() : nullptr, need, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   return THPVariable_Wrap(std::move(y));
 }
@@ -148,8 +164,10 @@ PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!stream_of(*x, &stream)) return nullptr;
   const int64_t M = x->size(0), K = x->size(1), ld = padded ? (M + 3) / 4 * 4 : M;
   at::Tensor q = at::empty({M, K}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({K / group, ld}, x->options().dtype(at::kFloat));
-  const int status = maxfp8_quantize_dynamic_scaled_fp8(q.data_ptr(), s.data_ptr(), x->data_ptr(), M, K, row_stride(*x), K, group, ld, MAXFP8_BF16,
-                                                        MAXFP8_F32, ub, stream);
+  const int status = unlocked([&] {
+    return maxfp8_quantize_dynamic_scaled_fp8(q.data_ptr(), s.data_ptr(), x->data_ptr(), M, K, row_stride(*x), K, group, ld, MAXFP8_BF16,
+        MAXFP8_F32, ub, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   return pair(std::move(q), std::move(s));
 }
@@ -166,8 +184,10 @@ PyObject* rms_norm_quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
   if (!stream_of(*x, &stream)) return nullptr;
   const int64_t M = x->size(0), K = x->size(1);
   at::Tensor q = at::empty({M, K}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({1, M}, x->options().dtype(at::kFloat));
-  const int status = maxfp8_rms_norm_fused_quantize_dynamic_scaled_fp8(q.data_ptr(), s.data_ptr(), x->data_ptr(), g->data_ptr(), M, K, row_stride(*x),
-                                                                       K, MAXFP8_BF16, MAXFP8_F32, eps, offset, ub, stream);
+  const int status = unlocked([&] {
+    return maxfp8_rms_norm_fused_quantize_dynamic_scaled_fp8(q.data_ptr(), s.data_ptr(), x->data_ptr(), g->data_ptr(), M, K, row_stride(*x),
+        K, MAXFP8_BF16, MAXFP8_F32, eps, offset, ub, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   return pair(std::move(q), std::move(s));
 }
@@ -191,10 +211,12 @@ PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const size_t need = maxfp8_matmul_auto_workspace_bytes(M, N, K);
   at::Tensor ws;
   if (need) ws = bytes_on(*a, need);
-  const int status = maxfp8_matmul_dynamic_scaled_fp8(
-      c.data_ptr(), a->data_ptr(), b->data_ptr(), sa->data_ptr(), sb->data_ptr(), M, N, K, row_stride(*a), row_stride(*b), N,
-      block ? MAXFP8_GRAN_BLOCK : MAXFP8_GRAN_COLWISE, granularity, block ? 1 : -1, block ? 128 : -1, block ? 128 : -1, row_stride(*sa), sb->size(1),
-      MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO, need ? ws.data_ptr() : nullptr, need, stream);
+  const int status = unlocked([&] {
+    return maxfp8_matmul_dynamic_scaled_fp8(
+        c.data_ptr(), a->data_ptr(), b->data_ptr(), sa->data_ptr(), sb->data_ptr(), M, N, K, row_stride(*a), row_stride(*b), N,
+        block ? MAXFP8_GRAN_BLOCK : MAXFP8_GRAN_COLWISE, granularity, block ? 1 : -1, block ? 128 : -1, block ? 128 : -1, row_stride(*sa), sb->size(1),
+        MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO, need ? ws.data_ptr() : nullptr, need, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   return THPVariable_Wrap(std::move(c));
 }
@@ -213,9 +235,11 @@ PyObject* batched_quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!stream_of(*x, &stream)) return nullptr;
   const int64_t B = x->size(0), M = x->size(1), K = x->size(2), ld = (M + 3) / 4 * 4;
   at::Tensor q = at::empty({B, M, K}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({B, K / group, ld}, x->options().dtype(at::kFloat));
-  const int status = maxfp8_batched_quantize_dynamic_scaled_fp8(
-      q.data_ptr(), s.data_ptr(), x->data_ptr(), B, M, K, B > 1 ? x->stride(0) : M * K, M > 1 ? x->stride(1) : K, M * K, K, group, (K / group) * ld, ld,
-      MAXFP8_BF16, MAXFP8_F32, ub, stream);
+  const int status = unlocked([&] {
+    return maxfp8_batched_quantize_dynamic_scaled_fp8(
+        q.data_ptr(), s.data_ptr(), x->data_ptr(), B, M, K, B > 1 ? x->stride(0) : M * K, M > 1 ? x->stride(1) : K, M * K, K, group, (K / group) * ld, ld,
+        MAXFP8_BF16, MAXFP8_F32, ub, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   return pair(std::move(q), std::move(s));
 }
@@ -234,9 +258,11 @@ PyObject* batched_matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!stream_of(*a, &stream)) return nullptr;
   at::Tensor c = at::empty({B, M, N}, a->options().dtype(at::kBFloat16));
   const int64_t ld = sa->size(2);
-  const int status = maxfp8_batched_matmul_dynamic_scaled_fp8(
-      c.data_ptr(), a->data_ptr(), b->data_ptr(), sa->data_ptr(), sb->data_ptr(), B, M, N, K, M * K, K, N * K, K, M * N, N, 1, 128, 128, kb * ld, ld,
-      nb * kb, kb, MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO, stream);
+  const int status = unlocked([&] {
+    return maxfp8_batched_matmul_dynamic_scaled_fp8(
+        c.data_ptr(), a->data_ptr(), b->data_ptr(), sa->data_ptr(), sb->data_ptr(), B, M, N, K, M * K, K, N * K, K, M * N, N, 1, 128, 128, kb * ld, ld,
+        nb * kb, kb, MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   return THPVariable_Wrap(std::move(c));
 }
@@ -271,14 +297,18 @@ PyObject* mlp(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const size_t partial = maxfp8_matmul_auto_workspace_bytes(M, H, F);
   at::Tensor ws = bytes_on(*x, at_partial + partial);
   uint8_t* q = static_cast<uint8_t*>(ws.data_ptr());
-  status = maxfp8_silu_quantize_dynamic_scaled_fp8(q, q + at_scales, both.data_ptr(), static_cast<const uint32_t*>(rows->data_ptr()), 2, M, F, 2 * F, F,
-                                                   group, ld, MAXFP8_BF16, 1, ub, stream);
+  status = unlocked([&] {
+    return maxfp8_silu_quantize_dynamic_scaled_fp8(q, q + at_scales, both.data_ptr(), static_cast<const uint32_t*>(rows->data_ptr()), 2, M, F, 2 * F, F,
+        group, ld, MAXFP8_BF16, 1, ub, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   at::Tensor y = at::empty({M, H}, x->options());
-  status = maxfp8_matmul_dynamic_scaled_fp8(y.data_ptr(), q, d->data_ptr(), q + at_scales, sd->data_ptr(), M, H, F, F, row_stride(*d), H,
-                                            block ? MAXFP8_GRAN_BLOCK : MAXFP8_GRAN_COLWISE, granularity, block ? 1 : -1, block ? 128 : -1,
-                                            block ? 128 : -1, ld, sd->size(1), MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO,
-                                            partial ? q + at_partial : nullptr, partial, stream);
+  status = unlocked([&] {
+    return maxfp8_matmul_dynamic_scaled_fp8(y.data_ptr(), q, d->data_ptr(), q + at_scales, sd->data_ptr(), M, H, F, F, row_stride(*d), H,
+        block ? MAXFP8_GRAN_BLOCK : MAXFP8_GRAN_COLWISE, granularity, block ? 1 : -1, block ? 128 : -1,
+        block ? 128 : -1, ld, sd->size(1), MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO,
+        partial ? q + at_partial : nullptr, partial, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   return THPVariable_Wrap(std::move(y));
 }
@@ -308,11 +338,13 @@ PyObject* qkv_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const size_t need = maxfp8_linear_qkv_workspace_bytes(T, N, K, granularity);
   at::Tensor ws;
   if (need) ws = bytes_on(*x, need);
-  const int status = maxfp8_linear_qkv_ragged_paged_scale(
-      q.data_ptr(), x->data_ptr(), row_stride(*x), static_cast<const uint32_t*>(offsets->data_ptr()), w->data_ptr(), s->data_ptr(), blocks->data_ptr(),
-      static_cast<const uint32_t*>(lengths->data_ptr()), static_cast<const uint32_t*>(table->data_ptr()), bias ? bias->data_ptr() : nullptr, T, N, K,
-      q_dim, batch, blocks->size(0), blocks->size(1), blocks->size(2), layer, blocks->size(3), blocks->size(4), blocks->size(5), table->size(1),
-      granularity, s->size(1), ub, need ? ws.data_ptr() : nullptr, need, stream);
+  const int status = unlocked([&] {
+    return maxfp8_linear_qkv_ragged_paged_scale(
+        q.data_ptr(), x->data_ptr(), row_stride(*x), static_cast<const uint32_t*>(offsets->data_ptr()), w->data_ptr(), s->data_ptr(), blocks->data_ptr(),
+        static_cast<const uint32_t*>(lengths->data_ptr()), static_cast<const uint32_t*>(table->data_ptr()), bias ? bias->data_ptr() : nullptr, T, N, K,
+        q_dim, batch, blocks->size(0), blocks->size(1), blocks->size(2), layer, blocks->size(3), blocks->size(4), blocks->size(5), table->size(1),
+        granularity, s->size(1), ub, need ? ws.data_ptr() : nullptr, need, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   return THPVariable_Wrap(std::move(q));
 }
@@ -338,27 +370,37 @@ PyObject* moe_experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   at::Tensor idx = at::empty({2 * T + 2 * E + 8}, x->options().dtype(at::kInt));
   uint32_t* order = static_cast<uint32_t*>(idx.data_ptr());
   uint32_t *restore = order + T, *start = restore + T, *ids = start + E + 1, *usage = ids + E;
-  int status = maxfp8_moe_create_indices(order, start, restore, reinterpret_cast<int32_t*>(ids), usage, r->data_ptr(), T, E, stream);
+  int status = unlocked([&] {
+    return maxfp8_moe_create_indices(order, start, restore, reinterpret_cast<int32_t*>(ids), usage, r->data_ptr(), T, E, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   // every token quantised once and stored to its k rows of the grouped order
   at::Tensor q = at::empty({T, H}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({H / 128, ld}, x->options().dtype(at::kFloat));
-  status = maxfp8_quantize_dynamic_scaled_fp8_scatter(q.data_ptr(), s.data_ptr(), x->data_ptr(), restore, k, seq, H, T, row_stride(*x), H, 128, ld,
-                                                      MAXFP8_BF16, MAXFP8_F32, ub, stream);
+  status = unlocked([&] {
+    return maxfp8_quantize_dynamic_scaled_fp8_scatter(q.data_ptr(), s.data_ptr(), x->data_ptr(), restore, k, seq, H, T, row_stride(*x), H, 128, ld,
+        MAXFP8_BF16, MAXFP8_F32, ub, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   // (the bounds of the two host scalars: every row on one expert, every expert in use)
   at::Tensor both = at::empty({T, 2 * F}, x->options());
-  status = maxfp8_grouped_matmul_dynamic_scaled_fp8(both.data_ptr(), q.data_ptr(), gu->data_ptr(), s.data_ptr(), sgu->data_ptr(), start,
-                                                    reinterpret_cast<const int32_t*>(ids), T, 2 * F, H, E, T, E, ld, MAXFP8_BF16, MAXFP8_F32,
-                                                    MAXFP8_ALGO_AUTO, stream);
+  status = unlocked([&] {
+    return maxfp8_grouped_matmul_dynamic_scaled_fp8(both.data_ptr(), q.data_ptr(), gu->data_ptr(), s.data_ptr(), sgu->data_ptr(), start,
+        reinterpret_cast<const int32_t*>(ids), T, 2 * F, H, E, T, E, ld, MAXFP8_BF16, MAXFP8_F32,
+        MAXFP8_ALGO_AUTO, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   at::Tensor hq = at::empty({T, F}, x->options().dtype(at::kFloat8_e4m3fn)), hs = at::empty({F / 128, ld}, x->options().dtype(at::kFloat));
-  status = maxfp8_silu_quantize_dynamic_scaled_fp8(hq.data_ptr(), hs.data_ptr(), both.data_ptr(), start, E + 1, T, F, 2 * F, F, 128, ld, MAXFP8_BF16, 0,
-                                                   ub, stream);
+  status = unlocked([&] {
+    return maxfp8_silu_quantize_dynamic_scaled_fp8(hq.data_ptr(), hs.data_ptr(), both.data_ptr(), start, E + 1, T, F, 2 * F, F, 128, ld, MAXFP8_BF16, 0,
+        ub, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   at::Tensor y = at::empty({seq, k, H}, x->options());
-  status = maxfp8_grouped_matmul_dynamic_scaled_fp8_scatter(y.data_ptr(), order, hq.data_ptr(), d->data_ptr(), hs.data_ptr(), sd->data_ptr(), start,
-                                                            reinterpret_cast<const int32_t*>(ids), T, H, F, E, T, E, ld, MAXFP8_BF16, MAXFP8_F32,
-                                                            MAXFP8_ALGO_AUTO, stream);
+  status = unlocked([&] {
+    return maxfp8_grouped_matmul_dynamic_scaled_fp8_scatter(y.data_ptr(), order, hq.data_ptr(), d->data_ptr(), hs.data_ptr(), sd->data_ptr(), start,
+        reinterpret_cast<const int32_t*>(ids), T, H, F, E, T, E, ld, MAXFP8_BF16, MAXFP8_F32,
+        MAXFP8_ALGO_AUTO, stream);
+  });
   if (status != MAXFP8_OK) return raise(status);
   return THPVariable_Wrap(std::move(y));
 }

@@ -166,7 +166,8 @@ class MLP(torch.nn.Module):
         module in its place, a bias, a static scale, another config or hooks."""
         down = self.down_proj
         return (type(down) is Linear and down.bias is None and down.input_scale is None
-                and (down.quant_config is self.quant_config or down.quant_config == self.quant_config) and not (down._forward_hooks or down._forward_pre_hooks or "forward" in down.__dict__))
+                and (down.quant_config is self.quant_config or down.quant_config == self.quant_config)
+                and not (down._forward_hooks or down._forward_pre_hooks or "forward" in down.__dict__))
 
     def _all_rows(self, rows: int, device: torch.device) -> torch.Tensor:
         """The row_offsets operand of the silu kernels for a dense block: [0, rows] (uint32, on the device).  Kept
