@@ -121,11 +121,17 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 PyObject* linear_static(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   NEED_ARGS(4)
   const at::Tensor *x = tensor(args[0]), *w = tensor(args[1]), *si = tensor(args[2]), *sw = tensor(args[3]);
-  auto scalar = [](const at::Tensor* t) { return t && !t->is_cuda() && t->scalar_type() == at::kFloat && t->numel() == 1 && t->dim() <= 1; };
-  if (!x || !w || !scalar(si) || !scalar(sw) || !bf16_rows(*x) || !fp8_rows(*w) || !on_gpu(*w, *x) || w->size(1) != x->size(1) || x->size(1) % 16 != 0)
+  // (a tensor on the meta device, or one that only has a shape while a program is traced, has no value to read)
+  auto scalar = [](const at::Tensor* t) -> const float* {
+    const bool ok = t && t->device().is_cpu() && t->scalar_type() == at::kFloat && t->numel() == 1 && t->dim() <= 1;
+    return ok ? static_cast<const float*>(t->data_ptr()) : nullptr;
+  };
+  const float *pi = scalar(si), *pw = scalar(sw);
+  if (!x || !w || !pi || !pw || !bf16_rows(*x) || !fp8_rows(*w) || !on_gpu(*w, *x) || w->size(1) != x->size(1) || x->size(1) % 16 != 0)
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
+  const float input_scale = *pi, weight_scale = *pw;
   const int64_t M = x->size(0), K = x->size(1), N = w->size(0);
   at::Tensor y = at::empty({M, N}, x->options());
   const size_t need = maxfp8_linear_workspace_bytes(M, N, K, MAXFP8_GRAN_TENSOR);
@@ -133,8 +139,7 @@ PyObject* linear_static(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (need) ws = bytes_on(*x, need);
   const int status = unlocked([&] {
     return maxfp8_linear_static_scaled_fp8(y.data_ptr(), x->data_ptr(), w->data_ptr(), M, N, K, row_stride(*x), row_stride(*w), N,
-        *static_cast<const float*>(si->data_ptr()), *static_cast<const float*>(sw->data_ptr()),
-        need ? ws.data_ptr() : nullptr, need, stream);
+        input_scale, weight_scale, need ? ws.data_ptr() : nullptr, need, stream);
   });
   if (status != MAXFP8_OK) return raise(status);
   return THPVariable_Wrap(std::move(y));
