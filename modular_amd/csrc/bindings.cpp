@@ -3,7 +3,7 @@
 // A decode linear takes 6 us on the GPU; the Python wrappers (argument checks one by one, three to four torch.empty, two
 // ctypes calls of some twenty arguments) took 26 us of host time around it.  Each function here handles the common case of
 // one wrapper and returns None for every other -- another dtype, layout, device, an empty tensor -- so that the wrapper's
-// own checks and messages decide those.  Nothing is kept between calls but the two Python functions found at import.
+// own checks and messages decide those.  Nothing is kept between calls but the Python function found at import.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -55,8 +55,9 @@ bool weight_scales_ok(const at::Tensor& s, const at::Tensor& w, int granularity)
 }
 at::Tensor bytes_on(const at::Tensor& like, size_t n) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
 
-// One call of the C ABI without the interpreter lock, as ctypes makes it: a launch waits where the queue is full, and other
-// threads go on meanwhile.  (The lock is back before an exception of the call's arguments leaves.)
+// An operator's allocations and launches without the interpreter lock, as torch's own calls and ctypes make them: an allocation
+// may reach the driver, a launch waits where the queue is full, and other threads go on meanwhile.  (The lock is back before an
+// exception of the call leaves.)
 struct Unlocked {
   PyThreadState* state = PyEval_SaveThread();
   ~Unlocked() { PyEval_RestoreThread(state); }
@@ -67,18 +68,15 @@ int unlocked(Call call) {
   return call();
 }
 
-// y = quantise(x) . w^T: [M, N] bf16.  Null with *status set where the library refuses.
-at::Tensor linear_of(const at::Tensor& x, const at::Tensor& w, const at::Tensor& s, int granularity, float scale_ub, void* stream, int* status) {
+// y = quantise(x) . w^T: [M, N] bf16; a status of the C ABI.  (Without the lock, like what the operators below do inside `unlocked`.)
+int linear_of(at::Tensor& y, const at::Tensor& x, const at::Tensor& w, const at::Tensor& s, int granularity, float scale_ub, void* stream) {
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  at::Tensor y = at::empty({M, N}, x.options());
+  y = at::empty({M, N}, x.options());
   const size_t need = maxfp8_linear_workspace_bytes(M, N, K, granularity);
   at::Tensor ws;
   if (need) ws = bytes_on(x, need);
-  *status = unlocked([&] {
-    return maxfp8_linear_dynamic_scaled_fp8(y.data_ptr(), x.data_ptr(), w.data_ptr(), s.data_ptr(), M, N, K, row_stride(x), row_stride(w), N,
-        granularity, s.size(1), scale_ub, need ? ws.data_ptr() : nullptr, need, stream);
-  });
-  return y;
+  return maxfp8_linear_dynamic_scaled_fp8(y.data_ptr(), x.data_ptr(), w.data_ptr(), s.data_ptr(), M, N, K, row_stride(x), row_stride(w), N,
+      granularity, s.size(1), scale_ub, need ? ws.data_ptr() : nullptr, need, stream);
 }
 bool linear_ok(const at::Tensor& x, const at::Tensor& w, const at::Tensor& s, int granularity) {
   return bf16_rows(x) && fp8_rows(w) && on_gpu(w, x) && w.size(1) == x.size(1) && weight_scales_ok(s, w, granularity);
@@ -111,8 +109,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!x || !w || !s || !linear_ok(*x, *w, *s, granularity)) Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
-  int status;
-  at::Tensor y = linear_of(*x, *w, *s, granularity, ub, stream, &status);
+  at::Tensor y;
+  const int status = unlocked([&] { return linear_of(y, *x, *w, *s, granularity, ub, stream); });
   if (status != MAXFP8_OK) return raise(status);
   return THPVariable_Wrap(std::move(y));
 }
@@ -133,11 +131,12 @@ PyObject* linear_static(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!stream_of(*x, &stream)) return nullptr;
   const float input_scale = *pi, weight_scale = *pw;
   const int64_t M = x->size(0), K = x->size(1), N = w->size(0);
-  at::Tensor y = at::empty({M, N}, x->options());
-  const size_t need = maxfp8_linear_workspace_bytes(M, N, K, MAXFP8_GRAN_TENSOR);
-  at::Tensor ws;
-  if (need) ws = bytes_on(*x, need);
+  at::Tensor y;
   const int status = unlocked([&] {
+    y = at::empty({M, N}, x->options());
+    const size_t need = maxfp8_linear_workspace_bytes(M, N, K, MAXFP8_GRAN_TENSOR);
+    at::Tensor ws;
+    if (need) ws = bytes_on(*x, need);
     return maxfp8_linear_static_scaled_fp8(y.data_ptr(), x->data_ptr(), w->data_ptr(), M, N, K, row_stride(*x), row_stride(*w), N,
         input_scale, weight_scale, need ? ws.data_ptr() : nullptr, need, stream);
   });
@@ -168,8 +167,10 @@ PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
   const int64_t M = x->size(0), K = x->size(1), ld = padded ? (M + 3) / 4 * 4 : M;
-  at::Tensor q = at::empty({M, K}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({K / group, ld}, x->options().dtype(at::kFloat));
+  at::Tensor q, s;
   const int status = unlocked([&] {
+    q = at::empty({M, K}, x->options().dtype(at::kFloat8_e4m3fn));
+    s = at::empty({K / group, ld}, x->options().dtype(at::kFloat));
     return maxfp8_quantize_dynamic_scaled_fp8(q.data_ptr(), s.data_ptr(), x->data_ptr(), M, K, row_stride(*x), K, group, ld, MAXFP8_BF16,
         MAXFP8_F32, ub, stream);
   });
@@ -188,8 +189,10 @@ PyObject* rms_norm_quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
   const int64_t M = x->size(0), K = x->size(1);
-  at::Tensor q = at::empty({M, K}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({1, M}, x->options().dtype(at::kFloat));
+  at::Tensor q, s;
   const int status = unlocked([&] {
+    q = at::empty({M, K}, x->options().dtype(at::kFloat8_e4m3fn));
+    s = at::empty({1, M}, x->options().dtype(at::kFloat));
     return maxfp8_rms_norm_fused_quantize_dynamic_scaled_fp8(q.data_ptr(), s.data_ptr(), x->data_ptr(), g->data_ptr(), M, K, row_stride(*x),
         K, MAXFP8_BF16, MAXFP8_F32, eps, offset, ub, stream);
   });
@@ -212,11 +215,12 @@ PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   void* stream;
   if (!stream_of(*a, &stream)) return nullptr;
   const int64_t M = a->size(0), K = a->size(1), N = b->size(0);
-  at::Tensor c = at::empty({M, N}, a->options().dtype(at::kBFloat16));
-  const size_t need = maxfp8_matmul_auto_workspace_bytes(M, N, K);
-  at::Tensor ws;
-  if (need) ws = bytes_on(*a, need);
+  at::Tensor c;
   const int status = unlocked([&] {
+    c = at::empty({M, N}, a->options().dtype(at::kBFloat16));
+    const size_t need = maxfp8_matmul_auto_workspace_bytes(M, N, K);
+    at::Tensor ws;
+    if (need) ws = bytes_on(*a, need);
     return maxfp8_matmul_dynamic_scaled_fp8(
         c.data_ptr(), a->data_ptr(), b->data_ptr(), sa->data_ptr(), sb->data_ptr(), M, N, K, row_stride(*a), row_stride(*b), N,
         block ? MAXFP8_GRAN_BLOCK : MAXFP8_GRAN_COLWISE, granularity, block ? 1 : -1, block ? 128 : -1, block ? 128 : -1, row_stride(*sa), sb->size(1),
@@ -239,8 +243,10 @@ PyObject* batched_quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
   const int64_t B = x->size(0), M = x->size(1), K = x->size(2), ld = (M + 3) / 4 * 4;
-  at::Tensor q = at::empty({B, M, K}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({B, K / group, ld}, x->options().dtype(at::kFloat));
+  at::Tensor q, s;
   const int status = unlocked([&] {
+    q = at::empty({B, M, K}, x->options().dtype(at::kFloat8_e4m3fn));
+    s = at::empty({B, K / group, ld}, x->options().dtype(at::kFloat));
     return maxfp8_batched_quantize_dynamic_scaled_fp8(
         q.data_ptr(), s.data_ptr(), x->data_ptr(), B, M, K, B > 1 ? x->stride(0) : M * K, M > 1 ? x->stride(1) : K, M * K, K, group, (K / group) * ld, ld,
         MAXFP8_BF16, MAXFP8_F32, ub, stream);
@@ -261,9 +267,10 @@ PyObject* batched_matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*a, &stream)) return nullptr;
-  at::Tensor c = at::empty({B, M, N}, a->options().dtype(at::kBFloat16));
   const int64_t ld = sa->size(2);
+  at::Tensor c;
   const int status = unlocked([&] {
+    c = at::empty({B, M, N}, a->options().dtype(at::kBFloat16));
     return maxfp8_batched_matmul_dynamic_scaled_fp8(
         c.data_ptr(), a->data_ptr(), b->data_ptr(), sa->data_ptr(), sb->data_ptr(), B, M, N, K, M * K, K, N * K, K, M * N, N, 1, 128, 128, kb * ld, ld,
         nb * kb, kb, MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO, stream);
@@ -292,23 +299,22 @@ PyObject* mlp(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
   const int64_t M = x->size(0), F = d->size(1), H = d->size(0);
-  int status;
-  at::Tensor both = linear_of(*x, *gu, *sgu, granularity, ub, stream, &status);
-  if (status != MAXFP8_OK) return raise(status);
   const bool block = granularity == MAXFP8_GRAN_BLOCK;
   const int64_t group = block ? 128 : F, ld = block ? (M + 3) / 4 * 4 : M;
   // one buffer: the quantised product, its scales, the down matmul's partial sums
   const size_t at_scales = ((size_t)M * (size_t)F + 255) / 256 * 256, at_partial = at_scales + ((size_t)(F / group) * (size_t)ld * 4 + 255) / 256 * 256;
-  const size_t partial = maxfp8_matmul_auto_workspace_bytes(M, H, F);
-  at::Tensor ws = bytes_on(*x, at_partial + partial);
-  uint8_t* q = static_cast<uint8_t*>(ws.data_ptr());
-  status = unlocked([&] {
-    return maxfp8_silu_quantize_dynamic_scaled_fp8(q, q + at_scales, both.data_ptr(), static_cast<const uint32_t*>(rows->data_ptr()), 2, M, F, 2 * F, F,
+  at::Tensor y;
+  const int status = unlocked([&] {
+    at::Tensor both;
+    int rc = linear_of(both, *x, *gu, *sgu, granularity, ub, stream);
+    if (rc != MAXFP8_OK) return rc;
+    const size_t partial = maxfp8_matmul_auto_workspace_bytes(M, H, F);
+    at::Tensor ws = bytes_on(*x, at_partial + partial);
+    uint8_t* q = static_cast<uint8_t*>(ws.data_ptr());
+    rc = maxfp8_silu_quantize_dynamic_scaled_fp8(q, q + at_scales, both.data_ptr(), static_cast<const uint32_t*>(rows->data_ptr()), 2, M, F, 2 * F, F,
         group, ld, MAXFP8_BF16, 1, ub, stream);
-  });
-  if (status != MAXFP8_OK) return raise(status);
-  at::Tensor y = at::empty({M, H}, x->options());
-  status = unlocked([&] {
+    if (rc != MAXFP8_OK) return rc;
+    y = at::empty({M, H}, x->options());
     return maxfp8_matmul_dynamic_scaled_fp8(y.data_ptr(), q, d->data_ptr(), q + at_scales, sd->data_ptr(), M, H, F, F, row_stride(*d), H,
         block ? MAXFP8_GRAN_BLOCK : MAXFP8_GRAN_COLWISE, granularity, block ? 1 : -1, block ? 128 : -1,
         block ? 128 : -1, ld, sd->size(1), MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO,
@@ -339,11 +345,12 @@ PyObject* qkv_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
-  at::Tensor q = at::empty({T, q_dim}, x->options());
-  const size_t need = maxfp8_linear_qkv_workspace_bytes(T, N, K, granularity);
-  at::Tensor ws;
-  if (need) ws = bytes_on(*x, need);
+  at::Tensor q;
   const int status = unlocked([&] {
+    q = at::empty({T, q_dim}, x->options());
+    const size_t need = maxfp8_linear_qkv_workspace_bytes(T, N, K, granularity);
+    at::Tensor ws;
+    if (need) ws = bytes_on(*x, need);
     return maxfp8_linear_qkv_ragged_paged_scale(
         q.data_ptr(), x->data_ptr(), row_stride(*x), static_cast<const uint32_t*>(offsets->data_ptr()), w->data_ptr(), s->data_ptr(), blocks->data_ptr(),
         static_cast<const uint32_t*>(lengths->data_ptr()), static_cast<const uint32_t*>(table->data_ptr()), bias ? bias->data_ptr() : nullptr, T, N, K,
@@ -371,40 +378,32 @@ PyObject* moe_experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(*x, &stream)) return nullptr;
-  // the grouping: order [T], restore [T], starts [E + 1], expert ids [E], usage [2]
-  at::Tensor idx = at::empty({2 * T + 2 * E + 8}, x->options().dtype(at::kInt));
-  uint32_t* order = static_cast<uint32_t*>(idx.data_ptr());
-  uint32_t *restore = order + T, *start = restore + T, *ids = start + E + 1, *usage = ids + E;
-  int status = unlocked([&] {
-    return maxfp8_moe_create_indices(order, start, restore, reinterpret_cast<int32_t*>(ids), usage, r->data_ptr(), T, E, stream);
-  });
-  if (status != MAXFP8_OK) return raise(status);
-  // every token quantised once and stored to its k rows of the grouped order
-  at::Tensor q = at::empty({T, H}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({H / 128, ld}, x->options().dtype(at::kFloat));
-  status = unlocked([&] {
-    return maxfp8_quantize_dynamic_scaled_fp8_scatter(q.data_ptr(), s.data_ptr(), x->data_ptr(), restore, k, seq, H, T, row_stride(*x), H, 128, ld,
+  at::Tensor y;
+  const int status = unlocked([&] {
+    // the grouping: order [T], restore [T], starts [E + 1], expert ids [E], usage [2]
+    at::Tensor idx = at::empty({2 * T + 2 * E + 8}, x->options().dtype(at::kInt));
+    uint32_t* order = static_cast<uint32_t*>(idx.data_ptr());
+    uint32_t *restore = order + T, *start = restore + T, *ids = start + E + 1, *usage = ids + E;
+    const int32_t* expert_ids = reinterpret_cast<const int32_t*>(ids);
+    int rc = maxfp8_moe_create_indices(order, start, restore, reinterpret_cast<int32_t*>(ids), usage, r->data_ptr(), T, E, stream);
+    if (rc != MAXFP8_OK) return rc;
+    // every token quantised once and stored to its k rows of the grouped order
+    at::Tensor q = at::empty({T, H}, x->options().dtype(at::kFloat8_e4m3fn)), s = at::empty({H / 128, ld}, x->options().dtype(at::kFloat));
+    rc = maxfp8_quantize_dynamic_scaled_fp8_scatter(q.data_ptr(), s.data_ptr(), x->data_ptr(), restore, k, seq, H, T, row_stride(*x), H, 128, ld,
         MAXFP8_BF16, MAXFP8_F32, ub, stream);
-  });
-  if (status != MAXFP8_OK) return raise(status);
-  // (the bounds of the two host scalars: every row on one expert, every expert in use)
-  at::Tensor both = at::empty({T, 2 * F}, x->options());
-  status = unlocked([&] {
-    return maxfp8_grouped_matmul_dynamic_scaled_fp8(both.data_ptr(), q.data_ptr(), gu->data_ptr(), s.data_ptr(), sgu->data_ptr(), start,
-        reinterpret_cast<const int32_t*>(ids), T, 2 * F, H, E, T, E, ld, MAXFP8_BF16, MAXFP8_F32,
-        MAXFP8_ALGO_AUTO, stream);
-  });
-  if (status != MAXFP8_OK) return raise(status);
-  at::Tensor hq = at::empty({T, F}, x->options().dtype(at::kFloat8_e4m3fn)), hs = at::empty({F / 128, ld}, x->options().dtype(at::kFloat));
-  status = unlocked([&] {
-    return maxfp8_silu_quantize_dynamic_scaled_fp8(hq.data_ptr(), hs.data_ptr(), both.data_ptr(), start, E + 1, T, F, 2 * F, F, 128, ld, MAXFP8_BF16, 0,
+    if (rc != MAXFP8_OK) return rc;
+    // (the bounds of the two host scalars: every row on one expert, every expert in use)
+    at::Tensor both = at::empty({T, 2 * F}, x->options());
+    rc = maxfp8_grouped_matmul_dynamic_scaled_fp8(both.data_ptr(), q.data_ptr(), gu->data_ptr(), s.data_ptr(), sgu->data_ptr(), start, expert_ids,
+        T, 2 * F, H, E, T, E, ld, MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO, stream);
+    if (rc != MAXFP8_OK) return rc;
+    at::Tensor hq = at::empty({T, F}, x->options().dtype(at::kFloat8_e4m3fn)), hs = at::empty({F / 128, ld}, x->options().dtype(at::kFloat));
+    rc = maxfp8_silu_quantize_dynamic_scaled_fp8(hq.data_ptr(), hs.data_ptr(), both.data_ptr(), start, E + 1, T, F, 2 * F, F, 128, ld, MAXFP8_BF16, 0,
         ub, stream);
-  });
-  if (status != MAXFP8_OK) return raise(status);
-  at::Tensor y = at::empty({seq, k, H}, x->options());
-  status = unlocked([&] {
+    if (rc != MAXFP8_OK) return rc;
+    y = at::empty({seq, k, H}, x->options());
     return maxfp8_grouped_matmul_dynamic_scaled_fp8_scatter(y.data_ptr(), order, hq.data_ptr(), d->data_ptr(), hs.data_ptr(), sd->data_ptr(), start,
-        reinterpret_cast<const int32_t*>(ids), T, H, F, E, T, E, ld, MAXFP8_BF16, MAXFP8_F32,
-        MAXFP8_ALGO_AUTO, stream);
+        expert_ids, T, H, F, E, T, E, ld, MAXFP8_BF16, MAXFP8_F32, MAXFP8_ALGO_AUTO, stream);
   });
   if (status != MAXFP8_OK) return raise(status);
   return THPVariable_Wrap(std::move(y));
