@@ -99,10 +99,10 @@ def expert_matmuls_fp8(
     The grouped matmul op takes two host scalars (most tokens on one expert, active experts), which
     the reference copies from the device between the grouping and the first matmul
     (max/python/max/nn/moe/quant_strategy.py:175).  This package's kernels read the offsets on the
-    device and use the scalars only as upper bounds for their grids, so the bounds themselves (every row
-    on one expert, every expert active) stand in: same result, nothing waits for the GPU, and the
-    whole function can be captured in a HIP graph.  With `host_sync=True` the step-by-step route (an operand that
-    the native operator leaves to it, or `fuse_activation_quant`) still copies them, once.
+    device and use the scalars only as upper bounds for their grids, so with `host_sync=False` the
+    bounds (every row on one expert, every expert active) stand in and nothing waits for the GPU:
+    same result, and the whole function can be captured in a HIP graph.  With `host_sync=True` the scalars are
+    copied, once: when the call returns, the grouping and all work in front of it is done.
 
     By default silu(gate) * up is rounded to bf16 and quantised for the down projection like any bf16 tensor
     (`silu_quantize`: the values of `fused_silu` followed by the quantiser, in one kernel).
@@ -114,7 +114,7 @@ def expert_matmuls_fp8(
         raise ValueError("the FP8 MoE path of this package is the block-scaled one")
     if not fuse_activation_quant and native_granularity(quant_config.input_scale, quant_config.weight_scale) == _lib.GRAN_BLOCK:
         ids = router_idx if router_idx.dtype == torch.int32 else router_idx.to(torch.int32)
-        done = _lib.native().moe_experts(x, ids, gate_up_proj, gate_up_proj_scales, down_proj, down_proj_scales, 1200.0)
+        done = _lib.native().moe_experts(x, ids, gate_up_proj, gate_up_proj_scales, down_proj, down_proj_scales, 1200.0, host_sync)
         if done is not None:
             return done
     strategy = Fp8Strategy(quant_config, gate_up_proj.dtype)

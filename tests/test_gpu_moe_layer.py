@@ -112,3 +112,28 @@ def test_expert_matmuls_replay_from_a_graph(dev):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want), f"replay {i}"
+
+
+def test_host_sync_waits_for_the_routing(dev):
+    """host_sync=True returns after the work in front of the call (a caller may read what it wrote from the host);
+    host_sync=False does not wait for it."""
+    seq, k, E, hidden, inter = 64, 2, 8, 256, 128
+    wgu, sgu = zip(*[synth.quantize_weight_block(synth.weights_f32(2 * inter, hidden, seed=10 + e)) for e in range(E)])
+    wd, sd = zip(*[synth.quantize_weight_block(synth.weights_f32(hidden, inter, seed=100 + e)) for e in range(E)])
+    wgu, sgu, wd, sd = (torch.stack(t).to(dev) for t in (wgu, sgu, wd, sd))
+    x = synth.activations(seq, hidden, seed=1).to(dev)
+    router_idx = torch.randn((seq, E), generator=torch.Generator().manual_seed(5)).topk(k, dim=1).indices.to(torch.int32).to(dev)
+    big = torch.randn((8192, 8192), device=dev)
+    run = lambda wait: mx.expert_matmuls_fp8(x, router_idx, wgu, sgu, wd, sd, BLK, host_sync=wait)
+    want = run(False)
+    torch.mm(big, big)
+    torch.cuda.synchronize()
+    for wait in (False, True):
+        for _ in range(10):                      # (a float32 product of this size takes about 10 ms)
+            torch.mm(big, big)
+        before = torch.cuda.Event()
+        before.record()
+        y = run(wait)
+        assert before.query() == wait
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
