@@ -478,7 +478,8 @@ int maxfp8_quantize_tensor_dynamic_scaled_fp8(
  * topk_ids[i] (int32 / uint32, values in [0, num_experts)) by expert:
  *   token_expert_order[n]   assignment indices grouped by expert slot
  *   expert_start_indices[num_experts + 1]  slot z owns token_expert_order[start[z] .. start[z+1])
- *   restore_token_order[n]  position of assignment i in token_expert_order
+ *   restore_token_order[n]  position of assignment i in token_expert_order; 0xffffffff for an id outside the range, whose
+ *                           assignment belongs to no expert and has no position (the quantiser's scatter form skips it)
  *   expert_ids[num_experts] expert of slot z
  *   expert_usage_stats[2]   {most assignments on one expert, number of slots = num_experts}
  * The reference assigns slots in the order its blocks reach a lock, so any permutation of the

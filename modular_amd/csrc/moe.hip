@@ -17,7 +17,11 @@
 namespace maxfp8 {
 
 // ---- moe_create_indices -----------------------------------------------------------------------
-// block e counts the assignments to expert e; the count waits in expert_start_indices[e + 1].
+// An id that is no expert's: its assignment has no position, and a consumer of restore_token_order skips it as out of range.
+constexpr uint32_t kMoeNoPosition = 0xffffffffu;
+
+// block e counts the assignments to expert e; the count waits in expert_start_indices[e + 1].  The block behind
+// the last expert's marks the assignments to none.
 // V ids per thread and iteration: a multiple of 4 (16-byte loads, topk_ids 16-byte aligned) or 1.  Every block reads all of topk_ids from
 // L2, so what counts is loads in flight: one id per load and iteration took 49 us for 32768 ids, four per load with
 // four loads in flight take a fifth of that.
@@ -38,9 +42,21 @@ __device__ __forceinline__ void moe_load_ids(const int32_t* __restrict__ topk_id
 }
 template <int V>
 __global__ __launch_bounds__(256) void moe_count_kernel(uint32_t* __restrict__ expert_start_indices,
+                                                        uint32_t* __restrict__ restore_token_order,
                                                         const int32_t* __restrict__ topk_ids, int n) {
   __shared__ int red[4];
-  const int e = blockIdx.x, tid = threadIdx.x;
+  const int e = blockIdx.x, tid = threadIdx.x, num_experts = (int)gridDim.x - 1;
+  if (e == num_experts) {
+#pragma unroll 4
+    for (int i = tid * V; i < n; i += 256 * V) {
+      int id[V];
+      moe_load_ids<V>(topk_ids, i, n, id);
+#pragma unroll
+      for (int j = 0; j < V; ++j)
+        if ((uint32_t)id[j] >= (uint32_t)num_experts && i + j < n) restore_token_order[i + j] = kMoeNoPosition;
+    }
+    return;
+  }
   int cnt = 0;
 #pragma unroll 4
   for (int i = tid * V; i < n; i += 256 * V) {
@@ -246,6 +262,8 @@ __global__ __launch_bounds__(1024) void moe_indices_one_block_kernel(uint32_t* _
       const uint32_t pos = counts[wave][id[s]] + rank[s];
       token_expert_order[pos] = (uint32_t)(first + 64 * s);
       restore_token_order[first + 64 * s] = pos;
+    } else if (first + 64 * s < n) {
+      restore_token_order[first + 64 * s] = kMoeNoPosition;
     }
   }
 }
@@ -261,8 +279,10 @@ int moe_create_indices_dispatch(uint32_t* token_expert_order, uint32_t* expert_s
     return launch_status("moe_create_indices");
   }
   const bool vec = (reinterpret_cast<uintptr_t>(topk_ids) & 15) == 0;
-  if (vec) hipLaunchKernelGGL(moe_count_kernel<4>, dim3((unsigned)num_experts), dim3(256), 0, stream, expert_start_indices, topk_ids, (int)n);
-  else hipLaunchKernelGGL(moe_count_kernel<1>, dim3((unsigned)num_experts), dim3(256), 0, stream, expert_start_indices, topk_ids, (int)n);
+  if (vec) hipLaunchKernelGGL(moe_count_kernel<4>, dim3((unsigned)num_experts + 1), dim3(256), 0, stream, expert_start_indices, restore_token_order,
+                              topk_ids, (int)n);
+  else hipLaunchKernelGGL(moe_count_kernel<1>, dim3((unsigned)num_experts + 1), dim3(256), 0, stream, expert_start_indices, restore_token_order,
+                          topk_ids, (int)n);
   hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(1024), 0, stream, expert_start_indices, expert_ids, expert_usage_stats,
                      (int)num_experts);
   if (n > 0) {
