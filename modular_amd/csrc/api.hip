@@ -593,12 +593,10 @@ extern "C" {
 int maxfp8_matmul_describe(int64_t M, int64_t N, int64_t K, int block_scaling, int with_workspace, char* buf, size_t len) {
   if (!buf || len == 0) return 0;
   if (M <= 0 || N <= 0 || K <= 0) return snprintf(buf, len, "nothing to do");
-  // ("skinny" names the launches whose blocks split K among their waves: up to 64 rows both kernels that do, beyond that
-  // the one there is with its tiles)
   int algo = choose_kernel(M, N, K);
   if (algo == MAXFP8_ALGO_TILED && M <= gemm_skinny_max_m() && !with_workspace && gemm_tiled_plan_workspace_bytes(M, N, K, block_scaling != 0) > 0)
     algo = without_workspace(M, N, K);
-  if (algo == MAXFP8_ALGO_SKINNY || (algo == kAlgoMid && M <= gemm_skinny_max_m())) return snprintf(buf, len, "skinny");
+  if (algo == MAXFP8_ALGO_SKINNY) return snprintf(buf, len, "skinny");
   if (algo == kAlgoMid) {
     float us;
     const int sel = tuning().mid > 0 ? tuning().mid : gemm_mid_shape(M, N, K, &us), bm = 16 * (sel / 10), bn = 16 * (sel % 10);

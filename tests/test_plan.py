@@ -15,10 +15,12 @@ def test_single_shapes_and_k_split():
     assert _lib.matmul_describe(2048, 6144, 4096) == "256x256 x192 persistent"
     assert _lib.matmul_describe(2040, 6144, 4096) == "256x256 x192"
     assert _lib.matmul_describe(8, 4096, 4096) == "skinny"
-    assert _lib.matmul_describe(64, 4096, 4096) == "skinny" and _lib.matmul_describe(32, 28672, 4096) == "skinny"
-    # 33 to 64 rows go to the tiles unless the weights are small (under 32 MB): wide matrices, and narrow ones split over K
+    assert _lib.matmul_describe(32, 28672, 4096) == "skinny"
+    # 33 to 64 rows go to the 128-row tiles unless the weights are small (under 32 MB): wide matrices, and narrow ones split over
+    # K; small weights to the tiles whose blocks split K among their waves where those are estimated quicker than the streaming
+    assert "block's waves" in _lib.matmul_describe(64, 4096, 4096) and "block's waves" in _lib.matmul_describe(33, 6144, 4096)
     assert _lib.matmul_describe(64, 28672, 4096).startswith("128x128")
-    assert "K split" in _lib.matmul_describe(48, 8192, 28672) and _lib.matmul_describe(33, 6144, 4096) == "skinny"
+    assert "K split" in _lib.matmul_describe(48, 8192, 28672)
     assert _lib.matmul_describe(48, 8192, 28672, True, False) == "skinny"  # no workspace, no split: the streaming kernel
     # 25 to 32 rows: the tiles only where K is long and N narrow
     assert "K split" in _lib.matmul_describe(32, 8192, 28672) and _lib.matmul_describe(24, 8192, 28672) == "skinny"
