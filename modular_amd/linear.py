@@ -163,11 +163,15 @@ class MLP(torch.nn.Module):
 
     def _down_is_plain(self) -> bool:
         """Whether `down_proj` is what the steps without a call of it compute: a program may have given the block another
-        module in its place, a bias, a static scale, another config or hooks."""
+        module in its place, a bias, a static scale, another config or hooks -- its own or those of every module, as
+        profilers and calibration register them -- or left its scales on another device, which the module's call moves."""
         down = self.down_proj
+        every = torch.nn.modules.module
         return (type(down) is Linear and down.bias is None and down.input_scale is None
                 and (down.quant_config is self.quant_config or down.quant_config == self.quant_config)
-                and not (down._forward_hooks or down._forward_pre_hooks or "forward" in down.__dict__))
+                and down.weight_scale.device == self.gate_up_weight.device
+                and not (down._forward_hooks or down._forward_pre_hooks or "forward" in down.__dict__
+                         or every._global_forward_hooks or every._global_forward_pre_hooks))
 
     def _all_rows(self, rows: int, device: torch.device) -> torch.Tensor:
         """The row_offsets operand of the silu kernels for a dense block: [0, rows] (uint32, on the device).  Kept
