@@ -112,7 +112,8 @@ def expert_matmuls_fp8(
         raise ValueError("expected x [seq, hidden] and router_idx [seq, k]")
     if not (quant_config.input_scale.is_block and quant_config.weight_scale.is_block):
         raise ValueError("the FP8 MoE path of this package is the block-scaled one")
-    if not fuse_activation_quant and native_granularity(quant_config.input_scale, quant_config.weight_scale) == _lib.GRAN_BLOCK:
+    if (not fuse_activation_quant and quant_config.weight_scale.dtype is torch.float32 and
+            native_granularity(quant_config.input_scale, quant_config.weight_scale) == _lib.GRAN_BLOCK):
         ids = router_idx if router_idx.dtype == torch.int32 else router_idx.to(torch.int32)
         done = _lib.native().moe_experts(x, ids, gate_up_proj, gate_up_proj_scales, down_proj, down_proj_scales, 1200.0, host_sync)
         if done is not None:

@@ -1,5 +1,6 @@
 """The native operators' argument checks, without a GPU: what they cannot take is left to the Python wrappers or raises, and
 never ends the process."""
+import dataclasses
 import os
 import subprocess
 import sys
@@ -8,7 +9,8 @@ import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
 
-from modular_amd import _lib
+import modular_amd as mx
+from modular_amd import _lib, moe
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -58,3 +60,32 @@ def test_static_scales_without_a_value(kind):
     done = subprocess.run([sys.executable, "-c", STATIC_SCALES, kind], capture_output=True, text=True, cwd=ROOT)
     assert done.returncode == 0, done.stderr[-2000:]
     assert done.stdout.startswith("raised"), done.stdout
+
+
+class Recorder:
+    """In the place of the native module: every operator takes its operands and says what it was given."""
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        def operator(*args):
+            self.calls.append((name, args))
+            return torch.zeros(1)
+        return operator
+
+
+def test_experts_with_scales_of_another_dtype_are_left_to_the_steps(monkeypatch):
+    """A config of bfloat16 scales with float32 scale tensors: the steps quantise with bfloat16 scales and refuse to mix them."""
+    native = Recorder()
+    monkeypatch.setattr(moe._lib, "native", lambda: native)
+    cfg = mx.blockwise_fp8_config()
+    x, ids = torch.zeros((4, 128), dtype=torch.bfloat16), torch.zeros((4, 2), dtype=torch.int32)
+    w, s = torch.zeros((3, 256, 128), dtype=torch.uint8).view(torch.float8_e4m3fn), torch.zeros((3, 2, 1))
+    moe.expert_matmuls_fp8(x, ids, w, s, w, s, cfg)
+    assert [name for name, _ in native.calls] == ["moe_experts"]
+    native.calls.clear()
+    cfg = dataclasses.replace(cfg, weight_scale=dataclasses.replace(cfg.weight_scale, dtype=torch.bfloat16))
+    with pytest.raises(RuntimeError):  # (the steps, which run on the GPU only)
+        moe.expert_matmuls_fp8(x, ids, w, s, w, s, cfg)
+    assert "moe_experts" not in [name for name, _ in native.calls]
