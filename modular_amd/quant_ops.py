@@ -112,7 +112,7 @@ def quantized_fused_qkv_matmul(
         kind = native_granularity(quant_config.input_scale, quant_config.weight_scale)
         if kind >= 0:
             done = _lib.native().qkv_linear(x, wqkv, weight_scale, kind, 1200.0, input_row_offsets, blocks, kv_collection.cache_lengths,
-                                            kv_collection.lookup_table, bias, layer_idx,
+                                            kv_collection.lookup_table, bias, int(layer_idx),
                                             _output_dim if _output_dim is not None else n_heads * kv_params.head_dim)
             if done is not None:
                 return done

@@ -10,7 +10,7 @@ import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
 
 import modular_amd as mx
-from modular_amd import _lib, moe
+from modular_amd import _lib, moe, quant_ops
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -89,3 +89,17 @@ def test_experts_with_scales_of_another_dtype_are_left_to_the_steps(monkeypatch)
     with pytest.raises(RuntimeError):  # (the steps, which run on the GPU only)
         moe.expert_matmuls_fp8(x, ids, w, s, w, s, cfg)
     assert "moe_experts" not in [name for name, _ in native.calls]
+
+
+@pytest.mark.parametrize("layer", [1, 1.0, torch.tensor(1)])
+def test_layer_index_of_another_type(monkeypatch, layer):
+    """The fused QKV projection's layer is whatever int() takes, as in the wrapper behind the native operator."""
+    native = Recorder()
+    monkeypatch.setattr(quant_ops._lib, "native", lambda: native)
+    kv = mx.KVCacheParams(torch.bfloat16, 1, 64, num_layers=2, page_size=16)
+    u32 = torch.zeros(2, dtype=torch.int32)
+    cache = mx.PagedCacheValues(torch.zeros(kv.blocks_shape(1), dtype=torch.bfloat16), u32[:1], u32[:1].reshape(1, 1))
+    w, s = torch.zeros((384, 128), dtype=torch.uint8).view(torch.float8_e4m3fn), torch.zeros((3, 1))
+    mx.quantized_fused_qkv_matmul(kv, torch.zeros((1, 128), dtype=torch.bfloat16), w, cache, layer, u32, 4, mx.blockwise_fp8_config(), s)
+    (name, args), = native.calls
+    assert name == "qkv_linear" and type(args[10]) is int and args[10] == 1
