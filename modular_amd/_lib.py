@@ -158,14 +158,30 @@ NATIVE_PATH = os.path.join(_HERE, "lib", "_native.so")
 _native = None
 
 
+class _NotBuilt:
+    """Stands for the native module where it was not built: a call with a tensor on the GPU raises, every other is left to the
+    wrapper, whose argument errors come before any library is needed."""
+
+    def __init__(self, path: str) -> None:
+        self.path = path
+
+    def __getattr__(self, name: str):
+        def operator(*args):
+            if any(getattr(a, "is_cuda", False) for a in args):
+                raise LibraryMissing(f"{self.path} not found: build it with `python -m modular_amd.build` (there is no fallback path)")
+            return None
+        return operator
+
+
 def native():
     """The CPython module of the hot operators (csrc/bindings.cpp): each of its functions returns None for what it leaves to
     the Python wrapper."""
     global _native
     if _native is None:
+        for path in (LIB_PATH, NATIVE_PATH):
+            if not os.path.exists(path):
+                return _NotBuilt(path)
         lib()
-        if not os.path.exists(NATIVE_PATH):
-            raise LibraryMissing(f"{NATIVE_PATH} not found: build it with `python -m modular_amd.build`")
         import importlib.machinery
         import importlib.util
 

@@ -103,3 +103,19 @@ def test_layer_index_of_another_type(monkeypatch, layer):
     mx.quantized_fused_qkv_matmul(kv, torch.zeros((1, 128), dtype=torch.bfloat16), w, cache, layer, u32, 4, mx.blockwise_fp8_config(), s)
     (name, args), = native.calls
     assert name == "qkv_linear" and type(args[10]) is int and args[10] == 1
+
+
+@pytest.mark.parametrize("path", ["LIB_PATH", "NATIVE_PATH"])
+def test_argument_errors_come_before_a_missing_library(monkeypatch, path):
+    """Without the built files the wrappers still say what is wrong with their operands; a call for the GPU says what is missing."""
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.setattr(_lib, path, "/nowhere/lib.so")
+    cfg = mx.blockwise_fp8_config()
+    x = torch.zeros((4, 256), dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match="rank 2"):
+        mx.quantize_dynamic_scaled_float8(x[0], cfg.input_scale, cfg.weight_scale, scales_type=torch.float32)
+    with pytest.raises(RuntimeError, match="GPU only"):
+        mx.quantize_dynamic_scaled_float8(x, cfg.input_scale, cfg.weight_scale, scales_type=torch.float32)
+    with FakeTensorMode(), pytest.raises(_lib.LibraryMissing, match="/nowhere/lib.so"):
+        mx.quantize_dynamic_scaled_float8(torch.empty((4, 256), dtype=torch.bfloat16, device="cuda"), cfg.input_scale, cfg.weight_scale,
+                                          scales_type=torch.float32)
