@@ -437,7 +437,8 @@ static int fused_silu_common(void* out, void* out_scales, const void* in, const 
   if (in_dtype != MAXFP8_BF16) MAXFP8_FAIL(MAXFP8_ERR_DTYPE, "fused_silu: input dtype %d is not bf16", in_dtype);
   if (max_rows < 0 || inter < 0 || num_offsets < 1) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused_silu: bad sizes");
   if (max_rows == 0 || inter == 0) return MAXFP8_OK;
-  if (max_rows >= ((int64_t)1 << 31) || inter >= ((int64_t)1 << 30)) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused_silu: sizes must fit 31 bits");
+  // (max_rows is a bound: only the form with one block per row makes it its grid)
+  if (inter >= ((int64_t)1 << 31) || (row_scales && max_rows >= ((int64_t)1 << 31))) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused_silu: sizes must fit 31 bits");
   if (inter % 128 != 0)
     MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused_silu: the output width %lld must be a multiple of 128", (long long)inter);
   const bool quant = mode != 0 && mode != 2;

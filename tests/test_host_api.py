@@ -290,3 +290,15 @@ def test_quantized_grouped_matmul_and_strategy_argument_rules():
     assert a is ws and b is off
     with pytest.raises(RuntimeError, match="GPU only"):
         st.quantize(x, 128)
+
+
+@pytest.mark.parametrize("rows, inter", [(1, (1 << 30) + 128), (1 << 31, 128)])
+def test_fused_silu_size_limits(rows, inter):
+    """Outputs of 2^30 and more columns, and a bound of 2^31 and more rows, are within the kernel's arithmetic: what is refused
+    here is the null pointer, which is looked at after the sizes."""
+    L = _lib.lib()
+    assert L.maxfp8_fused_silu(None, None, None, None, 2, rows, inter, 2 * inter, inter, 0, _lib.BF16, 0, None) == _lib.ERR_NULL
+    assert L.maxfp8_fused_silu(None, None, None, None, 2, 1, 1 << 31, 1 << 32, 1 << 31, 0, _lib.BF16, 0, None) == _lib.ERR_SHAPE
+    # (the form with one block per row launches one for every row of the bound)
+    assert L.maxfp8_silu_quantize_dynamic_scaled_fp8(None, None, None, None, 2, 1 << 31, 256, 512, 256, 256, 1, _lib.BF16, 0, 0.0,
+                                                     None) == _lib.ERR_SHAPE
