@@ -60,6 +60,7 @@ int gemm_skinny_dispatch(const GemmArgs&, bool, int64_t, hipStream_t);
 bool gemm_skinny_quant_ok(int64_t M, int64_t N, int64_t K, bool blockscale);
 int gemm_skinny_quant_dispatch(const GemmArgs&, bool, hipStream_t);
 int gemm_skinny_max_m();
+int compute_units();
 bool gemm_short_k_ok(const GemmArgs&, bool, int64_t);
 int gemm_short_k_dispatch(const GemmArgs&, int64_t, hipStream_t);
 int gemm_mid_dispatch(const GemmArgs&, bool, hipStream_t);
@@ -492,6 +493,14 @@ static int without_workspace(int64_t M, int64_t N, int64_t K) {
   return mid < 0.92f * gemm_skinny_cost(M, N, K) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
 }
 
+// A batch of short K and more than 32 rows on the tiles: one slab of K leaves three of the decode kernel's four waves idle, and
+// beyond one of its 16-row blocks per CU every block more reads the tokens again.  With one block per CU or less it is ahead from
+// two slabs on (decode kernel against tiles, 48 rows, us, cold: 32 x 512 -> 128 5.4 and 6.4, 48 of them 7.8 and 6.5, 128 12.7
+// and 6.7; 16 x 256 -> 256 4.8 and 5.3, 24 of them 6.3 and 5.3; 16 x 128 -> 512 5.6 and 4.8, 128 of them 28.7 and 6.7).
+static bool batch_on_tiles(int64_t batch, int64_t M, int64_t N, int64_t K) {
+  return M > 32 && K <= 512 && (K <= 128 || ceil_div(N, 16) * batch > (int64_t)compute_units());
+}
+
 static int matmul_common(void* c, const void* a, const void* b, const void* a_scales, const void* b_scales, int64_t M,
                          int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int input_granularity,
                          int weight_granularity, int64_t gm, int64_t gn, int64_t gk, int64_t a_scales_ld,
@@ -531,9 +540,7 @@ static int matmul_common(void* c, const void* a, const void* b, const void* a_sc
   if (automatic) {
     if (!fast_layout) algo = MAXFP8_ALGO_NAIVE;
     else if (bt.n == 1) algo = choose_kernel(M, N, K);
-    // (a batch of short K and more than 32 rows: the tiles -- 128 heads x 48 x 512 x 128: 6.6 us against the decode kernel's 31,
-    // 48 x 128 x 512: 6.6 against 14.5; 16 heads: 4.1 against 5.2 and 6.1 against 5.5)
-    else if (gemm_skinny_preferred(M, N, K) && !(bt.n > 1 && M > 32 && K <= 512)) algo = MAXFP8_ALGO_SKINNY;
+    else if (gemm_skinny_preferred(M, N, K) && !batch_on_tiles(bt.n, M, N, K)) algo = MAXFP8_ALGO_SKINNY;
     else algo = MAXFP8_ALGO_TILED;
     // 33 to 64 rows: the tiles win through their K split.  Without the workspace the split needs, a narrow weight
     // matrix would run on a fraction of the chip: the streaming kernel then.  (What this shape's own plan needs, not the

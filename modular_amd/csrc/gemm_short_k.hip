@@ -90,12 +90,14 @@ int compute_units();
 
 // Batches of at most 32 tokens, whole slabs and whole 32-column groups, bf16 results with 16-byte rows; every other shape
 // keeps the other kernels.  With three or four slabs the decode kernel's waves all have a share, and it stays ahead while its
-// 16-row blocks are at most two per CU (16 heads of 512 -> 128: 3.1 against 4.0 us at M = 1; 128 heads: 5.9 against 4.9).
+// 16-row blocks are at most two per CU (16 heads of 512 -> 128: 3.1 against 4.0 us at M = 1; 128 heads: 5.9 against 4.9) and,
+// with two groups of tokens, which are a wave each here and one pass over the weights there, at most one (17 to 32 tokens: 16 and
+// 32 heads of 512 -> 128 4.5 and 4.7 us against 5.4 and 5.3, 48 heads 6.3 against 5.9).
 bool gemm_short_k_ok(const GemmArgs& p, bool blockscale, int64_t batch) {
   if (!blockscale || !tuning().short_k || batch < 2 || p.kv_on || p.M > 32 || p.K % 128 != 0 || p.K > 512 || p.N % 32 != 0 ||
       p.c_dtype != MAXFP8_BF16 || !p.c_vec8_ok)
     return false;
-  return p.K <= 256 || p.M > 16 || ceil_div(p.N, 16) * batch > 2 * (int64_t)compute_units();
+  return p.K <= 256 || ceil_div(p.N, 16) * batch > (p.M > 16 ? 1 : 2) * (int64_t)compute_units();
 }
 
 template <int NS, int MT>

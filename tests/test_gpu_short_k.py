@@ -20,7 +20,8 @@ def reference(a, b, sa, sb):
 
 
 @pytest.mark.parametrize("B,M,N,K", [(2, 1, 32, 128), (3, 16, 160, 128), (5, 17, 512, 128), (2, 32, 96, 256), (3, 20, 288, 384),
-                                     (2, 17, 128, 512), (2, 31, 64, 512), (70, 5, 128, 512), (2, 33, 128, 128), (3, 12, 40, 128)])
+                                     (2, 17, 128, 512), (2, 31, 64, 512), (70, 5, 128, 512), (2, 33, 128, 128), (3, 12, 40, 128),
+                                     (40, 20, 288, 384), (40, 17, 128, 512), (70, 31, 64, 512)])
 @pytest.mark.parametrize("exact", [True, False])
 def test_short_k_batches(dev, B, M, N, K, exact):
     g = torch.Generator().manual_seed(B + M + N + K)
@@ -47,3 +48,18 @@ def test_short_k_batches(dev, B, M, N, K, exact):
     else:
         assert_rel(f32_np(y).reshape(B * M, N), want.reshape(B * M, N), 1e-2, "short K")
     assert bool((out[0] == 7).all()) and bool((out[M + 1] == 7).all()) and bool((out[:, :, N:] == 7).all())
+
+
+@pytest.mark.parametrize("B,M,N,K,decode", [(32, 48, 128, 512, True), (48, 48, 128, 512, False), (16, 33, 256, 256, True), (24, 64, 256, 256, False),
+                                            (2, 64, 1024, 384, True), (32, 32, 128, 512, True), (48, 32, 128, 512, False)])
+def test_decode_kernel_up_to_one_block_per_cu(dev, B, M, N, K, decode):
+    """From two slabs on the decode kernel runs while its 16-row blocks are at most one per CU (more than 16 tokens).  Seen in the
+    bits: it rounds a slab's scaled sum before it adds it, the others add in one fused step -- two float32 results in five differ,
+    and of the 131072 and more bf16 ones of 32 tokens (whose kernel has no float32 form) half a dozen."""
+    out_type = torch.float32 if M > 32 else torch.bfloat16
+    a, b = synth.random_fp8((B, M, K), 1).to(dev), synth.random_fp8((B, N, K), 2).to(dev)
+    sa, sb = synth.random_scales((B, K // 128, -(-M // 4) * 4), 3).to(dev), synth.random_scales((B, -(-N // 128), K // 128), 4).to(dev)
+    run = lambda algo: mx.batched_dynamic_scaled_fp8_matmul(a, b, sa, sb, BLK.input_scale, BLK.weight_scale, out_type, algo=algo)
+    assert torch.equal(run("auto"), run("skinny")) == decode
+    if M > 32:
+        assert torch.equal(run("auto"), run("tiled")) != decode
