@@ -66,7 +66,8 @@ int gemm_short_k_dispatch(const GemmArgs&, int64_t, hipStream_t);
 int gemm_mid_dispatch(const GemmArgs&, bool, hipStream_t);
 bool gemm_mid_ok(int64_t M, int64_t N, int64_t K);
 int gemm_mid_shape(int64_t M, int64_t N, int64_t K, float* us);
-float gemm_skinny_cost(int64_t M, int64_t N, int64_t K);
+bool gemm_mid_before_skinny(int64_t M, int64_t N, int64_t K, bool blockscale, bool qkv);
+float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
 float gemm_tiled_small_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
 float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool has_workspace);
 size_t gemm_tiled_qkv_workspace_bytes(int64_t M, int64_t N, int64_t K, bool blockscale);
@@ -208,74 +209,72 @@ constexpr int kAlgoMid = 100;
 
 // Which kernel MAXFP8_ALGO_AUTO gives a fast-layout matmul whose caller brings all the workspace it is asked for.  At most
 // 16 rows: the decode kernel.  Up to 64 rows: the decode kernel's own rule between itself and the tiles, the tiles also where
-// they are estimated 8 per cent quicker (the estimates' own error); up to 320 the tiles.  Against either the kernel in between,
-// by the same 8 per cent (up to 32 rows, where wide matrices miss their estimate by more, 15; against unsplit tiles, whose
-// estimate is the roughest, 25: 36 x 17632 x 3328 19 against 24 us, 140 x 1728 x 768 7.6 against 5.5).  Where the tiles' plan is none of the small ones (no estimate) they keep what they get.  Forced
-// shapes keep the other kernels out.
-static int choose_uncached(int64_t M, int64_t N, int64_t K) {
+// they are estimated 8 per cent quicker (the estimates' own error); up to 320 the tiles.  Against the decode kernel the one in
+// between by gemm_mid_before_skinny, against the tiles by the same 8 per cent (against unsplit tiles, whose estimate is the
+// roughest, 25: 36 x 17632 x 3328 19 against 24 us, 140 x 1728 x 768 7.6 against 5.5).  Where the tiles' plan is none of the small
+// ones (no estimate) they keep what they get.  Forced shapes keep the other kernels out.
+static int choose_uncached(int64_t M, int64_t N, int64_t K, bool block) {
   const Tuning& t = tuning();
   const int plain = gemm_skinny_preferred(M, N, K) ? MAXFP8_ALGO_SKINNY : MAXFP8_ALGO_TILED;
   if (t.mid > 0) return gemm_mid_ok(M, N, K) ? kAlgoMid : plain;
   if (M <= 16 || M > 320 || t.mid == 0 || t.tile || t.splitk || t.one_region || t.w4 >= 0 || t.w4_split == 1 || t.skinny) return plain;
   const float tiles = gemm_tiled_small_cost(M, N, K, true);
-  int algo = plain;
-  float us = tiles;
-  if (M <= 64) {
-    const float decode = gemm_skinny_cost(M, N, K);
-    if (plain == MAXFP8_ALGO_SKINNY) {
-      us = decode;
-      // (unsplit tiles in the decode kernel's range only for the shortest K, where four waves have no K to split: 48 x 32768 x 512
-      // 17.2 against 7.8 us; 49 x 20272 x 640 with row scales 10.9 against 13.0)
-      const bool splits = gemm_tiled_plan_workspace_bytes(M, N, K, true) > 0;
-      if (tiles > 0.f && tiles < 0.92f * decode && (splits || K <= 512)) {
-        us = tiles;
-        algo = MAXFP8_ALGO_TILED;
-      }
-    }
+  const bool splits = gemm_tiled_plan_workspace_bytes(M, N, K, true) > 0;
+  if (plain == MAXFP8_ALGO_SKINNY) {
+    // (unsplit tiles in the decode kernel's range only for the shortest K, where four waves have no K to split: 48 x 32768 x 512 with
+    // block scales 17.2 against 7.8 us; with row scales, which cost the decode kernel less, from its seventh block per CU on: 48 x
+    // 32768 x 512 14.8 against 10.1, but 57 x 20080 x 512 10.6 against 12.9, 62 x 8400 x 512 8.1 against 12.4, 24 x 32768 x 512 1.10)
+    const bool unsplit = K <= 512 && (block || (M > 32 && ceil_div(N, 16) > 6 * (int64_t)compute_units()));
+    // (up to 32 rows split tiles only from its fourth block per CU on: 24 x 17920 x 6528 31.5 against 28.7; its estimate is 10 to 20
+    // per cent high on narrow weights with long K)
+    const bool split = splits && (M > 32 || ceil_div(N, 16) > 3 * (int64_t)compute_units());
+    const bool on_tiles = tiles > 0.f && tiles < 0.92f * gemm_skinny_cost(M, N, K, block) && (split || (!splits && unsplit));
+    if (!on_tiles) return gemm_mid_before_skinny(M, N, K, block, false) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
   }
-  if (us == 0.f || !gemm_mid_ok(M, N, K)) return algo;
+  if (tiles == 0.f || M <= 32 || !gemm_mid_ok(M, N, K)) return MAXFP8_ALGO_TILED;
   float mid;
   gemm_mid_shape(M, N, K, &mid);
-  const float margin = algo == MAXFP8_ALGO_TILED && gemm_tiled_plan_workspace_bytes(M, N, K, true) == 0 ? 0.75f : M <= 32 ? 0.85f : 0.92f;
-  return mid < margin * us ? kAlgoMid : algo;
+  return mid < (splits ? 0.92f : 0.75f) * tiles ? kAlgoMid : MAXFP8_ALGO_TILED;
 }
-// (asked on every call: the answers are kept, keyed by the shape and the generation of the tuning switches)
-static int choose_kernel(int64_t M, int64_t N, int64_t K) {
-  if (M <= 16) return tuning().mid > 0 ? choose_uncached(M, N, K) : MAXFP8_ALGO_SKINNY;
+// (asked on every call: the answers are kept, keyed by the shape, the scaling and the generation of the tuning switches)
+static int choose_kernel(int64_t M, int64_t N, int64_t K, bool block) {
+  if (M <= 16) return tuning().mid > 0 ? choose_uncached(M, N, K, block) : MAXFP8_ALGO_SKINNY;
   if (M > 320) return MAXFP8_ALGO_TILED;
-  struct Entry { int64_t M, N, K; unsigned generation; int algo; };
+  struct Entry { int64_t M, N, K; unsigned generation; int algo; bool block; };
   static Entry table[128];  // (algo 0: empty)
   static std::mutex mu;
   const unsigned generation = tuning().generation;
-  const uint64_t h = ((uint64_t)M * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)N * 0xc2b2ae3d27d4eb4full) ^ ((uint64_t)K * 0x165667b19e3779f9ull);
+  const uint64_t h = ((uint64_t)M * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)N * 0xc2b2ae3d27d4eb4full) ^ ((uint64_t)K * 0x165667b19e3779f9ull) ^ (block ? 1ull << 32 : 0);
   Entry& e = table[(h >> 32) % 128];
   {
     std::lock_guard<std::mutex> lock(mu);
-    if (e.algo && e.M == M && e.N == N && e.K == K && e.generation == generation) return e.algo;
+    if (e.algo && e.M == M && e.N == N && e.K == K && e.block == block && e.generation == generation) return e.algo;
   }
-  const int algo = choose_uncached(M, N, K);
+  const int algo = choose_uncached(M, N, K, block);
   std::lock_guard<std::mutex> lock(mu);
-  e = Entry{M, N, K, generation, algo};
+  e = Entry{M, N, K, generation, algo, block};
   return algo;
+}
+// the workspace MAXFP8_ALGO_AUTO uses with this scaling
+static size_t auto_workspace(int64_t M, int64_t N, int64_t K, bool block) {
+  return choose_kernel(M, N, K, block) == MAXFP8_ALGO_TILED ? gemm_tiled_workspace_bytes(M, N, K) : 0;
 }
 
 // The same for the fused QKV matmul: decode kernel (at most 64 rows), the kernel in between (at most 320) or the tiles, whose
 // plan may cut them along K where the caller brings a workspace.
-static int choose_qkv(int64_t T, int64_t N, int64_t K, bool has_workspace) {
+static int choose_qkv(int64_t T, int64_t N, int64_t K, bool has_workspace, bool block) {
   const Tuning& t = tuning();
   const int plain = T <= gemm_skinny_max_m() ? MAXFP8_ALGO_SKINNY : MAXFP8_ALGO_TILED;
   if (t.mid > 0) return gemm_mid_ok(T, N, K) ? kAlgoMid : plain;
   if (T <= 16 || !gemm_mid_ok(T, N, K) || t.mid == 0 || t.tile || t.skinny) return plain;
+  const float tiles = gemm_tiled_qkv_cost(T, N, K, true, has_workspace);
+  if (plain == MAXFP8_ALGO_SKINNY) {
+    if (gemm_mid_before_skinny(T, N, K, block, true)) return kAlgoMid;
+    return tiles < 0.92f * gemm_skinny_cost(T, N, K, block) ? MAXFP8_ALGO_TILED : MAXFP8_ALGO_SKINNY;
+  }
   float mid;
   gemm_mid_shape(T, N, K, &mid);
-  const float tiles = gemm_tiled_qkv_cost(T, N, K, true, has_workspace);
-  float us = tiles;
-  int algo = MAXFP8_ALGO_TILED;
-  if (T <= gemm_skinny_max_m()) {
-    const float decode = gemm_skinny_cost(T, N, K);
-    if (decode < us) { us = decode; algo = MAXFP8_ALGO_SKINNY; }
-  }
-  return mid < 0.92f * us ? kAlgoMid : algo;
+  return mid < 0.92f * tiles ? kAlgoMid : MAXFP8_ALGO_TILED;
 }
 }  // namespace maxfp8
 
@@ -471,13 +470,14 @@ int maxfp8_silu_quantize_dynamic_scaled_fp8(void* out_fp8, void* out_scales, con
 }
 
 size_t maxfp8_matmul_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0 || K <= 0 || (gemm_skinny_preferred(M, N, K) && choose_kernel(M, N, K) != MAXFP8_ALGO_TILED)) return 0;
+  if (M <= 0 || N <= 0 || K <= 0 || (gemm_skinny_preferred(M, N, K) && !auto_workspace(M, N, K, true) && !auto_workspace(M, N, K, false))) return 0;
   return gemm_tiled_workspace_bytes(M, N, K);  // split-K partial sums; 0 when no split would be used
 }
 
 size_t maxfp8_matmul_auto_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0 || K <= 0 || choose_kernel(M, N, K) != MAXFP8_ALGO_TILED) return 0;
-  return gemm_tiled_workspace_bytes(M, N, K);
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const size_t block = auto_workspace(M, N, K, true);
+  return block ? block : auto_workspace(M, N, K, false);
 }
 
 }  // extern "C"
@@ -486,11 +486,9 @@ namespace maxfp8 {
 struct BatchStrides { int64_t n, a, b, c, a_scales, b_scales; };  // n batches; steps in elements
 
 // 17 to 64 rows whose tiles would split K, without the workspace for it
-static int without_workspace(int64_t M, int64_t N, int64_t K) {
-  float mid;
-  if (M <= 16 || tuning().mid == 0 || tuning().skinny || !gemm_mid_ok(M, N, K)) return MAXFP8_ALGO_SKINNY;
-  gemm_mid_shape(M, N, K, &mid);
-  return mid < 0.92f * gemm_skinny_cost(M, N, K) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
+static int without_workspace(int64_t M, int64_t N, int64_t K, bool block) {
+  if (M <= 16 || tuning().mid == 0 || tuning().skinny) return MAXFP8_ALGO_SKINNY;
+  return gemm_mid_before_skinny(M, N, K, block, false) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
 }
 
 // A batch of short K and more than 32 rows on the tiles: one slab of K leaves three of the decode kernel's four waves idle, and
@@ -539,7 +537,7 @@ static int matmul_common(void* c, const void* a, const void* b, const void* a_sc
   const bool automatic = algo == MAXFP8_ALGO_AUTO;
   if (automatic) {
     if (!fast_layout) algo = MAXFP8_ALGO_NAIVE;
-    else if (bt.n == 1) algo = choose_kernel(M, N, K);
+    else if (bt.n == 1) algo = choose_kernel(M, N, K, block);
     else if (gemm_skinny_preferred(M, N, K) && !batch_on_tiles(bt.n, M, N, K)) algo = MAXFP8_ALGO_SKINNY;
     else algo = MAXFP8_ALGO_TILED;
     // 33 to 64 rows: the tiles win through their K split.  Without the workspace the split needs, a narrow weight
@@ -547,7 +545,7 @@ static int matmul_common(void* c, const void* a, const void* b, const void* a_sc
     // worst case over all tile shapes: a plan that does not split runs the same with and without a workspace.)
     if (algo == MAXFP8_ALGO_TILED && M <= gemm_skinny_max_m() && bt.n == 1 &&
         gemm_tiled_plan_workspace_bytes(M, N, K, block) > (workspace ? workspace_bytes : 0))
-      algo = without_workspace(M, N, K);
+      algo = without_workspace(M, N, K, block);
   }
   if (algo == MAXFP8_ALGO_NAIVE) {
     if (block)
@@ -601,9 +599,9 @@ extern "C" {
 int maxfp8_matmul_describe(int64_t M, int64_t N, int64_t K, int block_scaling, int with_workspace, char* buf, size_t len) {
   if (!buf || len == 0) return 0;
   if (M <= 0 || N <= 0 || K <= 0) return snprintf(buf, len, "nothing to do");
-  int algo = choose_kernel(M, N, K);
+  int algo = choose_kernel(M, N, K, block_scaling != 0);
   if (algo == MAXFP8_ALGO_TILED && M <= gemm_skinny_max_m() && !with_workspace && gemm_tiled_plan_workspace_bytes(M, N, K, block_scaling != 0) > 0)
-    algo = without_workspace(M, N, K);
+    algo = without_workspace(M, N, K, block_scaling != 0);
   if (algo == MAXFP8_ALGO_SKINNY) return snprintf(buf, len, "skinny");
   if (algo == kAlgoMid) {
     float us;
@@ -636,8 +634,7 @@ int maxfp8_matmul_dynamic_scaled_fp8_noalloc(void* c, const void* a, const void*
   // entry points add the same partial sums in the same order.
   const bool block = input_granularity == MAXFP8_GRAN_BLOCK && weight_granularity == MAXFP8_GRAN_BLOCK;
   size_t need = 0;
-  const size_t useful = algo == MAXFP8_ALGO_AUTO ? maxfp8_matmul_auto_workspace_bytes(M, N, K) : maxfp8_matmul_workspace_bytes(M, N, K);
-  if (M > 0 && N > 0 && K > 0 && useful > 0) need = gemm_tiled_plan_workspace_bytes(M, N, K, block);
+  if (M > 0 && N > 0 && K > 0 && (algo == MAXFP8_ALGO_AUTO ? auto_workspace(M, N, K, block) : maxfp8_matmul_workspace_bytes(M, N, K)) > 0) need = gemm_tiled_plan_workspace_bytes(M, N, K, block);
   if (need > kScratchBytes)
     MAXFP8_FAIL(MAXFP8_ERR_WORKSPACE,
                 "matmul (no-alloc): the split of %lld x %lld x %lld uses %zu bytes of scratch, the library's static buffer holds "
@@ -666,13 +663,13 @@ static LinearLayout linear_layout(int64_t M, int64_t N, int64_t K, bool block, b
   l.scales_ld = block ? ceil_div(M, 4) * 4 : M;
   l.scales = up((size_t)M * (size_t)K);
   l.partial = l.scales + up((fixed ? 2 : block ? (size_t)(K / 128) * l.scales_ld : (size_t)M) * 4);
-  l.partial_bytes = maxfp8_matmul_auto_workspace_bytes(M, N, K);
+  l.partial_bytes = M > 0 && N > 0 && K > 0 ? auto_workspace(M, N, K, block) : 0;
   l.total = l.partial + l.partial_bytes;
   return l;
 }
 // does the decode kernel quantise by itself? (the layout as far as it is the operands': see linear_common)
 static bool linear_in_one(int64_t M, int64_t N, int64_t K, bool block) {
-  return M > 0 && N > 0 && K > 0 && choose_kernel(M, N, K) == MAXFP8_ALGO_SKINNY && gemm_skinny_quant_ok(M, N, K, block);
+  return M > 0 && N > 0 && K > 0 && choose_kernel(M, N, K, block) == MAXFP8_ALGO_SKINNY && gemm_skinny_quant_ok(M, N, K, block);
 }
 
 static int linear_common(void* y, const void* x, const void* w, const void* w_scales, int64_t M, int64_t N, int64_t K, int64_t ldx,
@@ -855,7 +852,7 @@ static int qkv_common(void* output, const void* input, const void* x, int64_t ld
     return gemm_skinny_quant_dispatch(p, block, st);
   }
   const bool automatic = algo == MAXFP8_ALGO_AUTO;
-  if (automatic) algo = choose_qkv(T, N, K, workspace != nullptr);
+  if (automatic) algo = choose_qkv(T, N, K, workspace != nullptr, block);
   if (automatic && algo == kAlgoMid) return gemm_mid_dispatch(p, block, st);
   if (algo == MAXFP8_ALGO_SKINNY) return gemm_skinny_dispatch(p, block, 1, st);
   if (algo != MAXFP8_ALGO_TILED) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused qkv matmul: algo %d is not available", algo);
@@ -879,11 +876,11 @@ int maxfp8_fused_qkv_matmul_ragged_paged_scale(void* output, const void* input, 
 }
 
 static bool qkv_in_one(int64_t T, int64_t N, int64_t K, bool block) {
-  return T > 0 && N > 0 && K > 0 && choose_qkv(T, N, K, true) == MAXFP8_ALGO_SKINNY && gemm_skinny_quant_ok(T, N, K, block);
+  return T > 0 && N > 0 && K > 0 && choose_qkv(T, N, K, true, block) == MAXFP8_ALGO_SKINNY && gemm_skinny_quant_ok(T, N, K, block);
 }
 // what follows the quantised activations and their scales: the sums of cut tiles
 static size_t qkv_partial_bytes(int64_t T, int64_t N, int64_t K, bool block) {
-  return choose_qkv(T, N, K, true) == MAXFP8_ALGO_TILED ? gemm_tiled_qkv_workspace_bytes(T, N, K, block) : 0;
+  return choose_qkv(T, N, K, true, block) == MAXFP8_ALGO_TILED ? gemm_tiled_qkv_workspace_bytes(T, N, K, block) : 0;
 }
 
 size_t maxfp8_linear_qkv_workspace_bytes(int64_t T, int64_t N, int64_t K, int weight_granularity) {

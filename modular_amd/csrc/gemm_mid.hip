@@ -27,6 +27,13 @@
 
 namespace maxfp8 {
 
+// Slabs in flight per wave: a quarter of the LDS, the 6-bit wait counter, at most six
+__host__ __device__ constexpr int mid_depth(int mt, int nt, bool blockscale) {
+  const int slot = (mt + nt) * 2048 + (blockscale ? 256 : 0), per = 2 * (mt + nt) + (blockscale ? 1 : 0);
+  const int lds = (160 * 1024 - 16 * mt * 8) / 4 / slot, counter = 63 / per + 1, least = lds < counter ? lds : counter;
+  return least > 6 ? 6 : least;
+}
+
 template <int MT, int NT, bool BLOCKSCALE>
 struct MidCfg {
   static constexpr int BM = 16 * MT, BN = 16 * NT;
@@ -34,10 +41,7 @@ struct MidCfg {
   static constexpr int SLOT = (MT + NT) * 2048 + SCALES;
   static constexpr int PER = 2 * (MT + NT) + (BLOCKSCALE ? 1 : 0);  // copies per wave and slab
   static constexpr int ROW_TABLE = BM * 8;                   // fused QKV: the cache row of every token
-  static constexpr int BUDGET = (160 * 1024 - ROW_TABLE) / 4;
-  static constexpr int D_LDS = BUDGET / SLOT, D_CNT = 63 / PER + 1;
-  static constexpr int D_MIN = D_LDS < D_CNT ? D_LDS : D_CNT;
-  static constexpr int DEPTH = D_MIN > 6 ? 6 : D_MIN;
+  static constexpr int DEPTH = mid_depth(MT, NT, BLOCKSCALE);
   static constexpr int RING = DEPTH * SLOT;
   static constexpr int RED_LD = BN + 4;                      // floats per token row of a partial tile
   static constexpr int RED = 4 * BM * RED_LD * 4;
@@ -274,6 +278,7 @@ static int launch_mid(const GemmArgs& p, hipStream_t stream) {
 }
 
 int compute_units();
+float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
 
 // Estimated times (microseconds), fitted to launches of every kernel on 26 weight matrices (K 512 ... 28672, N 576 ... 32768)
 // at 4 to 400 tokens in both scale modes, operands cold: within 15 per cent for nine launches in ten.
@@ -312,6 +317,34 @@ int gemm_mid_shape(int64_t M, int64_t N, int64_t K, float* us) {
     if (best == 0 || c < *us) { best = 10 * t.mt + t.nt; *us = c; }
   }
   return best;
+}
+
+// What that shape takes at 33 to 64 rows, for the comparison with the decode kernel: one estimate per scaling, with the slabs of
+// a wave in whole rounds of its ring (the launches of gemm_skinny_cost: within 9 per cent for nine in ten)
+float gemm_mid_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
+  float us;
+  const int sel = gemm_mid_shape(M, N, K, &us), mt = sel / 10, nt = sel % 10, depth = mid_depth(mt, nt, blockscale);
+  const float rounds = (float)ceil_div(ceil_div(M, 16 * mt) * ceil_div(N, 16 * nt), compute_units());
+  const int64_t slabs = ceil_div(K, 512);
+  const float walked = (float)(ceil_div(slabs, depth) * depth), stream = (float)N * (float)K * 1e-8f;
+  if (blockscale) return 1.91f + 12.6f * stream + rounds * (1.46f + 0.139f * (float)(mt * nt) + 0.049f * (float)(slabs * (mt + nt)) + 0.214f * walked);
+  return 1.58f + 10.9f * stream + rounds * (2.15f + 0.188f * (float)(mt * nt) + 0.058f * (float)(slabs * (mt + nt)) + 0.162f * walked);
+}
+
+// The kernel here or the decode kernel, 17 to 64 rows.
+// Up to 32 rows the decode kernel reads the tokens with half the loads and is ahead or level nearly everywhere (17 / 24 / 32 x 1536 x
+// 7168 8.8 / 9.9 / 11.0 us against 10.2 / 10.7 / 11.4, 20 x 5040 x 6528 11.0 against 12.4, 28 x 24624 x 2560 20.8 against 21.8) but
+// where its third block per CU runs all but alone: 22 x 9648 x 6912 0.81 of its time, 27 x 11328 x 1152 0.87 (shorter K: 1.0 to 1.1).
+// Beyond, by the estimates: 33 x 4096 x 4096 9.7 against 8.2 us, 47 x 9152 x 1024 9.9 against 7.1 -- but 36 x 6272 x 512 5.0 against
+// 5.8 and, with row scales, 39 x 21600 x 896 11.6 against 15.2 (block scales: 14.4 and 12.8).
+bool gemm_mid_before_skinny(int64_t M, int64_t N, int64_t K, bool blockscale, bool qkv) {
+  if (!gemm_mid_ok(M, N, K)) return false;
+  if (M <= 32) return K > 1024 && ceil_div(ceil_div(N, 16), compute_units()) == 3;
+  // (Beyond 3072 the estimate here is the higher one of the two by 6 per cent.  The fused QKV projection's epilogue costs more here, a
+  // microsecond per block and round: 48 x 2048 x 1536 7.0 against 7.7 us, 56 x 7168 x 5120 17.7 against 18.8, with row scales 18.2, 48 x
+  // 17408 x 2048 with row scales 20.9 against 26.7.)
+  const float margin = qkv ? (K < 3072 ? 0.90f : blockscale ? 0.95f : 1.06f) : K > 3072 ? 1.06f : 1.0f;
+  return gemm_mid_cost(M, N, K, blockscale) < margin * gemm_skinny_cost(M, N, K, blockscale);
 }
 
 template <bool BLOCKSCALE>

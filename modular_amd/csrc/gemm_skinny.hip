@@ -699,13 +699,22 @@ bool gemm_skinny_preferred(int64_t M, int64_t N, int64_t K) {
   return M <= 64 && small_weights;
 }
 
-// Estimated microseconds at 17 to 64 rows (fitted like gemm_mid_shape's: within 12 per cent for nine launches in ten)
-float gemm_skinny_cost(int64_t M, int64_t N, int64_t K) {
+// Estimated microseconds at 17 to 64 rows.  Up to 32 only the tiles are compared with it; beyond, the kernel for tens of tokens
+// too, so the estimate is one per scaling and counts the slabs a wave walks as its ring does, in whole rounds (fitted to 960
+// launches per scaling, 33 to 64 rows of 576 ... 32768 x 512 ... 12288, operands cold: within 6 per cent for nine in ten).
+float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
   const int ntw = skinny_shape(M, N, K) / 1000;
   const float blocks = (float)ceil_div(ceil_div(N, 16 * ntw), compute_units());  // per CU
-  const float w = blocks * (float)(ntw * 16) * (float)K * 1e-5f;                 // weight bytes per CU
-  if (M <= 32) return 3.0f + 0.84f * blocks + 2.62f * w + 1.62f * blocks * 32.f * (float)K * 1e-5f;
-  return 3.2f + 1.11f * blocks * (float)ntw + 2.88f * w + 1.41f * blocks * 64.f * (float)K * 1e-5f;
+  if (M <= 32) {
+    const float w = blocks * (float)(ntw * 16) * (float)K * 1e-5f;               // weight bytes per CU
+    return 3.0f + 0.84f * blocks + 2.62f * w + 1.62f * blocks * 32.f * (float)K * 1e-5f;
+  }
+  const int depth = ntw == 4   ? (blockscale ? SkinnyCfg<4, 4, true, 32, 4>::DEPTH : SkinnyCfg<4, 4, false, 32, 4>::DEPTH)
+                    : ntw == 2 ? (blockscale ? SkinnyCfg<2, 4, true, 8, 4>::DEPTH : SkinnyCfg<2, 4, false, 8, 4>::DEPTH)
+                               : (blockscale ? SkinnyCfg<1, 4, true, 8, 4>::DEPTH : SkinnyCfg<1, 4, false, 8, 4>::DEPTH);
+  const float slabs = (float)(ceil_div(ceil_div(K, 512), depth) * depth), k = (float)K;
+  if (blockscale) return 1.32f + blocks * (1.75f + 0.356f * (float)ntw + 0.24f * slabs + (3.80e-4f * (float)ntw + 1.62e-5f * (float)M) * k);
+  return 3.26f + blocks * (0.596f * (float)ntw + 0.099f * slabs + (4.20e-4f * (float)ntw + 1.88e-5f * (float)M) * k);
 }
 
 int gemm_skinny_dispatch(const GemmArgs& p, bool blockscale, int64_t batch, hipStream_t stream) {

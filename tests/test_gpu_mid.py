@@ -63,7 +63,7 @@ def test_every_tile_shape_is_exact(dev, forced, kind, shape):
 
 
 @pytest.mark.parametrize("kind", ["block", "row"])
-@pytest.mark.parametrize("M,N,K", [(17, 1536, 7168), (33, 576, 7168), (64, 4096, 4096), (65, 4096, 4096), (117, 6144, 4096),
+@pytest.mark.parametrize("M,N,K", [(17, 10240, 2176), (33, 576, 7168), (64, 4096, 4096), (65, 4096, 4096), (117, 6144, 4096),
                                    (256, 1536, 7168), (320, 576, 7168)])
 def test_chosen_shapes_against_the_oracle(dev, kind, M, N, K):
     assert "K split over the block's waves" in _lib.matmul_describe(M, N, K)

@@ -77,3 +77,26 @@ def test_four_wave_kernel_where_its_tile_count_fits_the_chip(tune):
     assert _lib.matmul_describe(4096, 7168, 16384) == "160x256 x728 persistent, four waves"
     assert "tail cut in pieces of 8 slabs" in _lib.matmul_describe(2040, 6144, 4096)
     assert "tail cut" not in _lib.matmul_describe(2040, 6144, 4096 + 256)
+
+
+def test_the_kernel_for_tens_of_tokens_against_the_decode_kernel():
+    """Up to 32 rows only where the decode kernel's third block per CU would run all but alone; beyond, by estimates of their own
+    for block and row scales; unsplit tiles for the shortest K."""
+    kind = lambda *a, **kw: "mid" if "block's waves" in _lib.matmul_describe(*a, **kw) else _lib.matmul_describe(*a, **kw)
+    for block in (True, False):
+        for M in (17, 24, 32):
+            for N, K in ((1536, 7168), (576, 7168), (2112, 7168), (4096, 4096), (6144, 4096), (704, 11520), (28672, 4096)):
+                assert kind(M, N, K, block) == "skinny", (M, N, K)
+            assert kind(M, 10240, 8192, block) == "mid"
+        for M in (33, 48, 64):
+            assert kind(M, 4096, 4096, block) == "mid" and kind(M, 1536, 7168, block) == "mid" and kind(M, 10240, 8192, block) == "mid"
+            assert kind(M, 6272, 512, block) == "skinny"
+        assert kind(17, 8208, 1024, block) == "skinny" and kind(17, 8208, 1152, block) == "mid" == kind(32, 12288, 1152, block)
+        assert kind(32, 8192, 1152, block) == "skinny" == kind(32, 12304, 1152, block)
+    # wide and short: the decode kernel pays for block scales, and is ahead without them
+    assert kind(39, 21600, 896) == "mid" and kind(39, 21600, 896, False) == "skinny"
+    assert "128x128" in kind(24, 32768, 512) and kind(24, 32768, 512, False) == "skinny"
+    assert "128x128" in kind(48, 32768, 512, False) and kind(57, 20080, 512, False) == "skinny"
+    # (no scaling is named: what either of them uses)
+    assert kind(20, 18784, 6656).endswith("K split 3") and _lib.lib().maxfp8_matmul_auto_workspace_bytes(20, 18784, 6656) > 0
+    assert _lib.lib().maxfp8_matmul_auto_workspace_bytes(24, 1536, 7168) == 0
