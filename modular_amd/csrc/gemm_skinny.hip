@@ -550,7 +550,8 @@ static int pick_ntw(const GemmArgs& p, int64_t batch, hipStream_t stream) {
 // Every block repeats the work, a third of a microsecond per 512 elements of a wave (its conversions come one after the
 // other, one wave per SIMD): with eight loads per wave the two ways are level (4 tokens of 4096: 9.1 and 8.6 us; 8 tokens 9.5
 // and 11.7).  With row scales every token costs a meeting of the waves on top, once per block of a CU: at most four tokens,
-// and together with the blocks a CU works on at most eight of them (4 tokens on 28672 x 4096: 24.9 and 26.3 us).
+// on at most three blocks per CU, and with those at most eight (2 tokens on 24576 x 4096, three blocks, 20.0 and 17.9 us; on 28672 x
+// 4096, four, 22.8 and 24.5; 4 tokens on 16384 x 4096, two blocks, 15.8 and 14.2).
 constexpr int kQuantLoads = 8;
 static int skinny_quant_loads(int64_t M, int64_t K) {
   return (int)(M * ceil_div(ceil_div(ceil_div(K, 128), 4), 4));
@@ -558,7 +559,7 @@ static int skinny_quant_loads(int64_t M, int64_t K) {
 template <int NTW, bool BLOCKSCALE, int RING_KB>
 static bool skinny_quant_fits(int64_t M, int64_t N, int64_t K) {
   const int64_t per_cu = ceil_div(ceil_div(N, 16 * NTW), (int64_t)compute_units());
-  if (skinny_quant_loads(M, K) > kQuantLoads || (!BLOCKSCALE && M > 1 && (M > 4 || M * per_cu > 8))) return false;
+  if (skinny_quant_loads(M, K) > kQuantLoads || (!BLOCKSCALE && M > 1 && (M > 4 || per_cu > 3 || M * per_cu > 8))) return false;
   // (the quantised activations of the blocks that are on a CU together -- three keep the weight stream full -- fit its LDS)
   const uint32_t per_wave = (uint32_t)ceil_div(ceil_div(K, 128), 4);
   const int64_t smem = SkinnyCfg<NTW, 1, BLOCKSCALE, RING_KB, 4, kQuantLoads>::SMEM +

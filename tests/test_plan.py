@@ -100,3 +100,11 @@ def test_the_kernel_for_tens_of_tokens_against_the_decode_kernel():
     # (no scaling is named: what either of them uses)
     assert kind(20, 18784, 6656).endswith("K split 3") and _lib.lib().maxfp8_matmul_auto_workspace_bytes(20, 18784, 6656) > 0
     assert _lib.lib().maxfp8_matmul_auto_workspace_bytes(24, 1536, 7168) == 0
+
+
+def test_rows_quantised_inside_the_decode_kernel():
+    """With row scales at most three blocks per CU for more than one token, and four tokens on two; with block scales four of them."""
+    need = lambda M, N, K, gran: _lib.lib().maxfp8_linear_workspace_bytes(M, N, K, gran)
+    for M, N, inside in ((1, 28672, True), (2, 24576, True), (2, 28672, False), (3, 16384, True), (3, 24576, False), (4, 16384, True), (5, 4096, False)):
+        assert (need(M, N, 4096, _lib.GRAN_ROWWISE) == 0) == inside, (M, N)
+    assert need(4, 28672, 4096, _lib.GRAN_BLOCK) == 0 < need(5, 28672, 4096, _lib.GRAN_BLOCK)
