@@ -283,7 +283,7 @@ size_t maxfp8_matmul_auto_workspace_bytes(int64_t M, int64_t N, int64_t K);
  * Either one launch -- a few tokens: the decode kernel quantises what it needs itself -- or the quantiser and
  * MAXFP8_ALGO_AUTO's matmul through the workspace, of maxfp8_linear_workspace_bytes bytes (0 for the one launch, which
  * takes 16-byte aligned rows; weight_granularity TENSOR for the static form).  Same results as the ops one by one.
- * The _qkv_ form is maxfp8_fused_qkv_matmul_ragged_paged_scale behind the same quantisation.
+ * The _qkv_ form is maxfp8_fused_qkv_matmul_ragged_paged_scale_workspace behind the same quantisation.
  */
 size_t maxfp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int weight_granularity);
 int maxfp8_linear_dynamic_scaled_fp8(
@@ -358,6 +358,24 @@ int maxfp8_fused_qkv_matmul_ragged_paged_scale(
     int64_t gm, int64_t gn, int64_t gk,
     int64_t input_scale_ld, int64_t weight_scale_ld,
     int scales_dtype, int algo, void* stream);
+
+/*
+ * The same with MAXFP8_ALGO_AUTO and a workspace, of maxfp8_fused_qkv_matmul_workspace_bytes bytes (often 0), for the sums of tiles
+ * that are cut along K.  Where tiles are cut the sums are added in another order than without, so the last bits may differ.
+ */
+size_t maxfp8_fused_qkv_matmul_workspace_bytes(int64_t T, int64_t N, int64_t K, int block_scaling);
+int maxfp8_fused_qkv_matmul_ragged_paged_scale_workspace(
+    void* output, const void* input, const uint32_t* input_row_offsets,
+    const void* wqkv, const void* input_scale, const void* weight_scale,
+    void* kv_blocks, const uint32_t* cache_lengths, const uint32_t* lookup_table,
+    const void* bias,
+    int64_t T, int64_t N, int64_t K, int64_t q_dim, int64_t batch_size,
+    int64_t num_blocks, int64_t kv_dim, int64_t num_layers, int64_t layer_idx,
+    int64_t page_size, int64_t num_kv_heads, int64_t head_dim, int64_t lut_ld,
+    int64_t gm, int64_t gn, int64_t gk,
+    int64_t input_scale_ld, int64_t weight_scale_ld,
+    int scales_dtype, void* workspace,
+    size_t workspace_bytes, void* stream);
 
 /*
  * Grouped (MoE) blockwise-scaled FP8 matmul over token rows sorted by expert.

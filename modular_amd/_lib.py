@@ -45,6 +45,8 @@ EXPORTS = (
     "maxfp8_grouped_matmul_dynamic_scaled_fp8",
     "maxfp8_grouped_matmul_rowwise_dynamic_scaled_fp8",
     "maxfp8_fused_qkv_matmul_ragged_paged_scale",
+    "maxfp8_fused_qkv_matmul_workspace_bytes",
+    "maxfp8_fused_qkv_matmul_ragged_paged_scale_workspace",
     "maxfp8_quantize_static_scaled_fp8",
     "maxfp8_quantize_tensor_dynamic_scaled_fp8",
     "maxfp8_moe_create_indices",
@@ -126,6 +128,10 @@ def lib() -> ctypes.CDLL:
     L.maxfp8_grouped_matmul_rowwise_dynamic_scaled_fp8.argtypes = [vp] * 7 + [i64] * 6 + [ci, ci, vp]
     L.maxfp8_fused_qkv_matmul_ragged_paged_scale.restype = ci
     L.maxfp8_fused_qkv_matmul_ragged_paged_scale.argtypes = [vp] * 10 + [i64] * 18 + [ci, ci, vp]
+    L.maxfp8_fused_qkv_matmul_workspace_bytes.restype = ctypes.c_size_t
+    L.maxfp8_fused_qkv_matmul_workspace_bytes.argtypes = [i64, i64, i64, ci]
+    L.maxfp8_fused_qkv_matmul_ragged_paged_scale_workspace.restype = ci
+    L.maxfp8_fused_qkv_matmul_ragged_paged_scale_workspace.argtypes = [vp] * 10 + [i64] * 18 + [ci, vp, ctypes.c_size_t, vp]
     L.maxfp8_quantize_static_scaled_fp8.restype = ci
     L.maxfp8_quantize_static_scaled_fp8.argtypes = [vp, vp, i64, i64, i64, i64, ci, cf, vp]
     L.maxfp8_quantize_tensor_dynamic_scaled_fp8.restype = ci

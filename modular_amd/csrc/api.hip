@@ -766,7 +766,8 @@ int maxfp8_batched_matmul_dynamic_scaled_fp8(void* c, const void* a, const void*
 
 }  // extern "C"
 
-// x != nullptr: the decode kernel quantises x (bf16 rows of ldx elements) by itself; input and input_scale are not used
+// x != nullptr: the decode kernel quantises x (bf16 rows of ldx elements) by itself; input and input_scale are not used.
+// with_workspace: the caller brings qkv_partial_bytes bytes (which may be none).
 static int qkv_common(void* output, const void* input, const void* x, int64_t ldx, float scale_ub, const uint32_t* input_row_offsets,
                                                const void* wqkv, const void* input_scale, const void* weight_scale,
                                                void* kv_blocks, const uint32_t* cache_lengths, const uint32_t* lookup_table,
@@ -774,8 +775,8 @@ static int qkv_common(void* output, const void* input, const void* x, int64_t ld
                                                int64_t batch_size, int64_t num_blocks, int64_t kv_dim, int64_t num_layers,
                                                int64_t layer_idx, int64_t page_size, int64_t num_kv_heads, int64_t head_dim,
                                                int64_t lut_ld, int64_t gm, int64_t gn, int64_t gk, int64_t input_scale_ld,
-                                               int64_t weight_scale_ld, int scales_dtype, int algo, void* workspace, size_t workspace_bytes,
-                                               void* stream) {
+                                               int64_t weight_scale_ld, int scales_dtype, int algo, bool with_workspace, void* workspace,
+                                               size_t workspace_bytes, void* stream) {
   if (T < 0 || N < 0 || K < 0 || q_dim < 0 || batch_size < 0) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused qkv matmul: negative size");
   if (batch_size == 0 || T == 0 || N == 0) return MAXFP8_OK;  // kv_cache_ragged.mojo:1193-1194
   if (T >= ((int64_t)1 << 31) || N >= ((int64_t)1 << 31) || K >= ((int64_t)1 << 31) || batch_size >= ((int64_t)1 << 31))
@@ -852,7 +853,7 @@ static int qkv_common(void* output, const void* input, const void* x, int64_t ld
     return gemm_skinny_quant_dispatch(p, block, st);
   }
   const bool automatic = algo == MAXFP8_ALGO_AUTO;
-  if (automatic) algo = choose_qkv(T, N, K, workspace != nullptr, block);
+  if (automatic) algo = choose_qkv(T, N, K, with_workspace, block);
   if (automatic && algo == kAlgoMid) return gemm_mid_dispatch(p, block, st);
   if (algo == MAXFP8_ALGO_SKINNY) return gemm_skinny_dispatch(p, block, 1, st);
   if (algo != MAXFP8_ALGO_TILED) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused qkv matmul: algo %d is not available", algo);
@@ -872,7 +873,7 @@ int maxfp8_fused_qkv_matmul_ragged_paged_scale(void* output, const void* input, 
                                                int64_t weight_scale_ld, int scales_dtype, int algo, void* stream) {
   return qkv_common(output, input, nullptr, 0, 0.f, input_row_offsets, wqkv, input_scale, weight_scale, kv_blocks, cache_lengths, lookup_table,
                     bias, T, N, K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads, head_dim, lut_ld, gm,
-                    gn, gk, input_scale_ld, weight_scale_ld, scales_dtype, algo, nullptr, 0, stream);
+                    gn, gk, input_scale_ld, weight_scale_ld, scales_dtype, algo, false, nullptr, 0, stream);
 }
 
 static bool qkv_in_one(int64_t T, int64_t N, int64_t K, bool block) {
@@ -881,6 +882,26 @@ static bool qkv_in_one(int64_t T, int64_t N, int64_t K, bool block) {
 // what follows the quantised activations and their scales: the sums of cut tiles
 static size_t qkv_partial_bytes(int64_t T, int64_t N, int64_t K, bool block) {
   return choose_qkv(T, N, K, true, block) == MAXFP8_ALGO_TILED ? gemm_tiled_qkv_workspace_bytes(T, N, K, block) : 0;
+}
+
+size_t maxfp8_fused_qkv_matmul_workspace_bytes(int64_t T, int64_t N, int64_t K, int block_scaling) {
+  return T > 0 && N > 0 && K > 0 ? qkv_partial_bytes(T, N, K, block_scaling != 0) : 0;
+}
+
+int maxfp8_fused_qkv_matmul_ragged_paged_scale_workspace(
+    void* output, const void* input, const uint32_t* input_row_offsets, const void* wqkv, const void* input_scale, const void* weight_scale,
+    void* kv_blocks, const uint32_t* cache_lengths, const uint32_t* lookup_table, const void* bias, int64_t T, int64_t N, int64_t K,
+    int64_t q_dim, int64_t batch_size, int64_t num_blocks, int64_t kv_dim, int64_t num_layers, int64_t layer_idx, int64_t page_size,
+    int64_t num_kv_heads, int64_t head_dim, int64_t lut_ld, int64_t gm, int64_t gn, int64_t gk, int64_t input_scale_ld,
+    int64_t weight_scale_ld, int scales_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  const bool block = !(gk == -1 && gm == gn && (gm == -1 || gm == 1));
+  const size_t need = maxfp8_fused_qkv_matmul_workspace_bytes(T, N, K, block);
+  if (need > 0 && (!workspace || workspace_bytes < need))
+    MAXFP8_FAIL(MAXFP8_ERR_WORKSPACE, "fused qkv matmul: needs %zu bytes of workspace, got %zu", need, workspace ? workspace_bytes : (size_t)0);
+  if (need > 0 && !is_aligned(workspace, 16)) MAXFP8_FAIL(MAXFP8_ERR_ALIGN, "fused qkv matmul: workspace must be 16-byte aligned");
+  return qkv_common(output, input, nullptr, 0, 0.f, input_row_offsets, wqkv, input_scale, weight_scale, kv_blocks, cache_lengths, lookup_table,
+                    bias, T, N, K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads, head_dim, lut_ld, gm,
+                    gn, gk, input_scale_ld, weight_scale_ld, scales_dtype, MAXFP8_ALGO_AUTO, true, need ? workspace : nullptr, need, stream);
 }
 
 size_t maxfp8_linear_qkv_workspace_bytes(int64_t T, int64_t N, int64_t K, int weight_granularity) {
@@ -906,7 +927,7 @@ int maxfp8_linear_qkv_ragged_paged_scale(void* output, const void* x, int64_t x_
   if (qkv_in_one(T, N, K, block) && is_aligned(x, 16) && x_row_stride % 8 == 0 && 32 * x_row_stride < ((int64_t)1 << 31))
     return qkv_common(output, nullptr, x, x_row_stride, scale_ub, input_row_offsets, wqkv, nullptr, weight_scale, kv_blocks, cache_lengths,
                       lookup_table, bias, T, N, K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads,
-                      head_dim, lut_ld, gm, gn, gk, 0, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_SKINNY, nullptr, 0, stream);
+                      head_dim, lut_ld, gm, gn, gk, 0, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_SKINNY, false, nullptr, 0, stream);
   const LinearLayout l = linear_layout(T, N, K, block, false);
   const size_t partial = qkv_partial_bytes(T, N, K, block), total = l.partial + partial;
   if (!workspace || workspace_bytes < total)
@@ -919,7 +940,7 @@ int maxfp8_linear_qkv_ragged_paged_scale(void* output, const void* x, int64_t x_
   if (rc != MAXFP8_OK) return rc;
   return qkv_common(output, q, nullptr, 0, 0.f, input_row_offsets, wqkv, scales, weight_scale, kv_blocks, cache_lengths, lookup_table, bias, T, N,
                     K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads, head_dim, lut_ld, gm, gn, gk,
-                    block ? l.scales_ld : T, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_AUTO, q + l.partial, partial, stream);
+                    block ? l.scales_ld : T, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_AUTO, true, partial ? q + l.partial : nullptr, partial, stream);
 }
 
 }  // extern "C"

@@ -601,12 +601,20 @@ def _qkv_cache_matmul(kv_params: KVCacheParams, input: torch.Tensor, input_row_o
     out = torch.empty((T, q_dim), dtype=torch.bfloat16, device=input.device)
     in_ld = input_scale.shape[1] if input_scale.dim() == 2 else 1
     w_ld = weight_scale.shape[1] if weight_scale.dim() == 2 else 1
-    st = _lib.lib().maxfp8_fused_qkv_matmul_ragged_paged_scale(
+    operands = (
         out.data_ptr() if q_dim else None, input.data_ptr(), row_offsets.data_ptr(), weight.data_ptr(),
         input_scale.data_ptr(), weight_scale.data_ptr(), blocks.data_ptr(), cache_lengths.data_ptr(), lut.data_ptr(),
         bias.data_ptr() if bias is not None else None, T, N, K, q_dim, batch, blocks.shape[0], kv_params.kv_dim,
         kv_params.num_layers, int(layer_idx), kv_params.page_size, kv_params.n_kv_heads, kv_params.head_dim,
-        lut.shape[1], *scales_granularity_mnk, in_ld, w_ld, _lib.F32, _ALGOS[algo], _stream(input))
+        lut.shape[1], *scales_granularity_mnk, in_ld, w_ld, _lib.F32)
+    if algo == "auto" and q_dim:
+        # the sums of tiles cut along K, as in the step from bfloat16 activations (maxfp8_linear_qkv_ragged_paged_scale)
+        need = _lib.lib().maxfp8_fused_qkv_matmul_workspace_bytes(T, N, K, int(tuple(scales_granularity_mnk) not in ((-1, -1, -1), (1, 1, -1))))
+        ws = torch.empty((need,), dtype=torch.uint8, device=input.device) if need else None
+        st = _lib.lib().maxfp8_fused_qkv_matmul_ragged_paged_scale_workspace(*operands, ws.data_ptr() if ws is not None else None, need,
+                                                                             _stream(input))
+    else:
+        st = _lib.lib().maxfp8_fused_qkv_matmul_ragged_paged_scale(*operands, _ALGOS[algo], _stream(input))
     _lib.check(st)
     return out
 

@@ -101,12 +101,17 @@ def test_experts_have_the_bits_of_their_steps(dev):
     assert torch.equal(y.reshape(seq * k, H), mm(hq, hs, d, sd, out_row_index=order))
 
 
+# a few tokens, more sequences, more tokens; a projection whose tiles are cut along K (150 tokens fill its two row tiles badly, 200 well)
 @pytest.mark.parametrize("kind", ["block", "row"])
 @pytest.mark.parametrize("bias", [False, True])
-@pytest.mark.parametrize("lens", [[1], [1, 1, 1], [2, 30, 1, 40]])
-def test_qkv_linear_has_the_bits_of_its_steps(dev, kind, bias, lens):
-    heads, kv_heads, D, K, page, cached = 4, 2, 64, 512, 16, 9
+@pytest.mark.parametrize("lens,shape", [([1], (4, 2, 64, 512)), ([1, 1, 1], (4, 2, 64, 512)), ([2, 30, 1, 40], (4, 2, 64, 512)),
+                                        ([60, 1, 89], (32, 8, 128, 8192)), ([130, 70], (32, 8, 128, 8192))])
+def test_qkv_linear_has_the_bits_of_its_steps(dev, kind, bias, lens, shape):
+    heads, kv_heads, D, K = shape
+    page, cached = 16, 9
     T, N = sum(lens), (heads + 2 * kv_heads) * D
+    if T == 200:
+        assert _lib.lib().maxfp8_fused_qkv_matmul_workspace_bytes(T, N, K, int(kind == "block")) > 0, "tiles cut along K"
     w, ws = weight(N, K, kind, dev, seed=1)
     x = synth.activations(T, K, seed=2, device=dev)
     kv = mx.KVCacheParams(torch.bfloat16, kv_heads, D, num_layers=2, page_size=page)
@@ -124,6 +129,10 @@ def test_qkv_linear_has_the_bits_of_its_steps(dev, kind, bias, lens):
     xq, xs = mx.quantize_dynamic_scaled_float8(x, cfg.input_scale, cfg.weight_scale, scales_type=torch.float32)
     want = mx.fused_qkv_ragged_matmul_scaled_float8(kv, xq, offsets, w, two, 1, heads, xs, ws, bias=b, quant_config=cfg)
     assert torch.equal(q, want) and torch.equal(one.kv_blocks, two.kv_blocks)
+    # an operand that the native operator leaves to the wrapper: channels that are not contiguous
+    three = cache()
+    q = mx.quantized_fused_qkv_matmul(kv, x.t().contiguous().t(), w, three, 1, offsets, heads, cfg, ws, bias=b)
+    assert torch.equal(q, want) and torch.equal(three.kv_blocks, two.kv_blocks)
 
 
 def test_what_the_native_operators_leave_to_the_wrappers(dev):
