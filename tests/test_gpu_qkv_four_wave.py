@@ -26,6 +26,15 @@ def test_whole_tiles_exact(dev, tune, tm, mnk, prompt, cached, page):
              algo="tiled", bias=True, exact=True)
 
 
+@pytest.mark.parametrize("mnk", [BLOCK, ROW])
+@pytest.mark.parametrize("kv_dim", [1, 2])
+def test_key_cache_only(dev, tune, mnk, kv_dim):
+    """No Q at all: every column of every tile goes to the pages, C is null with rows of no length (the K-cache matmul)."""
+    tune(MAXFP8_W4="5")
+    run_case(dev, [210, 0, 190], [100, 3, 37], Hq=0, H=21, D=16, K=512, mnk=mnk, page=128, layers=2, layer=1, nblocks=40, seed=8,
+             algo="tiled", k_only=True, kv_dim=kv_dim, exact=True)
+
+
 @pytest.mark.parametrize("mnk", [BLOCK, ROW, TENSOR])
 def test_whole_tiles(dev, tune, mnk):
     tune(MAXFP8_W4="6")
