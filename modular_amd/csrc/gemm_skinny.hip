@@ -315,7 +315,7 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in)
         }
       }
     } else {
-      // one scale per token: the waves' shares meet in LDS (word 16 * wave + t of the first wave's scale area)
+      // one scale per token: the waves' shares meet in LDS (word t of each wave's scale area)
       float* meet = reinterpret_cast<float*>(smem + Cfg::RINGS + (uint32_t)p.M * a_tok);
       constexpr uint32_t kWaveStep = 16;  // (each wave's area holds 32 words: 16 for the waves' values of ITS tokens, 16 scales)
       const uint32_t area = skinny_acts_bytes<ACTS, BLOCKSCALE>((uint32_t)p.M, (uint32_t)per_wave) / 4u;
