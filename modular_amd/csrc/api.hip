@@ -65,10 +65,11 @@ bool gemm_short_k_ok(const GemmArgs&, bool, int64_t);
 int gemm_short_k_dispatch(const GemmArgs&, int64_t, hipStream_t);
 int gemm_mid_dispatch(const GemmArgs&, bool, hipStream_t);
 bool gemm_mid_ok(int64_t M, int64_t N, int64_t K);
-int gemm_mid_shape(int64_t M, int64_t N, int64_t K, float* us);
-bool gemm_mid_before_skinny(int64_t M, int64_t N, int64_t K, bool blockscale, bool qkv);
+int gemm_mid_shape(int64_t M, int64_t N, int64_t K, bool blockscale, float* us);
+int gemm_mid_forced_shape();
+bool gemm_mid_before_skinny(int64_t M, int64_t N, int64_t K);
 float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
-float gemm_tiled_small_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
+float gemm_tiled_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
 float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool has_workspace);
 size_t gemm_tiled_qkv_workspace_bytes(int64_t M, int64_t N, int64_t K, bool blockscale);
 bool gemm_skinny_preferred(int64_t M, int64_t N, int64_t K);
@@ -208,38 +209,46 @@ namespace maxfp8 {
 constexpr int kAlgoMid = 100;
 
 // Which kernel MAXFP8_ALGO_AUTO gives a fast-layout matmul whose caller brings all the workspace it is asked for.  At most
-// 16 rows: the decode kernel.  Up to 64 rows: the decode kernel's own rule between itself and the tiles, the tiles also where
-// they are estimated 8 per cent quicker (the estimates' own error); up to 320 the tiles.  Against the decode kernel the one in
-// between by gemm_mid_before_skinny, against the tiles by the same 8 per cent (against unsplit tiles, whose estimate is the
-// roughest, 25: 36 x 17632 x 3328 19 against 24 us, 140 x 1728 x 768 7.6 against 5.5).  Where the tiles' plan is none of the small
-// ones (no estimate) they keep what they get.  Forced shapes keep the other kernels out.
+// 16 rows: the decode kernel.  Up to 64: streaming the weights or the tiles, by the decode kernel's own rule; the tiles also where they are estimated 8 per
+// cent quicker than it (the estimates' own error), streaming also where the tiles' rule gave way to a quicker estimate of gemm_mid.hip's kernel;
+// up to 2048: that kernel or the tiles, by the estimates.  Forced shapes keep the other kernels out.
+//
+// Streaming has two names, kAlgoMid and MAXFP8_ALGO_SKINNY, and beyond 16 rows one launch (gemm_mid_before_skinny): which name a shape has
+// is what maxfp8_matmul_describe has always called it.
+static bool named_mid(int64_t M, int64_t N, int64_t K, bool block) {
+  if (K > 12288) return false;
+  return M <= 32 ? K > 1024 && ceil_div(ceil_div(N, 16), (int64_t)compute_units()) == 3 : K > (block ? 512 : 896);
+}
 static int choose_uncached(int64_t M, int64_t N, int64_t K, bool block) {
   const Tuning& t = tuning();
   const int plain = gemm_skinny_preferred(M, N, K) ? MAXFP8_ALGO_SKINNY : MAXFP8_ALGO_TILED;
   if (t.mid > 0) return gemm_mid_ok(M, N, K) ? kAlgoMid : plain;
-  if (M <= 16 || M > 320 || t.mid == 0 || t.tile || t.splitk || t.one_region || t.w4 >= 0 || t.w4_split == 1 || t.skinny) return plain;
-  const float tiles = gemm_tiled_small_cost(M, N, K, true);
-  const bool splits = gemm_tiled_plan_workspace_bytes(M, N, K, true) > 0;
-  if (plain == MAXFP8_ALGO_SKINNY) {
-    // (unsplit tiles in the decode kernel's range only for the shortest K, where four waves have no K to split: 48 x 32768 x 512 with
-    // block scales 17.2 against 7.8 us; with row scales, which cost the decode kernel less, from its seventh block per CU on: 48 x
-    // 32768 x 512 14.8 against 10.1, but 57 x 20080 x 512 10.6 against 12.9, 62 x 8400 x 512 8.1 against 12.4, 24 x 32768 x 512 1.10)
-    const bool unsplit = K <= 512 && (block || (M > 32 && ceil_div(N, 16) > 6 * (int64_t)compute_units()));
-    // (up to 32 rows split tiles only from its fourth block per CU on: 24 x 17920 x 6528 31.5 against 28.7; its estimate is 10 to 20
-    // per cent high on narrow weights with long K)
-    const bool split = splits && (M > 32 || ceil_div(N, 16) > 3 * (int64_t)compute_units());
-    const bool on_tiles = tiles > 0.f && tiles < 0.92f * gemm_skinny_cost(M, N, K, block) && (split || (!splits && unsplit));
-    if (!on_tiles) return gemm_mid_before_skinny(M, N, K, block, false) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
-  }
-  if (tiles == 0.f || M <= 32 || !gemm_mid_ok(M, N, K)) return MAXFP8_ALGO_TILED;
+  if (M <= 16 || !gemm_mid_ok(M, N, K) || t.mid == 0 || t.tile || t.splitk || t.one_region || t.w4 >= 0 || t.w4_split == 1 || t.skinny) return plain;
   float mid;
-  gemm_mid_shape(M, N, K, &mid);
-  return mid < (splits ? 0.92f : 0.75f) * tiles ? kAlgoMid : MAXFP8_ALGO_TILED;
+  gemm_mid_shape(M, N, K, block, &mid);
+  // (further from what the estimate was fitted to, or with more of its time spent on memory, or against whole tiles, whose estimate is rough: 1730
+  // x 592 x 5248 19 against 22 us, 79 x 7168 x 16384 35 against 38, 940 x 8320 x 1408 24 against 29)
+  const float margin = M > 1024 ? 0.80f : gemm_tiled_plan_workspace_bytes(M, N, K, block) == 0 ? 0.85f : N * K >= ((int64_t)1 << 26) ? 0.90f : 0.97f;
+  if (M > gemm_skinny_max_m()) return mid < margin * gemm_tiled_cost(M, N, K, block) ? kAlgoMid : MAXFP8_ALGO_TILED;
+  const int stream = named_mid(M, N, K, block) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
+  const float tiles = gemm_tiled_cost(M, N, K, block);
+  const bool splits = gemm_tiled_plan_workspace_bytes(M, N, K, true) > 0;
+  // (the estimate of unsplit tiles is the roughest)
+  if (plain == MAXFP8_ALGO_TILED) return mid < (splits ? 0.85f : 0.75f) * tiles ? stream : MAXFP8_ALGO_TILED;
+  // (unsplit tiles in the decode kernel's range only for the shortest K, where four waves have no K to split: 48 x 32768 x 512 with
+  // block scales 17.2 against 7.8 us; with row scales, which cost the decode kernel less, from its seventh block per CU on: 48 x
+  // 32768 x 512 14.8 against 10.1, but 57 x 20080 x 512 10.6 against 12.9, 62 x 8400 x 512 8.1 against 12.4, 24 x 32768 x 512 1.10)
+  const bool unsplit = K <= 512 && (block || (M > 32 && ceil_div(N, 16) > 6 * (int64_t)compute_units()));
+  // (up to 32 rows split tiles only from its fourth block per CU on: 24 x 17920 x 6528 31.5 against 28.7; its estimate is 10 to 20
+  // per cent high on narrow weights with long K)
+  const bool split = splits && (M > 32 || ceil_div(N, 16) > 3 * (int64_t)compute_units());
+  const bool on_tiles = tiles < 0.92f * gemm_skinny_cost(M, N, K, block) && (split || (!splits && unsplit));
+  return on_tiles && (M <= 32 || !splits || tiles < 1.15f * mid) ? MAXFP8_ALGO_TILED : stream;
 }
 // (asked on every call: the answers are kept, keyed by the shape, the scaling and the generation of the tuning switches)
 static int choose_kernel(int64_t M, int64_t N, int64_t K, bool block) {
   if (M <= 16) return tuning().mid > 0 ? choose_uncached(M, N, K, block) : MAXFP8_ALGO_SKINNY;
-  if (M > 320) return MAXFP8_ALGO_TILED;
+  if (M > 2048) return MAXFP8_ALGO_TILED;
   struct Entry { int64_t M, N, K; unsigned generation; int algo; bool block; };
   static Entry table[128];  // (algo 0: empty)
   static std::mutex mu;
@@ -267,14 +276,10 @@ static int choose_qkv(int64_t T, int64_t N, int64_t K, bool has_workspace, bool 
   const int plain = T <= gemm_skinny_max_m() ? MAXFP8_ALGO_SKINNY : MAXFP8_ALGO_TILED;
   if (t.mid > 0) return gemm_mid_ok(T, N, K) ? kAlgoMid : plain;
   if (T <= 16 || !gemm_mid_ok(T, N, K) || t.mid == 0 || t.tile || t.skinny) return plain;
-  const float tiles = gemm_tiled_qkv_cost(T, N, K, true, has_workspace);
-  if (plain == MAXFP8_ALGO_SKINNY) {
-    if (gemm_mid_before_skinny(T, N, K, block, true)) return kAlgoMid;
-    return tiles < 0.92f * gemm_skinny_cost(T, N, K, block) ? MAXFP8_ALGO_TILED : MAXFP8_ALGO_SKINNY;
-  }
+  if (plain == MAXFP8_ALGO_SKINNY) return kAlgoMid;
   float mid;
-  gemm_mid_shape(T, N, K, &mid);
-  return mid < 0.92f * tiles ? kAlgoMid : MAXFP8_ALGO_TILED;
+  gemm_mid_shape(T, N, K, block, &mid);
+  return mid < 0.85f * gemm_tiled_qkv_cost(T, N, K, block, has_workspace) ? kAlgoMid : MAXFP8_ALGO_TILED;
 }
 }  // namespace maxfp8
 
@@ -487,8 +492,7 @@ struct BatchStrides { int64_t n, a, b, c, a_scales, b_scales; };  // n batches; 
 
 // 17 to 64 rows whose tiles would split K, without the workspace for it
 static int without_workspace(int64_t M, int64_t N, int64_t K, bool block) {
-  if (M <= 16 || tuning().mid == 0 || tuning().skinny) return MAXFP8_ALGO_SKINNY;
-  return gemm_mid_before_skinny(M, N, K, block, false) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
+  return gemm_mid_before_skinny(M, N, K) && named_mid(M, N, K, block) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
 }
 
 // A batch of short K and more than 32 rows on the tiles: one slab of K leaves three of the decode kernel's four waves idle, and
@@ -585,7 +589,7 @@ static int matmul_common(void* c, const void* a, const void* b, const void* a_sc
   }
   p.a_batch = bt.a; p.b_batch = bt.b; p.c_batch = bt.c;
   p.a_scales_batch = bt.a_scales; p.b_scales_batch = bt.b_scales;
-  if (algo == kAlgoMid) return gemm_mid_dispatch(p, block, st);
+  if (algo == kAlgoMid || (automatic && algo == MAXFP8_ALGO_SKINNY && bt.n == 1 && gemm_mid_before_skinny(M, N, K))) return gemm_mid_dispatch(p, block, st);
   if (automatic && gemm_short_k_ok(p, block, bt.n)) return gemm_short_k_dispatch(p, bt.n, st);
   if (algo == MAXFP8_ALGO_SKINNY) return gemm_skinny_dispatch(p, block, bt.n, st);
   if (workspace && !is_aligned(workspace, 16)) MAXFP8_FAIL(MAXFP8_ERR_ALIGN, "matmul: workspace must be 16-byte aligned");
@@ -605,8 +609,9 @@ int maxfp8_matmul_describe(int64_t M, int64_t N, int64_t K, int block_scaling, i
   if (algo == MAXFP8_ALGO_SKINNY) return snprintf(buf, len, "skinny");
   if (algo == kAlgoMid) {
     float us;
-    const int sel = tuning().mid > 0 ? tuning().mid : gemm_mid_shape(M, N, K, &us), bm = 16 * (sel / 10), bn = 16 * (sel % 10);
-    return snprintf(buf, len, "%dx%d x%lld, K split over the block's waves", bm, bn, (long long)(ceil_div(M, bm) * ceil_div(N, bn)));
+    const int sel = tuning().mid > 0 ? gemm_mid_forced_shape() : gemm_mid_shape(M, N, K, block_scaling != 0, &us);
+    const int bm = 16 * (sel / 10 % 10), bn = 16 * (sel % 10);
+    return snprintf(buf, len, "%dx%d x%lld, %d per CU, K split over the block's waves", bm, bn, (long long)(ceil_div(M, bm) * ceil_div(N, bn)), sel / 100);
   }
   return gemm_tiled_describe(M, N, K, block_scaling != 0, with_workspace != 0, buf, len);
 }

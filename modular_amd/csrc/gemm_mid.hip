@@ -1,22 +1,28 @@
-// Scaled FP8 matmul for batches between decode and prefill (tens to a few hundred tokens): C[M,N] = A[M,K] . B[N,K]^T.
+// Scaled FP8 matmul for batches between decode and prefill (a few to a thousand tokens): C[M,N] = A[M,K] . B[N,K]^T.
 //
 // Such a matmul is a few dozen 128 x 128 tiles: too few for the chip, so the tile kernels cut K over blocks and pay for it
 // with a second launch (or a hand-over) and the partial sums' way to memory and back.  Here the K split stays inside a
-// block: a block owns a small tile, 16 * MT tokens x 16 * NT weight rows, its four waves a quarter of K each, and the
-// four partial tiles meet in LDS.  Small tiles make enough blocks for the chip without a cut.
+// block: a block owns a small tile, 16 * MT tokens x 16 * NT weight rows, its waves a share of K each, and their
+// partial tiles meet in LDS.  Small tiles make enough blocks for the chip without a cut.
 //
 //   * Each wave has an LDS ring of its own: a slot holds one 128-wide slab of the tile's weight rows AND token rows (and
-//     their scales), copied by LDS-DMA in whole 128-byte lines.  No barrier in the loop; waits are exact counts.
-//   * A slot's fragments are read into registers at once and the slot is refilled before they are multiplied, so DEPTH
-//     slabs stay in flight per wave nearly all the time.
-//   * Epilogue: partial sums to LDS as [token][column], a thread adds the four (in wave order) for eight columns of a token,
-//     scales, converts and stores 16 bytes.  The fused QKV projection's page look-ups are made before the loop.
+//     their scales), copied by LDS-DMA in whole 128-byte lines.  No barrier in the loop; waits are exact counts.  (Token rows
+//     loaded straight into the MFMA's operand layout instead, 16 rows x 64 bytes per instruction, come in at 38 GB/s
+//     per CU, out of L2 too; copies of 8 rows x 128 bytes at 117.)
+//   * A slot's fragments are read into registers at once, and the copies that refill it go out between the MFMAs that multiply
+//     them: a CU takes a copy of 1 KB every 18 cycles, so a slab's copies sent together stop their wave for as long as its
+//     MFMAs take (117 x 6144 x 4096 in 64 x 48 tiles 12.5 -> 10.6 us).
+//   * How a CU is filled (BLOCKS per CU): one block of eight waves with the whole LDS, whose waves cover each other's waits (the same
+//     shape 10.2 us); or two, three or four blocks of four waves on a share of it, so that one block's start and end hide
+//     behind another's loop (432 x 3648 x 2432 in 64 x 64 tiles 16.3 -> 12.5 us, 730 x 1824 x 1536 12.1 -> 9.3).
+//   * Epilogue: partial sums to LDS as [token][column], a thread adds them (in wave order) for eight columns of a token,
+//     scales, converts and stores 16 bytes.  Row scales are loaded in front of the copies (their first use was the longest
+//     wait of the epilogue: 64 x 10240 x 8192 22.9 -> 19.9 us), the fused QKV projection's page look-ups made before the loop.
 //
-// Bound: what a CU can pull out of the L2s -- every block fetches its tokens and weights itself, 16 * (MT + NT) * K bytes, and
-// 40 KB per wave hold two to six slabs in flight.  Measured (graph timing, operands cold) against what ran these shapes
-// before: 117 x 6144 x 4096 20.0 -> 13.1 us, 117 x 4096 x 4096 19.9 -> 10.7, 64 x 4096 x 4096 12.3 -> 8.3, 256 x 1536 x 7168 16.9 ->
-// 11.2, 256 x 576 x 7168 15.2 -> 9.0; the fused QKV projection of 64 tokens (10240 x 8192) 36.9 -> 23.6.  Bytes at 6 TB/s: 4.5,
-// 3.0, 2.9, 2.3, 1.0 and 14.3.
+// Bound: what a CU can pull out of the L2s -- every block fetches its tokens and weights itself, 16 * (MT + NT) * K bytes.
+// Measured (graph timing, operands in the memory-side cache) against what ran these shapes before: 117 x 6144 x 4096 12.1 -> 10.2 us,
+// 64 x 10240 x 8192 with row scales 23.5 -> 19.8, 432 x 3648 x 2432 20.1 -> 12.5, 730 x 1824 x 1536 17.2 -> 8.8, 18 x 4096 x 14336 15.6 ->
+// 13.4, 28 x 6144 x 4096 8.9 -> 7.3.  Bytes at 7 TB/s: 3.9, 12.2, 2.1, 1.1, 8.4 and 3.7.
 #include <type_traits>
 #include <utility>
 
@@ -27,32 +33,39 @@
 
 namespace maxfp8 {
 
-// Slabs in flight per wave: a quarter of the LDS, the 6-bit wait counter, at most six
-__host__ __device__ constexpr int mid_depth(int mt, int nt, bool blockscale) {
-  const int slot = (mt + nt) * 2048 + (blockscale ? 256 : 0), per = 2 * (mt + nt) + (blockscale ? 1 : 0);
-  const int lds = (160 * 1024 - 16 * mt * 8) / 4 / slot, counter = 63 / per + 1, least = lds < counter ? lds : counter;
+// BLOCKS blocks per CU: their waves and their share of its LDS
+__host__ __device__ constexpr int mid_waves(int blocks) { return blocks == 1 ? 8 : 4; }
+__host__ __device__ constexpr int mid_lds(int blocks) { return (blocks == 1 ? 160 : blocks == 2 ? 79 : blocks == 3 ? 53 : 39) * 1024; }
+// Slabs in flight per wave: what the block's LDS holds, the 6-bit wait counter, at most six
+__host__ __device__ constexpr int mid_depth(int mt, int nt, bool blockscale, int blocks) {
+  const int groups = blockscale ? (mt + 3) / 4 : 0, slot = (mt + nt) * 2048 + 256 * groups, per = 2 * (mt + nt) + groups;
+  const int lds = (mid_lds(blocks) - 16 * mt * 8) / mid_waves(blocks) / slot, counter = 63 / per + 1, least = lds < counter ? lds : counter;
   return least > 6 ? 6 : least;
 }
 
-template <int MT, int NT, bool BLOCKSCALE>
+template <int MT, int NT, bool BLOCKSCALE, int BLOCKS>
 struct MidCfg {
-  static constexpr int BM = 16 * MT, BN = 16 * NT;
+  static constexpr int NWAVES = mid_waves(BLOCKS), BM = 16 * MT, BN = 16 * NT;
   static constexpr int SCALES = BLOCKSCALE ? 256 : 0;        // 64 activation scales: one copy
   static constexpr int SLOT = (MT + NT) * 2048 + SCALES;
   static constexpr int PER = 2 * (MT + NT) + (BLOCKSCALE ? 1 : 0);  // copies per wave and slab
   static constexpr int ROW_TABLE = BM * 8;                   // fused QKV: the cache row of every token
-  static constexpr int DEPTH = mid_depth(MT, NT, BLOCKSCALE);
+  static constexpr int DEPTH = mid_depth(MT, NT, BLOCKSCALE, BLOCKS);
   static constexpr int RING = DEPTH * SLOT;
   static constexpr int RED_LD = BN + 4;                      // floats per token row of a partial tile
-  static constexpr int RED = 4 * BM * RED_LD * 4;
-  static constexpr int SMEM = (4 * RING > RED ? 4 * RING : RED) + ROW_TABLE;
-  static_assert(MT <= 4 && DEPTH >= 2 && SMEM <= 160 * 1024);
+  static constexpr int RED = NWAVES * BM * RED_LD * 4;
+  static constexpr int SMEM = (NWAVES * RING > RED ? NWAVES * RING : RED) + ROW_TABLE;
+  static_assert(MT <= 4 && NT <= 4 && DEPTH >= 1 && SMEM <= mid_lds(BLOCKS));
 };
 
-template <int MT, int NT, bool BLOCKSCALE, int W_POLICY>
-__global__ __launch_bounds__(256) void gemm_mid_kernel(GemmArgs p, int tiles_m, int tiles_n) {
-  using Cfg = MidCfg<MT, NT, BLOCKSCALE>;
-  constexpr int BM = Cfg::BM, BN = Cfg::BN, DEPTH = Cfg::DEPTH, PER = Cfg::PER, SLOT = Cfg::SLOT;
+// Where the copies of a slab read.  A slab past the wave's share fetches nothing (and writes zeros), so the counts stay exact.
+struct MidSlabAt { uint32_t koff, kill, kill_s, scales; };
+
+// KV: the fused QKV projection's epilogue and its wave of page look-ups
+template <int MT, int NT, bool BLOCKSCALE, int W_POLICY, int BLOCKS, bool KV>
+__global__ __launch_bounds__((BLOCKS == 1 ? 512 : 256) + (KV ? 64 : 0)) __attribute__((amdgpu_waves_per_eu(1, (BLOCKS == 1 ? 2 : BLOCKS) + (KV ? 1 : 0)))) void gemm_mid_kernel(GemmArgs p, int tiles_m, int tiles_n) {
+  using Cfg = MidCfg<MT, NT, BLOCKSCALE, BLOCKS>;
+  constexpr int NWAVES = Cfg::NWAVES, BM = Cfg::BM, BN = Cfg::BN, DEPTH = Cfg::DEPTH, PER = Cfg::PER, SLOT = Cfg::SLOT;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   // block id -> tile: every XCD (id mod 8) takes a contiguous run of tiles, the row tiles of a column tile next to each
   // other: its L2 holds their weights
@@ -72,7 +85,7 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmArgs p, int tiles_m, 
   const __amdgpu_buffer_rsrc_t b_rsrc = t2_rsrc(p.b + (int64_t)n0 * p.ldb, t2_clamp_u32((int64_t)(cols_here - 1) * p.ldb + p.K));
   const int nslab = (p.K + 127) / 128;
   const bool k_tail = (p.K & 127) != 0;
-  const int per_wave = (nslab + 3) / 4;
+  const int per_wave = (nslab + NWAVES - 1) / NWAVES;
   const int s_begin = wave * per_wave;
   const int s_end = s_begin + per_wave < nslab ? s_begin + per_wave : nslab;
 
@@ -104,30 +117,48 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmArgs p, int tiles_m, 
   // 16-row groups of weights from here on belong to the second scale row
   const int nt_hi = NT == 3 ? (128 - n0 % 128) / 16 : NT;
 
+  // Row scaling: what the epilogue multiplies this thread's results by (eight columns of a token per item), loaded before
+  // the copies
+  constexpr int CHUNKS = BN / 8, ITEMS = (BM * CHUNKS + NWAVES * 64 - 1) / (NWAVES * 64);
+  float row_s[ITEMS], col_s[ITEMS][8];
+  if (!BLOCKSCALE && (!KV || wave < NWAVES)) {
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+      const int item = it * NWAVES * 64 + tid, row = item / CHUNKS, col = (item - row * CHUNKS) * 8;
+      row_s[it] = scale_at(p.a_scales, (int64_t)(m0 + (row < rows_here ? row : 0)) * p.a_scale_stride, p.scales_dtype);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int n = n0 + col + i;
+        col_s[it][i] = scale_at(p.b_scales, (int64_t)(n < p.N ? n : p.N - 1) * p.b_scale_stride, p.scales_dtype);
+      }
+    }
+  }
+
   v4f acc[MT][NT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
-  // the PER copies of a slab; a slab past the wave's share fetches nothing (and writes zeros), so the counts stay exact
-  auto issue = [&](int slab, int d) {
+  auto slab_at = [&](int slab) {
     const bool live = slab < s_end;
     const int sl = live ? slab : s_begin;
-    const uint32_t koff = __builtin_amdgcn_readfirstlane((uint32_t)sl * 128u);
-    uint32_t kill = live ? 0u : 0x80000000u;
-    const uint32_t kill_s = kill;
-    if (k_tail && koff + cchunk * 16 >= (uint32_t)p.K) kill = 0x80000000u;
+    MidSlabAt at;
+    at.koff = __builtin_amdgcn_readfirstlane((uint32_t)sl * 128u);
+    at.kill = at.kill_s = live ? 0u : 0x80000000u;
+    if (k_tail && at.koff + cchunk * 16 >= (uint32_t)p.K) at.kill = 0x80000000u;
+    at.scales = (uint32_t)sl * (uint32_t)p.a_scales_ld * 4u;
+    return at;
+  };
+  // copy i (0 .. PER - 1, known at compile time) of a slab into slot d: weight rows, token rows, token scales
+  auto copy = [&](const MidSlabAt& at, int d, int i) {
     uint8_t* slot = ring + d * SLOT;
-#pragma unroll
-    for (int i = 0; i < 2 * NT; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, (lds_ptr_t)(slot + i * 1024), 16, b_voff | kill, koff + i * b_step, 0, W_POLICY);
-#pragma unroll
-    for (int i = 0; i < 2 * MT; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (lds_ptr_t)(slot + (2 * NT + i) * 1024), 16, a_voff | kill, koff + i * a_step, 0, 0);
-    if constexpr (BLOCKSCALE)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(s_rsrc, (lds_ptr_t)(slot + (MT + NT) * 2048), 4, s_voff | kill_s,
-                                               (uint32_t)sl * (uint32_t)p.a_scales_ld * 4u, 0, 0);
+    if (i < 2 * NT)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, (lds_ptr_t)(slot + i * 1024), 16, b_voff | at.kill, at.koff + i * b_step, 0, W_POLICY);
+    else if (i < 2 * (NT + MT))
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (lds_ptr_t)(slot + i * 1024), 16, a_voff | at.kill, at.koff + (i - 2 * NT) * a_step, 0, 0);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(s_rsrc, (lds_ptr_t)(slot + (MT + NT) * 2048), 4, s_voff | at.kill_s, at.scales, 0, 0);
   };
   auto step = [&](int slab, int d) {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * PER) : "memory");
@@ -143,57 +174,82 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmArgs p, int tiles_m, 
 #pragma unroll
     for (int i = 0; i < MT; ++i) af[i] = frag(slot + (NT + i) * 2048);
     v4f as = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (BLOCKSCALE) as = *reinterpret_cast<const v4f*>(slot + (MT + NT) * 2048 + lm * 16);
-    // the slot's bytes are in registers before it is refilled
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    issue(slab + DEPTH, d);
+    float b0 = 0.f, b1 = 0.f;
     if constexpr (BLOCKSCALE) {
+      as = *reinterpret_cast<const v4f*>(slot + (MT + NT) * 2048 + lm * 16);
       // (a slab past the share's end multiplies zeros; its scales are finite)
       const int at = __builtin_amdgcn_readfirstlane(slab - s_begin);
-      const float b0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, bs_lo), at));
-      const float b1 = NT == 3 ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, bs_hi), at)) : b0;
-      const v4f zero = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          const v4f part = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[nt], af[mt], zero, 0, 0, 0, 0, 0, 0);
-          acc[mt][nt] += part * (as[mt] * (NT == 3 && nt >= nt_hi ? b1 : b0));
-        }
-    } else {
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-          acc[mt][nt] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[nt], af[mt], acc[mt][nt], 0, 0, 0, 0, 0, 0);
+      b0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, bs_lo), at));
+      b1 = NT == 3 ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, bs_hi), at)) : b0;
+    }
+    // the slot's bytes are in registers before it is refilled
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    // MFMA i, in front of it its share of the copies of the slab that takes this slot, and behind it the promotion of the
+    // product LAG MFMAs back, which has left the matrix pipe
+    const MidSlabAt next = slab_at(slab + DEPTH);
+    constexpr int NM = MT * NT, LAG = 3;
+    v4f part[LAG + 1];
+    auto promote = [&](auto j_c) {
+      constexpr int j = decltype(j_c)::value, mt = j / NT, nt = j % NT;
+      acc[mt][nt] += part[j % (LAG + 1)] * (as[mt] * (NT == 3 && nt >= nt_hi ? b1 : b0));
+    };
+    static_for<NM>([&](auto i_c) {
+      constexpr int i = decltype(i_c)::value, mt = i / NT, nt = i % NT, c0 = i * PER / NM, c1 = (i + 1) * PER / NM;
+      static_for<c1 - c0>([&](auto c_c) { copy(next, d, c0 + decltype(c_c)::value); });
+      if constexpr (BLOCKSCALE) {
+        const v4f zero = {0.f, 0.f, 0.f, 0.f};
+        part[i % (LAG + 1)] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[nt], af[mt], zero, 0, 0, 0, 0, 0, 0);
+        if constexpr (i >= LAG) promote(std::integral_constant<int, i - LAG>{});
+      } else {
+        acc[mt][nt] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[nt], af[mt], acc[mt][nt], 0, 0, 0, 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    if constexpr (BLOCKSCALE) {
+      constexpr int left = NM < LAG ? NM : LAG;
+      static_for<left>([&](auto j_c) { promote(std::integral_constant<int, NM - left + decltype(j_c)::value>{}); });
     }
   };
 
+  if (!KV || wave < NWAVES) {
 #pragma unroll
-  for (int d = 0; d < DEPTH; ++d) issue(s_begin + d, d);
-  if constexpr (BLOCKSCALE)  // (the weight scales are older than the copies: they arrive without waiting for those)
-    asm volatile("s_waitcnt vmcnt(%2)" : "+v"(bs_lo), "+v"(bs_hi) : "n"(DEPTH * PER < 63 ? DEPTH * PER : 63));
-  if (p.kv_on && tid < BM) row_table[tid] = tid < rows_here ? kv_row_offset(p.kv, m0 + tid) : -1;
-  for (int base = s_begin; base < s_end; base += DEPTH) {
+    for (int d = 0; d < DEPTH; ++d) {
+      const MidSlabAt at = slab_at(s_begin + d);
 #pragma unroll
-    for (int d = 0; d < DEPTH; ++d) step(base + d, d);
+      for (int i = 0; i < PER; ++i) copy(at, d, i);
+    }
+    if constexpr (BLOCKSCALE)  // (the weight scales are older than the copies: they arrive without waiting for those)
+      asm volatile("s_waitcnt vmcnt(%2)" : "+v"(bs_lo), "+v"(bs_hi) : "n"(DEPTH * PER < 63 ? DEPTH * PER : 63));
+    for (int base = s_begin; base < s_end; base += DEPTH) {
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) step(base + d, d);
+    }
+    // drain: the last DEPTH copies fetched nothing but still write their slots
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  } else if (lane < BM) {
+    // fused QKV: a wave of its own looks up the rows' pages.  Its loads depend on one another, a search among the sequences and two
+    // more; in one of the other waves each of them waited for all copies in front of it, and the wave's share of K for them
+    // (64 tokens of 64 sequences, 10240 x 8192 with row scales, quantiser included: 29.1 -> 26.6 us).
+    row_table[lane] = lane < rows_here ? kv_row_offset(p.kv, m0 + lane) : -1;
   }
-  // drain: the last DEPTH copies fetched nothing but still write their slots
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 
-  // ---- the four partial tiles meet ------------------------------------------------------------------------------
+  // ---- the waves' partial tiles meet ------------------------------------------------------------------------------
   float* red = reinterpret_cast<float*>(smem);
   constexpr int LD = Cfg::RED_LD;
+  if (!KV || wave < NWAVES) {
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-      *reinterpret_cast<v4f*>(red + (wave * BM + mt * 16 + lm) * LD + nt * 16 + lq * 4) = acc[mt][nt];
+      for (int nt = 0; nt < NT; ++nt)
+        *reinterpret_cast<v4f*>(red + (wave * BM + mt * 16 + lm) * LD + nt * 16 + lq * 4) = acc[mt][nt];
+  }
   __syncthreads();
-  constexpr int CHUNKS = BN / 8;
-  for (int item = tid; item < BM * CHUNKS; item += 256) {
-    const int row = item / CHUNKS, col = (item - row * CHUNKS) * 8;
+  if (KV && wave >= NWAVES) return;
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int item = it * NWAVES * 64 + tid, row = item / CHUNKS, col = (item - row * CHUNKS) * 8;
     if (row >= rows_here || col >= cols_here) continue;
     float v[8];
     {
@@ -201,23 +257,23 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmArgs p, int tiles_m, 
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[i] = at[i];
 #pragma unroll
-      for (int w = 1; w < 4; ++w)
+      for (int w = 1; w < NWAVES; ++w)
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] += at[w * BM * LD + i];
     }
     const int64_t m = m0 + row;
     const int n = n0 + col;
-    if (p.kv_on) {
+    if constexpr (KV) {
       // fused QKV: the reference's bf16 roundings, then C or the row's K / V page (see tile_body)
       const int64_t row_off = row_table[row];
       if (row_off < 0 && n >= p.kv.q_dim) continue;
       float a_s = 1.f;
-      if constexpr (!BLOCKSCALE) a_s = bf16_round(p.a_scales[m * p.a_scale_stride]);
+      if constexpr (!BLOCKSCALE) a_s = bf16_round(row_s[it]);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int nn = n + i < p.N ? n + i : p.N - 1;
         float r = bf16_round(v[i]);
-        if constexpr (!BLOCKSCALE) r = bf16_round(r * bf16_round(a_s * bf16_round(p.b_scales[(int64_t)nn * p.b_scale_stride])));
+        if constexpr (!BLOCKSCALE) r = bf16_round(r * bf16_round(a_s * bf16_round(col_s[it][i])));
         if (p.kv.bias) r = bf16_round(r + bf16_bits_to_f32(p.kv.bias[nn]));
         v[i] = r;
       }
@@ -226,12 +282,8 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmArgs p, int tiles_m, 
       continue;
     }
     if constexpr (!BLOCKSCALE) {
-      const float a_s = scale_at(p.a_scales, m * p.a_scale_stride, p.scales_dtype);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int nn = n + i < p.N ? n + i : p.N - 1;
-        v[i] = (v[i] * a_s) * scale_at(p.b_scales, (int64_t)nn * p.b_scale_stride, p.scales_dtype);
-      }
+      for (int i = 0; i < 8; ++i) v[i] = (v[i] * row_s[it]) * col_s[it][i];
     }
     if (p.c_dtype == MAXFP8_BF16) {
       uint16_t* dst = reinterpret_cast<uint16_t*>(p.c) + m * p.ldc + n;
@@ -257,13 +309,14 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmArgs p, int tiles_m, 
   }
 }
 
-template <int MT, int NT, bool BLOCKSCALE>
+template <int MT, int NT, bool BLOCKSCALE, int BLOCKS, bool KV>
 static int launch_mid(const GemmArgs& p, hipStream_t stream) {
-  using Cfg = MidCfg<MT, NT, BLOCKSCALE>;
+  using Cfg = MidCfg<MT, NT, BLOCKSCALE, BLOCKS>;
   // weights that are read once and are more than a quarter of the memory-side cache: non-temporal (10240 x 8192 at 64 tokens
   // 24.1 -> 23.2 us; smaller ones may still sit in that cache and then come quicker without: 1536 x 7168 9.4 against 12.8)
   const bool once = p.M <= Cfg::BM && (int64_t)p.N * p.K >= ((int64_t)1 << 26);
-  auto kern = once ? gemm_mid_kernel<MT, NT, BLOCKSCALE, kStreamOnce> : gemm_mid_kernel<MT, NT, BLOCKSCALE, 0>;
+  void (*kern)(GemmArgs, int, int) = gemm_mid_kernel<MT, NT, BLOCKSCALE, 0, BLOCKS, KV>;
+  if (once) kern = gemm_mid_kernel<MT, NT, BLOCKSCALE, kStreamOnce, BLOCKS, KV>;
   static PerDeviceFlag attrs[2];
   PerDeviceFlag& attr = attrs[once];
   bool& attr_done = attr.here();
@@ -273,103 +326,85 @@ static int launch_mid(const GemmArgs& p, hipStream_t stream) {
     attr_done = true;
   }
   const int64_t tiles_m = ceil_div(p.M, Cfg::BM), tiles_n = ceil_div(p.N, Cfg::BN);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), Cfg::SMEM, stream, p, (int)tiles_m, (int)tiles_n);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3((Cfg::NWAVES + (KV ? 1 : 0)) * 64), Cfg::SMEM, stream, p, (int)tiles_m, (int)tiles_n);
   return launch_status("gemm_mid");
 }
 
 int compute_units();
 float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
 
-// Estimated times (microseconds), fitted to launches of every kernel on 26 weight matrices (K 512 ... 28672, N 576 ... 32768)
-// at 4 to 400 tokens in both scale modes, operands cold: within 15 per cent for nine launches in ten.
-//
-// This kernel: a start, per round of blocks a fixed part and a slab's time of the tile shape, the bytes of all blocks'
-// operands (out of the L2s), and not less than the weights take from memory.
-struct MidShape { int mt, nt; float start, round, slab, traffic; };
-static const MidShape kMidShapes[12] = {
-    {2, 1, 1.84f, 3.33f, 0.037f, 3.32f}, {2, 2, 1.82f, 2.93f, 0.066f, 2.91f}, {2, 3, 2.07f, 2.97f, 0.093f, 3.17f}, {2, 4, 2.17f, 3.25f, 0.121f, 2.89f},
-    {3, 1, 2.01f, 2.75f, 0.061f, 2.31f}, {3, 2, 1.91f, 2.98f, 0.091f, 2.44f}, {3, 3, 2.55f, 3.87f, 0.115f, 2.80f}, {3, 4, 1.69f, 4.01f, 0.166f, 2.16f},
-    {4, 1, 1.75f, 2.91f, 0.069f, 2.30f}, {4, 2, 1.90f, 3.56f, 0.104f, 2.13f}, {4, 3, 1.45f, 4.38f, 0.144f, 1.90f}, {4, 4, 1.43f, 4.97f, 0.181f, 2.27f}};
-static float mid_cost(const MidShape& t, int64_t M, int64_t N, int64_t K) {
-  const int64_t blocks = ceil_div(M, 16 * t.mt) * ceil_div(N, 16 * t.nt);
-  const float slabs = (float)(ceil_div(K, 512) * 4);
-  float us = t.start + (float)ceil_div(blocks, compute_units()) * (t.round + slabs * t.slab) +
-                   t.traffic * (float)(blocks * 16 * (t.mt + t.nt)) * (float)K * 1e-8f;
-  // (the fit reads long K on weights from 32 MB short: 9728 x 5328 at 59 tokens 22.7 us against the K split's 19.7; on smaller
-  // ones it does not: 9600 x 2416 at 45 tokens 14.5 against the decode kernel's 19.3)
-  if (K > 9216 && N * K >= ((int64_t)1 << 25)) us *= 1.25f;
-  const float stream = 4.0f + (float)N * (float)K / 5.2e6f;
-  return us > stream ? us : stream;
+// The shapes that are built: 16 mt tokens x 16 nt weight rows, blocks per CU.  Of 78 measured on 300 matmuls (1 to 1000 tokens, K 512 ...
+// 28672, N 512 ... 57344, both scalings), these lose 1 per cent against choosing among all of them.
+struct MidShape { int mt, nt, blocks; };
+#define MAXFP8_MID_SHAPES(S)                                                                                               \
+  S(1, 1, 4) S(1, 2, 3) S(2, 1, 3) S(2, 2, 4) S(2, 2, 2) S(2, 3, 3) S(2, 3, 1) S(2, 4, 3) S(2, 4, 1) S(3, 1, 2) S(3, 2, 1) S(3, 3, 1) \
+  S(3, 4, 2) S(3, 4, 1) S(4, 1, 1) S(4, 2, 1) S(4, 3, 1) S(4, 4, 2)
+#define MAXFP8_MID_ROW(mt, nt, blocks) {mt, nt, blocks},
+static const MidShape kMidShapes[] = {MAXFP8_MID_SHAPES(MAXFP8_MID_ROW)};
+#undef MAXFP8_MID_ROW
+
+// Estimated microseconds, one estimate for all shapes (fitted to the launches above, operands in the memory-side cache where they fit:
+// within 8 per cent for half of the launches, 19 for nine in ten; what the shapes have in common cancels where they are
+// compared: the one it picks is 0.4 per cent behind the best of them on average, 10 at most).  A launch; per round of blocks on the
+// chip a start and end, the waits of the ring's rounds, and the MFMAs of a wave; per block of a CU the bytes of its slabs and
+// its MFMAs; the weights' way from memory.
+static float mid_cost(const MidShape& t, int64_t M, int64_t N, int64_t K, bool blockscale) {
+  const int64_t cus = compute_units(), blocks = ceil_div(M, 16 * t.mt) * ceil_div(N, 16 * t.nt);
+  const float rounds = (float)ceil_div(blocks, cus * t.blocks), per_cu = (float)ceil_div(blocks, cus);
+  const int64_t slabs = ceil_div(K, 128), wave_slabs = ceil_div(slabs, mid_waves(t.blocks)), depth = mid_depth(t.mt, t.nt, blockscale, t.blocks);
+  const float turns = (float)ceil_div(wave_slabs, depth), walked = turns * (float)depth, mfmas = (float)(t.mt * t.nt);
+  const float fetched = per_cu * (float)slabs * (float)(t.mt + t.nt), multiplied = per_cu * (float)slabs * mfmas, weights = (float)N * (float)K;
+  if (blockscale)
+    return 1.35f + rounds * (1.93f + 0.060f * turns + 0.0045f * walked * mfmas) + 0.0179f * fetched + 0.0033f * multiplied + 6.2e-8f * weights;
+  return 1.31f + rounds * (2.60f + 0.043f * turns + 0.0023f * walked * mfmas) + 0.0160f * fetched + 0.0033f * multiplied +
+         0.023f * per_cu * mfmas + 9.0e-8f * weights;
 }
 
-// What the estimate holds for: at most 320 tokens, K up to 12288 (beyond, the decode kernel and the K split's tiles win from
-// both sides: 14336 x 4096 at 24 tokens 17.4 against 20 us, at 117 tokens 26.6 against 28.4) and weights under 128 MB (25024 x
-// 6400 at 45 tokens 40 against 44).  (In any case at most 58 slabs per wave: their weight scales sit in its 64 lanes.)
-bool gemm_mid_ok(int64_t M, int64_t N, int64_t K) { return M <= 320 && K <= 12288 && N * K < ((int64_t)1 << 27); }
+// What the kernel takes (with block scaling a wave's weight scales sit in its 64 lanes) and where it may be the quicker one: at most 2048 tokens
+bool gemm_mid_ok(int64_t M, int64_t N, int64_t K) { return M <= 2048 && K <= 4 * 64 * 128 && ceil_div(M, 16) * ceil_div(N, 16) < ((int64_t)1 << 31); }
 
-// The shape for an M x N x K matmul (10 * MT + NT) and what it is estimated to take
-int gemm_mid_shape(int64_t M, int64_t N, int64_t K, float* us) {
-  int best = 0;
-  *us = 0.f;
+// The shape for an M x N x K matmul (100 * blocks per CU + 10 * mt + nt) and what it is estimated to take
+int gemm_mid_shape(int64_t M, int64_t N, int64_t K, bool blockscale, float* us) {
+  const MidShape* best = nullptr;
   for (const MidShape& t : kMidShapes) {
-    if (t.mt > 2 && M <= 16 * (t.mt - 1)) continue;
-    const float c = mid_cost(t, M, N, K);
-    if (best == 0 || c < *us) { best = 10 * t.mt + t.nt; *us = c; }
+    if (t.mt > 1 && M <= 16 * (t.mt - 1)) continue;
+    const float c = mid_cost(t, M, N, K, blockscale);
+    if (!best || c < *us) { best = &t; *us = c; }
   }
-  return best;
+  return 100 * best->blocks + 10 * best->mt + best->nt;
 }
 
-// What that shape takes at 33 to 64 rows, for the comparison with the decode kernel: one estimate per scaling, with the slabs of
-// a wave in whole rounds of its ring (the launches of gemm_skinny_cost: within 9 per cent for nine in ten)
-float gemm_mid_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
-  float us;
-  const int sel = gemm_mid_shape(M, N, K, &us), mt = sel / 10, nt = sel % 10, depth = mid_depth(mt, nt, blockscale);
-  const float rounds = (float)ceil_div(ceil_div(M, 16 * mt) * ceil_div(N, 16 * nt), compute_units());
-  const int64_t slabs = ceil_div(K, 512);
-  const float walked = (float)(ceil_div(slabs, depth) * depth), stream = (float)N * (float)K * 1e-8f;
-  if (blockscale) return 1.91f + 12.6f * stream + rounds * (1.46f + 0.139f * (float)(mt * nt) + 0.049f * (float)(slabs * (mt + nt)) + 0.214f * walked);
-  return 1.58f + 10.9f * stream + rounds * (2.15f + 0.188f * (float)(mt * nt) + 0.058f * (float)(slabs * (mt + nt)) + 0.162f * walked);
+// The kernel here or the decode kernel (gemm_skinny.hip), at most 64 rows.  From 17 on the decode kernel loads two or four groups of 16 tokens
+// straight into the MFMA's operand layout and is behind everywhere (17 x 7168 x 18432 27.0 against 27.6 us at best; 22 x 3312 x 512
+// 4.5 against 3.5, 28 x 4096 x 14336 19.1 against 13.5, 64 x 4096 x 14336 31.7 against 15.2).  Up to 16 it keeps more weights in flight:
+// 3 per cent behind with the weights in the memory-side cache, as much ahead where they come from memory.
+bool gemm_mid_before_skinny(int64_t M, int64_t N, int64_t K) {
+  if (!gemm_mid_ok(M, N, K) || tuning().skinny || tuning().mid == 0) return false;
+  return M > 16 || tuning().mid > 0;
 }
 
-// The kernel here or the decode kernel, 17 to 64 rows.
-// Up to 32 rows the decode kernel reads the tokens with half the loads and is ahead or level nearly everywhere (17 / 24 / 32 x 1536 x
-// 7168 8.8 / 9.9 / 11.0 us against 10.2 / 10.7 / 11.4, 20 x 5040 x 6528 11.0 against 12.4, 28 x 24624 x 2560 20.8 against 21.8) but
-// where its third block per CU runs all but alone: 22 x 9648 x 6912 0.81 of its time, 27 x 11328 x 1152 0.87 (shorter K: 1.0 to 1.1).
-// Beyond, by the estimates: 33 x 4096 x 4096 9.7 against 8.2 us, 47 x 9152 x 1024 9.9 against 7.1 -- but 36 x 6272 x 512 5.0 against
-// 5.8 and, with row scales, 39 x 21600 x 896 11.6 against 15.2 (block scales: 14.4 and 12.8).
-bool gemm_mid_before_skinny(int64_t M, int64_t N, int64_t K, bool blockscale, bool qkv) {
-  if (!gemm_mid_ok(M, N, K)) return false;
-  if (M <= 32) return K > 1024 && ceil_div(ceil_div(N, 16), compute_units()) == 3;
-  // (Beyond 3072 the estimate here is the higher one of the two by 6 per cent.  The fused QKV projection's epilogue costs more here, a
-  // microsecond per block and round: 48 x 2048 x 1536 7.0 against 7.7 us, 56 x 7168 x 5120 17.7 against 18.8, with row scales 18.2, 48 x
-  // 17408 x 2048 with row scales 20.9 against 26.7.)
-  const float margin = qkv ? (K < 3072 ? 0.90f : blockscale ? 0.95f : 1.06f) : K > 3072 ? 1.06f : 1.0f;
-  return gemm_mid_cost(M, N, K, blockscale) < margin * gemm_skinny_cost(M, N, K, blockscale);
-}
-
-template <bool BLOCKSCALE>
+template <bool BLOCKSCALE, bool KV>
 static int pick_mid(const GemmArgs& p, int sel, hipStream_t stream) {
-  switch (sel) {
-    case 21: return launch_mid<2, 1, BLOCKSCALE>(p, stream);
-    case 22: return launch_mid<2, 2, BLOCKSCALE>(p, stream);
-    case 23: return launch_mid<2, 3, BLOCKSCALE>(p, stream);
-    case 24: return launch_mid<2, 4, BLOCKSCALE>(p, stream);
-    case 31: return launch_mid<3, 1, BLOCKSCALE>(p, stream);
-    case 32: return launch_mid<3, 2, BLOCKSCALE>(p, stream);
-    case 33: return launch_mid<3, 3, BLOCKSCALE>(p, stream);
-    case 34: return launch_mid<3, 4, BLOCKSCALE>(p, stream);
-    case 41: return launch_mid<4, 1, BLOCKSCALE>(p, stream);
-    case 42: return launch_mid<4, 2, BLOCKSCALE>(p, stream);
-    case 43: return launch_mid<4, 3, BLOCKSCALE>(p, stream);
-    case 44: return launch_mid<4, 4, BLOCKSCALE>(p, stream);
-    default: MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "mid matmul: unknown shape selector %d", sel);
-  }
+#define MAXFP8_MID_CASE(mt, nt, blocks) if (sel == 100 * blocks + 10 * mt + nt) return launch_mid<mt, nt, BLOCKSCALE, blocks, KV>(p, stream);
+  MAXFP8_MID_SHAPES(MAXFP8_MID_CASE)
+#undef MAXFP8_MID_CASE
+  MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "mid matmul: unknown shape selector %d", sel);
+}
+
+// The tuning switch names a shape as <blocks per CU><mt><nt>, or a tile as <mt><nt>: the first shape above with that tile
+int gemm_mid_forced_shape() {
+  const int sel = tuning().mid;
+  if (sel >= 100) return sel;
+  for (const MidShape& t : kMidShapes)
+    if (10 * t.mt + t.nt == sel) return 100 * t.blocks + sel;
+  return sel;
 }
 
 int gemm_mid_dispatch(const GemmArgs& p, bool blockscale, hipStream_t stream) {
-  float us;
-  const int sel = tuning().mid > 0 ? tuning().mid : gemm_mid_shape(p.M, p.N, p.K, &us);
-  return blockscale ? pick_mid<true>(p, sel, stream) : pick_mid<false>(p, sel, stream);
+  float us = 0.f;
+  const int sel = tuning().mid > 0 ? gemm_mid_forced_shape() : gemm_mid_shape(p.M, p.N, p.K, blockscale, &us);
+  if (p.kv_on) return blockscale ? pick_mid<true, true>(p, sel, stream) : pick_mid<false, true>(p, sel, stream);
+  return blockscale ? pick_mid<true, false>(p, sel, stream) : pick_mid<false, false>(p, sel, stream);
 }
 
 }  // namespace maxfp8

@@ -74,6 +74,7 @@ struct SkinnyCfg {
   static constexpr int RING = DEPTH * SLOT;                  // per wave
   static constexpr int RED = WAVES * MT * NTW * 4 * 64 * 4;  // reduction buffer (reuses the rings)
   static constexpr int RINGS = WAVES * RING > RED ? WAVES * RING : RED;
+  static constexpr int ROW_TABLE = 16 * MT * 8;              // fused QKV only, behind everything else: the cache row of every token
   static constexpr int SMEM = RINGS;  // (ALDS: plus WAVES * M * the share's bytes, added at the launch)
 };
 
@@ -93,8 +94,9 @@ __host__ __device__ constexpr uint32_t skinny_acts_bytes(uint32_t M, uint32_t pe
   return ACTS > kActsLds ? rows + (BLOCKSCALE ? (M * per_wave * 4u + 15u) & ~15u : 128u) : rows;
 }
 
-template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, int ACTS = kActsPerSlab>
-__global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in) {
+// KV: the fused QKV projection's epilogue (a kernel of its own: the plain one would load its arguments all the same, 1 to 2 per cent)
+template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, int ACTS = kActsPerSlab, bool KV = false>
+__global__ __launch_bounds__(NWAVES * 64 + (KV ? 64 : 0)) void gemm_skinny_kernel(GemmArgs p_in) {
   const GemmArgs p = gridDim.y == 1 ? p_in : batch_view(p_in, blockIdx.y);
   using Cfg = SkinnyCfg<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ACTS>;
   constexpr bool ALDS = Cfg::ALDS, QUANT = Cfg::QUANT;
@@ -119,6 +121,22 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in)
   const int per_wave = (nslab + WAVES - 1) / WAVES;
   const int s_begin = wave * per_wave;
   const int s_end = (s_begin + per_wave) < nslab ? (s_begin + per_wave) : nslab;
+
+  // Fused QKV: a wave of its own looks up the rows' pages while the others walk their slabs.  Its loads depend on one another (a search
+  // among the sequences and two more) and stood at the end of the kernel before: 8 tokens of 8 sequences, 6144 x 4096, 11.5 -> 11.0 us, quantiser
+  // included.
+  [[maybe_unused]] int64_t* row_table = reinterpret_cast<int64_t*>(smem + Cfg::RINGS + WAVES * skinny_acts_bytes<ACTS, BLOCKSCALE>((uint32_t)p.M, (uint32_t)per_wave));
+  if constexpr (KV) {
+    if (wave == WAVES) {
+      if (lane < 16 * MT) row_table[lane] = lane < p.M ? kv_row_offset(p.kv, lane) : -1;
+      if constexpr (QUANT && !BLOCKSCALE) {
+        if (!p.x_static) __builtin_amdgcn_s_barrier();  // (the waves' meeting below)
+      }
+      __syncthreads();
+      __syncthreads();
+      return;
+    }
+  }
 
   // weight DMA: lane (cr = lane >> 3, cp = lane & 7) moves logical chunk cp ^ cr of row cr (then
   // row 8 + cr) of a 16-row group to LDS position lane * 16: row r, chunk c is stored at c ^ (r & 7)
@@ -235,6 +253,9 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, (sk_lds_ptr_t)(slot + t * 2048 + 1024), 16, w_voff | killw,
                                                koff + t * w_tile + w_half, 0, kWeightStream);
     }
+    // (the slabs' loads stay in this order: with another one in front of the loop, the waits the compiler adds for registers have to hold for
+    // both and were for everything in flight, once a round of the ring; 1 to 4 tokens, 102 matmuls, 3.6 per cent, up to 25)
+    __builtin_amdgcn_sched_barrier(0);
   };
   auto compute = [&](auto d_c, [[maybe_unused]] int slab) {
     constexpr int d = decltype(d_c)::value;
@@ -398,9 +419,9 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in)
       v[i] = sum;
     }
     if (m >= p.M || n >= p.N) continue;
-    if (p.kv_on) {
+    if constexpr (KV) {
       // fused QKV: the reference's bf16 roundings, then C or the row's K / V page (see tile_body)
-      const int64_t row_off = kv_row_offset(p.kv, m);
+      const int64_t row_off = row_table[m];
       float a_s = 1.f;
       if constexpr (!BLOCKSCALE) a_s = QUANT ? a_sc[16 + m] : p.a_scales[(int64_t)m * p.a_scale_stride];
 #pragma unroll
@@ -460,9 +481,12 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_skinny_kernel(GemmArgs p_in)
 }
 
 int compute_units();
-template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, int ACTS = kActsPerSlab>
+template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, int ACTS = kActsPerSlab, bool KV = false>
 static int launch_skinny_r(const GemmArgs& p, int64_t batch, hipStream_t stream) {
-  if constexpr (MT == 1 && ACTS == kActsPerSlab) {
+  if constexpr (!KV && ACTS != kActsLds) {
+    if (p.kv_on) return launch_skinny_r<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ACTS, true>(p, batch, stream);
+  }
+  if constexpr (MT == 1 && ACTS == kActsPerSlab && !KV) {
     // few tokens, a share of K per wave that fits, and a weight matrix small enough that the launch is about one round of
     // blocks: the activations go to LDS once (84 MB, M = 1: 17.8 -> 17.0 us; on a 470 MB matrix, where blocks come and
     // go, the per-slab loads cost nothing and this form measured 1 % slower).  Not for the fused QKV epilogue's build, a
@@ -474,15 +498,15 @@ static int launch_skinny_r(const GemmArgs& p, int64_t batch, hipStream_t stream)
     const int64_t a_bytes = (int64_t)p.M * ((per_wave * 128 + 1023) / 1024 * 1024);  // per wave
     const int64_t blocks_per_cu = ceil_div(ceil_div((int64_t)p.N, 16 * NTW) * batch, (int64_t)compute_units());
     using Plain = SkinnyCfg<NTW, MT, BLOCKSCALE, RING_KB, NWAVES>;
-    if (tuning().skinny_alds && !p.kv_on && (int64_t)p.N * p.K < ((int64_t)1 << 27) && a_bytes <= kSkinnyALdsBytes &&
+    if (tuning().skinny_alds && (int64_t)p.N * p.K < ((int64_t)1 << 27) && a_bytes <= kSkinnyALdsBytes &&
         blocks_per_cu * (Plain::SMEM + NWAVES * a_bytes) <= 160 * 1024)
       return launch_skinny_r<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, kActsLds>(p, batch, stream);
   }
   using Cfg = SkinnyCfg<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ACTS>;
-  auto kern = gemm_skinny_kernel<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ACTS>;
+  auto kern = gemm_skinny_kernel<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ACTS, KV>;
   static PerDeviceFlag attr;
   bool& attr_done = attr.here();
-  constexpr int smem_all = Cfg::QUANT ? 160 * 1024 : Cfg::SMEM + (Cfg::ALDS ? NWAVES * kSkinnyALdsBytes : 0);
+  constexpr int smem_all = Cfg::QUANT ? 160 * 1024 : Cfg::SMEM + Cfg::ROW_TABLE + (Cfg::ALDS ? NWAVES * kSkinnyALdsBytes : 0);
   constexpr int smem_max = smem_all < 160 * 1024 ? smem_all : 160 * 1024;  // (what a launch asks for was checked against the CU's LDS)
   if (!attr_done) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem_max);
@@ -490,9 +514,9 @@ static int launch_skinny_r(const GemmArgs& p, int64_t batch, hipStream_t stream)
     attr_done = true;
   }
   const uint32_t per_wave = (uint32_t)ceil_div(ceil_div(p.K, 128), NWAVES);
-  const int smem = Cfg::SMEM + NWAVES * (int)skinny_acts_bytes<ACTS, BLOCKSCALE>((uint32_t)p.M, per_wave);
+  const int smem = Cfg::SMEM + NWAVES * (int)skinny_acts_bytes<ACTS, BLOCKSCALE>((uint32_t)p.M, per_wave) + (KV ? Cfg::ROW_TABLE : 0);
   const int64_t blocks = ceil_div(p.N, 16 * NTW);
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)batch), dim3(NWAVES * 64), smem, stream, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)batch), dim3((NWAVES + (KV ? 1 : 0)) * 64), smem, stream, p);
   return launch_status("gemm_skinny");
 }
 
@@ -562,7 +586,8 @@ static bool skinny_quant_fits(int64_t M, int64_t N, int64_t K) {
   if (skinny_quant_loads(M, K) > kQuantLoads || (!BLOCKSCALE && M > 1 && (M > 4 || per_cu > 3 || M * per_cu > 8))) return false;
   // (the quantised activations of the blocks that are on a CU together -- three keep the weight stream full -- fit its LDS)
   const uint32_t per_wave = (uint32_t)ceil_div(ceil_div(K, 128), 4);
-  const int64_t smem = SkinnyCfg<NTW, 1, BLOCKSCALE, RING_KB, 4, kQuantLoads>::SMEM +
+  using Cfg = SkinnyCfg<NTW, 1, BLOCKSCALE, RING_KB, 4, kQuantLoads>;
+  const int64_t smem = Cfg::SMEM + Cfg::ROW_TABLE +
                        4 * (int64_t)skinny_acts_bytes<kQuantLoads, BLOCKSCALE>((uint32_t)M, per_wave);
   return (per_cu < 3 ? per_cu : 3) * smem <= 160 * 1024;
 }
@@ -700,9 +725,8 @@ bool gemm_skinny_preferred(int64_t M, int64_t N, int64_t K) {
   return M <= 64 && small_weights;
 }
 
-// Estimated microseconds at 17 to 64 rows.  Up to 32 only the tiles are compared with it; beyond, the kernel for tens of tokens
-// too, so the estimate is one per scaling and counts the slabs a wave walks as its ring does, in whole rounds (fitted to 960
-// launches per scaling, 33 to 64 rows of 576 ... 32768 x 512 ... 12288, operands cold: within 6 per cent for nine in ten).
+// Estimated microseconds at 17 to 64 rows, for the comparison with the tiles (beyond 32 fitted to 960 launches per scaling of 576 ... 32768 x
+// 512 ... 12288, the slabs a wave walks counted as its ring does, in whole rounds).
 float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
   const int ntw = skinny_shape(M, N, K) / 1000;
   const float blocks = (float)ceil_div(ceil_div(N, 16 * ntw), compute_units());  // per CU

@@ -1986,58 +1986,96 @@ static float persistent_cost(int64_t tiles, int slots, float t) {
 // index 0: 128 x 256, 1: 160 x 256, 2: 192 x 256.  Against the eight-wave persistent kernel's 1.63 / 1.40 per slab of a 256 x 256 tile
 // that is 6 ... 9 % less per flop with block scaling and level with row scaling; what decides between the three is
 // mostly how the tile count divides by the CUs.
-static const float kW4SlabBlock[3] = {0.90f, 1.00f, 1.14f}, kW4SlabRow[3] = {0.93f, 0.88f, 1.00f}, kW4Tile = 5.5f;
+static const float kW4SlabBlock[3] = {0.90f, 1.00f, 1.14f}, kW4SlabRow[3] = {0.80f, 0.88f, 1.00f}, kW4Tile = 5.5f;
+// ... and of its cut tiles, with few blocks to share the memory with
+static const float kW4CutSlabBlock[3] = {0.646f, 0.71f, 0.84f}, kW4CutSlabRow[3] = {0.56f, 0.72f, 0.80f};
 // With the tail cut: whole rounds, then a piece per block and the hand-over: a piece's sums written through to memory,
 // then read and added by the tile's last block, piece after piece (measured on 4096 x 7168 x 16384, 104 tiles in two
 // pieces each behind two whole rounds, and on 2048 x 7168 x 18432, 52 tiles in four pieces behind one).
-static const float kW4HandOver = 8.0f, kW4HandOverPiece = 7.0f;
+static const float kW4HandOver = 6.0f, kW4HandOverPiece = 4.5f;
 
 // The shapes the four-wave kernel takes (see gemm_w4_ok; pointers and strides are checked at the launch).
 static bool w4_shape(int64_t M, int64_t N, int64_t K) { return M > 0 && N > 0 && N % 8 == 0 && K >= 512 && K % 256 == 0; }
+
+// One round of three-stage 128 x 128 tiles (fitted: the shape's own time per slab is that of a full chip, and it runs where the chip is not)
+static float three_stage_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
+  const float slabs = (float)ceil_div(K, 128) * (float)ceil_div(ceil_div(M, 128) * ceil_div(N, 128), 256);
+  return (blockscale ? 4.9f + 0.559f * slabs : 6.8f + 0.473f * slabs) + 0.36f * (float)N * (float)K / 6e6f;
+}
+
+// What a plan on the four-wave kernel is estimated to take: tiles of 32 tm rows, whole, with their tail cut or each of them cut
+static float w4_plan_cost(int64_t M, int64_t N, int64_t K, bool blockscale, int tm, bool split) {
+  const int slots = compute_units(), nslab = (int)(K / 128);
+  const float t_slab = blockscale ? kW4SlabBlock[tm - 4] : kW4SlabRow[tm - 4], t = (float)nslab * t_slab + kW4Tile;
+  const int64_t tiles = ceil_div(M, 32 * tm) * ceil_div(N, 256);
+  // (part of one round, weights from memory: a block waits for its copies, and the chip's clock does not make up for it -- 166 x 36864 x 7168 in 144 tiles of 192 rows
+  // 1.17 us per slab, with row scales 260 x 17616 x 6144 in 138 of 160 rows 1.13, in 207 of 128 rows 0.96)
+  if (!split) return tiles < slots && N * K >= ((int64_t)1 << 26) ? (float)nslab * kW4SlabBlock[tm - 4] + kW4Tile : persistent_cost(tiles, slots, t);
+  const W4Split sp = gemm_w4_split(M, N, K, tm);
+  const float pieces = (float)ceil_div(nslab, sp.unit);
+  if (tiles * 2 <= slots)  // (fitted like gemm_mid_shape's estimates: within 5 per cent for nine launches in ten of 128-row tiles, 13 of taller ones)
+    return (blockscale ? 10.5f : 13.0f) + (blockscale ? kW4CutSlabBlock : kW4CutSlabRow)[tm - 4] * (float)sp.unit + 0.886f * pieces + 0.659f * (float)N * (float)K / 6e6f;
+  return (float)(tiles / sp.blocks) * t + (float)sp.unit * t_slab + kW4Tile + kW4HandOver + kW4HandOverPiece * (pieces - 1.f);
+}
 
 // Which four-wave tile height, if any, beats `other_cost` (microseconds, what the plan made of the eight-wave shapes
 // costs) by at least 3 %, and whether with its tail cut (*split; the workspace has to hold the pieces).
 //
 // other_splits: the other plan is a K split (two launches, the shares' sums through memory).  Then the matmul is at most
-// half a round of tiles, and the one candidate is the four-wave kernel with EVERY tile cut into pieces, the pieces
+// half a round of tiles, and the candidates are the four-wave kernel with EVERY tile cut into pieces, the pieces
 // exchanging their sums inside the one launch: measured ahead where the pieces fill three quarters of the chip and are at
 // least 16 slabs long (512 x 7168 x 16384: 67 against 84 us; 1024 x 2112 x 7168: 30 against 35; 384 x 6144 x 8192: 35
 // against 42; 768 x 2048 x 8192, 16 slabs: 27 against 32), behind with shorter pieces (8 slabs: 25 against 22) and with
 // fewer blocks (128 x 4096 x 14336, 16 tiles in 64 pieces: 38 against 27; 512 x 2048 x 28672, 128 pieces: 64 against 51).
-static int pick_w4(int64_t M, int64_t N, int64_t K, bool blockscale, float other_cost, bool other_splits, size_t workspace_bytes, bool* split) {
+// The height with the shortest pieces: 338 x 8192 x 28672 96 tiles of 128 rows in two pieces each 117 us, 64 of 192 rows in four 88.
+static int pick_w4(int64_t M, int64_t N, int64_t K, bool blockscale, float other_cost, bool other_splits, size_t workspace_bytes, bool kv_on, bool* split) {
   const int forced = tuning().w4, cut = tuning().w4_split;
   *split = false;
   if (forced == 0 || !tuning().persist || !w4_shape(M, N, K)) return 0;
   const int nslab = (int)(K / 128), slots = compute_units();
-  if (other_splits) {
-    const int tm = forced > 0 ? forced : 4;
+  // every tile of height tm cut, where its pieces are worth it (see above; forced: wherever there is a cut)
+  auto every_cut = [&](int tm) {
     const W4Split sp = gemm_w4_split(M, N, K, tm);
-    if (cut == 0 || sp.unit <= 0 || sp.bytes > workspace_bytes) return 0;
-    if (ceil_div(M, 32 * tm) * ceil_div(N, 256) * 2 > slots) return 0;  // (not the case meant here)
+    if (cut == 0 || sp.unit <= 0 || sp.bytes > workspace_bytes || ceil_div(M, 32 * tm) * ceil_div(N, 256) * 2 > slots) return false;
     // (more than four pieces only where they are long: 128 x 8192 x 28672 in eight pieces of 28 slabs 59 against 64 us,
     // 512 x 2048 x 28672 46 against 52; in eight of 16 slabs 128 x 8192 x 16384 47 against 41.  And only where the rows
-    // fill three quarters of the 128-row tiles: 48 ... 64 rows on 8192 x 28672 took 56 against 48 ... 51.)
+    // fill three quarters of the tiles: 48 ... 64 rows on 8192 x 28672 took 56 against 48 ... 51.)
     const int64_t pieces = ceil_div(nslab, sp.unit), rows_padded = ceil_div(M, 32 * tm) * 32 * tm;
-    if (forced <= 0 && cut != 1 &&
-        (sp.unit < (pieces > 4 ? 24 : 16) || (int64_t)sp.blocks * 4 < (int64_t)slots * 3 || M * 4 < rows_padded * 3))
-      return 0;
-    *split = true;
-    return tm;
+    return forced > 0 || cut == 1 ||
+           (sp.unit >= (pieces > 4 ? 24 : 16) && (int64_t)sp.blocks * 4 >= (int64_t)slots * 3 && M * 4 >= rows_padded * 3);
+  };
+  if (other_splits) {
+    int best = 0;
+    float best_cost = 0.f;
+    // (where the smallest tiles cut are not worth it, taller ones are not either: 164 x 8192 x 28672 in 32 tiles of 192 rows 71 us, K split 63)
+    if (forced <= 0 && !every_cut(4)) return 0;
+    for (int tm = 4; tm <= 6; ++tm) {
+      if ((forced > 0 && tm != forced) || !every_cut(tm)) continue;
+      const float cost = w4_plan_cost(M, N, K, blockscale, tm, true);
+      if (!best || cost < 0.95f * best_cost) { best = tm; best_cost = cost; }  // (the smaller tiles where it is level)
+    }
+    *split = best > 0;
+    return best;
   }
   int best = 0;
   float best_cost = forced > 0 ? 3.0e38f : 0.97f * other_cost;  // (a forced height is taken whatever it costs)
-  for (int i = 0; i < 3; ++i) {
-    const int tm = 4 + i;
+  for (int tm = 4; tm <= 6; ++tm) {
     if (forced > 0 && tm != forced) continue;
-    const float t_slab = blockscale ? kW4SlabBlock[i] : kW4SlabRow[i], t = (float)nslab * t_slab + kW4Tile;
     const int64_t tiles = ceil_div(M, 32 * tm) * ceil_div(N, 256);
-    if (forced <= 0 && tiles * 4 < (int64_t)slots * 3) continue;  // (well under one round: more, smaller tiles and a K split are the better fit)
-    const float whole = persistent_cost(tiles, slots, t);
+    // (half a round or less: more, smaller tiles and a K split are the better fit; a little more than half is not: 166 x 36864 x 7168 in
+    // 144 tiles of 192 rows 71 us, in 288 of 128 rows 101)
+    if (forced <= 0 && tiles * 2 <= slots) {
+      // (where the eight-wave shapes fill the chip without a K split, as one short round, the cut tiles may still be ahead: 1929 x 1536 x
+      // 7168 in 96 tiles of two pieces 30 against 38 us; the fused QKV projection not: 435 x 7168 x 5120 41 against 34)
+      const float cost = !kv_on && every_cut(tm) ? w4_plan_cost(M, N, K, blockscale, tm, true) : best_cost;
+      if (cost < 0.9f * best_cost) { best = tm; best_cost = cost; *split = true; }
+      continue;
+    }
+    const float whole = w4_plan_cost(M, N, K, blockscale, tm, false);
     if (whole < best_cost) { best = tm; best_cost = whole; *split = false; }
     const W4Split sp = gemm_w4_split(M, N, K, tm);
     if (cut != 0 && sp.unit > 0 && sp.bytes <= workspace_bytes) {
-      const float pieces = (float)ceil_div(nslab, sp.unit);
-      float with_cut = (float)(tiles / sp.blocks) * t + (float)sp.unit * t_slab + kW4Tile + kW4HandOver + kW4HandOverPiece * (pieces - 1.f);
+      float with_cut = w4_plan_cost(M, N, K, blockscale, tm, true);
       if (cut == 1) with_cut *= 1.0e-3f;  // (switched on: wherever there is one)
       if (with_cut < best_cost) { best = tm; best_cost = with_cut; *split = true; }
     }
@@ -2095,14 +2133,15 @@ static TiledPlan make_plan(int64_t M, int64_t N, int64_t K, bool blockscale, boo
   // on 128 x 128, 330 x 6144 x 4096 row 37.3 -> 27.7 us; 256 x 128 instead of 128 x 128, 512 x 10240 x 8192 row 65.0 -> 57.9.)
   if (batch == 1 && !plan.streamk && (free_choice || plan.variant == 1)) {
     float other = plan.two.axis ? plan.two.cost : region_cost(M, N, nslab, t, blockscale, kv_on);
+    if (!kv_on && !plan.two.axis && plan.variant == 4 && plan.splits == 1 && tiles <= t.slots) other = three_stage_cost(M, N, K, blockscale);
     if (!kv_on && !plan.two.axis && persist_shape(M, N, plan.variant))
       other = persistent_cost(tiles, t.slots, (float)nslab * (blockscale ? t.t_slab_block : t.t_slab_row) + tile_overhead(M, N, plan.variant - 1, 1));
     if (kv_on && has_workspace && free_choice) {
       const TileShape& u = kShapes[pick_shape(M, N, nslab, blockscale, true) - 1];
       if (pick_splits(ceil_div(M, u.bm) * ceil_div(N, u.bn), u.slots, nslab) > 1)
-        plan.w4 = pick_w4(M, N, K, blockscale, other, true, workspace_bytes, &plan.w4_split);
+        plan.w4 = pick_w4(M, N, K, blockscale, other, true, workspace_bytes, kv_on, &plan.w4_split);
     }
-    if (!plan.w4) plan.w4 = pick_w4(M, N, K, blockscale, other, wants_split, has_workspace ? workspace_bytes : 0, &plan.w4_split);
+    if (!plan.w4) plan.w4 = pick_w4(M, N, K, blockscale, other, wants_split, has_workspace ? workspace_bytes : 0, kv_on, &plan.w4_split);
     if (plan.w4) plan.splits = 1;
   }
   return plan;
@@ -2149,40 +2188,27 @@ static TiledPlan cached_plan(int64_t M, int64_t N, int64_t K, bool blockscale, b
   return plan;
 }
 
-// Estimated microseconds of this shape's plan with all the workspace it asks for, where the plan is one of those that small
-// matmuls get: a K split, every tile cut, one round of three-stage 128 x 128 tiles (fitted like gemm_mid_shape's estimates:
-// within 7, 5 and 20 per cent for nine launches in ten); 0 for every other plan.
-float gemm_tiled_small_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
+// Estimated microseconds of this shape's plan with all the workspace it asks for.  A K split, every tile cut, one round of three-stage
+// 128 x 128 tiles: fitted like gemm_mid_shape's estimates, within 7, 5 and 20 per cent for nine launches in ten; every other plan: what the planner
+// compares.
+float gemm_tiled_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
   const TiledPlan plan = cached_plan(M, N, K, blockscale, true, ~(size_t)0, 1, false);
   const float slabs = (float)ceil_div(K, 128), stream = (float)N * (float)K / 6e6f;
-  if (plan.w4) {
-    if (!plan.w4_split || ceil_div(M, 32 * plan.w4) * ceil_div(N, 256) * 2 > compute_units()) return 0.f;
-    const int unit = gemm_w4_split(M, N, K, plan.w4).unit;
-    return 10.5f + 0.646f * (float)unit + 0.886f * (float)ceil_div((int64_t)slabs, unit) + 0.659f * stream;
-  }
-  if (plan.two.axis || plan.streamk) return 0.f;
+  if (plan.w4) return w4_plan_cost(M, N, K, blockscale, plan.w4, plan.w4_split);
+  if (plan.two.axis) return plan.two.cost;
   if (plan.splits > 1)
     return 8.2f + 0.33f * (float)ceil_div((int64_t)slabs, plan.splits) * (kShapes[plan.variant - 1].bm == 128 ? 1.f : 1.25f) +
            1.024f * (float)plan.splits * (float)M * (float)N * 8.0f / 4.0e6f + 0.63f * stream;
-  if (plan.variant == 4) return 4.9f + 0.559f * slabs * (float)ceil_div(ceil_div(M, 128) * ceil_div(N, 128), 256) + 0.36f * stream;
-  return 0.f;
+  if (plan.variant == 4) return three_stage_cost(M, N, K, blockscale);
+  return region_cost(M, N, (int)slabs, kShapes[plan.variant - 1], blockscale);
 }
 
 // The same for a fused QKV matmul, of any plan (with the workspace it asks for, or without any)
 float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool has_workspace) {
   const TiledPlan plan = cached_plan(M, N, K, blockscale, has_workspace, has_workspace ? ~(size_t)0 : 0, 1, true);
-  const int64_t slabs = ceil_div(K, 128), slots = compute_units();
-  const float stream = (float)N * (float)K / 6e6f;
-  if (plan.w4) {
-    const int64_t tiles = ceil_div(M, 32 * plan.w4) * ceil_div(N, 256);
-    if (plan.w4_split && tiles * 2 <= slots) {
-      const int unit = gemm_w4_split(M, N, K, plan.w4).unit;
-      return 10.5f + 0.646f * (float)unit + 0.886f * (float)ceil_div(slabs, unit) + 0.659f * stream;
-    }
-    return persistent_cost(tiles, (int)slots, (float)slabs * (blockscale ? kW4SlabBlock : kW4SlabRow)[plan.w4 - 4] + kW4Tile);
-  }
-  if (plan.variant == 4) return 4.9f + 0.559f * (float)slabs * (float)ceil_div(ceil_div(M, 128) * ceil_div(N, 128), 256) + 0.36f * stream;
-  return region_cost(M, N, (int)slabs, kShapes[plan.variant - 1], blockscale, true);
+  if (plan.w4) return w4_plan_cost(M, N, K, blockscale, plan.w4, plan.w4_split);
+  if (plan.variant == 4) return three_stage_cost(M, N, K, blockscale);
+  return region_cost(M, N, (int)ceil_div(K, 128), kShapes[plan.variant - 1], blockscale, true);
 }
 
 // The workspace of a fused QKV matmul's plan (its cut tiles' sums; 0: none are cut)

@@ -19,7 +19,8 @@
 //   MAXFP8_SKINNY_ALDS=0       decode kernel: activations loaded per slab even where a wave's share of them fits LDS
 //   MAXFP8_SKINNY_QUANT=0      linears: always the quantiser's launch in front of the decode kernel
 //   MAXFP8_SKINNY=<ntw>4<KB>   force a shape of the weight-streaming kernel (e.g. 1408, 2416)
-//   MAXFP8_MID=0 / <MT><NT>    the kernel for tens to a few hundred tokens: never / always, in 16 MT x 16 NT tiles (e.g. 43)
+//   MAXFP8_MID=0 / [<b>]<MT><NT>  the kernel for tens to hundreds of tokens: never / always, in 16 MT x 16 NT tiles (e.g. 43), b blocks per
+//                              CU (e.g. 244; without b the first built shape with that tile)
 //   MAXFP8_SHORT_K=0           batches of short K: the decode and tile kernels only
 #pragma once
 

@@ -1,0 +1,65 @@
+"""Every built shape of the kernel whose blocks split K among their waves, by its tile and its blocks per CU: exact where the arithmetic is, on
+ragged sizes, K tails, shares of K without a slab and grids of one, several and many blocks; and the heights and cuts the planner
+takes for matmuls of little more than half a round of tiles."""
+import os
+
+import pytest
+import torch
+
+import modular_amd as mx
+from modular_amd import _lib
+
+CFG = {"block": mx.blockwise_fp8_config(), "row": mx.rowwise_fp8_config()}
+# blocks per CU, 16-token groups, 16-column groups
+SHAPES = [411, 312, 321, 422, 222, 323, 123, 324, 124, 231, 132, 133, 234, 134, 141, 142, 143, 244]
+
+
+@pytest.fixture
+def forced():
+    def use(value):
+        os.environ["MAXFP8_MID"] = str(value)
+        _lib.tuning_reload()
+    yield use
+    os.environ.pop("MAXFP8_MID", None)
+    _lib.tuning_reload()
+
+
+def exact_case(M, N, K, kind, seed):
+    """small integers times powers of two: every sum is exact in any order"""
+    g = torch.Generator().manual_seed(seed)
+    a = torch.randint(-2, 3, (M, K), generator=g).float().to(torch.float8_e4m3fn)
+    b = torch.randint(-2, 3, (N, K), generator=g).float().to(torch.float8_e4m3fn)
+    if kind == "block":
+        sa = 2.0 ** torch.randint(-1, 2, (-(-K // 128), -(-M // 4) * 4), generator=g).float()
+        sb = 2.0 ** torch.randint(-1, 2, (-(-N // 128), -(-K // 128)), generator=g).float()
+    else:
+        sa, sb = 2.0 ** torch.randint(-1, 2, (1, M), generator=g).float(), 2.0 ** torch.randint(-1, 2, (N, 1), generator=g).float()
+    return a, b, sa, sb
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["block", "row"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_every_built_shape_is_exact(dev, forced, kind, shape):
+    blocks, mt, nt = shape // 100, shape // 10 % 10, shape % 10
+    forced(shape)
+    assert f"{blocks} per CU" in _lib.matmul_describe(20, 512, 512)
+    waves = 8 if blocks == 1 else 4
+    # one slab; a slab more than the waves; a K tail; the longest share of a wave; several rounds of blocks; more tokens than the
+    # choice by estimates takes below the tiles
+    for i, (M, N, K) in enumerate([(16 * mt, 16 * nt, 128), (16 * mt + 1, 16 * nt * 9 + 8, 128 * (waves + 1)), (5, 16 * nt * 3 - 3, 1040),
+                                   (17, 16 * nt, 64 * waves * 128 if waves == 4 else 32768), (3 * 16 * mt - 7, 16 * nt * 601, 256), (1030, 16 * nt * 2, 640)]):
+        case = exact_case(M, N, K, kind, 100 * shape + i)
+        on = [t.to(dev) for t in case]
+        run = lambda algo: mx.dynamic_scaled_matmul(*on, CFG[kind].input_scale, CFG[kind].weight_scale, algo=algo)
+        assert torch.equal(run("auto"), run("naive")), f"shape {shape}, {M} x {N} x {K}"
+
+
+def test_heights_and_cuts_of_little_more_than_half_a_round():
+    # one row tile of 192 instead of two of 128: 144 tiles on 256 CUs
+    assert _lib.matmul_describe(166, 36864, 7168) == "192x256 x144 persistent, four waves"
+    # two row tiles of 192 in four pieces instead of three of 128 in two; where 128-row tiles do not pay, K splits as before
+    assert _lib.matmul_describe(338, 8192, 28672, False) == "192x256 x64 persistent, four waves, every tile cut in pieces of 56 slabs"
+    assert "K split" in _lib.matmul_describe(164, 8192, 28672, False) and "K split 3" in _lib.matmul_describe(2048, 2304, 16384)
+    # cut tiles against a short round of whole ones, with the workspace and without
+    assert "every tile cut" in _lib.matmul_describe(1929, 1536, 7168) and "cut" not in _lib.matmul_describe(1929, 1536, 7168, True, False)
