@@ -25,20 +25,34 @@ struct KvStore {
   int bf16_scaling;               // per-tensor / per-channel flavour: scales are applied in bf16
 };
 
-struct GemmArgs {
+// What the plain matmuls read.  (A base of its own, because a launch copies its arguments to the GPU's memory, over the bus: 480 bytes take
+// 0.6 us of host time, the decode kernel's 200 a third of it -- with two launches of 3 us in a small linear.)
+struct MatmulArgs {
   const uint8_t* a;        // [M, K] e4m3fn, row stride lda bytes
   const uint8_t* b;        // [N, K] e4m3fn (per expert when grouped), row stride ldb bytes
   void* c;                 // [M, N] bf16 or f32, row stride ldc elements
   const float* a_scales;   // block: [ceil(K/128), a_scales_ld]; row/tensor: element m * a_scale_stride
   const float* b_scales;   // block: [ceil(N/128), b_scales_ld]; row/tensor: element n * b_scale_stride
   int M, N, K;
+  int c_dtype;
   int64_t lda, ldb, ldc;
   int64_t a_scales_ld, b_scales_ld;
   int64_t a_scale_stride, b_scale_stride;
-  int c_dtype;
   int scales_dtype;        // row / tensor scaling: MAXFP8_F32, MAXFP8_BF16 or MAXFP8_F16 (block scaling is always f32)
   int c_vec_ok;            // C base and ldc allow 4-element vector stores
   int c_vec8_ok;           // ... and 8-element ones (16-byte aligned rows)
+  // decode kernel with the quantisation inside (a is not used then): the bf16 activations, their row stride in elements, and
+  // how they are quantised -- dynamically (scales bounded by x_scale_ub) or by a fixed scale (x_static; x_recip its reciprocal,
+  // x_scale what the result is multiplied by in place of a_scales and b_scales)
+  int x_static;
+  const uint16_t* x;
+  int64_t ldx;
+  float x_scale_ub, x_recip, x_scale;
+  // batched only: blockIdx.z (tiled) / blockIdx.y (skinny) steps the five base pointers, in elements
+  int64_t a_batch, b_batch, c_batch, a_scales_batch, b_scales_batch;
+};
+
+struct GemmArgs : MatmulArgs {
   // grouped only
   const uint32_t* offsets;
   const int32_t* expert_ids;
@@ -53,8 +67,6 @@ struct GemmArgs {
   int64_t b_expert_stride;   // bytes between experts in b
   int64_t bs_expert_stride;  // elements between experts in b_scales
   const uint32_t* c_row_index;  // grouped only, optional: row m of the result is stored at row c_row_index[m] of c
-  // batched only: blockIdx.z (tiled) / blockIdx.y (skinny) steps the five base pointers, in elements
-  int64_t a_batch, b_batch, c_batch, a_scales_batch, b_scales_batch;
   // split-K / skinny only
   float* workspace;
   int splits;
@@ -64,13 +76,6 @@ struct GemmArgs {
   // four-wave kernel only: slabs per block of the tail (the tiles beyond the last whole round of the chip, cut evenly along
   // K among the blocks; 0: every tile is computed whole by one block)
   int tail_units;           // the four-wave kernel: slabs of a run of its cut tail (0: whole tiles only)
-  // decode kernel with the quantisation inside (a is not used then): the bf16 activations, their row stride in elements, and
-  // how they are quantised -- dynamically (scales bounded by x_scale_ub) or by a fixed scale (x_static; x_recip its reciprocal,
-  // x_scale what the result is multiplied by in place of a_scales and b_scales)
-  const uint16_t* x;
-  int64_t ldx;
-  int x_static;
-  float x_scale_ub, x_recip, x_scale;
   // fused QKV only
   int kv_on;
   KvStore kv;
@@ -155,8 +160,9 @@ __device__ __forceinline__ uint16_t* kv_dst(const KvStore& kv, void* c, int64_t 
 }
 
 // the arguments of batch `b` of a batched matmul
-__device__ __forceinline__ GemmArgs batch_view(const GemmArgs& p, int64_t b) {
-  GemmArgs q = p;
+template <class Args>
+__device__ __forceinline__ Args batch_view(const Args& p, int64_t b) {
+  Args q = p;
   q.a += b * p.a_batch;
   q.b += b * p.b_batch;
   q.c = reinterpret_cast<uint8_t*>(p.c) + b * p.c_batch * (p.c_dtype == 0 /* bf16 */ ? 2 : 4);

@@ -63,7 +63,7 @@ struct MidSlabAt { uint32_t koff, kill, kill_s, scales; };
 
 // KV: the fused QKV projection's epilogue and its wave of page look-ups
 template <int MT, int NT, bool BLOCKSCALE, int W_POLICY, int BLOCKS, bool KV>
-__global__ __launch_bounds__((BLOCKS == 1 ? 512 : 256) + (KV ? 64 : 0)) __attribute__((amdgpu_waves_per_eu(1, (BLOCKS == 1 ? 2 : BLOCKS) + (KV ? 1 : 0)))) void gemm_mid_kernel(GemmArgs p, int tiles_m, int tiles_n) {
+__global__ __launch_bounds__((BLOCKS == 1 ? 512 : 256) + (KV ? 64 : 0)) __attribute__((amdgpu_waves_per_eu(1, (BLOCKS == 1 ? 2 : BLOCKS) + (KV ? 1 : 0)))) void gemm_mid_kernel(std::conditional_t<KV, GemmArgs, MatmulArgs> p, int tiles_m, int tiles_n) {
   using Cfg = MidCfg<MT, NT, BLOCKSCALE, BLOCKS>;
   constexpr int NWAVES = Cfg::NWAVES, BM = Cfg::BM, BN = Cfg::BN, DEPTH = Cfg::DEPTH, PER = Cfg::PER, SLOT = Cfg::SLOT;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -231,7 +231,7 @@ __global__ __launch_bounds__((BLOCKS == 1 ? 512 : 256) + (KV ? 64 : 0)) __attrib
     // fused QKV: a wave of its own looks up the rows' pages.  Its loads depend on one another, a search among the sequences and two
     // more; in one of the other waves each of them waited for all copies in front of it, and the wave's share of K for them
     // (64 tokens of 64 sequences, 10240 x 8192 with row scales, quantiser included: 29.1 -> 26.6 us).
-    row_table[lane] = lane < rows_here ? kv_row_offset(p.kv, m0 + lane) : -1;
+    if constexpr (KV) row_table[lane] = lane < rows_here ? kv_row_offset(p.kv, m0 + lane) : -1;
   }
   __syncthreads();
 
@@ -315,7 +315,8 @@ static int launch_mid(const GemmArgs& p, hipStream_t stream) {
   // weights that are read once and are more than a quarter of the memory-side cache: non-temporal (10240 x 8192 at 64 tokens
   // 24.1 -> 23.2 us; smaller ones may still sit in that cache and then come quicker without: 1536 x 7168 9.4 against 12.8)
   const bool once = p.M <= Cfg::BM && (int64_t)p.N * p.K >= ((int64_t)1 << 26);
-  void (*kern)(GemmArgs, int, int) = gemm_mid_kernel<MT, NT, BLOCKSCALE, 0, BLOCKS, KV>;
+  using Args = std::conditional_t<KV, GemmArgs, MatmulArgs>;
+  void (*kern)(Args, int, int) = gemm_mid_kernel<MT, NT, BLOCKSCALE, 0, BLOCKS, KV>;
   if (once) kern = gemm_mid_kernel<MT, NT, BLOCKSCALE, kStreamOnce, BLOCKS, KV>;
   static PerDeviceFlag attrs[2];
   PerDeviceFlag& attr = attrs[once];
@@ -326,7 +327,7 @@ static int launch_mid(const GemmArgs& p, hipStream_t stream) {
     attr_done = true;
   }
   const int64_t tiles_m = ceil_div(p.M, Cfg::BM), tiles_n = ceil_div(p.N, Cfg::BN);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3((Cfg::NWAVES + (KV ? 1 : 0)) * 64), Cfg::SMEM, stream, p, (int)tiles_m, (int)tiles_n);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3((Cfg::NWAVES + (KV ? 1 : 0)) * 64), Cfg::SMEM, stream, static_cast<const Args&>(p), (int)tiles_m, (int)tiles_n);
   return launch_status("gemm_mid");
 }
 

@@ -96,8 +96,8 @@ __host__ __device__ constexpr uint32_t skinny_acts_bytes(uint32_t M, uint32_t pe
 
 // KV: the fused QKV projection's epilogue (a kernel of its own: the plain one would load its arguments all the same, 1 to 2 per cent)
 template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, int ACTS = kActsPerSlab, bool KV = false>
-__global__ __launch_bounds__(NWAVES * 64 + (KV ? 64 : 0)) void gemm_skinny_kernel(GemmArgs p_in) {
-  const GemmArgs p = gridDim.y == 1 ? p_in : batch_view(p_in, blockIdx.y);
+__global__ __launch_bounds__(NWAVES * 64 + (KV ? 64 : 0)) void gemm_skinny_kernel(std::conditional_t<KV, GemmArgs, MatmulArgs> p_in) {
+  const auto p = gridDim.y == 1 ? p_in : batch_view(p_in, blockIdx.y);
   using Cfg = SkinnyCfg<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ACTS>;
   constexpr bool ALDS = Cfg::ALDS, QUANT = Cfg::QUANT;
   static_assert(!ALDS || MT == 1, "activations in LDS: one 16-token group");
@@ -516,7 +516,7 @@ static int launch_skinny_r(const GemmArgs& p, int64_t batch, hipStream_t stream)
   const uint32_t per_wave = (uint32_t)ceil_div(ceil_div(p.K, 128), NWAVES);
   const int smem = Cfg::SMEM + NWAVES * (int)skinny_acts_bytes<ACTS, BLOCKSCALE>((uint32_t)p.M, per_wave) + (KV ? Cfg::ROW_TABLE : 0);
   const int64_t blocks = ceil_div(p.N, 16 * NTW);
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)batch), dim3((NWAVES + (KV ? 1 : 0)) * 64), smem, stream, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)batch), dim3((NWAVES + (KV ? 1 : 0)) * 64), smem, stream, static_cast<const std::conditional_t<KV, GemmArgs, MatmulArgs>&>(p));
   return launch_status("gemm_skinny");
 }
 
