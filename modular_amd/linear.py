@@ -69,7 +69,12 @@ class Linear(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
-        y = quantized_matmul(x2, self.weight, self.weight_scale, self.input_scale, self.quant_config)
+        # (the buffers from their dictionary: torch's attribute look-up takes 0.3 us for each, in a call of 6.  A weight that is no buffer,
+        # as after a program has put a parameter in its place, is looked up.)
+        buffers = self._buffers
+        weight, scale = buffers.get("weight"), buffers.get("weight_scale")
+        y = quantized_matmul(x2, self.weight if weight is None else weight, self.weight_scale if scale is None else scale, self.input_scale,
+                             self.quant_config)
         if self.bias is not None:
             y = y + self.bias.to(y.dtype)
         return y if x.dim() == 2 else y.reshape(*x.shape[:-1], self.out_dim)
