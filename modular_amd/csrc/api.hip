@@ -269,7 +269,7 @@ static size_t auto_workspace(int64_t M, int64_t N, int64_t K, bool block) {
   return choose_kernel(M, N, K, block) == MAXFP8_ALGO_TILED ? gemm_tiled_workspace_bytes(M, N, K) : 0;
 }
 
-// The same for the fused QKV matmul: decode kernel (at most 64 rows), the kernel in between (at most 320) or the tiles, whose
+// The same for the fused QKV matmul: decode kernel (at most 16 rows), the kernel in between (17 to 64, beyond by its estimate) or the tiles, whose
 // plan may cut them along K where the caller brings a workspace.
 static int choose_qkv(int64_t T, int64_t N, int64_t K, bool has_workspace, bool block) {
   const Tuning& t = tuning();

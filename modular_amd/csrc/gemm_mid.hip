@@ -17,12 +17,12 @@
 //     behind another's loop (432 x 3648 x 2432 in 64 x 64 tiles 16.3 -> 12.5 us, 730 x 1824 x 1536 12.1 -> 9.3).
 //   * Epilogue: partial sums to LDS as [token][column], a thread adds them (in wave order) for eight columns of a token,
 //     scales, converts and stores 16 bytes.  Row scales are loaded in front of the copies (their first use was the longest
-//     wait of the epilogue: 64 x 10240 x 8192 22.9 -> 19.9 us), the fused QKV projection's page look-ups made before the loop.
+//     wait of the epilogue); a wave of its own makes the fused QKV projection's page look-ups during the loop.
 //
 // Bound: what a CU can pull out of the L2s -- every block fetches its tokens and weights itself, 16 * (MT + NT) * K bytes.
 // Measured (graph timing, operands in the memory-side cache) against what ran these shapes before: 117 x 6144 x 4096 12.1 -> 10.2 us,
-// 64 x 10240 x 8192 with row scales 23.5 -> 19.8, 432 x 3648 x 2432 20.1 -> 12.5, 730 x 1824 x 1536 17.2 -> 8.8, 18 x 4096 x 14336 15.6 ->
-// 13.4, 28 x 6144 x 4096 8.9 -> 7.3.  Bytes at 7 TB/s: 3.9, 12.2, 2.1, 1.1, 8.4 and 3.7.
+// 432 x 3648 x 2432 20.1 -> 12.5, 730 x 1824 x 1536 17.2 -> 8.8, 18 x 4096 x 14336 15.6 -> 13.4, 28 x 6144 x 4096 8.9 -> 7.3.  Bytes at
+// 7 TB/s: 3.9, 2.1, 1.1, 8.4 and 3.7.  64 x 10240 x 8192 with row scales, whose weights pass the L2s by (`once` below), stays at 23.7 (12.2).
 #include <type_traits>
 #include <utility>
 
@@ -230,7 +230,7 @@ __global__ __launch_bounds__((BLOCKS == 1 ? 512 : 256) + (KV ? 64 : 0)) __attrib
   } else if (lane < BM) {
     // fused QKV: a wave of its own looks up the rows' pages.  Its loads depend on one another, a search among the sequences and two
     // more; in one of the other waves each of them waited for all copies in front of it, and the wave's share of K for them
-    // (64 tokens of 64 sequences, 10240 x 8192 with row scales, quantiser included: 29.1 -> 26.6 us).
+    // (64 tokens of 64 sequences, 10240 x 8192 with row scales, quantiser and the new tiles included: 30.9 -> 30.5 us).
     if constexpr (KV) row_table[lane] = lane < rows_here ? kv_row_offset(p.kv, m0 + lane) : -1;
   }
   __syncthreads();

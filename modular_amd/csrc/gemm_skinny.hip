@@ -123,7 +123,7 @@ __global__ __launch_bounds__(NWAVES * 64 + (KV ? 64 : 0)) void gemm_skinny_kerne
   const int s_end = (s_begin + per_wave) < nslab ? (s_begin + per_wave) : nslab;
 
   // Fused QKV: a wave of its own looks up the rows' pages while the others walk their slabs.  Its loads depend on one another (a search
-  // among the sequences and two more) and stood at the end of the kernel before: 8 tokens of 8 sequences, 6144 x 4096, 11.5 -> 11.0 us, quantiser
+  // among the sequences and two more) and stood at the end of the kernel before: 10 tokens, 6144 x 4096, 11.5 -> 11.1 us, quantiser
   // included.
   [[maybe_unused]] int64_t* row_table = reinterpret_cast<int64_t*>(smem + Cfg::RINGS + WAVES * skinny_acts_bytes<ACTS, BLOCKSCALE>((uint32_t)p.M, (uint32_t)per_wave));
   if constexpr (KV) {
