@@ -313,7 +313,8 @@ template <int MT, int NT, bool BLOCKSCALE, int BLOCKS, bool KV>
 static int launch_mid(const GemmArgs& p, hipStream_t stream) {
   using Cfg = MidCfg<MT, NT, BLOCKSCALE, BLOCKS>;
   // weights that are read once and are more than a quarter of the memory-side cache: non-temporal (10240 x 8192 at 64 tokens
-  // 24.1 -> 23.2 us; smaller ones may still sit in that cache and then come quicker without: 1536 x 7168 9.4 against 12.8)
+  // 24.1 -> 23.2 us; smaller ones may still sit in that cache and then come quicker without: 1536 x 7168 9.4 against 12.8; from 2^23 on for tiles of
+  // up to 32 tokens: 1.7 per cent from memory, -5 from the cache)
   const bool once = p.M <= Cfg::BM && (int64_t)p.N * p.K >= ((int64_t)1 << 26);
   using Args = std::conditional_t<KV, GemmArgs, MatmulArgs>;
   void (*kern)(Args, int, int) = gemm_mid_kernel<MT, NT, BLOCKSCALE, 0, BLOCKS, KV>;
@@ -376,9 +377,11 @@ int gemm_mid_shape(int64_t M, int64_t N, int64_t K, bool blockscale, float* us) 
 }
 
 // The kernel here or the decode kernel (gemm_skinny.hip), at most 64 rows.  From 17 on the decode kernel loads two or four groups of 16 tokens
-// straight into the MFMA's operand layout and is behind everywhere (17 x 7168 x 18432 27.0 against 27.6 us at best; 22 x 3312 x 512
-// 4.5 against 3.5, 28 x 4096 x 14336 19.1 against 13.5, 64 x 4096 x 14336 31.7 against 15.2).  Up to 16 it keeps more weights in flight:
-// 3 per cent behind with the weights in the memory-side cache, as much ahead where they come from memory.
+// straight into the MFMA's operand layout and is behind with the weights in the memory-side cache (17 x 7168 x 18432 27.0 against 27.6 us at
+// best; 22 x 3312 x 512 4.5 against 3.5, 28 x 4096 x 14336 19.1 against 13.5, 64 x 4096 x 14336 31.7 against 15.2; 17 to 32 rows 1.2 on
+// average).  With weights that come from memory 17 to 32 rows are 1.07 on average, and up to 13 per cent behind on a quarter of the
+// shapes, most with row scales and one or two of the decode kernel's blocks per CU (18 x 2048 x 4880 5.9 against 6.8, the cache 6.3 against
+// 5.9).  Up to 16 rows the decode kernel keeps more weights in flight: 3 per cent behind in that cache, as much ahead from memory.
 bool gemm_mid_before_skinny(int64_t M, int64_t N, int64_t K) {
   if (!gemm_mid_ok(M, N, K) || tuning().skinny || tuning().mid == 0) return false;
   return M > 16 || tuning().mid > 0;
