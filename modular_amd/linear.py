@@ -69,10 +69,12 @@ class Linear(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
-        # (the buffers from their dictionary: torch's attribute look-up takes 0.3 us for each, in a call of 6.  A weight that is no buffer,
-        # as after a program has put a parameter in its place, is looked up.)
-        buffers = self._buffers
-        weight, scale = buffers.get("weight"), buffers.get("weight_scale")
+        # (the buffers from their dictionary: torch's attribute look-up takes 0.3 us for each, in a call of 6.  Only where that look-up would
+        # find them there: not in a subclass, which may define either name or the look-up itself, not behind an attribute of the
+        # object's own, and not where a program has put something else in a buffer's place, as a parameter.)
+        own, buffers = self.__dict__, self._buffers if type(self) is Linear else {}
+        weight = None if "weight" in own else buffers.get("weight")
+        scale = None if "weight_scale" in own else buffers.get("weight_scale")
         y = quantized_matmul(x2, self.weight if weight is None else weight, self.weight_scale if scale is None else scale, self.input_scale,
                              self.quant_config)
         if self.bias is not None:
