@@ -94,9 +94,13 @@ __host__ __device__ constexpr uint32_t skinny_acts_bytes(uint32_t M, uint32_t pe
   return ACTS > kActsLds ? rows + (BLOCKSCALE ? (M * per_wave * 4u + 15u) & ~15u : 128u) : rows;
 }
 
+// The fused QKV projection's form has a wave of its own for the page look-ups where the tokens are one group of 16.  (With five waves two share
+// a SIMD, so each has half of its registers: 256, which two or four groups do not fit.)
+__host__ __device__ constexpr int skinny_page_waves(int mt, bool kv) { return kv && mt == 1 ? 1 : 0; }
+
 // KV: the fused QKV projection's epilogue (a kernel of its own: the plain one would load its arguments all the same, 1 to 2 per cent)
 template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, int ACTS = kActsPerSlab, bool KV = false>
-__global__ __launch_bounds__(NWAVES * 64 + (KV ? 64 : 0)) void gemm_skinny_kernel(std::conditional_t<KV, GemmArgs, MatmulArgs> p_in) {
+__global__ __launch_bounds__((NWAVES + skinny_page_waves(MT, KV)) * 64) void gemm_skinny_kernel(std::conditional_t<KV, GemmArgs, MatmulArgs> p_in) {
   const auto p = gridDim.y == 1 ? p_in : batch_view(p_in, blockIdx.y);
   using Cfg = SkinnyCfg<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ACTS>;
   constexpr bool ALDS = Cfg::ALDS, QUANT = Cfg::QUANT;
@@ -126,7 +130,8 @@ __global__ __launch_bounds__(NWAVES * 64 + (KV ? 64 : 0)) void gemm_skinny_kerne
   // among the sequences and two more) and stood at the end of the kernel before: 10 tokens, 6144 x 4096, 11.5 -> 11.1 us, quantiser
   // included.
   [[maybe_unused]] int64_t* row_table = reinterpret_cast<int64_t*>(smem + Cfg::RINGS + WAVES * skinny_acts_bytes<ACTS, BLOCKSCALE>((uint32_t)p.M, (uint32_t)per_wave));
-  if constexpr (KV) {
+  constexpr bool PAGE_WAVE = skinny_page_waves(MT, KV) > 0;
+  if constexpr (PAGE_WAVE) {
     if (wave == WAVES) {
       if (lane < 16 * MT) row_table[lane] = lane < p.M ? kv_row_offset(p.kv, lane) : -1;
       if constexpr (QUANT && !BLOCKSCALE) {
@@ -254,8 +259,9 @@ __global__ __launch_bounds__(NWAVES * 64 + (KV ? 64 : 0)) void gemm_skinny_kerne
                                                koff + t * w_tile + w_half, 0, kWeightStream);
     }
     // (the slabs' loads stay in this order: with another one in front of the loop, the waits the compiler adds for registers have to hold for
-    // both and were for everything in flight, once a round of the ring; 1 to 4 tokens, 102 matmuls, 3.6 per cent, up to 25)
-    __builtin_amdgcn_sched_barrier(0);
+    // both and were for everything in flight, once a round of the ring; 1 to 4 tokens, 102 matmuls, 3.6 per cent, up to 25.  Not in the form
+    // that has no registers to spare for the order: it spilled a fifth more.)
+    if constexpr (NTW * MT < 16) __builtin_amdgcn_sched_barrier(0);
   };
   auto compute = [&](auto d_c, [[maybe_unused]] int slab) {
     constexpr int d = decltype(d_c)::value;
@@ -421,7 +427,9 @@ __global__ __launch_bounds__(NWAVES * 64 + (KV ? 64 : 0)) void gemm_skinny_kerne
     if (m >= p.M || n >= p.N) continue;
     if constexpr (KV) {
       // fused QKV: the reference's bf16 roundings, then C or the row's K / V page (see tile_body)
-      const int64_t row_off = row_table[m];
+      int64_t row_off;
+      if constexpr (PAGE_WAVE) row_off = row_table[m];
+      else row_off = kv_row_offset(p.kv, m);
       float a_s = 1.f;
       if constexpr (!BLOCKSCALE) a_s = QUANT ? a_sc[16 + m] : p.a_scales[(int64_t)m * p.a_scale_stride];
 #pragma unroll
@@ -516,7 +524,7 @@ static int launch_skinny_r(const GemmArgs& p, int64_t batch, hipStream_t stream)
   const uint32_t per_wave = (uint32_t)ceil_div(ceil_div(p.K, 128), NWAVES);
   const int smem = Cfg::SMEM + NWAVES * (int)skinny_acts_bytes<ACTS, BLOCKSCALE>((uint32_t)p.M, per_wave) + (KV ? Cfg::ROW_TABLE : 0);
   const int64_t blocks = ceil_div(p.N, 16 * NTW);
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)batch), dim3((NWAVES + (KV ? 1 : 0)) * 64), smem, stream, static_cast<const std::conditional_t<KV, GemmArgs, MatmulArgs>&>(p));
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)batch), dim3((NWAVES + skinny_page_waves(MT, KV)) * 64), smem, stream, static_cast<const std::conditional_t<KV, GemmArgs, MatmulArgs>&>(p));
   return launch_status("gemm_skinny");
 }
 
