@@ -1,8 +1,6 @@
 """The matmul kernel for tens to a few hundred tokens (small tiles, K split over the block's waves): every tile shape forced on
 ragged sizes, exact where the arithmetic is; the shape the estimates choose against the oracle on both sides of every edge; and
 its fused QKV epilogue against the decode kernel's."""
-import os
-
 import numpy as np
 import pytest
 import torch
@@ -10,6 +8,7 @@ import torch
 import modular_amd as mx
 import oracle
 from modular_amd import _lib, synth
+from mid_cases import SHAPES as BUILT, exact_case
 from qkv_cases import make_cache_case, make_operands
 from util import assert_rel, f32_np, fp8_bytes
 
@@ -19,29 +18,6 @@ CFG = {"block": mx.blockwise_fp8_config(), "row": mx.rowwise_fp8_config()}
 SHAPES = [10 * mt + nt for mt in (2, 3, 4) for nt in (1, 2, 3, 4)]
 
 
-@pytest.fixture
-def forced():
-    def use(value):
-        os.environ["MAXFP8_MID"] = str(value)
-        _lib.tuning_reload()
-    yield use
-    os.environ.pop("MAXFP8_MID", None)
-    _lib.tuning_reload()
-
-
-def exact_case(M, N, K, kind, seed):
-    """small integers times powers of two: every sum is exact in any order"""
-    g = torch.Generator().manual_seed(seed)
-    a = torch.randint(-2, 3, (M, K), generator=g).float().to(torch.float8_e4m3fn)
-    b = torch.randint(-2, 3, (N, K), generator=g).float().to(torch.float8_e4m3fn)
-    if kind == "block":
-        sa = 2.0 ** torch.randint(-1, 2, (-(-K // 128), -(-M // 4) * 4), generator=g).float()
-        sb = 2.0 ** torch.randint(-1, 2, (-(-N // 128), -(-K // 128)), generator=g).float()
-    else:
-        sa, sb = 2.0 ** torch.randint(-1, 2, (1, M), generator=g).float(), 2.0 ** torch.randint(-1, 2, (N, 1), generator=g).float()
-    return a, b, sa, sb
-
-
 def run(a, b, sa, sb, kind, dev, out_type, algo="auto"):
     return mx.dynamic_scaled_matmul(a.to(dev), b.to(dev), sa.to(dev), sb.to(dev), CFG[kind].input_scale, CFG[kind].weight_scale,
                                     out_type=out_type, algo=algo)
@@ -49,9 +25,9 @@ def run(a, b, sa, sb, kind, dev, out_type, algo="auto"):
 
 @pytest.mark.parametrize("kind", ["block", "row"])
 @pytest.mark.parametrize("shape", SHAPES)
-def test_every_tile_shape_is_exact(dev, forced, kind, shape):
+def test_every_tile_shape_is_exact(dev, tune, kind, shape):
     mt, nt = divmod(shape, 10)
-    forced(shape)
+    tune(MAXFP8_MID=shape)
     # one slab (three waves idle), slabs that do not divide by four, a K tail, ragged last tiles of rows and columns, N not
     # a multiple of 8, more tiles than the eight XCDs divide evenly
     for i, (M, N, K) in enumerate([(16 * mt, 16 * nt, 128), (16 * mt + 1, 16 * nt * 9 + 8, 640), (5, 16 * nt * 3 - 3, 1040),
@@ -85,10 +61,10 @@ def test_chosen_shapes_against_the_oracle(dev, kind, M, N, K):
 
 
 @pytest.mark.parametrize("mnk", [(-1, -1, -1), (1, 1, -1), (1, 128, 128)])
-@pytest.mark.parametrize("shape", [21, 33, 44])
+@pytest.mark.parametrize("shape", BUILT)
 @pytest.mark.parametrize("bias", [False, True])
-def test_fused_qkv_epilogue_matches_the_decode_kernel(dev, forced, mnk, shape, bias):
-    """Q and both caches, bit for bit, on exactly representable data: sequences that start inside a page, pages scattered
+def test_fused_qkv_epilogue_matches_the_decode_kernel(dev, tune, mnk, shape, bias):
+    """Every built shape: Q and both caches, bit for bit, on exactly representable data: sequences that start inside a page, pages scattered
     over the pool, a row without a page."""
     lens, cached, page, heads, kv_heads, D = [3, 1, 20, 9], [5, 127, 0, 60], 16, 4, 2, 64
     T, K, q_dim = sum(lens), 768, heads * D
@@ -111,7 +87,7 @@ def test_fused_qkv_epilogue_matches_the_decode_kernel(dev, forced, mnk, shape, b
         torch.cuda.synchronize()
         return q, blocks
 
-    forced(shape)
+    tune(MAXFP8_MID=shape)
     q, blocks = once("auto")
     want_q, want_blocks = once("skinny")
     assert torch.equal(q, want_q) and torch.equal(blocks, want_blocks)

@@ -1,49 +1,23 @@
 """Every built shape of the kernel whose blocks split K among their waves, by its tile and its blocks per CU: exact where the arithmetic is, on
 ragged sizes, K tails, shares of K without a slab and grids of one, several and many blocks; and the heights and cuts the planner
 takes for matmuls of little more than half a round of tiles."""
-import os
-
 import pytest
 import torch
 
 import modular_amd as mx
 from modular_amd import _lib
+from mid_cases import SHAPES, describe_of, exact_case, exact_operands, exact_scales
 
 CFG = {"block": mx.blockwise_fp8_config(), "row": mx.rowwise_fp8_config()}
-# blocks per CU, 16-token groups, 16-column groups
-SHAPES = [411, 312, 321, 422, 222, 323, 123, 324, 124, 231, 132, 133, 234, 134, 141, 142, 143, 244]
-
-
-@pytest.fixture
-def forced():
-    def use(value):
-        os.environ["MAXFP8_MID"] = str(value)
-        _lib.tuning_reload()
-    yield use
-    os.environ.pop("MAXFP8_MID", None)
-    _lib.tuning_reload()
-
-
-def exact_case(M, N, K, kind, seed):
-    """small integers times powers of two: every sum is exact in any order"""
-    g = torch.Generator().manual_seed(seed)
-    a = torch.randint(-2, 3, (M, K), generator=g).float().to(torch.float8_e4m3fn)
-    b = torch.randint(-2, 3, (N, K), generator=g).float().to(torch.float8_e4m3fn)
-    if kind == "block":
-        sa = 2.0 ** torch.randint(-1, 2, (-(-K // 128), -(-M // 4) * 4), generator=g).float()
-        sb = 2.0 ** torch.randint(-1, 2, (-(-N // 128), -(-K // 128)), generator=g).float()
-    else:
-        sa, sb = 2.0 ** torch.randint(-1, 2, (1, M), generator=g).float(), 2.0 ** torch.randint(-1, 2, (N, 1), generator=g).float()
-    return a, b, sa, sb
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["block", "row"])
 @pytest.mark.parametrize("shape", SHAPES)
-def test_every_built_shape_is_exact(dev, forced, kind, shape):
+def test_every_built_shape_is_exact(dev, tune, kind, shape):
     blocks, mt, nt = shape // 100, shape // 10 % 10, shape % 10
-    forced(shape)
-    assert f"{blocks} per CU" in _lib.matmul_describe(20, 512, 512)
+    tune(MAXFP8_MID=shape)
+    assert all(part in _lib.matmul_describe(20, 512, 512) for part in describe_of(shape))
     waves = 8 if blocks == 1 else 4
     # one slab; a slab more than the waves; a K tail; the longest share of a wave; several rounds of blocks; more tokens than the
     # choice by estimates takes below the tiles
@@ -53,6 +27,33 @@ def test_every_built_shape_is_exact(dev, forced, kind, shape):
         on = [t.to(dev) for t in case]
         run = lambda algo: mx.dynamic_scaled_matmul(*on, CFG[kind].input_scale, CFG[kind].weight_scale, algo=algo)
         assert torch.equal(run("auto"), run("naive")), f"shape {shape}, {M} x {N} x {K}"
+
+
+@pytest.fixture(scope="module")
+def large(dev):
+    """64 MB of weights and a few tokens: what the kernel reads past the caches; and the naive kernel's results"""
+    M, N, K = 50, 262152, 256
+    a, b, g = exact_operands(M, N, K, 5, dev)
+    scales, want = {}, {}
+    for kind in CFG:
+        scales[kind] = exact_scales(M, N, K, kind, g, dev)
+        want[kind] = mx.dynamic_scaled_matmul(a, b, *scales[kind], CFG[kind].input_scale, CFG[kind].weight_scale, algo="naive")
+    return a, b, scales, want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["block", "row"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_weights_that_are_read_once_are_exact(large, tune, kind, shape):
+    """One row tile and 2^26 bytes of weights or more: the form with non-temporal loads.  The last column tile is ragged."""
+    a, b, scales, want = large
+    M = min(16 * (shape // 10 % 10) - 3, 50)
+    assert b.numel() >= 1 << 26
+    sa, sb = scales[kind]
+    sa = sa[:, :-(-M // 4) * 4] if kind == "block" else sa[:, :M]
+    tune(MAXFP8_MID=shape)
+    y = mx.dynamic_scaled_matmul(a[:M], b, sa.contiguous(), sb, CFG[kind].input_scale, CFG[kind].weight_scale)
+    assert torch.equal(y, want[kind][:M])
 
 
 def test_heights_and_cuts_of_little_more_than_half_a_round():
