@@ -63,7 +63,7 @@ int gemm_skinny_max_m();
 int compute_units();
 bool gemm_short_k_ok(const GemmArgs&, bool, int64_t);
 int gemm_short_k_dispatch(const GemmArgs&, int64_t, hipStream_t);
-int gemm_mid_dispatch(const GemmArgs&, bool, hipStream_t);
+int gemm_mid_dispatch(const GemmArgs&, bool, int, hipStream_t);
 bool gemm_mid_ok(int64_t M, int64_t N, int64_t K);
 int gemm_mid_shape(int64_t M, int64_t N, int64_t K, bool blockscale, float* us);
 int gemm_mid_forced_shape();
@@ -207,6 +207,37 @@ void maxfp8_tuning_reload(void) { tuning_reload(); }
 namespace maxfp8 {
 // The kernel for tens to a few hundred tokens (gemm_mid.hip), beside the ABI's algo values.
 constexpr int kAlgoMid = 100;
+// A kernel, and which of its shapes where it is that one.
+struct Choice { int algo, shape; };
+static Choice mid_choice(int64_t M, int64_t N, int64_t K, bool block) {
+  float us;
+  return {kAlgoMid, tuning().mid > 0 ? gemm_mid_forced_shape() : gemm_mid_shape(M, N, K, block, &us)};
+}
+
+// What is chosen: for a matmul whose caller brings all the workspace it is asked for, or none for the sums of a K split; for a fused QKV
+// matmul with and without that workspace.
+enum class Asked : int { kMatmul, kMatmulNoSplit, kQkv, kQkvWorkspace };
+static Choice choose_uncached(Asked what, int64_t M, int64_t N, int64_t K, bool block);
+
+// The choice is asked for several times on every call and walks all shapes of the small tiles (1 to 3 us of host time, as much as a
+// launch): the answers are kept, keyed by all that they depend on, the generation of the tuning switches included.
+static Choice choose(Asked what, int64_t M, int64_t N, int64_t K, bool block) {
+  struct Entry { int64_t M, N, K; unsigned generation; Asked what; bool block; Choice choice; };
+  static Entry table[256];  // (algo 0: empty)
+  static std::mutex mu;
+  const unsigned generation = tuning().generation;
+  const uint64_t h = ((uint64_t)M * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)N * 0xc2b2ae3d27d4eb4full) ^ ((uint64_t)K * 0x165667b19e3779f9ull) ^
+                     ((uint64_t)(2 * (int)what + (block ? 1 : 0)) * 0xd6e8feb86659fd93ull);
+  Entry& e = table[(h >> 32) % 256];
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (e.choice.algo && e.M == M && e.N == N && e.K == K && e.what == what && e.block == block && e.generation == generation) return e.choice;
+  }
+  const Choice choice = choose_uncached(what, M, N, K, block);
+  std::lock_guard<std::mutex> lock(mu);
+  e = Entry{M, N, K, generation, what, block, choice};
+  return choice;
+}
 
 // Which kernel MAXFP8_ALGO_AUTO gives a fast-layout matmul whose caller brings all the workspace it is asked for.  At most
 // 16 rows: the decode kernel.  Up to 64: streaming the weights or the tiles, by the decode kernel's own rule; the tiles also where they are estimated 8 per
@@ -219,7 +250,7 @@ static bool named_mid(int64_t M, int64_t N, int64_t K, bool block) {
   if (K > 12288) return false;
   return M <= 32 ? K > 1024 && ceil_div(ceil_div(N, 16), (int64_t)compute_units()) == 3 : K > (block ? 512 : 896);
 }
-static int choose_uncached(int64_t M, int64_t N, int64_t K, bool block) {
+static int choose_matmul(int64_t M, int64_t N, int64_t K, bool block) {
   const Tuning& t = tuning();
   const int plain = gemm_skinny_preferred(M, N, K) ? MAXFP8_ALGO_SKINNY : MAXFP8_ALGO_TILED;
   if (t.mid > 0) return gemm_mid_ok(M, N, K) ? kAlgoMid : plain;
@@ -245,33 +276,19 @@ static int choose_uncached(int64_t M, int64_t N, int64_t K, bool block) {
   const bool on_tiles = tiles < 0.92f * gemm_skinny_cost(M, N, K, block) && (split || (!splits && unsplit));
   return on_tiles && (M <= 32 || !splits || tiles < 1.15f * mid) ? MAXFP8_ALGO_TILED : stream;
 }
-// (asked on every call: the answers are kept, keyed by the shape, the scaling and the generation of the tuning switches)
-static int choose_kernel(int64_t M, int64_t N, int64_t K, bool block) {
-  if (M <= 16) return tuning().mid > 0 ? choose_uncached(M, N, K, block) : MAXFP8_ALGO_SKINNY;
-  if (M > 2048) return MAXFP8_ALGO_TILED;
-  struct Entry { int64_t M, N, K; unsigned generation; int algo; bool block; };
-  static Entry table[128];  // (algo 0: empty)
-  static std::mutex mu;
-  const unsigned generation = tuning().generation;
-  const uint64_t h = ((uint64_t)M * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)N * 0xc2b2ae3d27d4eb4full) ^ ((uint64_t)K * 0x165667b19e3779f9ull) ^ (block ? 1ull << 32 : 0);
-  Entry& e = table[(h >> 32) % 128];
-  {
-    std::lock_guard<std::mutex> lock(mu);
-    if (e.algo && e.M == M && e.N == N && e.K == K && e.block == block && e.generation == generation) return e.algo;
-  }
-  const int algo = choose_uncached(M, N, K, block);
-  std::lock_guard<std::mutex> lock(mu);
-  e = Entry{M, N, K, generation, algo, block};
-  return algo;
+static Choice choose_kernel(int64_t M, int64_t N, int64_t K, bool block) {
+  if (M <= 16 && tuning().mid <= 0) return {MAXFP8_ALGO_SKINNY, 0};
+  if (M > 2048) return {MAXFP8_ALGO_TILED, 0};
+  return choose(Asked::kMatmul, M, N, K, block);
 }
 // the workspace MAXFP8_ALGO_AUTO uses with this scaling
 static size_t auto_workspace(int64_t M, int64_t N, int64_t K, bool block) {
-  return choose_kernel(M, N, K, block) == MAXFP8_ALGO_TILED ? gemm_tiled_workspace_bytes(M, N, K) : 0;
+  return choose_kernel(M, N, K, block).algo == MAXFP8_ALGO_TILED ? gemm_tiled_workspace_bytes(M, N, K) : 0;
 }
 
 // The same for the fused QKV matmul: decode kernel (at most 16 rows), the kernel in between (17 to 64, beyond by its estimate) or the tiles, whose
 // plan may cut them along K where the caller brings a workspace.
-static int choose_qkv(int64_t T, int64_t N, int64_t K, bool has_workspace, bool block) {
+static int choose_qkv_matmul(int64_t T, int64_t N, int64_t K, bool has_workspace, bool block) {
   const Tuning& t = tuning();
   const int plain = T <= gemm_skinny_max_m() ? MAXFP8_ALGO_SKINNY : MAXFP8_ALGO_TILED;
   if (t.mid > 0) return gemm_mid_ok(T, N, K) ? kAlgoMid : plain;
@@ -280,6 +297,23 @@ static int choose_qkv(int64_t T, int64_t N, int64_t K, bool has_workspace, bool 
   float mid;
   gemm_mid_shape(T, N, K, block, &mid);
   return mid < 0.85f * gemm_tiled_qkv_cost(T, N, K, block, has_workspace) ? kAlgoMid : MAXFP8_ALGO_TILED;
+}
+static Choice choose_qkv(int64_t T, int64_t N, int64_t K, bool has_workspace, bool block) {
+  if (T <= 16 && tuning().mid <= 0) return {MAXFP8_ALGO_SKINNY, 0};
+  if (T > 2048) return {MAXFP8_ALGO_TILED, 0};
+  return choose(has_workspace ? Asked::kQkvWorkspace : Asked::kQkv, T, N, K, block);
+}
+
+// 17 to 64 rows whose tiles would split K, without the workspace for it
+static int without_workspace(int64_t M, int64_t N, int64_t K, bool block) {
+  return gemm_mid_before_skinny(M, N, K) && named_mid(M, N, K, block) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
+}
+static Choice choose_uncached(Asked what, int64_t M, int64_t N, int64_t K, bool block) {
+  const int algo = what == Asked::kMatmul          ? choose_matmul(M, N, K, block)
+                   : what == Asked::kMatmulNoSplit ? without_workspace(M, N, K, block)
+                                                   : choose_qkv_matmul(M, N, K, what == Asked::kQkvWorkspace, block);
+  const bool streamed = (what == Asked::kMatmul || what == Asked::kMatmulNoSplit) && algo == MAXFP8_ALGO_SKINNY && gemm_mid_before_skinny(M, N, K);
+  return algo == kAlgoMid || streamed ? Choice{algo, mid_choice(M, N, K, block).shape} : Choice{algo, 0};
 }
 }  // namespace maxfp8
 
@@ -490,11 +524,6 @@ size_t maxfp8_matmul_auto_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 namespace maxfp8 {
 struct BatchStrides { int64_t n, a, b, c, a_scales, b_scales; };  // n batches; steps in elements
 
-// 17 to 64 rows whose tiles would split K, without the workspace for it
-static int without_workspace(int64_t M, int64_t N, int64_t K, bool block) {
-  return gemm_mid_before_skinny(M, N, K) && named_mid(M, N, K, block) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
-}
-
 // A batch of short K and more than 32 rows on the tiles: one slab of K leaves three of the decode kernel's four waves idle, and
 // beyond one of its 16-row blocks per CU every block more reads the tokens again.  With one block per CU or less it is ahead from
 // two slabs on (decode kernel against tiles, 48 rows, us, cold: 32 x 512 -> 128 5.4 and 6.4, 48 of them 7.8 and 6.5, 128 12.7
@@ -539,17 +568,21 @@ static int matmul_common(void* c, const void* a, const void* b, const void* a_sc
                            K > 0 && (!block || (gm == 1 && gn == 128 && gk == 128)) &&
                            (bt.n == 1 || (bt.a % 16 == 0 && bt.b % 16 == 0)) && offsets_fit(K, lda, ldb, a_scales_ld, block);
   const bool automatic = algo == MAXFP8_ALGO_AUTO;
+  int shape = 0;  // of the small tiles
   if (automatic) {
     if (!fast_layout) algo = MAXFP8_ALGO_NAIVE;
-    else if (bt.n == 1) algo = choose_kernel(M, N, K, block);
+    else if (bt.n == 1) { const Choice c = choose_kernel(M, N, K, block); algo = c.algo; shape = c.shape; }
     else if (gemm_skinny_preferred(M, N, K) && !batch_on_tiles(bt.n, M, N, K)) algo = MAXFP8_ALGO_SKINNY;
     else algo = MAXFP8_ALGO_TILED;
     // 33 to 64 rows: the tiles win through their K split.  Without the workspace the split needs, a narrow weight
     // matrix would run on a fraction of the chip: the streaming kernel then.  (What this shape's own plan needs, not the
     // worst case over all tile shapes: a plan that does not split runs the same with and without a workspace.)
     if (algo == MAXFP8_ALGO_TILED && M <= gemm_skinny_max_m() && bt.n == 1 &&
-        gemm_tiled_plan_workspace_bytes(M, N, K, block) > (workspace ? workspace_bytes : 0))
-      algo = without_workspace(M, N, K, block);
+        gemm_tiled_plan_workspace_bytes(M, N, K, block) > (workspace ? workspace_bytes : 0)) {
+      const Choice c = choose(Asked::kMatmulNoSplit, M, N, K, block);
+      algo = c.algo;
+      shape = c.shape;
+    }
   }
   if (algo == MAXFP8_ALGO_NAIVE) {
     if (block)
@@ -589,7 +622,7 @@ static int matmul_common(void* c, const void* a, const void* b, const void* a_sc
   }
   p.a_batch = bt.a; p.b_batch = bt.b; p.c_batch = bt.c;
   p.a_scales_batch = bt.a_scales; p.b_scales_batch = bt.b_scales;
-  if (algo == kAlgoMid || (automatic && algo == MAXFP8_ALGO_SKINNY && bt.n == 1 && gemm_mid_before_skinny(M, N, K))) return gemm_mid_dispatch(p, block, st);
+  if (shape) return gemm_mid_dispatch(p, block, shape, st);
   if (automatic && gemm_short_k_ok(p, block, bt.n)) return gemm_short_k_dispatch(p, bt.n, st);
   if (algo == MAXFP8_ALGO_SKINNY) return gemm_skinny_dispatch(p, block, bt.n, st);
   if (workspace && !is_aligned(workspace, 16)) MAXFP8_FAIL(MAXFP8_ERR_ALIGN, "matmul: workspace must be 16-byte aligned");
@@ -603,13 +636,12 @@ extern "C" {
 int maxfp8_matmul_describe(int64_t M, int64_t N, int64_t K, int block_scaling, int with_workspace, char* buf, size_t len) {
   if (!buf || len == 0) return 0;
   if (M <= 0 || N <= 0 || K <= 0) return snprintf(buf, len, "nothing to do");
-  int algo = choose_kernel(M, N, K, block_scaling != 0);
-  if (algo == MAXFP8_ALGO_TILED && M <= gemm_skinny_max_m() && !with_workspace && gemm_tiled_plan_workspace_bytes(M, N, K, block_scaling != 0) > 0)
-    algo = without_workspace(M, N, K, block_scaling != 0);
-  if (algo == MAXFP8_ALGO_SKINNY) return snprintf(buf, len, "skinny");
-  if (algo == kAlgoMid) {
-    float us;
-    const int sel = tuning().mid > 0 ? gemm_mid_forced_shape() : gemm_mid_shape(M, N, K, block_scaling != 0, &us);
+  Choice c = choose_kernel(M, N, K, block_scaling != 0);
+  if (c.algo == MAXFP8_ALGO_TILED && M <= gemm_skinny_max_m() && !with_workspace && gemm_tiled_plan_workspace_bytes(M, N, K, block_scaling != 0) > 0)
+    c = choose(Asked::kMatmulNoSplit, M, N, K, block_scaling != 0);
+  if (c.algo == MAXFP8_ALGO_SKINNY) return snprintf(buf, len, "skinny");
+  if (c.algo == kAlgoMid) {
+    const int sel = c.shape;
     const int bm = 16 * (sel / 10 % 10), bn = 16 * (sel % 10);
     return snprintf(buf, len, "%dx%d x%lld, %d per CU, K split over the block's waves", bm, bn, (long long)(ceil_div(M, bm) * ceil_div(N, bn)), sel / 100);
   }
@@ -662,19 +694,20 @@ int maxfp8_matmul_dynamic_scaled_fp8_noalloc(void* c, const void* a, const void*
 }  // extern "C"
 namespace maxfp8 {
 struct LinearLayout { size_t scales, partial, partial_bytes, total; int64_t scales_ld; };
-static LinearLayout linear_layout(int64_t M, int64_t N, int64_t K, bool block, bool fixed) {
+// (plain: the matmul behind it is the plain one, whose workspace comes last)
+static LinearLayout linear_layout(int64_t M, int64_t N, int64_t K, bool block, bool fixed, bool plain = true) {
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
   LinearLayout l;
   l.scales_ld = block ? ceil_div(M, 4) * 4 : M;
   l.scales = up((size_t)M * (size_t)K);
   l.partial = l.scales + up((fixed ? 2 : block ? (size_t)(K / 128) * l.scales_ld : (size_t)M) * 4);
-  l.partial_bytes = M > 0 && N > 0 && K > 0 ? auto_workspace(M, N, K, block) : 0;
+  l.partial_bytes = plain && M > 0 && N > 0 && K > 0 ? auto_workspace(M, N, K, block) : 0;
   l.total = l.partial + l.partial_bytes;
   return l;
 }
 // does the decode kernel quantise by itself? (the layout as far as it is the operands': see linear_common)
 static bool linear_in_one(int64_t M, int64_t N, int64_t K, bool block) {
-  return M > 0 && N > 0 && K > 0 && choose_kernel(M, N, K, block) == MAXFP8_ALGO_SKINNY && gemm_skinny_quant_ok(M, N, K, block);
+  return M > 0 && N > 0 && K > 0 && choose_kernel(M, N, K, block).algo == MAXFP8_ALGO_SKINNY && gemm_skinny_quant_ok(M, N, K, block);
 }
 
 static int linear_common(void* y, const void* x, const void* w, const void* w_scales, int64_t M, int64_t N, int64_t K, int64_t ldx,
@@ -772,7 +805,7 @@ int maxfp8_batched_matmul_dynamic_scaled_fp8(void* c, const void* a, const void*
 }  // extern "C"
 
 // x != nullptr: the decode kernel quantises x (bf16 rows of ldx elements) by itself; input and input_scale are not used.
-// with_workspace: the caller brings qkv_partial_bytes bytes (which may be none).
+// chosen: what the caller has found for MAXFP8_ALGO_AUTO, with the workspace that takes; nullptr: it is chosen here, without any.
 static int qkv_common(void* output, const void* input, const void* x, int64_t ldx, float scale_ub, const uint32_t* input_row_offsets,
                                                const void* wqkv, const void* input_scale, const void* weight_scale,
                                                void* kv_blocks, const uint32_t* cache_lengths, const uint32_t* lookup_table,
@@ -780,7 +813,7 @@ static int qkv_common(void* output, const void* input, const void* x, int64_t ld
                                                int64_t batch_size, int64_t num_blocks, int64_t kv_dim, int64_t num_layers,
                                                int64_t layer_idx, int64_t page_size, int64_t num_kv_heads, int64_t head_dim,
                                                int64_t lut_ld, int64_t gm, int64_t gn, int64_t gk, int64_t input_scale_ld,
-                                               int64_t weight_scale_ld, int scales_dtype, int algo, bool with_workspace, void* workspace,
+                                               int64_t weight_scale_ld, int scales_dtype, int algo, const Choice* chosen, void* workspace,
                                                size_t workspace_bytes, void* stream) {
   if (T < 0 || N < 0 || K < 0 || q_dim < 0 || batch_size < 0) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused qkv matmul: negative size");
   if (batch_size == 0 || T == 0 || N == 0) return MAXFP8_OK;  // kv_cache_ragged.mojo:1193-1194
@@ -858,8 +891,9 @@ static int qkv_common(void* output, const void* input, const void* x, int64_t ld
     return gemm_skinny_quant_dispatch(p, block, st);
   }
   const bool automatic = algo == MAXFP8_ALGO_AUTO;
-  if (automatic) algo = choose_qkv(T, N, K, with_workspace, block);
-  if (automatic && algo == kAlgoMid) return gemm_mid_dispatch(p, block, st);
+  const Choice choice = !automatic ? Choice{algo, 0} : chosen ? *chosen : choose_qkv(T, N, K, false, block);
+  if (automatic) algo = choice.algo;
+  if (automatic && algo == kAlgoMid) return gemm_mid_dispatch(p, block, choice.shape, st);
   if (algo == MAXFP8_ALGO_SKINNY) return gemm_skinny_dispatch(p, block, 1, st);
   if (algo != MAXFP8_ALGO_TILED) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused qkv matmul: algo %d is not available", algo);
   p.workspace = (float*)workspace;
@@ -878,19 +912,21 @@ int maxfp8_fused_qkv_matmul_ragged_paged_scale(void* output, const void* input, 
                                                int64_t weight_scale_ld, int scales_dtype, int algo, void* stream) {
   return qkv_common(output, input, nullptr, 0, 0.f, input_row_offsets, wqkv, input_scale, weight_scale, kv_blocks, cache_lengths, lookup_table,
                     bias, T, N, K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads, head_dim, lut_ld, gm,
-                    gn, gk, input_scale_ld, weight_scale_ld, scales_dtype, algo, false, nullptr, 0, stream);
+                    gn, gk, input_scale_ld, weight_scale_ld, scales_dtype, algo, nullptr, nullptr, 0, stream);
 }
 
-static bool qkv_in_one(int64_t T, int64_t N, int64_t K, bool block) {
-  return T > 0 && N > 0 && K > 0 && choose_qkv(T, N, K, true, block) == MAXFP8_ALGO_SKINNY && gemm_skinny_quant_ok(T, N, K, block);
+// does the decode kernel quantise by itself?
+static bool qkv_in_one(const Choice& choice, int64_t T, int64_t N, int64_t K, bool block) {
+  return choice.algo == MAXFP8_ALGO_SKINNY && gemm_skinny_quant_ok(T, N, K, block);
 }
 // what follows the quantised activations and their scales: the sums of cut tiles
-static size_t qkv_partial_bytes(int64_t T, int64_t N, int64_t K, bool block) {
-  return choose_qkv(T, N, K, true, block) == MAXFP8_ALGO_TILED ? gemm_tiled_qkv_workspace_bytes(T, N, K, block) : 0;
+static size_t qkv_partial_bytes(const Choice& choice, int64_t T, int64_t N, int64_t K, bool block) {
+  return choice.algo == MAXFP8_ALGO_TILED ? gemm_tiled_qkv_workspace_bytes(T, N, K, block) : 0;
 }
 
 size_t maxfp8_fused_qkv_matmul_workspace_bytes(int64_t T, int64_t N, int64_t K, int block_scaling) {
-  return T > 0 && N > 0 && K > 0 ? qkv_partial_bytes(T, N, K, block_scaling != 0) : 0;
+  const bool block = block_scaling != 0;
+  return T > 0 && N > 0 && K > 0 ? qkv_partial_bytes(choose_qkv(T, N, K, true, block), T, N, K, block) : 0;
 }
 
 int maxfp8_fused_qkv_matmul_ragged_paged_scale_workspace(
@@ -900,19 +936,25 @@ int maxfp8_fused_qkv_matmul_ragged_paged_scale_workspace(
     int64_t num_kv_heads, int64_t head_dim, int64_t lut_ld, int64_t gm, int64_t gn, int64_t gk, int64_t input_scale_ld,
     int64_t weight_scale_ld, int scales_dtype, void* workspace, size_t workspace_bytes, void* stream) {
   const bool block = !(gk == -1 && gm == gn && (gm == -1 || gm == 1));
-  const size_t need = maxfp8_fused_qkv_matmul_workspace_bytes(T, N, K, block);
+  Choice choice = {MAXFP8_ALGO_AUTO, 0};
+  size_t need = 0;
+  if (T > 0 && N > 0 && K > 0) {
+    choice = choose_qkv(T, N, K, true, block);
+    need = qkv_partial_bytes(choice, T, N, K, block);
+  }
   if (need > 0 && (!workspace || workspace_bytes < need))
     MAXFP8_FAIL(MAXFP8_ERR_WORKSPACE, "fused qkv matmul: needs %zu bytes of workspace, got %zu", need, workspace ? workspace_bytes : (size_t)0);
   if (need > 0 && !is_aligned(workspace, 16)) MAXFP8_FAIL(MAXFP8_ERR_ALIGN, "fused qkv matmul: workspace must be 16-byte aligned");
   return qkv_common(output, input, nullptr, 0, 0.f, input_row_offsets, wqkv, input_scale, weight_scale, kv_blocks, cache_lengths, lookup_table,
                     bias, T, N, K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads, head_dim, lut_ld, gm,
-                    gn, gk, input_scale_ld, weight_scale_ld, scales_dtype, MAXFP8_ALGO_AUTO, true, need ? workspace : nullptr, need, stream);
+                    gn, gk, input_scale_ld, weight_scale_ld, scales_dtype, MAXFP8_ALGO_AUTO, &choice, need ? workspace : nullptr, need, stream);
 }
 
 size_t maxfp8_linear_qkv_workspace_bytes(int64_t T, int64_t N, int64_t K, int weight_granularity) {
   if (T <= 0 || N <= 0 || K <= 0) return 0;
   const bool block = weight_granularity == MAXFP8_GRAN_BLOCK;
-  return qkv_in_one(T, N, K, block) ? 0 : linear_layout(T, N, K, block, false).partial + qkv_partial_bytes(T, N, K, block);
+  const Choice choice = choose_qkv(T, N, K, true, block);
+  return qkv_in_one(choice, T, N, K, block) ? 0 : linear_layout(T, N, K, block, false, false).partial + qkv_partial_bytes(choice, T, N, K, block);
 }
 
 int maxfp8_linear_qkv_ragged_paged_scale(void* output, const void* x, int64_t x_row_stride, const uint32_t* input_row_offsets,
@@ -929,12 +971,13 @@ int maxfp8_linear_qkv_ragged_paged_scale(void* output, const void* x, int64_t x_
   if (batch_size == 0 || T == 0 || N == 0) return MAXFP8_OK;
   if (!x) MAXFP8_FAIL(MAXFP8_ERR_NULL, "qkv linear: null pointer");
   if (x_row_stride < K || K <= 0 || K % (block ? 128 : 16) != 0) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "qkv linear: K = %lld does not suit the scaling", (long long)K);
-  if (qkv_in_one(T, N, K, block) && is_aligned(x, 16) && x_row_stride % 8 == 0 && 32 * x_row_stride < ((int64_t)1 << 31))
+  const Choice choice = choose_qkv(T, N, K, true, block);
+  if (qkv_in_one(choice, T, N, K, block) && is_aligned(x, 16) && x_row_stride % 8 == 0 && 32 * x_row_stride < ((int64_t)1 << 31))
     return qkv_common(output, nullptr, x, x_row_stride, scale_ub, input_row_offsets, wqkv, nullptr, weight_scale, kv_blocks, cache_lengths,
                       lookup_table, bias, T, N, K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads,
-                      head_dim, lut_ld, gm, gn, gk, 0, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_SKINNY, false, nullptr, 0, stream);
-  const LinearLayout l = linear_layout(T, N, K, block, false);
-  const size_t partial = qkv_partial_bytes(T, N, K, block), total = l.partial + partial;
+                      head_dim, lut_ld, gm, gn, gk, 0, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_SKINNY, nullptr, nullptr, 0, stream);
+  const LinearLayout l = linear_layout(T, N, K, block, false, false);
+  const size_t partial = qkv_partial_bytes(choice, T, N, K, block), total = l.partial + partial;
   if (!workspace || workspace_bytes < total)
     MAXFP8_FAIL(MAXFP8_ERR_WORKSPACE, "qkv linear: needs %zu bytes of workspace, got %zu", total, workspace ? workspace_bytes : (size_t)0);
   if (!is_aligned(workspace, 16)) MAXFP8_FAIL(MAXFP8_ERR_ALIGN, "qkv linear: workspace must be 16-byte aligned");
@@ -945,7 +988,7 @@ int maxfp8_linear_qkv_ragged_paged_scale(void* output, const void* x, int64_t x_
   if (rc != MAXFP8_OK) return rc;
   return qkv_common(output, q, nullptr, 0, 0.f, input_row_offsets, wqkv, scales, weight_scale, kv_blocks, cache_lengths, lookup_table, bias, T, N,
                     K, q_dim, batch_size, num_blocks, kv_dim, num_layers, layer_idx, page_size, num_kv_heads, head_dim, lut_ld, gm, gn, gk,
-                    block ? l.scales_ld : T, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_AUTO, true, partial ? q + l.partial : nullptr, partial, stream);
+                    block ? l.scales_ld : T, weight_scale_ld, MAXFP8_F32, MAXFP8_ALGO_AUTO, &choice, partial ? q + l.partial : nullptr, partial, stream);
 }
 
 }  // extern "C"

@@ -404,9 +404,8 @@ int gemm_mid_forced_shape() {
   return sel;
 }
 
-int gemm_mid_dispatch(const GemmArgs& p, bool blockscale, hipStream_t stream) {
-  float us = 0.f;
-  const int sel = tuning().mid > 0 ? gemm_mid_forced_shape() : gemm_mid_shape(p.M, p.N, p.K, blockscale, &us);
+// sel: the shape, as gemm_mid_shape names it
+int gemm_mid_dispatch(const GemmArgs& p, bool blockscale, int sel, hipStream_t stream) {
   if (p.kv_on) return blockscale ? pick_mid<true, true>(p, sel, stream) : pick_mid<false, true>(p, sel, stream);
   return blockscale ? pick_mid<true, false>(p, sel, stream) : pick_mid<false, false>(p, sel, stream);
 }
