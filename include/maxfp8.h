@@ -263,8 +263,7 @@ int maxfp8_batched_matmul_dynamic_scaled_fp8(
 /*
  * Diagnostic: which launches MAXFP8_ALGO_AUTO makes for a fast-layout M x N x K matmul, as text
  * ("256x256 x768 + columns from 24576: 256x128 x256", "256x128 x112, K split 4", "64x48 x86, 1 per CU, K split over the block's waves"
- * -- the small tiles of gemm_mid_kernel, blocks per CU --, "skinny" -- streaming the weights as MAXFP8_ALGO_SKINNY does: the decode kernel, beyond
- * 16 rows the small tiles).
+ * -- the small tiles of gemm_mid_kernel, blocks per CU --, "skinny" -- the decode kernel, as MAXFP8_ALGO_SKINNY).
  * Returns the length snprintf would have written.  No counterpart in the reference.
  */
 int maxfp8_matmul_describe(int64_t M, int64_t N, int64_t K, int block_scaling, int with_workspace,

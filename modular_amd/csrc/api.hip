@@ -240,16 +240,9 @@ static Choice choose(Asked what, int64_t M, int64_t N, int64_t K, bool block) {
 }
 
 // Which kernel MAXFP8_ALGO_AUTO gives a fast-layout matmul whose caller brings all the workspace it is asked for.  At most
-// 16 rows: the decode kernel.  Up to 64: streaming the weights or the tiles, by the decode kernel's own rule; the tiles also where they are estimated 8 per
-// cent quicker than it (the estimates' own error), streaming also where the tiles' rule gave way to a quicker estimate of gemm_mid.hip's kernel;
-// up to 2048: that kernel or the tiles, by the estimates.  Forced shapes keep the other kernels out.
-//
-// Streaming has two names, kAlgoMid and MAXFP8_ALGO_SKINNY, and beyond 16 rows one launch (gemm_mid_before_skinny): which name a shape has
-// is what maxfp8_matmul_describe has always called it.
-static bool named_mid(int64_t M, int64_t N, int64_t K, bool block) {
-  if (K > 12288) return false;
-  return M <= 32 ? K > 1024 && ceil_div(ceil_div(N, 16), (int64_t)compute_units()) == 3 : K > (block ? 512 : 896);
-}
+// 16 rows: the decode kernel.  Up to 64: the small tiles or the tiles, by the decode kernel's own rule; the tiles also where they are estimated 8 per
+// cent quicker than it (the estimates' own error), the small tiles also where the tiles' rule gave way to their quicker estimate;
+// up to 2048: either of them, by the estimates.  Forced shapes keep the other kernels out.
 static int choose_matmul(int64_t M, int64_t N, int64_t K, bool block) {
   const Tuning& t = tuning();
   const int plain = gemm_skinny_preferred(M, N, K) ? MAXFP8_ALGO_SKINNY : MAXFP8_ALGO_TILED;
@@ -261,11 +254,10 @@ static int choose_matmul(int64_t M, int64_t N, int64_t K, bool block) {
   // x 592 x 5248 19 against 22 us, 79 x 7168 x 16384 35 against 38, 940 x 8320 x 1408 24 against 29)
   const float margin = M > 1024 ? 0.80f : gemm_tiled_plan_workspace_bytes(M, N, K, block) == 0 ? 0.85f : N * K >= ((int64_t)1 << 26) ? 0.90f : 0.97f;
   if (M > gemm_skinny_max_m()) return mid < margin * gemm_tiled_cost(M, N, K, block) ? kAlgoMid : MAXFP8_ALGO_TILED;
-  const int stream = named_mid(M, N, K, block) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
   const float tiles = gemm_tiled_cost(M, N, K, block);
   const bool splits = gemm_tiled_plan_workspace_bytes(M, N, K, true) > 0;
   // (the estimate of unsplit tiles is the roughest)
-  if (plain == MAXFP8_ALGO_TILED) return mid < (splits ? 0.85f : 0.75f) * tiles ? stream : MAXFP8_ALGO_TILED;
+  if (plain == MAXFP8_ALGO_TILED) return mid < (splits ? 0.85f : 0.75f) * tiles ? kAlgoMid : MAXFP8_ALGO_TILED;
   // (unsplit tiles in the decode kernel's range only for the shortest K, where four waves have no K to split: 48 x 32768 x 512 with
   // block scales 17.2 against 7.8 us; with row scales, which cost the decode kernel less, from its seventh block per CU on: 48 x
   // 32768 x 512 14.8 against 10.1, but 57 x 20080 x 512 10.6 against 12.9, 62 x 8400 x 512 8.1 against 12.4, 24 x 32768 x 512 1.10)
@@ -274,7 +266,7 @@ static int choose_matmul(int64_t M, int64_t N, int64_t K, bool block) {
   // per cent high on narrow weights with long K)
   const bool split = splits && (M > 32 || ceil_div(N, 16) > 3 * (int64_t)compute_units());
   const bool on_tiles = tiles < 0.92f * gemm_skinny_cost(M, N, K, block) && (split || (!splits && unsplit));
-  return on_tiles && (M <= 32 || !splits || tiles < 1.15f * mid) ? MAXFP8_ALGO_TILED : stream;
+  return on_tiles && (M <= 32 || !splits || tiles < 1.15f * mid) ? MAXFP8_ALGO_TILED : kAlgoMid;
 }
 static Choice choose_kernel(int64_t M, int64_t N, int64_t K, bool block) {
   if (M <= 16 && tuning().mid <= 0) return {MAXFP8_ALGO_SKINNY, 0};
@@ -305,15 +297,14 @@ static Choice choose_qkv(int64_t T, int64_t N, int64_t K, bool has_workspace, bo
 }
 
 // 17 to 64 rows whose tiles would split K, without the workspace for it
-static int without_workspace(int64_t M, int64_t N, int64_t K, bool block) {
-  return gemm_mid_before_skinny(M, N, K) && named_mid(M, N, K, block) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
+static int without_workspace(int64_t M, int64_t N, int64_t K) {
+  return gemm_mid_before_skinny(M, N, K) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
 }
 static Choice choose_uncached(Asked what, int64_t M, int64_t N, int64_t K, bool block) {
   const int algo = what == Asked::kMatmul          ? choose_matmul(M, N, K, block)
-                   : what == Asked::kMatmulNoSplit ? without_workspace(M, N, K, block)
+                   : what == Asked::kMatmulNoSplit ? without_workspace(M, N, K)
                                                    : choose_qkv_matmul(M, N, K, what == Asked::kQkvWorkspace, block);
-  const bool streamed = (what == Asked::kMatmul || what == Asked::kMatmulNoSplit) && algo == MAXFP8_ALGO_SKINNY && gemm_mid_before_skinny(M, N, K);
-  return algo == kAlgoMid || streamed ? Choice{algo, mid_choice(M, N, K, block).shape} : Choice{algo, 0};
+  return algo == kAlgoMid ? mid_choice(M, N, K, block) : Choice{algo, 0};
 }
 }  // namespace maxfp8
 
@@ -622,7 +613,7 @@ static int matmul_common(void* c, const void* a, const void* b, const void* a_sc
   }
   p.a_batch = bt.a; p.b_batch = bt.b; p.c_batch = bt.c;
   p.a_scales_batch = bt.a_scales; p.b_scales_batch = bt.b_scales;
-  if (shape) return gemm_mid_dispatch(p, block, shape, st);
+  if (algo == kAlgoMid) return gemm_mid_dispatch(p, block, shape, st);
   if (automatic && gemm_short_k_ok(p, block, bt.n)) return gemm_short_k_dispatch(p, bt.n, st);
   if (algo == MAXFP8_ALGO_SKINNY) return gemm_skinny_dispatch(p, block, bt.n, st);
   if (workspace && !is_aligned(workspace, 16)) MAXFP8_FAIL(MAXFP8_ERR_ALIGN, "matmul: workspace must be 16-byte aligned");

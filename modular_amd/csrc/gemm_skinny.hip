@@ -717,8 +717,9 @@ int gemm_skinny_read_probe(const void* b, int64_t M, int64_t N, int64_t K, int64
 
 int gemm_skinny_max_m() { return 64; }
 
-// What MAXFP8_ALGO_AUTO gives the weight-streaming kernel: every matmul of at most 32 rows (but see below), and those
-// of 33 to 64 rows whose weights take less than 32 MB.  With four 16-token groups per weight fragment every block re-reads 64 rows of
+// Where streaming the weights is preferred to the tiles by size alone: every matmul of at most 32 rows (but see below), and those
+// of 33 to 64 rows whose weights take less than 32 MB.  (Batches, and what the small tiles of gemm_mid.hip do not take, go by it; the choice
+// between those, the tiles and this kernel is made in api.hip.)  With four 16-token groups per weight fragment every block re-reads 64 rows of
 // activations through its L1 (about 8 TB/s over the chip) and its time grows with M, while the three-stage 128 x 128
 // tiles share the activations through LDS, split K over the chip when their column tiles are few, and take the same
 // time from 1 to 128 rows: at M = 64 they measured 54 us against 75 (N = 8192, K = 28672), 19 against 36 (2304 x

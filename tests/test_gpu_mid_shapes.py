@@ -1,6 +1,8 @@
 """Every built shape of the kernel whose blocks split K among their waves, by its tile and its blocks per CU: exact where the arithmetic is, on
 ragged sizes, K tails, shares of K without a slab and grids of one, several and many blocks; and the heights and cuts the planner
 takes for matmuls of little more than half a round of tiles."""
+import re
+
 import pytest
 import torch
 
@@ -64,3 +66,34 @@ def test_heights_and_cuts_of_little_more_than_half_a_round():
     assert "K split" in _lib.matmul_describe(164, 8192, 28672, False) and "K split 3" in _lib.matmul_describe(2048, 2304, 16384)
     # cut tiles against a short round of whole ones, with the workspace and without
     assert "every tile cut" in _lib.matmul_describe(1929, 1536, 7168) and "cut" not in _lib.matmul_describe(1929, 1536, 7168, True, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["block", "row"])
+def test_the_name_is_that_of_the_kernel_that_runs(dev, kind):
+    from torch.profiler import ProfilerActivity, profile
+
+    sizes = [(8, 4096, 4096), (16, 6144, 4096), (17, 1536, 7168), (18, 2048, 4880), (20, 4096, 4096), (28, 4096, 14336), (32, 28672, 4096),
+             (48, 8192, 28672), (64, 4096, 4096), (64, 32768, 512), (117, 6144, 4096), (1500, 4096, 4096)]
+
+    def call(M, N, K):
+        a, b = (torch.ones(rows, K, device=dev).to(torch.float8_e4m3fn) for rows in (M, N))
+        ones = lambda *shape: torch.ones(shape, device=dev)
+        scales = (ones(-(-K // 128), -(-M // 4) * 4), ones(-(-N // 128), -(-K // 128))) if kind == "block" else (ones(1, M), ones(N, 1))
+        mx.dynamic_scaled_matmul(a, b, *scales, CFG[kind].input_scale, CFG[kind].weight_scale)
+    with profile(activities=[ProfilerActivity.CUDA]) as seen:
+        for size in sizes:
+            call(*size)
+        torch.cuda.synchronize()
+    ran = sorted((e.time_range.start, e.name) for e in seen.events() if "maxfp8::gemm_" in e.name)
+    assert len(ran) == len(sizes)
+    for (M, N, K), (_, name) in zip(sizes, ran):
+        text = _lib.matmul_describe(M, N, K, kind == "block")
+        small = [shape for shape in SHAPES if all(part in text for part in describe_of(shape))]
+        if small:
+            blocks, mt, nt = small[0] // 100, small[0] // 10 % 10, small[0] % 10
+            assert re.search(rf"gemm_mid_kernel<{mt}, {nt}, \w+, \d+, {blocks}, ", name), (text, name)
+        elif text == "skinny":
+            assert "gemm_skinny_kernel" in name, (text, name)
+        else:
+            assert ("gemm_w4_kernel" if "four waves" in text else "gemm_tiled_kernel") in name, (text, name)

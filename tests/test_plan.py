@@ -15,16 +15,18 @@ def test_single_shapes_and_k_split():
     assert _lib.matmul_describe(2048, 6144, 4096) == "256x256 x192 persistent"
     assert _lib.matmul_describe(2040, 6144, 4096) == "256x256 x192"
     assert _lib.matmul_describe(8, 4096, 4096) == "skinny"
-    assert _lib.matmul_describe(32, 28672, 4096) == "skinny"
+    assert "block's waves" in _lib.matmul_describe(32, 28672, 4096)
     # 33 to 64 rows go to the 128-row tiles unless the weights are small (under 32 MB): wide matrices, and narrow ones split over
     # K; small weights to the tiles whose blocks split K among their waves where those are estimated quicker than the streaming
     assert "block's waves" in _lib.matmul_describe(64, 4096, 4096) and "block's waves" in _lib.matmul_describe(33, 6144, 4096)
     assert _lib.matmul_describe(64, 28672, 4096).startswith("128x128")
     assert "K split" in _lib.matmul_describe(48, 8192, 28672)
-    assert _lib.matmul_describe(48, 8192, 28672, True, False) == "skinny"  # no workspace, no split: the streaming kernel
+    assert "block's waves" in _lib.matmul_describe(48, 8192, 28672, True, False)  # no workspace, no split: the small tiles
     # 25 to 32 rows: the tiles only where K is long and N narrow
-    assert "K split" in _lib.matmul_describe(32, 8192, 28672) and _lib.matmul_describe(24, 8192, 28672) == "skinny"
-    assert _lib.matmul_describe(32, 8192, 8192) == "skinny" and _lib.matmul_describe(32, 10240, 16384) == "skinny"
+    assert "K split" in _lib.matmul_describe(32, 8192, 28672) and "block's waves" in _lib.matmul_describe(24, 8192, 28672)
+    assert "block's waves" in _lib.matmul_describe(32, 8192, 8192) and "block's waves" in _lib.matmul_describe(32, 10240, 16384)
+    # (K longer than the small tiles' registers hold scales of: the decode kernel)
+    assert _lib.matmul_describe(24, 4096, 32768 + 128) == "skinny"
     with_ws, without = _lib.matmul_describe(256, 4096, 14336), _lib.matmul_describe(256, 4096, 14336, True, False)
     assert "K split" in with_ws and "K split" not in without
     # where the pieces of a K split would fill three quarters of the chip with at least 16 slabs each, the four-wave kernel
@@ -79,27 +81,29 @@ def test_four_wave_kernel_where_its_tile_count_fits_the_chip(tune):
     assert "tail cut" not in _lib.matmul_describe(2040, 6144, 4096 + 256)
 
 
-def test_the_kernel_for_tens_of_tokens_against_the_decode_kernel():
-    """Up to 32 rows only where the decode kernel's third block per CU would run all but alone; beyond, by estimates of their own
-    for block and row scales; unsplit tiles for the shortest K."""
+def test_the_kernel_for_tens_of_tokens(tune):
+    """From 17 rows on the small tiles wherever the decode kernel ran; the tiles for unsplit ones of the shortest K."""
     kind = lambda *a, **kw: "mid" if "block's waves" in _lib.matmul_describe(*a, **kw) else _lib.matmul_describe(*a, **kw)
     for block in (True, False):
+        for M in (1, 16):
+            assert kind(M, 4096, 4096, block) == "skinny"
         for M in (17, 24, 32):
-            for N, K in ((1536, 7168), (576, 7168), (2112, 7168), (4096, 4096), (6144, 4096), (704, 11520), (28672, 4096)):
-                assert kind(M, N, K, block) == "skinny", (M, N, K)
-            assert kind(M, 10240, 8192, block) == "mid"
+            for N, K in ((1536, 7168), (576, 7168), (2112, 7168), (4096, 4096), (6144, 4096), (704, 11520), (28672, 4096), (10240, 8192), (8208, 1024)):
+                assert kind(M, N, K, block) == "mid", (M, N, K)
         for M in (33, 48, 64):
-            assert kind(M, 4096, 4096, block) == "mid" and kind(M, 1536, 7168, block) == "mid" and kind(M, 10240, 8192, block) == "mid"
-            assert kind(M, 6272, 512, block) == "skinny"
-        assert kind(17, 8208, 1024, block) == "skinny" and kind(17, 8208, 1152, block) == "mid" == kind(32, 12288, 1152, block)
-        assert kind(32, 8192, 1152, block) == "skinny" == kind(32, 12304, 1152, block)
-    # wide and short: the decode kernel pays for block scales, and is ahead without them
-    assert kind(39, 21600, 896) == "mid" and kind(39, 21600, 896, False) == "skinny"
-    assert "128x128" in kind(24, 32768, 512) and kind(24, 32768, 512, False) == "skinny"
-    assert "128x128" in kind(48, 32768, 512, False) and kind(57, 20080, 512, False) == "skinny"
+            for N, K in ((4096, 4096), (1536, 7168), (10240, 8192), (6272, 512)):
+                assert kind(M, N, K, block) == "mid", (M, N, K)
+        assert kind(39, 21600, 896, block) == "mid"
+    assert "128x128" in kind(24, 32768, 512) and kind(24, 32768, 512, False) == "mid"
+    assert "128x128" in kind(48, 32768, 512, False) and kind(57, 20080, 512, False) == "mid"
     # (no scaling is named: what either of them uses)
     assert kind(20, 18784, 6656).endswith("K split 3") and _lib.lib().maxfp8_matmul_auto_workspace_bytes(20, 18784, 6656) > 0
     assert _lib.lib().maxfp8_matmul_auto_workspace_bytes(24, 1536, 7168) == 0
+    # switches of the other kernels, and the small tiles' own, leave the decode kernel in their place
+    for switch in ({"MAXFP8_MID": "0"}, {"MAXFP8_TILE": "2"}, {"MAXFP8_SPLITK": "2"}, {"MAXFP8_W4": "4"}, {"MAXFP8_SKINNY": "1408"}):
+        tune(**switch)
+        assert kind(24, 4096, 4096) == "skinny", switch
+        tune(**{name: None for name in switch})
 
 
 def test_rows_quantised_inside_the_decode_kernel():
