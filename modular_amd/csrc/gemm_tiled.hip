@@ -2009,8 +2009,12 @@ static float w4_plan_cost(int64_t M, int64_t N, int64_t K, bool blockscale, int 
   const float t_slab = blockscale ? kW4SlabBlock[tm - 4] : kW4SlabRow[tm - 4], t = (float)nslab * t_slab + kW4Tile;
   const int64_t tiles = ceil_div(M, 32 * tm) * ceil_div(N, 256);
   // (part of one round, weights from memory: a block waits for its copies, and the chip's clock does not make up for it -- 166 x 36864 x 7168 in 144 tiles of 192 rows
-  // 1.17 us per slab, with row scales 260 x 17616 x 6144 in 138 of 160 rows 1.13, in 207 of 128 rows 0.96)
-  if (!split) return tiles < slots && N * K >= ((int64_t)1 << 26) ? (float)nslab * kW4SlabBlock[tm - 4] + kW4Tile : persistent_cost(tiles, slots, t);
+  // 1.17 us per slab, with row scales 260 x 17616 x 6144 in 138 of 160 rows 1.13, in 207 of 128 rows 0.96.  From five row tiles on, which share the weights,
+  // row scales are quicker than block scales again in the taller tiles, where those fill three quarters of the chip: 1352 x 5856 x 15104 in 207 tiles of
+  // 160 rows 110 us, on 128 x 128 tiles 131; 1072 x 7168 x 18432 138 and 158; but 776 x 7168 x 18432 in 140 of them 142, on 256 x 128 tiles 124, and
+  // 598 x 12128 x 10496 in 192 of them, four row tiles, 81, in 240 of 128 rows 76)
+  const bool alone = blockscale || tm == 4 || M <= 4 * 32 * tm || tiles * 4 < slots * 3;
+  if (!split) return alone && tiles < slots && N * K >= ((int64_t)1 << 26) ? (float)nslab * kW4SlabBlock[tm - 4] + kW4Tile : persistent_cost(tiles, slots, t);
   const W4Split sp = gemm_w4_split(M, N, K, tm);
   const float pieces = (float)ceil_div(nslab, sp.unit);
   if (tiles * 2 <= slots)  // (fitted like gemm_mid_shape's estimates: within 5 per cent for nine launches in ten of 128-row tiles, 13 of taller ones)
@@ -2068,7 +2072,10 @@ static int pick_w4(int64_t M, int64_t N, int64_t K, bool blockscale, float other
       // (where the eight-wave shapes fill the chip without a K split, as one short round, the cut tiles may still be ahead: 1929 x 1536 x
       // 7168 in 96 tiles of two pieces 30 against 38 us; the fused QKV projection not: 435 x 7168 x 5120 41 against 34)
       const float cost = !kv_on && every_cut(tm) ? w4_plan_cost(M, N, K, blockscale, tm, true) : best_cost;
-      if (cost < 0.9f * best_cost) { best = tm; best_cost = cost; *split = true; }
+      // (with row scales less of a margin against whole tiles of this kernel, which wait for 16 MB of weights and more from memory: 600 x 7168 x 5120 31
+      // against 33 us, from memory 36 and 46; with less of them 2823 x 2016 x 4608 36 against 31, 37 and 35)
+      const bool waits = best && !*split && !blockscale && N * K >= ((int64_t)1 << 24);
+      if (cost < (waits ? 0.97f : 0.9f) * best_cost) { best = tm; best_cost = cost; *split = true; }
       continue;
     }
     const float whole = w4_plan_cost(M, N, K, blockscale, tm, false);

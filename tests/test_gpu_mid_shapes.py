@@ -64,6 +64,13 @@ def test_heights_and_cuts_of_little_more_than_half_a_round():
     # two row tiles of 192 in four pieces instead of three of 128 in two; where 128-row tiles do not pay, K splits as before
     assert _lib.matmul_describe(338, 8192, 28672, False) == "192x256 x64 persistent, four waves, every tile cut in pieces of 56 slabs"
     assert "K split" in _lib.matmul_describe(164, 8192, 28672, False) and "K split 3" in _lib.matmul_describe(2048, 2304, 16384)
+    # row scales: taller tiles whose row tiles share the weights, not 504 tiles of 128 x 128; where they fill too little of the chip, not
+    assert _lib.matmul_describe(1072, 7168, 18432, False) == "160x256 x196 persistent, four waves"
+    assert _lib.matmul_describe(1352, 5856, 15104, False) == "160x256 x207 persistent, four waves"
+    assert "four waves" not in _lib.matmul_describe(776, 7168, 18432, False)
+    assert _lib.matmul_describe(598, 12128, 10496, False) == "128x256 x240 persistent, four waves"
+    # ... and cut tiles rather than whole ones of little more than half a round
+    assert _lib.matmul_describe(600, 7168, 5120, False) == "160x256 x112 persistent, four waves, every tile cut in pieces of 20 slabs"
     # cut tiles against a short round of whole ones, with the workspace and without
     assert "every tile cut" in _lib.matmul_describe(1929, 1536, 7168) and "cut" not in _lib.matmul_describe(1929, 1536, 7168, True, False)
 
