@@ -67,8 +67,7 @@ int gemm_mid_dispatch(const GemmArgs&, bool, int, hipStream_t);
 bool gemm_mid_ok(int64_t M, int64_t N, int64_t K);
 int gemm_mid_shape(int64_t M, int64_t N, int64_t K, bool blockscale, float* us);
 int gemm_mid_forced_shape();
-bool gemm_mid_before_skinny(int64_t M, int64_t N, int64_t K);
-float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
+float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool* alone);
 float gemm_tiled_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
 float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool has_workspace);
 size_t gemm_tiled_qkv_workspace_bytes(int64_t M, int64_t N, int64_t K, bool blockscale);
@@ -239,10 +238,18 @@ static Choice choose(Asked what, int64_t M, int64_t N, int64_t K, bool block) {
   return choice;
 }
 
-// Which kernel MAXFP8_ALGO_AUTO gives a fast-layout matmul whose caller brings all the workspace it is asked for.  At most
-// 16 rows: the decode kernel.  Up to 64: the small tiles or the tiles, by the decode kernel's own rule; the tiles also where they are estimated 8 per
-// cent quicker than it (the estimates' own error), the small tiles also where the tiles' rule gave way to their quicker estimate;
-// up to 2048: either of them, by the estimates.  Forced shapes keep the other kernels out.
+// Do the small tiles, at `mid` microseconds, stand back behind the decode kernel?  At 17 to 32 rows with row scales and one of its blocks per CU: with its
+// whole share of K in flight it is up to 13 per cent ahead with the weights from memory (22 x 5536 x 640 4.3 us against 4.8, 18 x 6144 x 4096 8.5 and 9.1), as a
+// model's are, and 5 to 20 behind with them in the memory-side cache (4.9 and 4.5, 8.6 and 8.1).  Block scales cost it more (20 x 6144 x 4096 8.4 and
+// 8.6, 8.5 and 7.5), and at up to 16 rows, where it always runs, the two are 3 per cent apart either way.
+static bool decode_ahead(int64_t M, int64_t N, int64_t K, bool block, float mid) {
+  bool alone;
+  return M <= 32 && !block && gemm_skinny_cost(M, N, K, block, &alone) < 1.02f * mid && alone;
+}
+
+// Which kernel MAXFP8_ALGO_AUTO gives a fast-layout matmul whose caller brings all the workspace it is asked for.  At most 16 rows: the decode kernel.  Up to
+// 2048: the small tiles or the tiles, by the estimates, or, up to 32, the decode kernel.  Forced shapes keep the other kernels out, and beyond what the small
+// tiles take the sizes alone decide.
 static int choose_matmul(int64_t M, int64_t N, int64_t K, bool block) {
   const Tuning& t = tuning();
   const int plain = gemm_skinny_preferred(M, N, K) ? MAXFP8_ALGO_SKINNY : MAXFP8_ALGO_TILED;
@@ -250,23 +257,19 @@ static int choose_matmul(int64_t M, int64_t N, int64_t K, bool block) {
   if (M <= 16 || !gemm_mid_ok(M, N, K) || t.mid == 0 || t.tile || t.splitk || t.one_region || t.w4 >= 0 || t.w4_split == 1 || t.skinny) return plain;
   float mid;
   gemm_mid_shape(M, N, K, block, &mid);
-  // (further from what the estimate was fitted to, or with more of its time spent on memory, or against whole tiles, whose estimate is rough: 1730
-  // x 592 x 5248 19 against 22 us, 79 x 7168 x 16384 35 against 38, 940 x 8320 x 1408 24 against 29)
-  const float margin = M > 1024 ? 0.80f : gemm_tiled_plan_workspace_bytes(M, N, K, block) == 0 ? 0.85f : N * K >= ((int64_t)1 << 26) ? 0.90f : 0.97f;
-  if (M > gemm_skinny_max_m()) return mid < margin * gemm_tiled_cost(M, N, K, block) ? kAlgoMid : MAXFP8_ALGO_TILED;
+  if (decode_ahead(M, N, K, block, mid)) return MAXFP8_ALGO_SKINNY;
   const float tiles = gemm_tiled_cost(M, N, K, block);
-  const bool splits = gemm_tiled_plan_workspace_bytes(M, N, K, true) > 0;
-  // (the estimate of unsplit tiles is the roughest)
-  if (plain == MAXFP8_ALGO_TILED) return mid < (splits ? 0.85f : 0.75f) * tiles ? kAlgoMid : MAXFP8_ALGO_TILED;
-  // (unsplit tiles in the decode kernel's range only for the shortest K, where four waves have no K to split: 48 x 32768 x 512 with
-  // block scales 17.2 against 7.8 us; with row scales, which cost the decode kernel less, from its seventh block per CU on: 48 x
-  // 32768 x 512 14.8 against 10.1, but 57 x 20080 x 512 10.6 against 12.9, 62 x 8400 x 512 8.1 against 12.4, 24 x 32768 x 512 1.10)
-  const bool unsplit = K <= 512 && (block || (M > 32 && ceil_div(N, 16) > 6 * (int64_t)compute_units()));
-  // (up to 32 rows split tiles only from its fourth block per CU on: 24 x 17920 x 6528 31.5 against 28.7; its estimate is 10 to 20
-  // per cent high on narrow weights with long K)
-  const bool split = splits && (M > 32 || ceil_div(N, 16) > 3 * (int64_t)compute_units());
-  const bool on_tiles = tiles < 0.92f * gemm_skinny_cost(M, N, K, block) && (split || (!splits && unsplit));
-  return on_tiles && (M <= 32 || !splits || tiles < 1.15f * mid) ? MAXFP8_ALGO_TILED : kAlgoMid;
+  const bool large = N * K >= ((int64_t)1 << 26), whole = gemm_tiled_plan_workspace_bytes(M, N, K, block) == 0;
+  // The tiles' estimate at up to 64 rows is of weights from memory and the small tiles' is not: the tiles may take more where the small ones need it -- large
+  // weights, of long K above all (42 x 8192 x 28672 46 us on tiles, 54 on small ones, estimates 51 and 47), and few slabs in many blocks (45 x 24576 x 1536
+  // 11.6 and 13.1, 12.7 and 9.9; 50 x 32768 x 512 7.0 and 8.6, 24 of them 6.7 and 7.0).
+  if (M <= 64) {
+    const float margin = whole && K <= 512 ? 1.36f : M <= 32 ? 0.95f : large ? (K >= 16384 ? 1.15f : whole ? 1.12f : 1.05f) : whole ? 1.30f : 0.95f;
+    return tiles < margin * mid ? MAXFP8_ALGO_TILED : kAlgoMid;
+  }
+  // Beyond, both by their prices of the chip at work.  (Further from what the estimate was fitted to, or with more of its time spent on memory, or against whole
+  // tiles, whose estimate is rough: 1730 x 592 x 5248 19 against 22 us, 79 x 7168 x 16384 35 against 38, 940 x 8320 x 1408 24 against 29.)
+  return mid < (M > 1024 ? 0.80f : whole ? 0.85f : large ? 0.90f : 0.97f) * tiles ? kAlgoMid : MAXFP8_ALGO_TILED;
 }
 static Choice choose_kernel(int64_t M, int64_t N, int64_t K, bool block) {
   if (M <= 16 && tuning().mid <= 0) return {MAXFP8_ALGO_SKINNY, 0};
@@ -297,12 +300,17 @@ static Choice choose_qkv(int64_t T, int64_t N, int64_t K, bool has_workspace, bo
 }
 
 // 17 to 64 rows whose tiles would split K, without the workspace for it
-static int without_workspace(int64_t M, int64_t N, int64_t K) {
-  return gemm_mid_before_skinny(M, N, K) ? kAlgoMid : MAXFP8_ALGO_SKINNY;
+static int without_workspace(int64_t M, int64_t N, int64_t K, bool block) {
+  const Tuning& t = tuning();
+  if (!gemm_mid_ok(M, N, K) || t.skinny || t.mid == 0 || (M <= 16 && t.mid < 0)) return MAXFP8_ALGO_SKINNY;
+  if (t.mid > 0) return kAlgoMid;
+  float mid;
+  gemm_mid_shape(M, N, K, block, &mid);
+  return decode_ahead(M, N, K, block, mid) ? MAXFP8_ALGO_SKINNY : kAlgoMid;
 }
 static Choice choose_uncached(Asked what, int64_t M, int64_t N, int64_t K, bool block) {
   const int algo = what == Asked::kMatmul          ? choose_matmul(M, N, K, block)
-                   : what == Asked::kMatmulNoSplit ? without_workspace(M, N, K)
+                   : what == Asked::kMatmulNoSplit ? without_workspace(M, N, K, block)
                                                    : choose_qkv_matmul(M, N, K, what == Asked::kQkvWorkspace, block);
   return algo == kAlgoMid ? mid_choice(M, N, K, block) : Choice{algo, 0};
 }

@@ -333,7 +333,6 @@ static int launch_mid(const GemmArgs& p, hipStream_t stream) {
 }
 
 int compute_units();
-float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
 
 // The shapes that are built: 16 mt tokens x 16 nt weight rows, blocks per CU.  Of 78 measured on 300 matmuls (1 to 1000 tokens, K 512 ...
 // 28672, N 512 ... 57344, both scalings), these lose 1 per cent against choosing among all of them.
@@ -345,11 +344,13 @@ struct MidShape { int mt, nt, blocks; };
 static const MidShape kMidShapes[] = {MAXFP8_MID_SHAPES(MAXFP8_MID_ROW)};
 #undef MAXFP8_MID_ROW
 
-// Estimated microseconds, one estimate for all shapes (fitted to the launches above, operands in the memory-side cache where they fit:
+// Estimated microseconds, one estimate for all shapes.  Fitted to the launches above with the operands in the memory-side cache where they fit:
 // within 8 per cent for half of the launches, 19 for nine in ten; what the shapes have in common cancels where they are
-// compared: the one it picks is 0.4 per cent behind the best of them on average, 10 at most).  A launch; per round of blocks on the
-// chip a start and end, the waits of the ring's rounds, and the MFMAs of a wave; per block of a CU the bytes of its slabs and
-// its MFMAs; the weights' way from memory.
+// compared: the one it picks is 0.4 per cent behind the best of them on average there, 10 at most, and 0.8 with the weights from memory.  From memory a launch takes
+// 1.07 to 1.2 times as long, the more the longer K is; the rules that compare it with other kernels (api.hip) were made for that.  An estimate fitted to times from
+// memory instead picked no better there beyond 64 tokens (1066 matmuls: 0.6 per cent behind the best kernel and shape with either) and worse in the cache.
+// Its terms: a launch; per round of blocks on the chip a start and end, the waits of the ring's rounds, and the MFMAs of a wave; per block of a CU the bytes of its
+// slabs and its MFMAs; the weights' way.
 static float mid_cost(const MidShape& t, int64_t M, int64_t N, int64_t K, bool blockscale) {
   const int64_t cus = compute_units(), blocks = ceil_div(M, 16 * t.mt) * ceil_div(N, 16 * t.nt);
   const float rounds = (float)ceil_div(blocks, cus * t.blocks), per_cu = (float)ceil_div(blocks, cus);
@@ -374,17 +375,6 @@ int gemm_mid_shape(int64_t M, int64_t N, int64_t K, bool blockscale, float* us) 
     if (!best || c < *us) { best = &t; *us = c; }
   }
   return 100 * best->blocks + 10 * best->mt + best->nt;
-}
-
-// The kernel here or the decode kernel (gemm_skinny.hip), at most 64 rows.  From 17 on the decode kernel loads two or four groups of 16 tokens
-// straight into the MFMA's operand layout and is behind with the weights in the memory-side cache (17 x 7168 x 18432 27.0 against 27.6 us at
-// best; 22 x 3312 x 512 4.5 against 3.5, 28 x 4096 x 14336 19.1 against 13.5, 64 x 4096 x 14336 31.7 against 15.2; 17 to 32 rows 1.2 on
-// average).  With weights that come from memory 17 to 32 rows are 1.07 on average, and up to 13 per cent behind on a quarter of the
-// shapes, most with row scales and one or two of the decode kernel's blocks per CU (18 x 2048 x 4880 5.9 against 6.8, the cache 6.3 against
-// 5.9).  Up to 16 rows the decode kernel keeps more weights in flight: 3 per cent behind in that cache, as much ahead from memory.
-bool gemm_mid_before_skinny(int64_t M, int64_t N, int64_t K) {
-  if (!gemm_mid_ok(M, N, K) || tuning().skinny || tuning().mid == 0) return false;
-  return M > 16 || tuning().mid > 0;
 }
 
 template <bool BLOCKSCALE, bool KV>

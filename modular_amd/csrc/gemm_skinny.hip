@@ -734,21 +734,15 @@ bool gemm_skinny_preferred(int64_t M, int64_t N, int64_t K) {
   return M <= 64 && small_weights;
 }
 
-// Estimated microseconds at 17 to 64 rows, for the comparison with the tiles (beyond 32 fitted to 960 launches per scaling of 576 ... 32768 x
-// 512 ... 12288, the slabs a wave walks counted as its ring does, in whole rounds).
-float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
+// Estimated microseconds at 17 to 32 rows, fitted to 700 matmuls with the weights from memory and, with less weight, in the memory-side cache: within 3 per cent
+// for half of the launches, 7 for nine in ten.  *alone: a CU has one block, of at most 32 weight rows
+float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool* alone) {
   const int ntw = skinny_shape(M, N, K) / 1000;
-  const float blocks = (float)ceil_div(ceil_div(N, 16 * ntw), compute_units());  // per CU
-  if (M <= 32) {
-    const float w = blocks * (float)(ntw * 16) * (float)K * 1e-5f;               // weight bytes per CU
-    return 3.0f + 0.84f * blocks + 2.62f * w + 1.62f * blocks * 32.f * (float)K * 1e-5f;
-  }
-  const int depth = ntw == 4   ? (blockscale ? SkinnyCfg<4, 4, true, 32, 4>::DEPTH : SkinnyCfg<4, 4, false, 32, 4>::DEPTH)
-                    : ntw == 2 ? (blockscale ? SkinnyCfg<2, 4, true, 8, 4>::DEPTH : SkinnyCfg<2, 4, false, 8, 4>::DEPTH)
-                               : (blockscale ? SkinnyCfg<1, 4, true, 8, 4>::DEPTH : SkinnyCfg<1, 4, false, 8, 4>::DEPTH);
-  const float slabs = (float)(ceil_div(ceil_div(K, 512), depth) * depth), k = (float)K;
-  if (blockscale) return 1.32f + blocks * (1.75f + 0.356f * (float)ntw + 0.24f * slabs + (3.80e-4f * (float)ntw + 1.62e-5f * (float)M) * k);
-  return 3.26f + blocks * (0.596f * (float)ntw + 0.099f * slabs + (4.20e-4f * (float)ntw + 1.88e-5f * (float)M) * k);
+  const int64_t per_cu = ceil_div(ceil_div(N, 16 * ntw), (int64_t)compute_units());
+  *alone = per_cu == 1 && ntw <= 2;
+  const float blocks = (float)per_cu, k = (float)K * 1e-4f, weights = (float)N * (float)K * 1e-6f;
+  if (blockscale) return 2.70f + blocks * (0.81f + (3.26f * (float)ntw + 0.88f + 0.195f * (float)M) * k) + 0.026f * weights;
+  return 3.07f + blocks * (0.76f + (3.32f * (float)ntw + 0.42f + 0.192f * (float)M) * k) + 0.025f * weights;
 }
 
 int gemm_skinny_dispatch(const GemmArgs& p, bool blockscale, int64_t batch, hipStream_t stream) {

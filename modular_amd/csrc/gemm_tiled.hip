@@ -2195,12 +2195,39 @@ static TiledPlan cached_plan(int64_t M, int64_t N, int64_t K, bool blockscale, b
   return plan;
 }
 
+// At most 64 rows, where the planner's prices (of a full chip) are furthest off: one round of tiles or less, and a K split.  Fitted to 700 matmuls (K 512 ...
+// 28672, N 512 ... 57344, in every shape and split that suits them), weights from memory; from the memory-side cache the eight-wave tiles take the same.
+struct LaunchCost { float slab, more, launch, stream; };
+// microseconds per slab with the chip empty and what a full one adds, per launch, per MB of weights: within 3 per cent for half of the launches, 5 to 17 for
+// nine in ten.  The shapes of kShapes and the four-wave kernel's lowest tiles.
+static const LaunchCost kFewBlock[5] = {{1.21f, 0.45f, 7.4f, 0.029f}, {0.69f, 0.24f, 5.4f, 0.f}, {0.77f, 0.28f, 4.4f, 0.058f}, {0.53f, 0.06f, 4.4f, 0.036f}, {0.53f, 0.28f, 5.2f, 0.092f}};
+static const LaunchCost kFewRow[5] = {{1.31f, 0.25f, 11.6f, 0.023f}, {0.64f, 0.19f, 8.0f, 0.003f}, {0.83f, 0.19f, 7.4f, 0.058f}, {0.50f, 0.02f, 7.5f, 0.040f}, {0.55f, 0.18f, 8.7f, 0.094f}};
+// ... per slab of a share, per MB of the shares' sums, both launches, per MB of weights: within 3 per cent for half, 8 for nine in ten
+static const LaunchCost kFewSplitBlock[4] = {{1.56f, 0.70f, 7.4f, 0.027f}, {0.80f, 0.82f, 7.7f, 0.025f}, {0.90f, 0.71f, 7.4f, 0.060f}, {0.54f, 0.97f, 6.9f, 0.048f}};
+static const LaunchCost kFewSplitRow[4] = {{1.55f, 0.70f, 8.9f, 0.017f}, {0.72f, 0.91f, 7.7f, 0.016f}, {0.92f, 0.71f, 8.1f, 0.049f}, {0.50f, 0.98f, 7.1f, 0.049f}};
+static float few_rows_cost(const TiledPlan& plan, int64_t M, int64_t N, int64_t K, bool blockscale) {
+  const int64_t slabs = ceil_div(K, 128);
+  const float weights = (float)N * (float)K * 1e-6f;
+  const int shape = plan.w4 ? 4 : plan.variant - 1, slots = plan.w4 ? compute_units() : kShapes[shape].slots;
+  const int64_t tiles = plan.w4 ? ceil_div(M, 128) * ceil_div(N, 256) : ceil_div(M, kShapes[shape].bm) * ceil_div(N, kShapes[shape].bn);
+  if (plan.splits > 1) {
+    const LaunchCost& c = (blockscale ? kFewSplitBlock : kFewSplitRow)[shape];
+    return c.launch + c.slab * (float)(ceil_div(tiles * plan.splits, slots) * ceil_div(slabs, plan.splits)) + c.more * (float)plan.splits * (float)M * (float)N * 2e-6f + c.stream * weights;
+  }
+  if (tiles > slots || plan.w4_split || plan.w4 > 4) return 0.f;  // (none of these)
+  const LaunchCost& c = (blockscale ? kFewBlock : kFewRow)[shape];
+  return (float)slabs * (c.slab + c.more * (float)tiles / (float)slots) + c.launch + c.stream * weights;
+}
+
 // Estimated microseconds of this shape's plan with all the workspace it asks for.  A K split, every tile cut, one round of three-stage
-// 128 x 128 tiles: fitted like gemm_mid_shape's estimates, within 7, 5 and 20 per cent for nine launches in ten; every other plan: what the planner
-// compares.
+// 128 x 128 tiles: within 7, 5 and 20 per cent for nine launches in ten; every other plan: what the planner compares.
 float gemm_tiled_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
   const TiledPlan plan = cached_plan(M, N, K, blockscale, true, ~(size_t)0, 1, false);
   const float slabs = (float)ceil_div(K, 128), stream = (float)N * (float)K / 6e6f;
+  if (M <= 64 && !plan.two.axis) {
+    const float few = few_rows_cost(plan, M, N, K, blockscale);
+    if (few > 0.f) return few;
+  }
   if (plan.w4) return w4_plan_cost(M, N, K, blockscale, plan.w4, plan.w4_split);
   if (plan.two.axis) return plan.two.cost;
   if (plan.splits > 1)

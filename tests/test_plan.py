@@ -16,14 +16,14 @@ def test_single_shapes_and_k_split():
     assert _lib.matmul_describe(2040, 6144, 4096) == "256x256 x192"
     assert _lib.matmul_describe(8, 4096, 4096) == "skinny"
     assert "block's waves" in _lib.matmul_describe(32, 28672, 4096)
-    # 33 to 64 rows go to the 128-row tiles unless the weights are small (under 32 MB): wide matrices, and narrow ones split over
-    # K; small weights to the tiles whose blocks split K among their waves where those are estimated quicker than the streaming
+    # 33 to 64 rows: the tiles whose blocks split K among their waves, or the 128-row tiles: wide matrices of short K, and narrow ones
+    # of long K split over the chip
     assert "block's waves" in _lib.matmul_describe(64, 4096, 4096) and "block's waves" in _lib.matmul_describe(33, 6144, 4096)
-    assert _lib.matmul_describe(64, 28672, 4096).startswith("128x128")
+    assert _lib.matmul_describe(64, 32768, 512).startswith("128x128")
     assert "K split" in _lib.matmul_describe(48, 8192, 28672)
     assert "block's waves" in _lib.matmul_describe(48, 8192, 28672, True, False)  # no workspace, no split: the small tiles
-    # 25 to 32 rows: the tiles only where K is long and N narrow
-    assert "K split" in _lib.matmul_describe(32, 8192, 28672) and "block's waves" in _lib.matmul_describe(24, 8192, 28672)
+    # up to 32 rows
+    assert "block's waves" in _lib.matmul_describe(32, 8192, 28672) and "block's waves" in _lib.matmul_describe(24, 8192, 28672)
     assert "block's waves" in _lib.matmul_describe(32, 8192, 8192) and "block's waves" in _lib.matmul_describe(32, 10240, 16384)
     # (K longer than the small tiles' registers hold scales of: the decode kernel)
     assert _lib.matmul_describe(24, 4096, 32768 + 128) == "skinny"
@@ -82,22 +82,28 @@ def test_four_wave_kernel_where_its_tile_count_fits_the_chip(tune):
 
 
 def test_the_kernel_for_tens_of_tokens(tune):
-    """From 17 rows on the small tiles wherever the decode kernel ran; the tiles for unsplit ones of the shortest K."""
+    """Up to 16 rows the decode kernel; beyond, the small tiles but for row scales on weights of one decode block per CU, up to 32, and where
+    the tiles' estimate is the better one."""
     kind = lambda *a, **kw: "mid" if "block's waves" in _lib.matmul_describe(*a, **kw) else _lib.matmul_describe(*a, **kw)
     for block in (True, False):
         for M in (1, 16):
             assert kind(M, 4096, 4096, block) == "skinny"
         for M in (17, 24, 32):
-            for N, K in ((1536, 7168), (576, 7168), (2112, 7168), (4096, 4096), (6144, 4096), (704, 11520), (28672, 4096), (10240, 8192), (8208, 1024)):
+            for N, K in ((28672, 4096), (10240, 8192), (16384, 1024), (576, 7168)):
                 assert kind(M, N, K, block) == "mid", (M, N, K)
         for M in (33, 48, 64):
             for N, K in ((4096, 4096), (1536, 7168), (10240, 8192), (6272, 512)):
                 assert kind(M, N, K, block) == "mid", (M, N, K)
-        assert kind(39, 21600, 896, block) == "mid"
-    assert "128x128" in kind(24, 32768, 512) and kind(24, 32768, 512, False) == "mid"
-    assert "128x128" in kind(48, 32768, 512, False) and kind(57, 20080, 512, False) == "mid"
+        assert "K split" in kind(42, 8192, 28672, block) and "K split" in kind(55, 7168, 18432, block)
+    for M, N, K in ((18, 6144, 4096), (22, 5536, 640), (24, 5536, 1280), (17, 4096, 14336)):
+        assert kind(M, N, K, False) == "skinny" and kind(M, N, K, True) == "mid", (M, N, K)
+        assert kind(33, N, K, False) != "skinny"
+    # wide weights of few slabs: 128 x 128 tiles with block scales
+    assert "128x128" in kind(45, 24576, 1536) and "128x128" in kind(50, 32768, 512) and "128x128" in kind(24, 32768, 512)
+    # ... and as many blocks as the chip holds at once, of 64 columns
+    assert kind(64, 28672, 4096) == "mid" == kind(20, 18784, 6656)
     # (no scaling is named: what either of them uses)
-    assert kind(20, 18784, 6656).endswith("K split 3") and _lib.lib().maxfp8_matmul_auto_workspace_bytes(20, 18784, 6656) > 0
+    assert kind(42, 8192, 28672).endswith("K split 8") and _lib.lib().maxfp8_matmul_auto_workspace_bytes(42, 8192, 28672) > 0
     assert _lib.lib().maxfp8_matmul_auto_workspace_bytes(24, 1536, 7168) == 0
     # switches of the other kernels, and the small tiles' own, leave the decode kernel in their place
     for switch in ({"MAXFP8_MID": "0"}, {"MAXFP8_TILE": "2"}, {"MAXFP8_SPLITK": "2"}, {"MAXFP8_W4": "4"}, {"MAXFP8_SKINNY": "1408"}):
