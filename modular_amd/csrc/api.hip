@@ -281,17 +281,19 @@ static size_t auto_workspace(int64_t M, int64_t N, int64_t K, bool block) {
   return choose_kernel(M, N, K, block).algo == MAXFP8_ALGO_TILED ? gemm_tiled_workspace_bytes(M, N, K) : 0;
 }
 
-// The same for the fused QKV matmul: decode kernel (at most 16 rows), the kernel in between (17 to 64, beyond by its estimate) or the tiles, whose
-// plan may cut them along K where the caller brings a workspace.
+// The same for the fused QKV matmul: decode kernel (at most 16 rows, and up to 32 where it is ahead -- more often than of a plain matmul, since the small tiles' store
+// of K and V costs them 1 us with row scales: 18 x 6144 x 4096 9.4 us from memory against 10.5, in the cache 9.5 both --), the small tiles (17 to 64, beyond by their estimate) or
+// the tiles, whose plan may cut them along K where the caller brings a workspace.  (348 x 5120 x 2048 15.6 us on tiles, on small ones 15.1 and from memory 16.8;
+// 491 x 3072 x 2048 with row scales 16.4 and 17.9, 17.4 and 19.3; 209 x 4608 x 3584 21 and 14, 23 and 16.)
 static int choose_qkv_matmul(int64_t T, int64_t N, int64_t K, bool has_workspace, bool block) {
   const Tuning& t = tuning();
   const int plain = T <= gemm_skinny_max_m() ? MAXFP8_ALGO_SKINNY : MAXFP8_ALGO_TILED;
   if (t.mid > 0) return gemm_mid_ok(T, N, K) ? kAlgoMid : plain;
   if (T <= 16 || !gemm_mid_ok(T, N, K) || t.mid == 0 || t.tile || t.skinny) return plain;
-  if (plain == MAXFP8_ALGO_SKINNY) return kAlgoMid;
   float mid;
   gemm_mid_shape(T, N, K, block, &mid);
-  return mid < 0.85f * gemm_tiled_qkv_cost(T, N, K, block, has_workspace) ? kAlgoMid : MAXFP8_ALGO_TILED;
+  if (plain == MAXFP8_ALGO_SKINNY) return decode_ahead(T, N, K, block, 1.07f * mid) ? MAXFP8_ALGO_SKINNY : kAlgoMid;
+  return mid < (T > 256 ? 0.73f : 0.85f) * gemm_tiled_qkv_cost(T, N, K, block, has_workspace) ? kAlgoMid : MAXFP8_ALGO_TILED;
 }
 static Choice choose_qkv(int64_t T, int64_t N, int64_t K, bool has_workspace, bool block) {
   if (T <= 16 && tuning().mid <= 0) return {MAXFP8_ALGO_SKINNY, 0};

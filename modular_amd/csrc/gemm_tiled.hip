@@ -2068,6 +2068,10 @@ static int pick_w4(int64_t M, int64_t N, int64_t K, bool blockscale, float other
     const int64_t tiles = ceil_div(M, 32 * tm) * ceil_div(N, 256);
     // (half a round or less: more, smaller tiles and a K split are the better fit; a little more than half is not: 166 x 36864 x 7168 in
     // 144 tiles of 192 rows 71 us, in 288 of 128 rows 101)
+    // (the fused QKV projection's tiles, with a store of their own, want three quarters of a round: 526 x 8192 x 6144 with row scales in 160 tiles of 128 rows 42 us and 55
+    // from memory, on 256 x 128 tiles 42 and 44; 639 x 7168 x 5120 with block scales in 140 36 and 48, 41 and 42; but not on large weights, 434 x 9216 x
+    // 7168 in 144 45 and 52, 50 and 52)
+    if (forced <= 0 && kv_on && tiles * 4 < slots * 3 && (!blockscale || N * K < ((int64_t)3 << 24))) continue;
     if (forced <= 0 && tiles * 2 <= slots) {
       // (where the eight-wave shapes fill the chip without a K split, as one short round, the cut tiles may still be ahead: 1929 x 1536 x
       // 7168 in 96 tiles of two pieces 30 against 38 us; the fused QKV projection not: 435 x 7168 x 5120 41 against 34)
@@ -2078,7 +2082,10 @@ static int pick_w4(int64_t M, int64_t N, int64_t K, bool blockscale, float other
       if (cost < (waits ? 0.97f : 0.9f) * best_cost) { best = tm; best_cost = cost; *split = true; }
       continue;
     }
-    const float whole = w4_plan_cost(M, N, K, blockscale, tm, false);
+    // (... and with row scales seven eighths of one, or its smallest take more per slab: 939 x 6144 x 4096 34 us in 192 tiles of 128 rows, from memory 39, on 256 x 128
+    // tiles 33 and 34; 937 x 8192 x 6144 in 256 of them 48 and 57, 51 and 69)
+    const bool slow = kv_on && !blockscale && tm == 4 && tiles * 8 < slots * 7;
+    const float whole = slow ? persistent_cost(tiles, slots, (float)nslab * 0.93f + kW4Tile) : w4_plan_cost(M, N, K, blockscale, tm, false);
     if (whole < best_cost) { best = tm; best_cost = whole; *split = false; }
     const W4Split sp = gemm_w4_split(M, N, K, tm);
     if (cut != 0 && sp.unit > 0 && sp.bytes <= workspace_bytes) {
