@@ -269,7 +269,11 @@ static int choose_matmul(int64_t M, int64_t N, int64_t K, bool block) {
   }
   // Beyond, both by their prices of the chip at work.  (Further from what the estimate was fitted to, or with more of its time spent on memory, or against whole
   // tiles, whose estimate is rough: 1730 x 592 x 5248 19 against 22 us, 79 x 7168 x 16384 35 against 38, 940 x 8320 x 1408 24 against 29.)
-  return mid < (M > 1024 ? 0.80f : whole ? 0.85f : large ? 0.90f : 0.97f) * tiles ? kAlgoMid : MAXFP8_ALGO_TILED;
+  // Up to 512 rows, from 64 slabs on, where the tiles split K: 0.95 of that, as the longest shares of K lose most when the weights come from memory (239 x 4784 x 9984 30 us on
+  // tiles, on small ones 31 and from memory 36; 223 x 4096 x 14336 32, 30 and 36; 142 x 4096 x 14336 with row scales 29, 23 and 31; beyond 512 rows level from
+  // memory and 6 per cent behind in the cache).
+  const float margin = M > 1024 ? 0.80f : whole ? 0.85f : large ? 0.90f : 0.97f;
+  return mid < (M <= 512 && !whole && K >= 8192 ? 0.95f * margin : margin) * tiles ? kAlgoMid : MAXFP8_ALGO_TILED;
 }
 static Choice choose_kernel(int64_t M, int64_t N, int64_t K, bool block) {
   if (M <= 16 && tuning().mid <= 0) return {MAXFP8_ALGO_SKINNY, 0};

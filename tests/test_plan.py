@@ -112,6 +112,16 @@ def test_the_kernel_for_tens_of_tokens(tune):
         tune(**{name: None for name in switch})
 
 
+def test_small_tiles_stand_back_where_long_k_comes_from_memory():
+    """65 to 512 rows, from 64 slabs of K on: near the tiles' estimate a K split is the quicker one with the weights from memory.  Further from it, with
+    fewer slabs or with whole tiles on the other side the small tiles stay."""
+    small = lambda *a: "block's waves" in _lib.matmul_describe(*a)
+    for M, N, K, block in ((239, 4784, 9984, True), (223, 4096, 14336, True), (182, 2176, 14464, True), (142, 4096, 14336, False), (212, 2544, 12544, False), (73, 7056, 12032, True)):
+        assert "K split" in _lib.matmul_describe(M, N, K, block) and not small(M, N, K, block), (M, N, K)
+    for M, N, K, block in ((197, 1632, 14464, True), (99, 4096, 14336, True), (87, 4096, 14336, False), (207, 7168, 5120, False), (204, 4096, 4096, True), (380, 576, 7168, True), (601, 1312, 9856, False)):
+        assert small(M, N, K, block), (M, N, K)
+
+
 def test_rows_quantised_inside_the_decode_kernel():
     """With row scales at most three blocks per CU for more than one token, and four tokens on two; with block scales four of them."""
     need = lambda M, N, K, gran: _lib.lib().maxfp8_linear_workspace_bytes(M, N, K, gran)
