@@ -2241,7 +2241,12 @@ float gemm_tiled_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
     return 8.2f + 0.33f * (float)ceil_div((int64_t)slabs, plan.splits) * (kShapes[plan.variant - 1].bm == 128 ? 1.f : 1.25f) +
            1.024f * (float)plan.splits * (float)M * (float)N * 8.0f / 4.0e6f + 0.63f * stream;
   if (plan.variant == 4) return three_stage_cost(M, N, K, blockscale);
-  return region_cost(M, N, (int)slabs, kShapes[plan.variant - 1], blockscale);
+  const float cost = region_cost(M, N, (int)slabs, kShapes[plan.variant - 1], blockscale);
+  // (one round of block-scaled 256 x 128 tiles is 4 us quicker than the planner's price, and of 256 x 256 ones 3 and more:
+  // 148 x 16656 x 384 7.5 us priced 11.8, on small tiles 9.5; 169 x 20240 x 640 10.2, 13.6 and 12.6; 278 x 12272 x 1152 13.3, 17.2 and 14.1.  With row scales it is right)
+  const TileShape& shape = kShapes[plan.variant - 1];
+  const bool one_round = blockscale && shape.bm == 256 && ceil_div(M, shape.bm) * ceil_div(N, shape.bn) <= shape.slots;
+  return one_round ? cost - (shape.bn == 128 ? 4.f : 3.f) : cost;
 }
 
 // The same for a fused QKV matmul, of any plan (with the workspace it asks for, or without any)

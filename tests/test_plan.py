@@ -122,6 +122,13 @@ def test_small_tiles_stand_back_where_long_k_comes_from_memory():
         assert small(M, N, K, block), (M, N, K)
 
 
+def test_small_tiles_stand_back_behind_one_round_of_large_ones():
+    """Few slabs of block scales on at most one round of whole 256-row tiles: 1.2 to 1.4 times as quick as small tiles at every size measured."""
+    for M, N, K in ((148, 16656, 384), (674, 5408, 384), (257, 21792, 384), (169, 20240, 640), (1602, 2496, 640), (181, 18112, 896), (162, 18160, 1152), (812, 4848, 1152), (301, 12960, 1408), (1423, 2720, 1664)):
+        text = _lib.matmul_describe(M, N, K)
+        assert text.startswith("256x") and "K split" not in text, (M, N, K, text)
+
+
 def test_rows_quantised_inside_the_decode_kernel():
     """With row scales at most three blocks per CU for more than one token, and four tokens on two; with block scales four of them."""
     need = lambda M, N, K, gran: _lib.lib().maxfp8_linear_workspace_bytes(M, N, K, gran)
