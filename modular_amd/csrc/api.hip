@@ -67,7 +67,7 @@ int gemm_mid_dispatch(const GemmArgs&, bool, int, hipStream_t);
 bool gemm_mid_ok(int64_t M, int64_t N, int64_t K);
 int gemm_mid_shape(int64_t M, int64_t N, int64_t K, bool blockscale, float* us);
 int gemm_mid_forced_shape();
-float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool* alone);
+float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool* alone);
 float gemm_tiled_cost(int64_t M, int64_t N, int64_t K, bool blockscale);
 float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool has_workspace);
 size_t gemm_tiled_qkv_workspace_bytes(int64_t M, int64_t N, int64_t K, bool blockscale);
@@ -244,7 +244,7 @@ static Choice choose(Asked what, int64_t M, int64_t N, int64_t K, bool block) {
 // 8.6, 8.5 and 7.5), and at up to 16 rows, where it always runs, the two are 3 per cent apart either way.
 static bool decode_ahead(int64_t M, int64_t N, int64_t K, bool block, float mid) {
   bool alone;
-  return M <= 32 && !block && gemm_skinny_cost(M, N, K, block, &alone) < 1.02f * mid && alone;
+  return M <= 32 && !block && gemm_skinny_cost(M, N, K, &alone) < 1.02f * mid && alone;
 }
 
 // Which kernel MAXFP8_ALGO_AUTO gives a fast-layout matmul whose caller brings all the workspace it is asked for.  At most 16 rows: the decode kernel.  Up to
@@ -286,8 +286,8 @@ static size_t auto_workspace(int64_t M, int64_t N, int64_t K, bool block) {
 }
 
 // The same for the fused QKV matmul: decode kernel (at most 16 rows, and up to 32 where it is ahead -- more often than of a plain matmul, since the small tiles' store
-// of K and V costs them 1 us with row scales: 18 x 6144 x 4096 9.4 us from memory against 10.5, in the cache 9.5 both --), the small tiles (17 to 64, beyond by their estimate) or
-// the tiles, whose plan may cut them along K where the caller brings a workspace.  (348 x 5120 x 2048 15.6 us on tiles, on small ones 15.1 and from memory 16.8;
+// of K and V costs them 1 us with row scales: 18 x 6144 x 4096 9.4 us from memory against 10.5, in the cache 9.5 both --), the small tiles (17 to 64, where the tiles, whole, take 1.7 to 3 times
+// as long, and beyond by their estimate) or the tiles, whose plan may cut them along K where the caller brings a workspace.  (348 x 5120 x 2048 15.6 us on tiles, on small ones 15.1 and from memory 16.8;
 // 491 x 3072 x 2048 with row scales 16.4 and 17.9, 17.4 and 19.3; 209 x 4608 x 3584 21 and 14, 23 and 16.)
 static int choose_qkv_matmul(int64_t T, int64_t N, int64_t K, bool has_workspace, bool block) {
   const Tuning& t = tuning();

@@ -12,7 +12,7 @@
 //   * A slot's fragments are read into registers at once, and the copies that refill it go out between the MFMAs that multiply
 //     them: a CU takes a copy of 1 KB every 18 cycles, so a slab's copies sent together stop their wave for as long as its
 //     MFMAs take (117 x 6144 x 4096 in 64 x 48 tiles 12.5 -> 10.6 us).
-//   * How a CU is filled (BLOCKS per CU): one block of eight waves with the whole LDS, whose waves cover each other's waits (the same
+//   * How a CU is filled (BLOCKS per CU): one block of eight waves with the whole LDS, all on one tile where there is one for each CU (the same
 //     shape 10.2 us); or two, three or four blocks of four waves on a share of it, so that one block's start and end hide
 //     behind another's loop (432 x 3648 x 2432 in 64 x 64 tiles 16.3 -> 12.5 us, 730 x 1824 x 1536 12.1 -> 9.3).
 //   * Epilogue: partial sums to LDS as [token][column], a thread adds them (in wave order) for eight columns of a token,
@@ -36,11 +36,11 @@ namespace maxfp8 {
 // BLOCKS blocks per CU: their waves and their share of its LDS
 __host__ __device__ constexpr int mid_waves(int blocks) { return blocks == 1 ? 8 : 4; }
 __host__ __device__ constexpr int mid_lds(int blocks) { return (blocks == 1 ? 160 : blocks == 2 ? 79 : blocks == 3 ? 53 : 39) * 1024; }
-// Slabs in flight per wave: what the block's LDS holds, the 6-bit wait counter, at most six
+// Slabs in flight per wave: what the block's LDS holds and the 6-bit wait counter counts -- of the shapes below one, or two in the smaller tiles of four waves
 __host__ __device__ constexpr int mid_depth(int mt, int nt, bool blockscale, int blocks) {
   const int groups = blockscale ? (mt + 3) / 4 : 0, slot = (mt + nt) * 2048 + 256 * groups, per = 2 * (mt + nt) + groups;
-  const int lds = (mid_lds(blocks) - 16 * mt * 8) / mid_waves(blocks) / slot, counter = 63 / per + 1, least = lds < counter ? lds : counter;
-  return least > 6 ? 6 : least;
+  const int lds = (mid_lds(blocks) - 16 * mt * 8) / mid_waves(blocks) / slot, counter = 63 / per + 1;
+  return lds < counter ? lds : counter;
 }
 
 template <int MT, int NT, bool BLOCKSCALE, int BLOCKS>

@@ -734,14 +734,13 @@ bool gemm_skinny_preferred(int64_t M, int64_t N, int64_t K) {
   return M <= 64 && small_weights;
 }
 
-// Estimated microseconds at 17 to 32 rows, fitted to 700 matmuls with the weights from memory and, with less weight, in the memory-side cache: within 3 per cent
+// Estimated microseconds at 17 to 32 rows with row scales, fitted to 700 matmuls with the weights from memory and, with less weight, in the memory-side cache: within 3 per cent
 // for half of the launches, 7 for nine in ten.  *alone: a CU has one block, of at most 32 weight rows
-float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool* alone) {
+float gemm_skinny_cost(int64_t M, int64_t N, int64_t K, bool* alone) {
   const int ntw = skinny_shape(M, N, K) / 1000;
   const int64_t per_cu = ceil_div(ceil_div(N, 16 * ntw), (int64_t)compute_units());
   *alone = per_cu == 1 && ntw <= 2;
   const float blocks = (float)per_cu, k = (float)K * 1e-4f, weights = (float)N * (float)K * 1e-6f;
-  if (blockscale) return 2.70f + blocks * (0.81f + (3.26f * (float)ntw + 0.88f + 0.195f * (float)M) * k) + 0.026f * weights;
   return 3.07f + blocks * (0.76f + (3.32f * (float)ntw + 0.42f + 0.192f * (float)M) * k) + 0.025f * weights;
 }
 

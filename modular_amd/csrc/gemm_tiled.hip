@@ -2017,7 +2017,7 @@ static float w4_plan_cost(int64_t M, int64_t N, int64_t K, bool blockscale, int 
   if (!split) return alone && tiles < slots && N * K >= ((int64_t)1 << 26) ? (float)nslab * kW4SlabBlock[tm - 4] + kW4Tile : persistent_cost(tiles, slots, t);
   const W4Split sp = gemm_w4_split(M, N, K, tm);
   const float pieces = (float)ceil_div(nslab, sp.unit);
-  if (tiles * 2 <= slots)  // (fitted like gemm_mid_shape's estimates: within 5 per cent for nine launches in ten of 128-row tiles, 13 of taller ones)
+  if (tiles * 2 <= slots)  // (fitted with the weights from memory, which gemm_mid_shape's estimates are not: within 5 per cent for nine launches in ten of 128-row tiles, 13 of taller ones)
     return (blockscale ? 10.5f : 13.0f) + (blockscale ? kW4CutSlabBlock : kW4CutSlabRow)[tm - 4] * (float)sp.unit + 0.886f * pieces + 0.659f * (float)N * (float)K / 6e6f;
   return (float)(tiles / sp.blocks) * t + (float)sp.unit * t_slab + kW4Tile + kW4HandOver + kW4HandOverPiece * (pieces - 1.f);
 }
