@@ -12,6 +12,8 @@
 //     128 outputs, scales transposed (max/kernels/src/shmem/ep_comm.mojo:4409-4500, 4505-4624).
 //     Note the quantiser of this op: scale = max(amax, 1e-4) / 448 and out / scale (a division),
 //     not the min(amax, ub) / 448 and x * (1 / scale) of quantize_dynamic_scaled_fp8.
+#include <type_traits>
+
 #include "common.h"
 
 namespace maxfp8 {
@@ -316,55 +318,86 @@ __device__ __forceinline__ float div_by(float a, float b, float y) {
   return a == 0.0f ? q0 : q;  // (keeps the sign of a zero quotient)
 }
 __device__ __forceinline__ bool div_b_ok(float b) {
-  return b >= 0x1p-63f && b < 0x1p64f && (__float_as_uint(b) & 0x007fffffu) != 0x007fffffu;
+  return (b >= 0x1p-63f) & (b < 0x1p64f) & ((__float_as_uint(b) & 0x007fffffu) != 0x007fffffu);
 }
 __device__ __forceinline__ bool div_q_ok(float a, float q) {
-  return a == 0.0f || (fabsf(a) >= 0x1p-63f && fabsf(q) >= 0x1p-63f && fabsf(q) < 0x1p64f);
+  return (a == 0.0f) | ((fabsf(a) >= 0x1p-63f) & (fabsf(q) >= 0x1p-63f) & (fabsf(q) < 0x1p64f));
 }
-// Eight quotients a[j] / b[j] (SHARED: one divisor b[0] for all) with one test for the lane and one branch for the wave
-template <bool SHARED>
-__device__ __forceinline__ void exact_div8(const float (&a)[8], const float (&b)[8], float (&q)[8]) {
-  bool ok = true;
-  float y = 0.f;
-  if constexpr (SHARED) {
-    y = refined_rcp(b[0]);
-    ok = div_b_ok(b[0]);
-  }
+// Eight quotients a[j] / b by one divisor, with one test for the lane and one branch for the wave
+__device__ __forceinline__ void exact_div8(const float (&a)[8], float b, float (&q)[8]) {
+  const float y = refined_rcp(b);
+  bool ok = div_b_ok(b);
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    if constexpr (!SHARED) {
-      y = refined_rcp(b[j]);
-      ok = ok && div_b_ok(b[j]);
-    }
-    q[j] = div_by(a[j], b[SHARED ? 0 : j], y);
-    ok = ok && div_q_ok(a[j], q[j]);
+    q[j] = div_by(a[j], b, y);
+    ok = ok & div_q_ok(a[j], q[j]);
   }
   if (__builtin_amdgcn_ballot_w64(!ok) != 0ull) {
     if (!ok) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) q[j] = a[j] / b[SHARED ? 0 : j];
+      for (int j = 0; j < 8; ++j) q[j] = a[j] / b;
     }
   }
 }
 
-// gate / (1 + exp(-gate)) * up, every step rounded to f32 (ep_comm.mojo:4494-4497), for eight outputs.
-// (1 + exp(-gate) = inf, gate < -88: outside the fast division's range, and gate / inf = -0 is what the IEEE division gives)
+__device__ __forceinline__ void unpack_bf16x8(const uint4& v, float (&f)[8]) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    f[2 * j] = __uint_as_float(w[j] << 16);
+    f[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
+  }
+}
+
+__device__ __forceinline__ uint4 pack_bf16x8(const float (&f)[8]) {
+  return make_uint4(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7]));
+}
+
+// gate / (1 + exp(-gate)), every step rounded to f32 (ep_comm.mojo:4494-4497), of eight gates that are bf16 values.
+//   BF16 = false: the bits of expf and the IEEE division in 13 instructions instead of 30.  log2(e) comes in two parts, the first of
+//     16 bits, whose product t with the gate's 8 is exact: the argument of the power of two has one rounding and no range checks.  The
+//     quotient is corrected once by its exact residual (v_div_fixup: signed zeros, NaN).
+//   BF16 = true, for a caller that rounds the result to bf16: 7 instructions, some ulp of f32 away, which bf16 does not show.
+// Gates of 86 and beyond, where the exponential leaves the range, and infinities take expf and the division, in a branch the wave
+// skips unless one of its lanes needs it.  (There are 65536 gates: all of them have been compared with that path, BF16 after
+// the rounding: the same bits.)
+template <bool BF16>
+__device__ __forceinline__ void silu8(const uint4& bits, const float (&gate)[8], float (&sig)[8]) {
+  constexpr float kHi = 0x1.7154p+0f, kLo = (float)(1.4426950408889634074 - 0x1.7154p+0);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    if constexpr (BF16) {
+      sig[j] = gate[j] * refined_rcp(1.0f + __builtin_amdgcn_exp2f(gate[j] * -1.4426950408889634074f));
+    } else {
+      const float t = gate[j] * -kHi, n = rintf(t);
+      const float d = 1.0f + ldexpf(__builtin_amdgcn_exp2f(fmaf(gate[j], -kLo, t - n)), (int)n);
+      const float y = __builtin_amdgcn_rcpf(d), q0 = gate[j] * y;
+      sig[j] = __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q0, gate[j]), y, q0), d, gate[j]);
+    }
+  }
+  // (compared as integers, two a word: a NaN is larger than every number, where a float maximum may lose the largest to it)
+  typedef unsigned short u2 __attribute__((ext_vector_type(2)));
+  auto size = [](uint32_t w) { return __builtin_bit_cast(u2, w & 0x7fff7fffu); };
+  const u2 most = __builtin_elementwise_max(__builtin_elementwise_max(size(bits.x), size(bits.y)), __builtin_elementwise_max(size(bits.z), size(bits.w)));
+  const bool beyond = (most.x >= 0x42acu) | (most.y >= 0x42acu);
+  if (__builtin_amdgcn_ballot_w64(beyond) != 0ull) {
+    if (beyond) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sig[j] = gate[j] / (1.0f + expf(-gate[j]));
+    }
+  }
+}
+
+// silu(gate) * up for eight outputs.
 // ROUND_ACT: the activation is rounded to bf16 before the product, as where silu and the multiplication are two bf16
 // operations (the dense gated MLP, max/python/max/nn/linear.py:1072: ops.silu(gate) * up).
 template <bool ROUND_ACT>
-__device__ __forceinline__ void silu_mul8(const float (&gate)[8], const float (&up)[8], float (&f)[8]) {
-  float d[8], sig[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) d[j] = 1.0f + expf(-gate[j]);
-  exact_div8<false>(gate, d, sig);
-  if constexpr (ROUND_ACT) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t w = pack_bf16x2(sig[2 * j], sig[2 * j + 1]);
-      sig[2 * j] = __uint_as_float(w << 16);
-      sig[2 * j + 1] = __uint_as_float(w & 0xffff0000u);
-    }
-  }
+__device__ __forceinline__ void silu_mul8(const uint4& gate_bits, const uint4& up_bits, float (&f)[8]) {
+  float gate[8], up[8], sig[8];
+  unpack_bf16x8(gate_bits, gate);
+  unpack_bf16x8(up_bits, up);
+  silu8<ROUND_ACT>(gate_bits, gate, sig);
+  if constexpr (ROUND_ACT) unpack_bf16x8(pack_bf16x8(sig), sig);
 #pragma unroll
   for (int j = 0; j < 8; ++j) f[j] = sig[j] * up[j];
 }
@@ -385,25 +418,16 @@ __device__ __forceinline__ uint2 pack_e4m3fn8(const float (&q)[8]) {
   hi = cvt_pk_e4m3fn(q[6], q[7], hi, true);
   return make_uint2((uint32_t)lo, (uint32_t)hi);
 }
-__device__ __forceinline__ void unpack_bf16x8(const uint4& v, float (&f)[8]) {
-  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    f[2 * j] = __uint_as_float(w[j] << 16);
-    f[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
-  }
-}
-__device__ __forceinline__ uint4 pack_bf16x8(const float (&f)[8]) {
-  return make_uint4(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7]));
-}
 
-// 16 lanes own 128 consecutive outputs of one row (8 each): one 16-byte load of gate and of up
-// per lane; quantised: amax over the 16 lanes by DPP, 8-byte packed fp8 store, lane 0 writes the scale.
-// Bound by the bytes (5 per output where the result is quantised) with the exponential and the division close behind.  Graph
-// timing, operands cold: 2048 x 14336 as kSiluBf16 and the quantiser behind it 46.7 us, as kSiluBf16Quant 35.9 (147 MB:
-// 4.1 TB/s); 32768 x 2048 104.6 and 80; 16 x 14336 6.5 and 3.7.
-template <SiluOut OUT, bool ROUND_ACT>
-__global__ __launch_bounds__(256) void fused_silu_bf16_kernel(void* __restrict__ out, float* __restrict__ scales,
+// A block takes tiles of ROWS rows x U groups of 128 outputs: 16 lanes own a row's group (8 outputs each, one 16-byte load of gate
+// and of up per lane), a thread the tile's U groups of its row, whose loads go out together; quantised: amax over the 16 lanes by
+// DPP, 8-byte packed fp8 store.  A group's scales leave as ROWS consecutive floats: with 32 rows a whole line, which no other XCD's L2
+// holds a part of (32768 x 2048: 16 groups of a row per block, every scale alone, 73 us; 4 rows 113; 16 rows 68; 32 rows 62).
+// Bound by the bytes (5 per output where the result is quantised) and, as close, by the arithmetic: 30 instructions per output, two of
+// them four times as long.  Graph timing, operands cold, before this form and now: 2048 x 14336 rounding twice and quantising 45 -> 32 us
+// (147 MB: 4.6 TB/s), 32768 x 2048 rounding once 82 -> 65, 512 x 14336 13 -> 10, 16 x 14336 3.6 -> 2.7.
+template <SiluOut OUT, bool ROUND_ACT, int ROWS, int U>
+__global__ __launch_bounds__(16 * ROWS) void fused_silu_bf16_kernel(void* __restrict__ out, float* __restrict__ scales,
                                                               const uint16_t* __restrict__ in,
                                                               const uint32_t* __restrict__ row_offsets, int num_offsets,
                                                               int64_t max_rows, int inter, int64_t in_stride,
@@ -412,51 +436,62 @@ __global__ __launch_bounds__(256) void fused_silu_bf16_kernel(void* __restrict__
   // turn into accesses outside them)
   const uint32_t rows_dev = row_offsets[num_offsets - 1];
   const int64_t rows = (int64_t)rows_dev < max_rows ? (int64_t)rows_dev : max_rows;
-  const int groups = inter >> 7;
+  const uint32_t groups = (uint32_t)inter >> 7, nxb = (groups + U - 1) / U;
+  const uint32_t tiles = (uint32_t)((rows + ROWS - 1) / ROWS) * nxb;  // (an output is 4 bytes of input and more: far below 2^32)
   const int tid = threadIdx.x, sub = tid & 15;
-  const int64_t total = rows * groups;
-  const bool narrow = total < ((int64_t)1 << 31);
-  for (int64_t item = (int64_t)blockIdx.x * 16 + (tid >> 4); item < total; item += (int64_t)gridDim.x * 16) {
-    // (a 64-bit division is half as many instructions as the item's arithmetic)
-    const int64_t m = narrow ? (int64_t)((uint32_t)item / (uint32_t)groups) : item / groups;
-    const int g = (int)(item - m * groups);
-    const uint16_t* src = in + m * in_stride + g * 128 + sub * 8;
-    float gate[8], up[8], f[8];
-    const uint4 gv = *reinterpret_cast<const uint4*>(src);
-    const uint4 uv = *reinterpret_cast<const uint4*>(src + inter);
-    unpack_bf16x8(gv, gate);
-    unpack_bf16x8(uv, up);
-    silu_mul8<ROUND_ACT>(gate, up, f);
-    if constexpr (OUT == kSiluBf16) {
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out) + m * out_stride + g * 128 + sub * 8) = pack_bf16x8(f);
-    } else {
-      if constexpr (OUT == kSiluBf16Quant) unpack_bf16x8(pack_bf16x8(f), f);
-      float amax = 0.0f;
+  for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const uint32_t rb = tile / nxb, g0 = (tile - rb * nxb) * U;
+    const int64_t row = (int64_t)rb * ROWS + (tid >> 4);
+    const bool row_ok = row < rows;
+    const uint16_t* src = in + row * in_stride + g0 * 128u + sub * 8;
+    uint4 gate[U], up[U];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(f[j]));
-      amax = row16_max(amax);
-      float scale, q[8];
-      if constexpr (OUT == kSiluQuant) {
-        scale = fmaxf(amax, 1e-4f) / 448.0f;
-        const float divisor[8] = {scale, scale, scale, scale, scale, scale, scale, scale};
-        exact_div8<true>(f, divisor, q);   // (one reciprocal and one test of the divisor for the lane's eight quotients)
-      } else {
-        float recip;
-        dynamic_scale_f32(amax, scale_ub, scale, recip);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) q[j] = f[j] * recip;
+    for (int u = 0; u < U; ++u) {
+      gate[u] = up[u] = make_uint4(0, 0, 0, 0);
+      if (row_ok && g0 + u < groups) {
+        gate[u] = *reinterpret_cast<const uint4*>(src + u * 128);
+        up[u] = *reinterpret_cast<const uint4*>(src + u * 128 + inter);
       }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) q[j] = clamp448(q[j]);
-      *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(out) + m * out_stride + g * 128 + sub * 8) = pack_e4m3fn8(q);
-      if (sub == 0) scales[(int64_t)g * scales_ld + m] = scale;
     }
+    const int64_t at = row * out_stride + g0 * 128u + sub * 8;
+    float my_scale = 0.0f;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool live = row_ok && g0 + u < groups;
+      float f[8];
+      silu_mul8<ROUND_ACT>(gate[u], up[u], f);
+      if constexpr (OUT == kSiluBf16) {
+        if (live) *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out) + at + u * 128) = pack_bf16x8(f);
+      } else {
+        if constexpr (OUT == kSiluBf16Quant) unpack_bf16x8(pack_bf16x8(f), f);
+        float amax = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(f[j]));
+        amax = row16_max(amax);
+        float scale, q[8];
+        if constexpr (OUT == kSiluQuant) {
+          scale = fmaxf(amax, 1e-4f) / 448.0f;
+          exact_div8(f, scale, q);
+        } else {
+          float recip;
+          dynamic_scale_f32(amax, scale_ub, scale, recip);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) q[j] = f[j] * recip;
+        }
+        if (sub == u) my_scale = scale;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = clamp448(q[j]);
+        if (live) *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(out) + at + u * 128) = pack_e4m3fn8(q);
+      }
+    }
+    if (OUT != kSiluBf16 && row_ok && sub < U && g0 + sub < groups) scales[(int64_t)(g0 + sub) * scales_ld + row] = my_scale;
   }
 }
 
 // The same with one scale per row (per-token quantisation of the bf16 product): one block per row, NV 16-byte vectors of
 // bf16 products per thread stay in registers between the amax and the convert pass; inter <= THREADS * 8 * NV.
-// 2048 x 14336: 45.6 us as two kernels, 38.0 as one; 32768 x 2048 (256 threads: every one has its vector) 105 and 79.
+// 2048 x 14336: 45.6 us as two kernels, 28 as one; 32768 x 2048 (256 threads: every one has its vector) 105 and 58.  (As one with expf and
+// the IEEE division 38 and 79.)
 template <int THREADS, int NV, bool ROUND_ACT>
 __global__ __launch_bounds__(THREADS) void fused_silu_row_quant_kernel(uint8_t* __restrict__ out, float* __restrict__ scales,
                                                                                const uint16_t* __restrict__ in,
@@ -478,10 +513,8 @@ __global__ __launch_bounds__(THREADS) void fused_silu_row_quant_kernel(uint8_t* 
     const int idx = tid + i * THREADS;
     h[i] = make_uint4(0, 0, 0, 0);
     if (idx < nvec) {
-      float gate[8], up[8], f[8];
-      unpack_bf16x8(gate_row[idx], gate);
-      unpack_bf16x8(up_row[idx], up);
-      silu_mul8<ROUND_ACT>(gate, up, f);
+      float f[8];
+      silu_mul8<ROUND_ACT>(gate_row[idx], up_row[idx], f);
       h[i] = pack_bf16x8(f);
       unpack_bf16x8(h[i], f);
 #pragma unroll
@@ -537,20 +570,29 @@ int fused_silu_dispatch(void* out, float* scales, const void* in, const uint32_t
     if (!ok) MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "fused_silu: one scale per row takes rows of at most 32768 outputs");
     return launch_status("fused_silu_quantized (row)");
   }
-  // the number of rows in use is only known on the device: the grid is sized for max_rows and
-  // walks the items in strides
-  const int64_t items = max_rows * (inter / 128);
-  const unsigned blocks = (unsigned)(ceil_div(items, 16) < 8192 ? ceil_div(items, 16) : 8192);
-  auto launch = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, stream, out, scales, (const uint16_t*)in, row_offsets, (int)num_offsets, max_rows,
-                       (int)inter, in_stride, out_stride, scales_ld, scale_ub);
+  // The number of rows in use is only known on the device: the grid is sized for max_rows and walks the tiles in strides.  Tiles of
+  // 32 rows x 2 groups, or of 16 x 1 where those would leave half of the CUs without one (16 x 14336 3.2 and 2.7 us, 333 x 1408 3.3 and
+  // 2.7, 128 x 14336 3.7 and 5.0).
+  const int64_t large = ceil_div(max_rows, 32) * ceil_div(inter / 128, 2);
+  auto launch = [&](auto kern, int rows, int64_t tiles) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)(tiles < 16384 ? tiles : 16384)), dim3(16 * rows), 0, stream, out, scales, (const uint16_t*)in, row_offsets,
+                       (int)num_offsets, max_rows, (int)inter, in_stride, out_stride, scales_ld, scale_ub);
   };
+  auto either = [&](auto out_c, auto round_c) {
+    constexpr SiluOut OUT = decltype(out_c)::value;
+    constexpr bool ROUND_ACT = decltype(round_c)::value;
+    if (large >= 128) launch(fused_silu_bf16_kernel<OUT, ROUND_ACT, 32, 2>, 32, large);
+    else launch(fused_silu_bf16_kernel<OUT, ROUND_ACT, 16, 1>, 16, ceil_div(max_rows, 16) * (inter / 128));
+  };
+  constexpr std::integral_constant<SiluOut, kSiluBf16> plain{};
+  constexpr std::integral_constant<SiluOut, kSiluQuant> quant{};
+  constexpr std::integral_constant<SiluOut, kSiluBf16Quant> bf16_quant{};
   switch (mode) {
-    case 1: launch(fused_silu_bf16_kernel<kSiluQuant, false>); break;
-    case 2: launch(fused_silu_bf16_kernel<kSiluBf16, true>); break;
-    case 3: launch(fused_silu_bf16_kernel<kSiluBf16Quant, false>); break;
-    case 4: launch(fused_silu_bf16_kernel<kSiluBf16Quant, true>); break;
-    default: launch(fused_silu_bf16_kernel<kSiluBf16, false>); break;
+    case 1: either(quant, std::false_type{}); break;
+    case 2: either(plain, std::true_type{}); break;
+    case 3: either(bf16_quant, std::false_type{}); break;
+    case 4: either(bf16_quant, std::true_type{}); break;
+    default: either(plain, std::false_type{}); break;
   }
   return launch_status(mode == 0 || mode == 2 ? "fused_silu" : "fused_silu_quantized");
 }
