@@ -101,6 +101,23 @@ __device__ __forceinline__ float scale_at(const float* base, int64_t idx, int dt
   return (float)__builtin_bit_cast(_Float16, h);
 }
 
+// out[i] = element at(i) of such a vector, for N of them.  The type is asked for once, in front of all loads: asked for load by load it made a
+// chain of loads that each waited for the one before, 38 of them in front of a 192 x 256 tile's stores (linears with row scales and the
+// quantiser, graph timing: 1777 x 6144 x 4096 46.7 -> 44.4 us, 1024 x 6144 x 4096 34.0 -> 30.8, 100 x 28672 x 4096 30.9 -> 28.5, 48 x 4096 x 4096 8.8 -> 7.6).
+template <int N, class At>
+__device__ __forceinline__ void scales_at(float (&out)[N], const float* base, int dtype, At at) {
+  if (dtype == 2 /* MAXFP8_F32 */) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) out[i] = base[at(i)];
+    return;
+  }
+  uint16_t h[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) h[i] = reinterpret_cast<const uint16_t*>(base)[at(i)];
+#pragma unroll
+  for (int i = 0; i < N; ++i) out[i] = dtype == 0 /* MAXFP8_BF16 */ ? __uint_as_float((uint32_t)h[i] << 16) : (float)__builtin_bit_cast(_Float16, h[i]);
+}
+
 // offsets (elements from k_base / v_base) of the cache rows that receive rows m[0..R); -1 for a
 // row that is not live or that the lookup table has no page for (nothing is stored then).  The R
 // binary searches run in lockstep with a trip count that only depends on the batch size, so

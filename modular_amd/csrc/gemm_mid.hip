@@ -58,8 +58,8 @@ struct MidCfg {
   static_assert(MT <= 4 && NT <= 4 && DEPTH >= 1 && SMEM <= mid_lds(BLOCKS));
 };
 
-// Where the copies of a slab read.  A slab past the wave's share fetches nothing (and writes zeros), so the counts stay exact.
-struct MidSlabAt { uint32_t koff, kill, kill_s, scales; };
+// Where the copies of a slab read
+struct MidSlabAt { uint32_t koff, kill, scales; };
 
 // KV: the fused QKV projection's epilogue and its wave of page look-ups
 template <int MT, int NT, bool BLOCKSCALE, int W_POLICY, int BLOCKS, bool KV>
@@ -125,12 +125,10 @@ __global__ __launch_bounds__((BLOCKS == 1 ? 512 : 256) + (KV ? 64 : 0)) __attrib
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
       const int item = it * NWAVES * 64 + tid, row = item / CHUNKS, col = (item - row * CHUNKS) * 8;
-      row_s[it] = scale_at(p.a_scales, (int64_t)(m0 + (row < rows_here ? row : 0)) * p.a_scale_stride, p.scales_dtype);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int n = n0 + col + i;
-        col_s[it][i] = scale_at(p.b_scales, (int64_t)(n < p.N ? n : p.N - 1) * p.b_scale_stride, p.scales_dtype);
-      }
+      scales_at(col_s[it], p.b_scales, p.scales_dtype, [&](int i) { return (int64_t)(n0 + col + i < p.N ? n0 + col + i : p.N - 1) * p.b_scale_stride; });
+      float one[1];
+      scales_at(one, p.a_scales, p.scales_dtype, [&](int) { return (int64_t)(m0 + (row < rows_here ? row : 0)) * p.a_scale_stride; });
+      row_s[it] = one[0];
     }
   }
 
@@ -141,13 +139,10 @@ __global__ __launch_bounds__((BLOCKS == 1 ? 512 : 256) + (KV ? 64 : 0)) __attrib
     for (int j = 0; j < NT; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
   auto slab_at = [&](int slab) {
-    const bool live = slab < s_end;
-    const int sl = live ? slab : s_begin;
     MidSlabAt at;
-    at.koff = __builtin_amdgcn_readfirstlane((uint32_t)sl * 128u);
-    at.kill = at.kill_s = live ? 0u : 0x80000000u;
-    if (k_tail && at.koff + cchunk * 16 >= (uint32_t)p.K) at.kill = 0x80000000u;
-    at.scales = (uint32_t)sl * (uint32_t)p.a_scales_ld * 4u;
+    at.koff = __builtin_amdgcn_readfirstlane((uint32_t)slab * 128u);
+    at.kill = k_tail && at.koff + cchunk * 16 >= (uint32_t)p.K ? 0x80000000u : 0u;
+    at.scales = (uint32_t)slab * (uint32_t)p.a_scales_ld * 4u;
     return at;
   };
   // copy i (0 .. PER - 1, known at compile time) of a slab into slot d: weight rows, token rows, token scales
@@ -158,10 +153,14 @@ __global__ __launch_bounds__((BLOCKS == 1 ? 512 : 256) + (KV ? 64 : 0)) __attrib
     else if (i < 2 * (NT + MT))
       __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (lds_ptr_t)(slot + i * 1024), 16, a_voff | at.kill, at.koff + (i - 2 * NT) * a_step, 0, 0);
     else
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(s_rsrc, (lds_ptr_t)(slot + (MT + NT) * 2048), 4, s_voff | at.kill_s, at.scales, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(s_rsrc, (lds_ptr_t)(slot + (MT + NT) * 2048), 4, s_voff, at.scales, 0, 0);
   };
-  auto step = [&](int slab, int d) {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * PER) : "memory");
+  // One slab, in slot d.  REFILLS: slab + DEPTH is one of the wave's too and takes the slot.  behind: DEPTH - 1 slabs are in flight behind this one
+  // (fewer only at the end of the share, where the wait is for everything).
+  auto step = [&](int slab, int d, auto refills_c, bool behind) {
+    constexpr bool REFILLS = decltype(refills_c)::value;
+    if (DEPTH > 1 && behind) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * PER) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const uint8_t* slot = ring + d * SLOT;
     v8i wf[NT], af[MT];
     auto frag = [&](const uint8_t* g) {
@@ -177,7 +176,6 @@ __global__ __launch_bounds__((BLOCKS == 1 ? 512 : 256) + (KV ? 64 : 0)) __attrib
     float b0 = 0.f, b1 = 0.f;
     if constexpr (BLOCKSCALE) {
       as = *reinterpret_cast<const v4f*>(slot + (MT + NT) * 2048 + lm * 16);
-      // (a slab past the share's end multiplies zeros; its scales are finite)
       const int at = __builtin_amdgcn_readfirstlane(slab - s_begin);
       b0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, bs_lo), at));
       b1 = NT == 3 ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, bs_hi), at)) : b0;
@@ -196,7 +194,7 @@ __global__ __launch_bounds__((BLOCKS == 1 ? 512 : 256) + (KV ? 64 : 0)) __attrib
     };
     static_for<NM>([&](auto i_c) {
       constexpr int i = decltype(i_c)::value, mt = i / NT, nt = i % NT, c0 = i * PER / NM, c1 = (i + 1) * PER / NM;
-      static_for<c1 - c0>([&](auto c_c) { copy(next, d, c0 + decltype(c_c)::value); });
+      if constexpr (REFILLS) static_for<c1 - c0>([&](auto c_c) { copy(next, d, c0 + decltype(c_c)::value); });
       if constexpr (BLOCKSCALE) {
         const v4f zero = {0.f, 0.f, 0.f, 0.f};
         part[i % (LAG + 1)] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[nt], af[mt], zero, 0, 0, 0, 0, 0, 0);
@@ -212,22 +210,30 @@ __global__ __launch_bounds__((BLOCKS == 1 ? 512 : 256) + (KV ? 64 : 0)) __attrib
     }
   };
 
-  if (!KV || wave < NWAVES) {
+  if ((!KV || wave < NWAVES) && s_begin < s_end) {
+    // (copies are sent for the wave's own slabs only: those of a slab past its share, of nothing, kept the counts of the waits exact and
+    // took a CU's 18 cycles each all the same, a fifth of the copies of a share of four slabs)
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
+      if (d > 0 && s_begin + d >= s_end) break;
       const MidSlabAt at = slab_at(s_begin + d);
 #pragma unroll
       for (int i = 0; i < PER; ++i) copy(at, d, i);
     }
     if constexpr (BLOCKSCALE)  // (the weight scales are older than the copies: they arrive without waiting for those)
       asm volatile("s_waitcnt vmcnt(%2)" : "+v"(bs_lo), "+v"(bs_hi) : "n"(DEPTH * PER < 63 ? DEPTH * PER : 63));
-    for (int base = s_begin; base < s_end; base += DEPTH) {
+    int slab = s_begin;
+    for (; slab + 2 * DEPTH <= s_end; slab += DEPTH) {
 #pragma unroll
-      for (int d = 0; d < DEPTH; ++d) step(base + d, d);
+      for (int d = 0; d < DEPTH; ++d) step(slab + d, d, std::true_type{}, true);
     }
-    // drain: the last DEPTH copies fetched nothing but still write their slots
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  } else if (lane < BM) {
+    const int left = s_end - slab;  // 1 .. 2 DEPTH - 1
+    static_for<2 * DEPTH - 1>([&](auto t_c) {
+      constexpr int t = decltype(t_c)::value;
+      if (t + 1 < DEPTH && t + DEPTH < left) step(slab + t, t % DEPTH, std::true_type{}, true);
+      else if (t < left) step(slab + t, t % DEPTH, std::false_type{}, t + DEPTH <= left);
+    });
+  } else if (KV && wave >= NWAVES && lane < BM) {
     // fused QKV: a wave of its own looks up the rows' pages.  Its loads depend on one another, a search among the sequences and two
     // more; in one of the other waves each of them waited for all copies in front of it, and the wave's share of K for them
     // (64 tokens of 64 sequences, 10240 x 8192 with row scales, quantiser and the new tiles included: 30.9 -> 30.5 us).

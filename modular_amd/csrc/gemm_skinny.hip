@@ -460,12 +460,13 @@ __global__ __launch_bounds__((NWAVES + skinny_page_waves(MT, KV)) * 64) void gem
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] *= p.x_scale;
     } else if constexpr (!BLOCKSCALE) {
+      float b_s[4];
+      scales_at(b_s, p.b_scales, p.scales_dtype, [&](int i) { return (int64_t)(n + i < p.N ? n + i : p.N - 1) * p.b_scale_stride; });
       const float a_s = QUANT ? a_sc[16 + m] : scale_at(p.a_scales, (int64_t)m * p.a_scale_stride, p.scales_dtype);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int nn = (n + i < p.N) ? n + i : p.N - 1;
         const float t = v[i] * a_s;
-        v[i] = t * scale_at(p.b_scales, (int64_t)nn * p.b_scale_stride, p.scales_dtype);
+        v[i] = t * b_s[i];
       }
     }
     if (p.c_dtype == MAXFP8_BF16) {

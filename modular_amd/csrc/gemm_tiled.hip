@@ -522,24 +522,28 @@ const ScaleRow<TM> a_sc = read_scales<TM>(sa + s_rd);
     if (p.c_dtype == MAXFP8_BF16 && p.c_vec8_ok && n0 + BN <= p.N) {
       __syncthreads();  // every wave has finished reading the stages
       uint8_t* wbuf = smem + wave * (WM * WN * 2);
+      float b_s[TN * 4], a_s_all[TM];
+      if constexpr (!BLOCKSCALE) {
+        scales_at(b_s, p.b_scales, p.scales_dtype, [&](int i) { return (int64_t)(n0 + wn * WN + (i >> 3) * 32 + lq * 8 + (i & 7)) * p.b_scale_stride; });
+        scales_at(a_s_all, p.a_scales, p.scales_dtype, [&](int mt) {
+          const int64_t mm = row_begin + wm * WM + mt * 16 + lm;
+          return (mm < p.M ? mm : p.M - 1) * p.a_scale_stride;
+        });
+      }
 #pragma unroll
       for (int mt = 0; mt < TM; ++mt) {
         const int r = mt * 16 + lm;
         float a_s = 1.f;
-        if constexpr (!BLOCKSCALE) {
-          const int64_t mm = row_begin + wm * WM + r;
-          a_s = scale_at(p.a_scales, (mm < p.M ? mm : p.M - 1) * p.a_scale_stride, p.scales_dtype);
-        }
+        if constexpr (!BLOCKSCALE) a_s = a_s_all[mt];
 #pragma unroll
         for (int q = 0; q < TN / 2; ++q) {
           v4f lo = acc[mt][2 * q], hi = acc[mt][2 * q + 1];
           if constexpr (!BLOCKSCALE) {
-            const int n = n0 + wn * WN + q * 32 + lq * 8;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               const float t_lo = lo[i] * a_s, t_hi = hi[i] * a_s;
-              lo[i] = t_lo * scale_at(p.b_scales, (int64_t)(n + i) * p.b_scale_stride, p.scales_dtype);
-              hi[i] = t_hi * scale_at(p.b_scales, (int64_t)(n + 4 + i) * p.b_scale_stride, p.scales_dtype);
+              lo[i] = t_lo * b_s[q * 8 + i];
+              hi[i] = t_hi * b_s[q * 8 + 4 + i];
             }
           }
           const int chunk = (q * 4 + lq) ^ (r & 7);
@@ -559,6 +563,17 @@ const ScaleRow<TM> a_sc = read_scales<TM>(sa + s_rd);
       return;
     }
   }
+  float b_s[TN * 4], a_s_all[TM];
+  if constexpr (!BLOCKSCALE) {
+    scales_at(b_s, bs_ptr, p.scales_dtype, [&](int i) {  // (bs_ptr: this expert's scales when grouped)
+      const int n = n0 + wn * WN + (i >> 3) * 32 + lq * 8 + (i & 7);
+      return (int64_t)(n < p.N ? n : p.N - 1) * p.b_scale_stride;
+    });
+    scales_at(a_s_all, p.a_scales, p.scales_dtype, [&](int mt) {
+      const int ml = wm * WM + mt * 16 + lm;
+      return (row_begin + (ml < rows_here ? ml : 0)) * p.a_scale_stride;
+    });
+  }
 #pragma unroll
   for (int mt = 0; mt < TM; ++mt) {
     const int ml = wm * WM + mt * 16 + lm;
@@ -568,7 +583,7 @@ const ScaleRow<TM> a_sc = read_scales<TM>(sa + s_rd);
     if constexpr (GROUPED)
       if (p.c_row_index) cm = p.c_row_index[m];
     float a_s = 1.f;
-    if constexpr (!BLOCKSCALE) a_s = scale_at(p.a_scales, m * p.a_scale_stride, p.scales_dtype);
+    if constexpr (!BLOCKSCALE) a_s = a_s_all[mt];
 #pragma unroll
     for (int q = 0; q < TN / 2; ++q) {
       const int n = n0 + wn * WN + q * 32 + lq * 8;
@@ -577,11 +592,9 @@ const ScaleRow<TM> a_sc = read_scales<TM>(sa + s_rd);
       if constexpr (!BLOCKSCALE) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int n_lo = (n + i < p.N) ? n + i : p.N - 1;
-          const int n_hi = (n + 4 + i < p.N) ? n + 4 + i : p.N - 1;
           const float t_lo = lo[i] * a_s, t_hi = hi[i] * a_s;
-          lo[i] = t_lo * scale_at(bs_ptr, (int64_t)n_lo * p.b_scale_stride, p.scales_dtype);  // (bs_ptr: this expert's scales when grouped)
-          hi[i] = t_hi * scale_at(bs_ptr, (int64_t)n_hi * p.b_scale_stride, p.scales_dtype);
+          lo[i] = t_lo * b_s[q * 8 + i];
+          hi[i] = t_hi * b_s[q * 8 + 4 + i];
         }
       }
       store8(cm, n, lo, hi);
@@ -981,16 +994,10 @@ const ScaleRow<TM> a_sc = read_scales<TM>(sa + s_rd);
       // ---- the tile leaves, 16 rows of the wave's part at a time
       // (row scaling: every scale of the tile is loaded before the first store, so that no later wait for a
       // load also waits for the stores in front of it)
-      float b_s[TN / 2][8], a_s_all[TM];
+      float b_s[TN * 4], a_s_all[TM];
       if constexpr (!BLOCKSCALE) {
-#pragma unroll
-        for (int q = 0; q < TN / 2; ++q)
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            b_s[q][i] = scale_at(p.b_scales, (int64_t)(tn * BN + wn * WN + q * 32 + lq * 8 + i) * p.b_scale_stride, p.scales_dtype);
-#pragma unroll
-        for (int mt = 0; mt < TM; ++mt)
-          a_s_all[mt] = scale_at(p.a_scales, ((int64_t)tm * BM + wm * WM + mt * 16 + lm) * p.a_scale_stride, p.scales_dtype);
+        scales_at(b_s, p.b_scales, p.scales_dtype, [&](int i) { return (int64_t)(tn * BN + wn * WN + (i >> 3) * 32 + lq * 8 + (i & 7)) * p.b_scale_stride; });
+        scales_at(a_s_all, p.a_scales, p.scales_dtype, [&](int mt) { return ((int64_t)tm * BM + wm * WM + mt * 16 + lm) * p.a_scale_stride; });
         asm volatile("" ::: "memory");
       }
       // (C goes out through a buffer descriptor: one 32-bit lane offset for all of a lane's stores, the rest scalar)
@@ -1006,8 +1013,8 @@ const ScaleRow<TM> a_sc = read_scales<TM>(sa + s_rd);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               const float t_lo = lo[i] * a_s, t_hi = hi[i] * a_s;
-              lo[i] = t_lo * b_s[q][i];
-              hi[i] = t_hi * b_s[q][4 + i];
+              lo[i] = t_lo * b_s[q * 8 + i];
+              hi[i] = t_hi * b_s[q * 8 + 4 + i];
             }
           }
           // (written and read back through the same vector type: to the compiler a store through one type and a load
@@ -1367,6 +1374,14 @@ __device__ __forceinline__ void grouped_stream_body(const GemmArgs& p, uint8_t* 
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last issues were out of range, but they still target the ring
 
   // lane (lm, lq) holds rows 4 * lq .. + 3 of a 16-row weight group for token lm: four consecutive columns of C
+  float b_s[NTW * 4], a_s_all[MT];
+  if constexpr (!BLOCKSCALE) {
+    scales_at(b_s, bs_ptr, p.scales_dtype, [&](int i) {
+      const int n = nw + (i >> 2) * 16 + lq * 4 + (i & 3);
+      return (int64_t)(n < p.N ? n : p.N - 1) * p.b_scale_stride;
+    });
+    scales_at(a_s_all, p.a_scales, p.scales_dtype, [&](int mt) { return (row_begin + (mt * 16 + lm < rows_here ? mt * 16 + lm : 0)) * p.a_scale_stride; });
+  }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int ml = mt * 16 + lm;
@@ -1374,7 +1389,7 @@ __device__ __forceinline__ void grouped_stream_body(const GemmArgs& p, uint8_t* 
     const int64_t m = row_begin + ml;
     const int64_t cm = p.c_row_index ? (int64_t)p.c_row_index[m] : m;
     float a_s = 1.f;
-    if constexpr (!BLOCKSCALE) a_s = scale_at(p.a_scales, m * p.a_scale_stride, p.scales_dtype);
+    if constexpr (!BLOCKSCALE) a_s = a_s_all[mt];
 #pragma unroll
     for (int nt = 0; nt < NTW; ++nt) {
       const int n = nw + nt * 16 + lq * 4;
@@ -1383,9 +1398,8 @@ __device__ __forceinline__ void grouped_stream_body(const GemmArgs& p, uint8_t* 
       if constexpr (!BLOCKSCALE) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int nn = (n + i < p.N) ? n + i : p.N - 1;
           const float t = v[i] * a_s;
-          v[i] = t * scale_at(bs_ptr, (int64_t)nn * p.b_scale_stride, p.scales_dtype);
+          v[i] = t * b_s[nt * 4 + i];
         }
       }
       if (p.c_dtype == MAXFP8_BF16) {
@@ -1805,10 +1819,12 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmArgs p) {
       const int64_t n = i - m * p.N;
       if constexpr (!BLOCKSCALE) {
         const float a_s = scale_at(p.a_scales, m * p.a_scale_stride, p.scales_dtype);
+        float b_s[4];
+        scales_at(b_s, p.b_scales, p.scales_dtype, [&](int j) { return (n + j) * p.b_scale_stride; });
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const float r = v[j] * a_s;
-          v[j] = r * scale_at(p.b_scales, (n + j) * p.b_scale_stride, p.scales_dtype);
+          v[j] = r * b_s[j];
         }
       }
       if (p.c_dtype == MAXFP8_BF16)

@@ -789,7 +789,7 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
     // ---- the tile leaves, 16 rows x 64 columns of the wave's part at a time
     // (row scaling: every scale of the tile is loaded before the first store, so that no later wait for a load also
     // waits for the stores in front of it)
-    float b_s[TN / 2][8], a_s_all[TM];
+    float b_s[TN * 4], a_s_all[TM];  // (b_s: eight of each pair of fragments)
     [[maybe_unused]] uint32_t bias[TN / 2][4];  // (two bf16 a word)
     if constexpr (KV) {
       if (p.kv.bias) {
@@ -803,23 +803,17 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
       }
     }
     if constexpr (!BLOCKSCALE) {
-#pragma unroll
-      for (int q = 0; q < TN / 2; ++q)
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          b_s[q][i] = scale_at(p.b_scales, (int64_t)cur_at.bs0 + (int64_t)min(tn * BN + wn * WN + q * 32 + lq * 8 + i, p.N - 1) * p.b_scale_stride,
-                               p.scales_dtype);  // (grouped: bs0 = where the expert's scales begin)
-#pragma unroll
-      for (int mt = 0; mt < TM; ++mt) {
-        int64_t m = (int64_t)cur_at.row0 + wm * WM + mt * 16 + lm;
-        if (m >= p.M) m = p.M - 1;
-        a_s_all[mt] = scale_at(p.a_scales, m * p.a_scale_stride, p.scales_dtype);
-      }
+      // (grouped: bs0 = where the expert's scales begin)
+      scales_at(b_s, p.b_scales, p.scales_dtype, [&](int i) {
+        return (int64_t)cur_at.bs0 + (int64_t)min(tn * BN + wn * WN + (i >> 3) * 32 + lq * 8 + (i & 7), p.N - 1) * p.b_scale_stride;
+      });
+      scales_at(a_s_all, p.a_scales, p.scales_dtype, [&](int mt) {
+        const int64_t m = (int64_t)cur_at.row0 + wm * WM + mt * 16 + lm;
+        return (m < p.M ? m : p.M - 1) * p.a_scale_stride;
+      });
       if constexpr (KV) {  // (this op's scales are rounded to bf16)
 #pragma unroll
-        for (int q = 0; q < TN / 2; ++q)
-#pragma unroll
-          for (int i = 0; i < 8; ++i) b_s[q][i] = bf16_round(b_s[q][i]);
+        for (int i = 0; i < TN * 4; ++i) b_s[i] = bf16_round(b_s[i]);
 #pragma unroll
         for (int mt = 0; mt < TM; ++mt) a_s_all[mt] = bf16_round(a_s_all[mt]);
       }
@@ -852,7 +846,7 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
           for (int i = 0; i < 4; ++i) {
             w[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
             if constexpr (!BLOCKSCALE) {
-              const uint32_t sc = pack_bf16x2(a_s * b_s[q][2 * i], a_s * b_s[q][2 * i + 1]);
+              const uint32_t sc = pack_bf16x2(a_s * b_s[q * 8 + 2 * i], a_s * b_s[q * 8 + 2 * i + 1]);
               w[i] = pack_bf16x2(__uint_as_float(w[i] << 16) * __uint_as_float(sc << 16),
                                  __uint_as_float(w[i] & 0xffff0000u) * __uint_as_float(sc & 0xffff0000u));
             }
@@ -867,8 +861,8 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const float t_lo = lo[i] * a_s, t_hi = hi[i] * a_s;
-            lo[i] = t_lo * b_s[q][i];
-            hi[i] = t_hi * b_s[q][4 + i];
+            lo[i] = t_lo * b_s[q * 8 + i];
+            hi[i] = t_hi * b_s[q * 8 + 4 + i];
           }
         }
         // (written and read back through the same vector type: to the compiler a store through one type and a load
