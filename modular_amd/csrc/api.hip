@@ -151,6 +151,7 @@ static const Tuning* read_tuning(unsigned generation) {
   t->big_rows = num("MAXFP8_BIG_ROWS", 1024);
   t->grouped_overlap = num("MAXFP8_GROUPED_OVERLAP", 1) != 0;
   t->grouped_persist = num("MAXFP8_GROUPED_PERSIST", 1) != 0;
+  t->grouped_decode = num("MAXFP8_GROUPED_DECODE", t->grouped_decode);
   const int w4 = num("MAXFP8_W4", -1);
   t->w4 = (w4 == 0 || w4 == 4 || w4 == 5 || w4 == 6) ? w4 : -1;
   const int w4_split = num("MAXFP8_W4_SPLIT", -1);

@@ -98,21 +98,20 @@ __host__ __device__ constexpr uint32_t skinny_acts_bytes(uint32_t M, uint32_t pe
 // a SIMD, so each has half of its registers: 256, which two or four groups do not fit.)
 __host__ __device__ constexpr int skinny_page_waves(int mt, bool kv) { return kv && mt == 1 ? 1 : 0; }
 
+// One block: columns [n0, n0 + 16 * NTW) of C.
 // KV: the fused QKV projection's epilogue (a kernel of its own: the plain one would load its arguments all the same, 1 to 2 per cent)
-template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, int ACTS = kActsPerSlab, bool KV = false>
-__global__ __launch_bounds__((NWAVES + skinny_page_waves(MT, KV)) * 64) void gemm_skinny_kernel(std::conditional_t<KV, GemmArgs, MatmulArgs> p_in) {
-  const auto p = gridDim.y == 1 ? p_in : batch_view(p_in, blockIdx.y);
+// c_rows (GROUPED, may be null): row m of the result goes to row c_rows[m] of C
+template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, int ACTS, bool KV, bool GROUPED = false, class Args>
+__device__ __forceinline__ void skinny_body(const Args& p, uint8_t* smem, const int n0, [[maybe_unused]] const uint32_t* c_rows = nullptr) {
   using Cfg = SkinnyCfg<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ACTS>;
   constexpr bool ALDS = Cfg::ALDS, QUANT = Cfg::QUANT;
   static_assert(!ALDS || MT == 1, "activations in LDS: one 16-token group");
   constexpr int WAVES = Cfg::WAVES, DEPTH = Cfg::DEPTH, SLOT = Cfg::SLOT, PER = Cfg::PER;
   static_assert((DEPTH - 1) * PER < 64, "vmcnt is a 6-bit counter");
-  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lm = lane & 15, lq = lane >> 4;
-  const int n0 = blockIdx.x * (16 * NTW);
   const int cols_here = (p.N - n0) < 16 * NTW ? (p.N - n0) : 16 * NTW;
 
   const uint8_t* b_tile = p.b + (int64_t)n0 * p.ldb;
@@ -469,8 +468,12 @@ __global__ __launch_bounds__((NWAVES + skinny_page_waves(MT, KV)) * 64) void gem
         v[i] = t * b_s[i];
       }
     }
+    int64_t cm = m;
+    if constexpr (GROUPED) {
+      if (c_rows) cm = c_rows[m];
+    }
     if (p.c_dtype == MAXFP8_BF16) {
-      uint16_t* dst = reinterpret_cast<uint16_t*>(p.c) + (int64_t)m * p.ldc + n;
+      uint16_t* dst = reinterpret_cast<uint16_t*>(p.c) + cm * p.ldc + n;
       if (p.c_vec_ok && n + 3 < p.N) {
         const uint32_t lo = pack_bf16x2(v[0], v[1]);
         const uint32_t hi = pack_bf16x2(v[2], v[3]);
@@ -481,12 +484,19 @@ __global__ __launch_bounds__((NWAVES + skinny_page_waves(MT, KV)) * 64) void gem
           if (n + i < p.N) dst[i] = (uint16_t)f32_to_bf16_bits(v[i]);
       }
     } else {
-      float* dst = reinterpret_cast<float*>(p.c) + (int64_t)m * p.ldc + n;
+      float* dst = reinterpret_cast<float*>(p.c) + cm * p.ldc + n;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         if (n + i < p.N) dst[i] = v[i];
     }
   }
+}
+
+template <int NTW, int MT, bool BLOCKSCALE, int RING_KB, int NWAVES, int ACTS = kActsPerSlab, bool KV = false>
+__global__ __launch_bounds__((NWAVES + skinny_page_waves(MT, KV)) * 64) void gemm_skinny_kernel(std::conditional_t<KV, GemmArgs, MatmulArgs> p_in) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  const auto p = gridDim.y == 1 ? p_in : batch_view(p_in, blockIdx.y);
+  skinny_body<NTW, MT, BLOCKSCALE, RING_KB, NWAVES, ACTS, KV>(p, smem, (int)blockIdx.x * (16 * NTW));
 }
 
 int compute_units();
@@ -625,6 +635,122 @@ int gemm_skinny_quant_dispatch(const GemmArgs& p, bool blockscale, hipStream_t s
   if (skinny_quant_loads(p.M, p.K) > kQuantLoads)
     MAXFP8_FAIL(MAXFP8_ERR_SHAPE, "decode matmul with the quantisation inside: M = %d, K = %d do not fit", p.M, p.K);
   return blockscale ? pick_quant<true>(p, stream) : pick_quant<false>(p, stream);
+}
+
+// ---- grouped: the experts of a few tokens ------------------------------------------------------------------------
+// The MoE matmul (rows sorted by expert, slot z = rows [offsets[z], offsets[z + 1]) times the weights of expert expert_ids[z], zeros where that is
+// -1: max/kernels/src/linalg/grouped_matmul_sm100_blockwise_fp8.mojo:2938-3105) when its slots hold a few rows each: the decode matmul of every
+// slot in use, 16 * NTW weight rows per tile, K split over the block's waves.  Bound by the weights of the experts in use.  A block works out from
+// the offsets which slots are in use (a list in LDS, once), then takes every gridDim.x-th tile: no claims, and four blocks per CU, so that one
+// block's start and end hide behind the others' streams.  The persistent launch of gemm_tiled.hip, made for mixed sizes, gives
+// a CU tiles of 512 weight rows that its block claims from counters in memory: a tile is 21 us and more for one CU however few there are.
+// A slot of more than 32 rows is computed 32 rows at a time, its weights read again for each.  (Four groups of 16 rows per pass take 168 registers,
+// three blocks per CU and spills: one token of 8 experts 7168 x 2048 70 -> 93 us, 64 tokens 467 -> 560.)
+template <int NTW, bool BLOCKSCALE>
+struct GroupedSkinnyCfg {
+  static constexpr int WAVES = 4, RING_KB = NTW == 1 ? 6 : 8, THREADS = 64 * WAVES;
+  using One = SkinnyCfg<NTW, 1, BLOCKSCALE, RING_KB, WAVES>;
+  using Two = SkinnyCfg<NTW, 2, BLOCKSCALE, RING_KB, WAVES>;
+  static constexpr int LIST = One::SMEM > Two::SMEM ? One::SMEM : Two::SMEM;  // the slots in use, 16 bits each, behind the rings and sums
+  static constexpr int MAX_SLOTS = 512, SMEM = LIST + MAX_SLOTS * 2 + 2 * WAVES * 4;
+};
+template <int NTW, bool BLOCKSCALE>
+__global__ __launch_bounds__(256, 4) void gemm_grouped_skinny_kernel(GemmArgs g, int ncol) {
+  using Cfg = GroupedSkinnyCfg<NTW, BLOCKSCALE>;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  uint16_t* const list = reinterpret_cast<uint16_t*>(smem + Cfg::LIST);
+  int* const counts = reinterpret_cast<int*>(list + Cfg::MAX_SLOTS);
+  // (rows held inside [0, M): a stale routing tensor must not turn into accesses outside the operands)
+  auto rows_of = [&](int z, int64_t& begin) {
+    const int64_t M = g.M, b = g.offsets[z], e = g.offsets[z + 1];
+    begin = b < M ? b : M;
+    const int64_t end = e < M ? e : M;
+    return (int)(end > begin ? end - begin : 0);
+  };
+  int used = 0;
+#pragma unroll
+  for (int half = 0; half < Cfg::MAX_SLOTS / Cfg::THREADS; ++half) {
+    const int z = half * Cfg::THREADS + tid;
+    int64_t begin;
+    const bool in_use = z < g.num_active && rows_of(z, begin) > 0;
+    const uint64_t with = __ballot(in_use);
+    if (lane == 0) counts[half * Cfg::WAVES + wave] = __popcll(with);
+    __syncthreads();
+    int before = used;
+    for (int w = 0; w < Cfg::WAVES; ++w) {
+      const int c = counts[half * Cfg::WAVES + w];
+      if (w < wave) before += c;
+      used += c;
+    }
+    if (in_use) list[before + __popcll(with & (((uint64_t)1 << lane) - 1))] = (uint16_t)z;
+  }
+  used = __builtin_amdgcn_readfirstlane(used);
+  for (int t = (int)blockIdx.x; t < used * ncol; t += (int)gridDim.x) {
+    __syncthreads();  // the list is there; the last tile's sums have been read
+    const int j = t / ncol, n0 = (t - j * ncol) * 16 * NTW;
+    const int slot = __builtin_amdgcn_readfirstlane((int)list[j]);
+    int64_t begin;
+    const int rows = rows_of(slot, begin);
+    const int e = g.expert_ids[slot];
+    const int64_t esize = g.c_dtype == MAXFP8_BF16 ? 2 : 4;
+    if (e < 0) {
+      const int cols = g.N - n0 < 16 * NTW ? g.N - n0 : 16 * NTW;
+      for (int i = tid; i < rows * cols; i += Cfg::THREADS) {
+        const int r = i / cols;
+        const int64_t m = begin + r, at = (g.c_row_index ? (int64_t)g.c_row_index[m] : m) * g.ldc + n0 + (i - r * cols);
+        if (esize == 2) reinterpret_cast<uint16_t*>(g.c)[at] = 0;
+        else reinterpret_cast<float*>(g.c)[at] = 0.f;
+      }
+      continue;
+    }
+    MatmulArgs p = g;
+    p.b = g.b + (int64_t)e * g.b_expert_stride;
+    p.b_scales = g.b_scales + (int64_t)e * g.bs_expert_stride;
+    for (int r0 = 0; r0 < rows; r0 += 32) {
+      if (r0 > 0) __syncthreads();
+      const int64_t row = begin + r0;
+      p.M = rows - r0 < 32 ? rows - r0 : 32;
+      p.a = g.a + row * g.lda;
+      p.a_scales = g.a_scales + (BLOCKSCALE ? row : row * g.a_scale_stride);
+      const uint32_t* c_rows = g.c_row_index ? g.c_row_index + row : nullptr;
+      p.c = g.c_row_index ? g.c : reinterpret_cast<uint8_t*>(g.c) + row * g.ldc * esize;
+      if (p.M <= 16) skinny_body<NTW, 1, BLOCKSCALE, Cfg::RING_KB, Cfg::WAVES, kActsPerSlab, false, true>(p, smem, n0, c_rows);
+      else skinny_body<NTW, 2, BLOCKSCALE, Cfg::RING_KB, Cfg::WAVES, kActsPerSlab, false, true>(p, smem, n0, c_rows);
+    }
+  }
+}
+
+template <int NTW, bool BLOCKSCALE>
+static int launch_grouped_skinny(const GemmArgs& p, int64_t most_tiles, hipStream_t stream) {
+  using Cfg = GroupedSkinnyCfg<NTW, BLOCKSCALE>;
+  auto kern = gemm_grouped_skinny_kernel<NTW, BLOCKSCALE>;
+  static PerDeviceFlag attr;
+  bool& attr_done = attr.here();
+  if (!attr_done) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::SMEM);
+    if (e != hipSuccess) MAXFP8_FAIL(MAXFP8_ERR_LAUNCH, "gemm_grouped_skinny: cannot reserve %d bytes of LDS: %s", Cfg::SMEM, hipGetErrorString(e));
+    attr_done = true;
+  }
+  const int64_t resident = 4 * (int64_t)compute_units();
+  hipLaunchKernelGGL(kern, dim3((unsigned)(most_tiles < resident ? most_tiles : resident)), dim3(Cfg::THREADS), Cfg::SMEM, stream, p,
+                     (int)ceil_div(p.N, 16 * NTW));
+  return launch_status("gemm_grouped_skinny");
+}
+
+// Total rows up to which a grouped matmul comes here.  The experts' two matmuls with what is around them, persistent launch and this one, us: 256
+// experts of 7168 x 2048, 8 per token, 1 / 8 / 32 / 48 / 64 / 128 tokens 137 / 213 / 395 / 408 / 453 / 565 and 71 / 173 / 323 / 401 / 469 / 713; 128 of 4096 x 1536,
+// 8 per token, 1 / 16 / 64 / 80 tokens 95 / 146 / 251 / 254 and 45 / 116 / 240 / 274; 64 of 2048 x 1408, 6 per token, 1 / 16 / 80 / 96 tokens 70 / 88 / 121 /
+// 121 and 32 / 52 / 115 / 126.  Level at 400, 576 and 510 rows: what turns it is the slots of more than 32 rows, whose weights are read more than once.
+bool gemm_grouped_skinny_ok(const GemmArgs& p) {
+  return p.M <= tuning().grouped_decode && p.num_active <= GroupedSkinnyCfg<2, true>::MAX_SLOTS;
+}
+int gemm_grouped_skinny_dispatch(const GemmArgs& p, bool blockscale, hipStream_t stream) {
+  const int64_t slots = p.M < p.num_active ? p.M : p.num_active, wide = slots * ceil_div(p.N, 32);
+  if (wide >= 4 * (int64_t)compute_units())
+    return blockscale ? launch_grouped_skinny<2, true>(p, wide, stream) : launch_grouped_skinny<2, false>(p, wide, stream);
+  const int64_t narrow = slots * ceil_div(p.N, 16);
+  return blockscale ? launch_grouped_skinny<1, true>(p, narrow, stream) : launch_grouped_skinny<1, false>(p, narrow, stream);
 }
 
 // ---- read-only probe ---------------------------------------------------------------------------

@@ -1,0 +1,89 @@
+"""The grouped form of the decode kernel (a few rows per slot in use): against the naive kernel and the persistent launch, exactly, on small
+integers and powers of two, where a slot's rows pass a group of 16 or a pass of 32, slots are empty or without an expert, columns do not
+fill a tile and slabs do not fill the waves; and stale offsets stay inside the operands."""
+import pytest
+import torch
+
+import modular_amd as mx
+from modular_amd import _lib
+
+pytestmark = pytest.mark.gpu
+BLK = mx.blockwise_fp8_config()
+
+# rows of the slots, their experts, N, K: one slab of one row; every edge of a slot; one tile per slot; more tiles than blocks on the chip (32 weight rows each),
+# fewer (16); a tile of two columns
+CASES = [([1], [0], 16, 128), ([1, 0, 16, 17, 31, 0, 32, 33, 64, 65], [3, 0, 1, 9, -1, 2, 5, 4, 6, 7], 200, 640), ([2, 0, 3], [2, 1, 0], 32, 2176),
+         ([1] * 24, list(range(24)), 1536, 256), ([40, 1], [1, 0], 66, 7168), ([3, 5, 2], [0, -1, 2], 8, 384)]
+
+
+def exact(counts, ids, N, K, kind, dev, spare=3):
+    g = torch.Generator().manual_seed(N + K + len(counts))
+    T, E = sum(counts) + spare, max(len(counts), max(ids) + 1)
+    ints = lambda *s: torch.randint(-2, 3, s, generator=g).float().to(torch.float8_e4m3fn).to(dev)
+    power = lambda *s: (2.0 ** torch.randint(-1, 2, s, generator=g).float()).to(dev)
+    off = torch.zeros(len(counts) + 1, dtype=torch.int64)
+    off[1:] = torch.cumsum(torch.tensor(counts), 0)
+    scales = (power(K // 128, -(-T // 4) * 4), power(E, -(-N // 128), K // 128)) if kind == "block" else (power(T, 1), power(E, N, 1))
+    return ints(T, K), ints(E, N, K), *scales, off.to(torch.uint32).to(dev), torch.tensor(list(ids) + [-1] * (E - len(ids)), dtype=torch.int32).to(dev)
+
+
+def run(case, kind, out, active, row_index=None):
+    a, b, sa, sb, off, ids = case
+    stats = torch.tensor([a.shape[0], active], dtype=torch.int64).to(torch.uint32)
+    if kind == "row":
+        return mx.grouped_matmul_rowwise_dynamic_scaled_fp8(a, b, sa, sb, off, ids, stats, out_type=out)
+    return mx.grouped_dynamic_scaled_fp8_matmul(a, b, sa, sb, off, ids, stats, BLK.input_scale, BLK.weight_scale, out_type=out,
+                                                **({} if row_index is None else {"out_row_index": row_index}))
+
+
+@pytest.mark.parametrize("kind", ["block", "row"])
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_bits_of_the_persistent_launch(dev, tune, case, kind):
+    counts, ids, N, K = CASES[case]
+    operands, used = exact(counts, ids, N, K, kind, dev), sum(counts)
+    for out in (torch.bfloat16, torch.float32):
+        tune(MAXFP8_GROUPED_DECODE=100000)
+        got = run(operands, kind, out, len(counts))
+        tune(MAXFP8_GROUPED_DECODE=0)
+        want = run(operands, kind, out, len(counts))
+        assert torch.equal(got[:used], want[:used])
+        # ... which is the sum itself
+        a, b, sa, sb = (t.double().cpu() for t in operands[:4])
+        at = 0
+        for rows, e in zip(counts, ids):
+            x = a[at:at + rows]
+            if e < 0 or rows == 0:
+                ref = torch.zeros(rows, N, dtype=torch.float64)
+            elif kind == "row":
+                ref = (x @ b[e].T) * sa[at:at + rows] * sb[e].T
+            else:
+                xs = x * sa[:, at:at + rows].repeat_interleave(128, 0).T
+                ref = xs @ (b[e] * sb[e].repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)).T
+            assert torch.equal(got[at:at + rows].cpu(), ref.to(out))
+            at += rows
+
+
+def test_row_index_many_slots_and_stale_offsets(dev, tune):
+    tune(MAXFP8_GROUPED_DECODE=100000)
+    counts = [1 if z % 7 == 3 else 0 for z in range(512)]         # 73 of 512 slots, in both halves of the list
+    operands = exact(counts, list(range(512)), 48, 256, "block", dev, spare=0)
+    T = sum(counts)
+    order = torch.randperm(T, generator=torch.Generator().manual_seed(1))
+    plain, moved = run(operands, "block", torch.bfloat16, 512), run(operands, "block", torch.bfloat16, 512, order.to(torch.int64).to(torch.uint32).to(dev))
+    assert torch.equal(moved[order.to(dev)], plain)
+    # offsets past the rows there are: held to them
+    a, b, sa, sb, off, ids = exact([5, 6], [1, 0], 40, 384, "block", dev, spare=0)
+    want = run((a, b, sa, sb, off, ids), "block", torch.bfloat16, 2)
+    stale = torch.tensor([0, 5, 1 << 30], dtype=torch.int64).to(torch.uint32).to(dev)
+    assert torch.equal(run((a, b, sa, sb, stale, ids), "block", torch.bfloat16, 2), want)
+
+
+def test_up_to_how_many_rows(dev):
+    from torch.profiler import ProfilerActivity, profile
+
+    for rows, name in ((448, "gemm_grouped_skinny_kernel"), (449, "gemm_grouped_persist_kernel")):
+        operands = exact([rows - 1, 1], [0, 1], 32, 128, "block", dev, spare=0)
+        with profile(activities=[ProfilerActivity.CUDA]) as seen:
+            run(operands, "block", torch.bfloat16, 2)
+            torch.cuda.synchronize()
+        assert any(name in e.name for e in seen.events()), rows
