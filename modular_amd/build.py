@@ -29,7 +29,8 @@ COMMON = [
 # the naive kernels must round every product and sum like a scalar host loop
 # the four-wave kernels keep their MFMA results in ordinary VGPRs (the promotions are VALU work) and their operand
 # fragments in AGPRs: left to itself the compiler writes every MFMA result to AGPRs once a kernel uses any
-PER_FILE = {"naive.hip": ["-ffp-contract=off"], "gemm_w4.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "gemm_mid.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+PER_FILE = {"naive.hip": ["-ffp-contract=off"], "gemm_w4.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "gemm_mid.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+            "gemm_short_k.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def hipcc() -> str:

@@ -63,6 +63,8 @@ int gemm_skinny_max_m();
 int compute_units();
 bool gemm_short_k_ok(const GemmArgs&, bool, int64_t);
 int gemm_short_k_dispatch(const GemmArgs&, int64_t, hipStream_t);
+bool gemm_one_slab_ok(const GemmArgs&, bool, int64_t);
+int gemm_one_slab_dispatch(const GemmArgs&, int64_t, hipStream_t);
 int gemm_mid_dispatch(const GemmArgs&, bool, int, hipStream_t);
 bool gemm_mid_ok(int64_t M, int64_t N, int64_t K);
 int gemm_mid_shape(int64_t M, int64_t N, int64_t K, bool blockscale, float* us);
@@ -530,8 +532,8 @@ size_t maxfp8_matmul_auto_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 namespace maxfp8 {
 struct BatchStrides { int64_t n, a, b, c, a_scales, b_scales; };  // n batches; steps in elements
 
-// A batch of short K and more than 32 rows on the tiles: one slab of K leaves three of the decode kernel's four waves idle, and
-// beyond one of its 16-row blocks per CU every block more reads the tokens again.  With one block per CU or less it is ahead from
+// A batch of short K and more than 32 rows on the tiles (one slab mostly has a kernel of its own): one slab of K leaves three of the decode
+// kernel's four waves idle, and beyond one of its 16-row blocks per CU every block more reads the tokens again.  With one block per CU or less it is ahead from
 // two slabs on (decode kernel against tiles, 48 rows, us, cold: 32 x 512 -> 128 5.4 and 6.4, 48 of them 7.8 and 6.5, 128 12.7
 // and 6.7; 16 x 256 -> 256 4.8 and 5.3, 24 of them 6.3 and 5.3; 16 x 128 -> 512 5.6 and 4.8, 128 of them 28.7 and 6.7).
 static bool batch_on_tiles(int64_t batch, int64_t M, int64_t N, int64_t K) {
@@ -629,6 +631,7 @@ static int matmul_common(void* c, const void* a, const void* b, const void* a_sc
   p.a_batch = bt.a; p.b_batch = bt.b; p.c_batch = bt.c;
   p.a_scales_batch = bt.a_scales; p.b_scales_batch = bt.b_scales;
   if (algo == kAlgoMid) return gemm_mid_dispatch(p, block, shape, st);
+  if (automatic && gemm_one_slab_ok(p, block, bt.n)) return gemm_one_slab_dispatch(p, bt.n, st);
   if (automatic && gemm_short_k_ok(p, block, bt.n)) return gemm_short_k_dispatch(p, bt.n, st);
   if (algo == MAXFP8_ALGO_SKINNY) return gemm_skinny_dispatch(p, block, bt.n, st);
   if (workspace && !is_aligned(workspace, 16)) MAXFP8_FAIL(MAXFP8_ERR_ALIGN, "matmul: workspace must be 16-byte aligned");

@@ -1894,6 +1894,15 @@ static float tile_overhead(int64_t M, int64_t N, int i, int splits, bool kv_on =
 
 // cost of a shape (microseconds) = rounds of resident blocks * time of one tile
 static int pick_shape(int64_t M, int64_t N, int nslab, bool blockscale, bool can_split, int64_t batch = 1, bool kv_on = false) {
+  // A batch of one slab of K (what gemm_one_slab_kernel does not take: other result types, ragged columns) is starts, ends and stores: 128 x 128 tiles, whose stores overlap the start of the CU's other block, but where
+  // 256 x 256 tiles are little more than whole rounds of the CUs and the small ones more than one.  Fitted to 27 batches (16, 64, 128 heads,
+  // 48 to 1024 tokens, N = 512, from the cache; us, 256 x 256 and 128 x 128): 16 heads of 256 / 1024 tokens 7.5 / 9.8 and 5.0 / 7.9, 64 of 256 / 512 9.7 / 13.5 and
+  // 8.4 / 14.7, 128 of 200 / 256 / 777 10.5 / 13.3 / 38.7 and 14.1 / 16.0 / 31.8.
+  if (batch > 1 && nslab == 1 && !kv_on) {
+    const float large = (float)(ceil_div(M, 256) * ceil_div(N, 256) * batch), small = (float)(ceil_div(M, 128) * ceil_div(N, 128) * batch);
+    const float fill = 0.5f + 0.5f * (float)M / (float)(ceil_div(M, 128) * 128);
+    return 5.5f + 0.0331f * large < 4.0f + 0.0094f * small * fill + (small > 512.f ? 1.5f : 0.f) ? 1 : 3;
+  }
   int best = 0;
   float best_cost = 0.f;
   for (int i = 0; i < 4; ++i) {

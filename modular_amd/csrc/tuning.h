@@ -22,7 +22,7 @@
 //   MAXFP8_SKINNY=<ntw>4<KB>   force a shape of the weight-streaming kernel (e.g. 1408, 2416)
 //   MAXFP8_MID=0 / [<b>]<MT><NT>  the kernel for tens to hundreds of tokens: never / always, in 16 MT x 16 NT tiles (e.g. 43), b blocks per
 //                              CU (e.g. 244; without b the first built shape with that tile)
-//   MAXFP8_SHORT_K=0           batches of short K: the decode and tile kernels only
+//   MAXFP8_SHORT_K=0           batches of short K: the decode and tile kernels only (gemm_short_k.hip)
 #pragma once
 
 namespace maxfp8 {
