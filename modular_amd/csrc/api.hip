@@ -155,7 +155,7 @@ static const Tuning* read_tuning(unsigned generation) {
   t->grouped_persist = num("MAXFP8_GROUPED_PERSIST", 1) != 0;
   t->grouped_decode = num("MAXFP8_GROUPED_DECODE", t->grouped_decode);
   const int w4 = num("MAXFP8_W4", -1);
-  t->w4 = (w4 == 0 || w4 == 4 || w4 == 5 || w4 == 6) ? w4 : -1;
+  t->w4 = (w4 == 0 || w4 == 4 || w4 == 5 || w4 == 6 || w4 == 8) ? w4 : -1;
   const int w4_split = num("MAXFP8_W4_SPLIT", -1);
   t->w4_split = (w4_split == 0 || w4_split == 1) ? w4_split : -1;
   t->skinny_quant = num("MAXFP8_SKINNY_QUANT", 1) != 0;

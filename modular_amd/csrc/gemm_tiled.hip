@@ -2009,11 +2009,20 @@ static float persistent_cost(int64_t tiles, int slots, float t) {
   return (float)full * t + (rest ? t * (0.75f + 0.3f * (float)rest / (float)slots) : 0.f);
 }
 
-// Per-slab and per-tile times (microseconds, chip full, operands from HBM) of the four-wave kernel's three tile heights:
-// index 0: 128 x 256, 1: 160 x 256, 2: 192 x 256.  Against the eight-wave persistent kernel's 1.63 / 1.40 per slab of a 256 x 256 tile
+// Per-slab and per-tile times (microseconds, chip full, operands from HBM) of the four-wave kernel's tile heights (tm - 4):
+// index 0: 128 x 256, 1: 160 x 256, 2: 192 x 256, 4: 256 x 192.  Against the eight-wave persistent kernel's 1.63 / 1.40 per slab of a 256 x 256 tile
 // that is 6 ... 9 % less per flop with block scaling and level with row scaling; what decides between the three is
 // mostly how the tile count divides by the CUs.
-static const float kW4SlabBlock[3] = {0.90f, 1.00f, 1.14f}, kW4SlabRow[3] = {0.80f, 0.88f, 1.00f}, kW4Tile = 5.5f;
+static const float kW4SlabBlock[5] = {0.90f, 1.00f, 1.14f, 0.f, 1.08f}, kW4SlabRow[5] = {0.80f, 0.88f, 1.00f, 0.f, 1.00f}, kW4Tile = 5.5f;
+// (256 x 192, fitted to K = 1024 ... 28672: its results leave in shorter runs, and the tile costs more and the slab less than its flops; with block scaling
+// a slab past the 64th, when the blocks of an XCD have drifted apart, 1.20: 16384 x 8192 x 28672 3.52 ms in 2752 of these tiles, 3.29 in as many of 192 x 256)
+static const float kW4TallTileBlock = 10.0f, kW4TallTileRow = 6.5f, kW4TallLateSlab = 0.12f;
+static float w4_slab(bool blockscale, int tm) { return (blockscale ? kW4SlabBlock : kW4SlabRow)[tm - 4]; }
+static float w4_tile(bool blockscale, int tm, int nslab) {
+  return tm != 8 ? kW4Tile : !blockscale ? kW4TallTileRow : kW4TallTileBlock + (nslab > 64 ? (float)(nslab - 64) * kW4TallLateSlab : 0.f);
+}
+static const int kW4Heights[4] = {4, 5, 6, 8};
+static int64_t w4_tiles(int64_t M, int64_t N, int tm) { return ceil_div(M, 32 * tm) * ceil_div(N, tm == 8 ? 192 : 256); }
 // ... and of its cut tiles, with few blocks to share the memory with
 static const float kW4CutSlabBlock[3] = {0.646f, 0.71f, 0.84f}, kW4CutSlabRow[3] = {0.56f, 0.72f, 0.80f};
 // With the tail cut: whole rounds, then a piece per block and the hand-over: a piece's sums written through to memory,
@@ -2033,15 +2042,15 @@ static float three_stage_cost(int64_t M, int64_t N, int64_t K, bool blockscale) 
 // What a plan on the four-wave kernel is estimated to take: tiles of 32 tm rows, whole, with their tail cut or each of them cut
 static float w4_plan_cost(int64_t M, int64_t N, int64_t K, bool blockscale, int tm, bool split) {
   const int slots = compute_units(), nslab = (int)(K / 128);
-  const float t_slab = blockscale ? kW4SlabBlock[tm - 4] : kW4SlabRow[tm - 4], t = (float)nslab * t_slab + kW4Tile;
-  const int64_t tiles = ceil_div(M, 32 * tm) * ceil_div(N, 256);
+  const float t_slab = w4_slab(blockscale, tm), t = (float)nslab * t_slab + w4_tile(blockscale, tm, nslab);
+  const int64_t tiles = w4_tiles(M, N, tm);
   // (part of one round, weights from memory: a block waits for its copies, and the chip's clock does not make up for it -- 166 x 36864 x 7168 in 144 tiles of 192 rows
   // 1.17 us per slab, with row scales 260 x 17616 x 6144 in 138 of 160 rows 1.13, in 207 of 128 rows 0.96.  From five row tiles on, which share the weights,
   // row scales are quicker than block scales again in the taller tiles, where those fill three quarters of the chip: 1352 x 5856 x 15104 in 207 tiles of
   // 160 rows 110 us, on 128 x 128 tiles 131; 1072 x 7168 x 18432 138 and 158; but 776 x 7168 x 18432 in 140 of them 142, on 256 x 128 tiles 124, and
   // 598 x 12128 x 10496 in 192 of them, four row tiles, 81, in 240 of 128 rows 76)
   const bool alone = blockscale || tm == 4 || M <= 4 * 32 * tm || tiles * 4 < slots * 3;
-  if (!split) return alone && tiles < slots && N * K >= ((int64_t)1 << 26) ? (float)nslab * kW4SlabBlock[tm - 4] + kW4Tile : persistent_cost(tiles, slots, t);
+  if (!split) return alone && tiles < slots && N * K >= ((int64_t)1 << 26) ? (float)nslab * kW4SlabBlock[tm - 4] + w4_tile(true, tm, nslab) : persistent_cost(tiles, slots, t);
   const W4Split sp = gemm_w4_split(M, N, K, tm);
   const float pieces = (float)ceil_div(nslab, sp.unit);
   if (tiles * 2 <= slots)  // (fitted with the weights from memory, which gemm_mid_shape's estimates are not: within 5 per cent for nine launches in ten of 128-row tiles, 13 of taller ones)
@@ -2067,7 +2076,7 @@ static int pick_w4(int64_t M, int64_t N, int64_t K, bool blockscale, float other
   // every tile of height tm cut, where its pieces are worth it (see above; forced: wherever there is a cut)
   auto every_cut = [&](int tm) {
     const W4Split sp = gemm_w4_split(M, N, K, tm);
-    if (cut == 0 || sp.unit <= 0 || sp.bytes > workspace_bytes || ceil_div(M, 32 * tm) * ceil_div(N, 256) * 2 > slots) return false;
+    if (tm == 8 || cut == 0 || sp.unit <= 0 || sp.bytes > workspace_bytes || ceil_div(M, 32 * tm) * ceil_div(N, 256) * 2 > slots) return false;
     // (more than four pieces only where they are long: 128 x 8192 x 28672 in eight pieces of 28 slabs 59 against 64 us,
     // 512 x 2048 x 28672 46 against 52; in eight of 16 slabs 128 x 8192 x 16384 47 against 41.  And only where the rows
     // fill three quarters of the tiles: 48 ... 64 rows on 8192 x 28672 took 56 against 48 ... 51.)
@@ -2090,9 +2099,9 @@ static int pick_w4(int64_t M, int64_t N, int64_t K, bool blockscale, float other
   }
   int best = 0;
   float best_cost = forced > 0 ? 3.0e38f : 0.97f * other_cost;  // (a forced height is taken whatever it costs)
-  for (int tm = 4; tm <= 6; ++tm) {
+  for (const int tm : kW4Heights) {
     if (forced > 0 && tm != forced) continue;
-    const int64_t tiles = ceil_div(M, 32 * tm) * ceil_div(N, 256);
+    const int64_t tiles = w4_tiles(M, N, tm);
     // (half a round or less: more, smaller tiles and a K split are the better fit; a little more than half is not: 166 x 36864 x 7168 in
     // 144 tiles of 192 rows 71 us, in 288 of 128 rows 101)
     // (the fused QKV projection's tiles, with a store of their own, want three quarters of a round: 526 x 8192 x 6144 with row scales in 160 tiles of 128 rows 42 us and 55
@@ -2113,6 +2122,13 @@ static int pick_w4(int64_t M, int64_t N, int64_t K, bool blockscale, float other
     // tiles 33 and 34; 937 x 8192 x 6144 in 256 of them 48 and 57, 51 and 69)
     const bool slow = kv_on && !blockscale && tm == 4 && tiles * 8 < slots * 7;
     const float whole = slow ? persistent_cost(tiles, slots, (float)nslab * 0.93f + kW4Tile) : w4_plan_cost(M, N, K, blockscale, tm, false);
+    if (tm == 8) {
+      // (no cut.  Against another height it has to be 2 per cent ahead, and against whole tiles of 128 rows with block scaling, which are quicker than
+      // priced where the weights are small, 7: 1024 x 24576 x 1536 47.2 us in 512 of these tiles, 46.0 in 768 of those, 4096 x 6144 x 1024 39.9 and 39.0)
+      const float ahead = !best || forced > 0 ? 1.f : (best == 4 && blockscale && !*split ? 0.93f : 0.98f);
+      if (whole < ahead * best_cost) { best = tm; best_cost = whole; *split = false; }
+      continue;
+    }
     if (whole < best_cost) { best = tm; best_cost = whole; *split = false; }
     const W4Split sp = gemm_w4_split(M, N, K, tm);
     if (cut != 0 && sp.unit > 0 && sp.bytes <= workspace_bytes) {
@@ -2303,7 +2319,7 @@ int gemm_tiled_describe(int64_t M, int64_t N, int64_t K, bool blockscale, bool h
                     n_tiles * 2 <= compute_units() ? "every tile" : "tail", sp.unit);
   }
   if (plan.w4)
-    return snprintf(buf, len, "%dx256 x%lld persistent, four waves", 32 * plan.w4, (long long)(ceil_div(M, 32 * plan.w4) * ceil_div(N, 256)));
+    return snprintf(buf, len, "%dx%d x%lld persistent, four waves", 32 * plan.w4, plan.w4 == 8 ? 192 : 256, (long long)w4_tiles(M, N, plan.w4));
   if (plan.two.axis && !plan.streamk) {
     const TileShape &a = kShapes[plan.two.v1 - 1], &b = kShapes[plan.two.v2 - 1];
     const bool cols = plan.two.axis == 1;

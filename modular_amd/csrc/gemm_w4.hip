@@ -30,7 +30,14 @@
 // Promotion: the MFMA of (16-row group mt, fragment nt) writes a fresh product, and the four FMAs that fold it into the
 // accumulators are issued LAG MFMAs later, when the product has left the matrix pipe.
 //
-// Tiles: any M and any N that is a multiple of 8 (rows of either operand past the end read as zero through the buffer
+// Tile shapes: 128, 160 or 192 rows by 256 columns (a wave: 64, 80 or 96 x 128), and 256 x 192 (128 x 96), for the same
+// matrix work as 192 x 256 and other remainders: 8 row tiles where 192 rows make 11, a whole number of columns where
+// N = 6144.  A wave's 96 columns may lie in two blocks of weight scales: the product of the two scales is formed per
+// pair of fragments, 24 multiplications a slab instead of 8.  Measured with the quantiser in front: 2011 x 6144 x 4096
+// 67.6 us on 256 x 256 tiles in three quarters of a round, 54.6 in one whole round of these (row scales 57.1, 46.7);
+// 1024 x 12288 x 6144 89.4 and 71.0; 2048 x 24576 x 7168 306 and 289.
+//
+// Edges: any M and any N that is a multiple of 8 (rows of either operand past the end read as zero through the buffer
 // descriptors, stores of rows past M fall outside C's descriptor, lanes whose columns lie past N store nothing), K an
 // even number (at least four) of whole 128-byte slabs (the two sets of fragment registers alternate).
 // Sums are formed in the same order as by the eight-wave kernels (one product per slab, promoted in slab order):
@@ -131,18 +138,21 @@ constexpr int kW4GroupedTableBytes = (16 + 4 * kW4GroupedSlots + 8) * 4 + 4 * 96
 // Bound like the plain kernel, by the matrix pipe; the projection ran on the one-tile-per-block kernels before (quantiser
 // included, block scaling): 777 x 10240 x 8192 102.7 -> 72.5 us, 2011 x 10240 x 8192 207 -> 157, 3000 x 6144 x 4096 101 -> 80,
 // 4096 x 10240 x 8192 381 -> 299, 200 x 10240 x 8192 (every tile cut) 66 -> 38; the plain linear of those sizes: 64, 149, 72, 287, 35.
+template <int TN>
+__host__ __device__ constexpr int w4_side_bytes() { return TN == 6 ? 16 * 208 : 2048; }
 template <int TM, int TN, bool BLOCKSCALE, int PROBE, int GROUPED = 0, bool KV = false>
 __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
   constexpr int WM = TM * 16, WN = TN * 16, BM = 2 * WM, BN = 2 * WN;
   constexpr int IA = BM / 32, IB = BN / 32;                  // copy instructions per wave and slab (8 rows each)
   constexpr int SCALE_BYTES = BLOCKSCALE ? 1024 : 0;         // 2 wave rows x 16 lane rows x 8 words
   constexpr int A_STAGE = BM * 128 + SCALE_BYTES, B_STAGE = BN * 128;
-  constexpr int B_BASE = 2 * A_STAGE, SIDE_BASE = B_BASE + 3 * B_STAGE, SIDE_BYTES = 2048;
+  // (a wave's results leave 16 rows x 64 columns at a time, or, of its 96 columns, 16 x 96 with rows 13 x 16 bytes apart)
+  constexpr int B_BASE = 2 * A_STAGE, SIDE_BASE = B_BASE + 3 * B_STAGE, SIDE_BYTES = w4_side_bytes<TN>();
   constexpr int PER_A = IA + (BLOCKSCALE ? 1 : 0), PER_B = IB;
   constexpr int NSTORE = TM * TN / 2;                        // 16-byte stores per lane and tile
   // a product is folded in LAG MFMAs after its own (2: 4 ... 6 % slower, the FMAs then wait for the matrix pipe; 4: the same)
   constexpr int LAG = 3;
-  static_assert(TN == 8 && TM >= 3 && TM <= 8, "wave tile");
+  static_assert((TN == 8 && TM >= 3 && TM <= 6) || (TN == 6 && TM == 8 && !GROUPED && PROBE == 0), "wave tile");
   // Row tiles that share weight columns in the tile order: the 32 blocks of an XCD work on a patch of kGroupM row tiles
   // x 32 / kGroupM column tiles at a time, and what the XCD's L2 fetches for it is the patch's rows of both operands --
   // least for a square patch: 8 x 4 for 128-row tiles (q_b M = 1024: 47 -> 43 us against 4 x 8; o_proj M = 1024: 112 ->
@@ -266,7 +276,7 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
   auto plan_of = [&]() {
     const int bid = opaque_uniform((int)blockIdx.x), G = GROUPED ? grouped_hdr(1) : (int)gridDim.x;
     const int xcd = bid & 7, my = bid >> 3;
-    const int tail_u = PROBE || GROUPED ? 0 : p.tail_units;
+    const int tail_u = PROBE || GROUPED || TN != 8 ? 0 : p.tail_units;
     const int main_total = tail_u > 0 ? (total / G) * G : total;
     const int run_begin = xcd * (main_total >> 3) + (xcd < (main_total & 7) ? xcd : (main_total & 7));
     const int run_len = (main_total >> 3) + (xcd < (main_total & 7) ? 1 : 0);
@@ -530,16 +540,28 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 
-  // (BN = 256: two weight-scale blocks per tile, one per wave column)
+  // (BN = 256: two weight-scale blocks per tile, one per wave column.  BN = 192: a wave's 96 columns may lie in two, the pairs of fragments
+  // from hi_from on in the second, whose scale sits hi_step elements behind the first's: none where there is one block)
   auto bs_block = [&](int tile_n) {
     if constexpr (PROBE != 0) return wn;
-    const int blk = 2 * tile_n + wn;
+    const int blk = (tile_n * BN + wn * WN) / 128;
     return blk < bs_rows ? blk : bs_rows - 1;
   };
+  constexpr bool TWO = BLOCKSCALE && TN == 6;
+  [[maybe_unused]] auto bs_hi_step = [&](int tile_n) {
+    const int c0 = tile_n * BN + wn * WN, blk = c0 / 128;
+    return (c0 + WN - 1) / 128 != blk && blk + 1 < bs_rows ? (uint32_t)p.b_scales_ld : 0u;
+  };
+  [[maybe_unused]] auto hi_from = [&](int tile_n) { return (128 - (tile_n * BN + wn * WN) % 128) / 32; };
   // The weight-block scale of a slab is element bs_cur of the weight scales: that of the slab to come is loaded a slab ahead.
   uint32_t bs_cur = cur_at.bs0 + (uint32_t)(bs_block(tn) * p.b_scales_ld + job.s0);
-  float bs_nxt = 1.f;
+  float bs_nxt = 1.f, bs_nxt_hi = 1.f;
   if constexpr (BLOCKSCALE) bs_nxt = scalar_load_f32(p.b_scales + bs_cur);
+  [[maybe_unused]] uint32_t hi_cur = 0;
+  if constexpr (TWO) {
+    hi_cur = bs_hi_step(tn);
+    bs_nxt_hi = scalar_load_f32(p.b_scales + bs_cur + hi_cur);
+  }
 
   // two sets of fragment registers: a slab is multiplied from one while the next slab's fragments arrive in the other
   v8i bf[2][TN], af[2][TM];
@@ -587,6 +609,8 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
     const SlabAt next0 = slab_at(next_at, next_job.s0, has_next ? 0u : 0x80000000u);
     const uint32_t next_bs0 = next_at.bs0 + (uint32_t)(bs_block(tn2) * p.b_scales_ld + next_job.s0);
     const int job_end = job.s1;
+    [[maybe_unused]] const uint32_t next_hi = TWO ? bs_hi_step(tn2) : 0u;
+    [[maybe_unused]] const int from = TWO ? hi_from(tn) : 0;
     if constexpr (KV) {
       if (tn * BN + wn * WN + WN > p.kv.q_dim && tn * BN + wn * WN < p.N) look_up_rows(cur_at.row0 + wm * WM);
     }
@@ -633,16 +657,32 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
         cur.b = slab + 4 == job_end ? next0.b : cur.b + 128u;
       }
 
-      float s_cur[TM];
+      float s_cur[TWO ? 1 : TM];
+      [[maybe_unused]] float bs_of[TN / 2];  // TWO: of each pair of fragments
       if constexpr (BLOCKSCALE) {
         const float bs = bs_nxt;
+        if constexpr (TWO) {
 #pragma unroll
-        for (int mt = 0; mt < TM; ++mt) s_cur[mt] = sraw[PAR].v[mt] * bs;
+          for (int q = 0; q < TN / 2; ++q) bs_of[q] = q >= from ? bs_nxt_hi : bs;
+        } else {
+#pragma unroll
+          for (int mt = 0; mt < TM; ++mt) s_cur[mt] = sraw[PAR].v[mt] * bs;
+        }
         // the weight-block scale of the next slab (of the next tile behind this tile's last slab)
         if constexpr (PROBE != 0) bs_cur = (bs_cur & ~7u) | ((bs_cur + 1u) & 7u);
         else bs_cur = slab + 1 == job_end ? next_bs0 : bs_cur + 1u;
         bs_nxt = scalar_load_f32(p.b_scales + bs_cur);
+        if constexpr (TWO) {
+          hi_cur = slab + 1 == job_end ? next_hi : hi_cur;
+          bs_nxt_hi = scalar_load_f32(p.b_scales + bs_cur + hi_cur);
+        }
       }
+      // product j folded in: its row group's activation scale times its columns' weight scale (TWO: formed with the first of a pair of fragments)
+      auto fold = [&](auto J, const v4f& product) {
+        constexpr int j = decltype(J)::value, mt = j / TN, nt = j % TN;
+        if constexpr (TWO && nt % 2 == 0) s_cur[0] = sraw[PAR].v[mt] * bs_of[nt / 2];
+        acc[mt][nt] += product * s_cur[TWO ? 0 : mt];
+      };
       [[maybe_unused]] v4f part[LAG + 1];
       // Slot i = MFMA i of the slab, the four FMAs of the product that left the pipe LAG MFMAs ago, and at most one
       // piece of memory work: a fragment read of slab s + 1 (two 16-byte LDS reads) or one copy instruction -- spread
@@ -654,7 +694,7 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
           part[i % (LAG + 1)] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf[PAR][nt], af[PAR][mt], zero, 0, 0, 0, 0, 0, 0);
           if constexpr (i >= LAG) {
             constexpr int j = i - LAG;
-            acc[j / TN][j % TN] += part[j % (LAG + 1)] * s_cur[j / TN];
+            fold(std::integral_constant<int, j>{}, part[j % (LAG + 1)]);
           }
         } else {
           acc[mt][nt] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf[PAR][nt], af[PAR][mt], acc[mt][nt], 0, 0, 0, 0, 0, 0);
@@ -685,8 +725,10 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
       });
       // (the slab's last products: folding them in during the first MFMAs of the next slab instead measured 7 % slower)
       if constexpr (BLOCKSCALE) {
-#pragma unroll
-        for (int j = NSLOT - LAG; j < NSLOT; ++j) acc[j / TN][j % TN] += part[j % (LAG + 1)] * s_cur[j / TN];
+        static_for<LAG>([&](auto L) {
+          constexpr int j = NSLOT - LAG + decltype(L)::value;
+          fold(std::integral_constant<int, j>{}, part[j % (LAG + 1)]);
+        });
       }
       // (the hint sits at the slab's end, where the whole set has arrived: right behind a read it would be a use of the
       // value, and the compiler would wait for the read on the spot)
@@ -718,8 +760,8 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
     }
     // the steps of the epilogue (16 rows x 64 columns of a wave's part: step = 2 * group of rows + half of the columns)
     // that this block converts and stores: all of them, or its share of a tile that is cut
-    int st_lo = 0, st_hi = 2 * TM;
-    if (!GROUPED && job.kind == PIECE) {
+    [[maybe_unused]] int st_lo = 0, st_hi = 2 * TM;
+    if constexpr (!GROUPED && TN == 8) if (job.kind == PIECE) {
       const Plan pl = plan_of();
       const int tail_c = pl.tail_c, T = total - pl.main_total, P = (nslab + pl.tail_u - 1) / pl.tail_u;
       const int q = tail_c / T, t = tail_c - q * T;
@@ -825,8 +867,79 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
     const int lane_e = lane_here();
     const int lm_e = lane_e & 15, lq_e = lane_e >> 4, rr = lane_e >> 3, cc = lane_e & 7;
     const uint32_t c_lane = (uint32_t)rr * c_row_bytes + (uint32_t)cc * 16u;
+    // a lane's eight results of a pair of fragments, as stored
+    auto finish = [&](v4f lo, v4f hi, int q, float a_s) -> v4u_t {
+      if constexpr (KV) {
+        // the sum to bf16, the scales' product to bf16, their product to bf16, then the bias in bf16 (see tile_body)
+        const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          w[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
+          if constexpr (!BLOCKSCALE) {
+            const uint32_t sc = pack_bf16x2(a_s * b_s[q * 8 + 2 * i], a_s * b_s[q * 8 + 2 * i + 1]);
+            w[i] = pack_bf16x2(__uint_as_float(w[i] << 16) * __uint_as_float(sc << 16),
+                               __uint_as_float(w[i] & 0xffff0000u) * __uint_as_float(sc & 0xffff0000u));
+          }
+          if (p.kv.bias)
+            w[i] = pack_bf16x2(__uint_as_float(w[i] << 16) + __uint_as_float(bias[q][i] << 16),
+                               __uint_as_float(w[i] & 0xffff0000u) + __uint_as_float(bias[q][i] & 0xffff0000u));
+        }
+        return v4u_t{w[0], w[1], w[2], w[3]};
+      }
+      if constexpr (!BLOCKSCALE) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float t_lo = lo[i] * a_s, t_hi = hi[i] * a_s;
+          lo[i] = t_lo * b_s[q * 8 + i];
+          hi[i] = t_hi * b_s[q * 8 + 4 + i];
+        }
+      }
+      return v4u_t{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]), pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
+    };
     // (the last column tile may reach past N, which is a multiple of 8: a lane whose eight columns lie there stores out of
     // the descriptor's range, i.e. nothing -- every store is still issued, so the counts of the waits stay exact)
+    if constexpr (TN == 6) {
+      // 16 rows x 96 columns at a time: converted, written to the side buffer and read back as 12 chunks of 16 bytes a row, so that a store
+      // instruction writes five and a third rows of 192 consecutive bytes (a line at a wave's edge is two waves' of one CU)
+      constexpr int PITCH = 208;
+      auto stage = [&](int mt) {
+        float a_s = 1.f;
+        if constexpr (!BLOCKSCALE) a_s = a_s_all[mt];
+#pragma unroll
+        for (int q = 0; q < TN / 2; ++q) {
+          const v4f lo = acc[mt][2 * q], hi = acc[mt][2 * q + 1];
+          *reinterpret_cast<v4u_t*>(wbuf + lm_e * PITCH + (q * 4 + lq_e) * 16) = finish(lo, hi, q, a_s);
+        }
+      };
+      uint32_t rd[3], dst[3];
+      int row_at[3], col_at[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int chunk = i * 64 + lane_e;
+        row_at[i] = chunk / 12;
+        col_at[i] = tn * BN + wn * WN + (chunk - row_at[i] * 12) * 8;
+        rd[i] = (uint32_t)(row_at[i] * PITCH + (chunk - row_at[i] * 12) * 16);
+        dst[i] = col_at[i] < (KV ? p.kv.q_dim : p.N) ? (uint32_t)row_at[i] * c_row_bytes + (uint32_t)(chunk - row_at[i] * 12) * 16u : 0x80000000u;
+      }
+      stage(0);
+      static_for<TM>([&](auto S) {
+        constexpr int mt = decltype(S)::value;
+        v4u_t v[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) v[i] = *reinterpret_cast<const v4u_t*>(wbuf + rd[i]);
+        if constexpr (mt + 1 < TM) stage(mt + 1);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) buffer_store_b128_guarded<2>(v[i], c_rsrc, dst[i], c_tile + (uint32_t)(mt * 16) * c_row_bytes);
+        if constexpr (KV) if (tn * BN + wn * WN + WN > p.kv.q_dim) {
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            const int64_t off = row_tab[mt * 16 + row_at[i]];
+            if (col_at[i] >= p.kv.q_dim && col_at[i] < p.N && off >= 0) *reinterpret_cast<v4u_t*>(kv_dst(p.kv, nullptr, 0, 0, off, col_at[i])) = v[i];
+          }
+        }
+      });
+    } else {
     uint32_t c_lane_h[TN / 4];
 #pragma unroll
     for (int h = 0; h < TN / 4; ++h) c_lane_h[h] = tn * BN + wn * WN + h * 64 + cc * 8 < (KV ? p.kv.q_dim : p.N) ? c_lane : 0x80000000u;
@@ -837,38 +950,9 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
 #pragma unroll
       for (int qq = 0; qq < 2; ++qq) {
         const int q = 2 * h + qq;
-        v4f lo = acc[mt][2 * q], hi = acc[mt][2 * q + 1];
-        if constexpr (KV) {
-          // the sum to bf16, the scales' product to bf16, their product to bf16, then the bias in bf16 (see tile_body)
-          const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-          uint32_t w[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            w[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
-            if constexpr (!BLOCKSCALE) {
-              const uint32_t sc = pack_bf16x2(a_s * b_s[q * 8 + 2 * i], a_s * b_s[q * 8 + 2 * i + 1]);
-              w[i] = pack_bf16x2(__uint_as_float(w[i] << 16) * __uint_as_float(sc << 16),
-                                 __uint_as_float(w[i] & 0xffff0000u) * __uint_as_float(sc & 0xffff0000u));
-            }
-            if (p.kv.bias)
-              w[i] = pack_bf16x2(__uint_as_float(w[i] << 16) + __uint_as_float(bias[q][i] << 16),
-                                 __uint_as_float(w[i] & 0xffff0000u) + __uint_as_float(bias[q][i] & 0xffff0000u));
-          }
-          *reinterpret_cast<v4u_t*>(wbuf + lm_e * 128 + (((qq * 4 + lq_e) ^ (lm_e & 7)) * 16)) = v4u_t{w[0], w[1], w[2], w[3]};
-          continue;
-        }
-        if constexpr (!BLOCKSCALE) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float t_lo = lo[i] * a_s, t_hi = hi[i] * a_s;
-            lo[i] = t_lo * b_s[q * 8 + i];
-            hi[i] = t_hi * b_s[q * 8 + 4 + i];
-          }
-        }
         // (written and read back through the same vector type: to the compiler a store through one type and a load
         // through another need not alias, and it may then move the load in front of the store)
-        *reinterpret_cast<v4u_t*>(wbuf + lm_e * 128 + (((qq * 4 + lq_e) ^ (lm_e & 7)) * 16)) =
-            v4u_t{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]), pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
+        *reinterpret_cast<v4u_t*>(wbuf + lm_e * 128 + (((qq * 4 + lq_e) ^ (lm_e & 7)) * 16)) = finish(acc[mt][2 * q], acc[mt][2 * q + 1], q, a_s);
       }
     };
     // ... read back as 8 rows x one whole 128-byte line per instruction (a wave reads back only what it wrote itself, and
@@ -942,6 +1026,7 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
         }
       }
     }
+    }
     stored = true;
     job = next_job;
     tm = tm2;
@@ -975,7 +1060,7 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
 
 template <int TM, int TN, bool BLOCKSCALE>
 constexpr int w4_lds_bytes() {
-  return 2 * (TM * 32 * 128 + (BLOCKSCALE ? 1024 : 0)) + 3 * (TN * 32 * 128) + 4 * 2048;
+  return 2 * (TM * 32 * 128 + (BLOCKSCALE ? 1024 : 0)) + 3 * (TN * 32 * 128) + 4 * w4_side_bytes<TN>();
 }
 
 // The shapes this kernel takes: bf16 C with 16-byte aligned rows, N a multiple of 8, K a whole and even number of slabs,
@@ -992,15 +1077,21 @@ bool gemm_w4_ok(const GemmArgs& p, bool blockscale) {
   if (rows * p.ldc * 2 >= lim) return false;
   return true;
 }
+// ... and for tiles of 256 x 192, which reach up to 255 rows and 191 columns past the end
+static bool w4_tall_ok(const GemmArgs& p, bool blockscale) {
+  const int64_t lim = 0x7ff00000ll, rows = (int64_t)p.M + 256;
+  return rows * p.lda < lim && ((int64_t)p.N + 192) * p.ldb < lim && rows * p.ldc * 2 < lim && (!blockscale || (p.K / 128 * p.a_scales_ld + rows) * 4 < lim);
+}
 
 template <int TM, bool BLOCKSCALE, int PROBE, bool KV = false>
 static int launch_w4(const GemmArgs& p, unsigned blocks, hipStream_t stream, const char* name) {
   static PerDeviceFlag attr_done;
-  constexpr int lds = w4_lds_bytes<TM, 8, BLOCKSCALE>() + (KV ? 4 * TM * 16 * 8 : 0);  // (the cache rows of each wave's rows)
+  constexpr int TN = TM == 8 ? 6 : 8;
+  constexpr int lds = w4_lds_bytes<TM, TN, BLOCKSCALE>() + (KV ? 4 * TM * 16 * 8 : 0);  // (the cache rows of each wave's rows)
   static_assert(lds <= 160 * 1024, "one block's LDS");
   void (*kern)(GemmArgs);
-  if constexpr (KV) kern = gemm_w4_qkv_kernel<TM, 8, BLOCKSCALE>;
-  else kern = gemm_w4_kernel<TM, 8, BLOCKSCALE, PROBE>;
+  if constexpr (KV) kern = gemm_w4_qkv_kernel<TM, TN, BLOCKSCALE>;
+  else kern = gemm_w4_kernel<TM, TN, BLOCKSCALE, PROBE>;
   bool& done = attr_done.here();
   if (!done) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -1043,11 +1134,12 @@ W4Split gemm_w4_split(int64_t M, int64_t N, int64_t K, int tm) {
   return W4Split{g, (int)u, (size_t)g * 32 * tm * 256 * 4};
 }
 
-// rows of a tile: 32 * tm (tm = 4, 5 or 6 sixteen-row groups per wave); split: cut the tail (p.workspace holds what
-// gemm_w4_split asks for)
+// rows of a tile: 32 * tm (tm = 4, 5 or 6 sixteen-row groups per wave, by 256 columns; 8, by 192); split: cut the tail (p.workspace holds what
+// gemm_w4_split asks for; not with tm = 8)
 int gemm_w4_launch(const GemmArgs& p_in, bool blockscale, int tm, bool split, hipStream_t stream) {
   GemmArgs p = p_in;
-  const int64_t tiles = ceil_div(p.M, 32 * tm) * ceil_div(p.N, 256);
+  if (tm == 8 && !w4_tall_ok(p, blockscale)) tm = 6;
+  const int64_t tiles = ceil_div(p.M, 32 * tm) * ceil_div(p.N, tm == 8 ? 192 : 256);
   const int cus = compute_units();
   unsigned blocks = (unsigned)(tiles < cus ? tiles : cus);
   p.tail_units = 0;
@@ -1067,6 +1159,10 @@ int gemm_w4_launch(const GemmArgs& p_in, bool blockscale, int tm, bool split, hi
       p.streamk_slot = status == hipStreamCaptureStatusNone ? (int)(issued.fetch_add(1, std::memory_order_relaxed) % (kW4FlagSets / 2))
                                                             : kW4FlagSets / 2 + (int)(recorded.fetch_add(1, std::memory_order_relaxed) % (kW4FlagSets / 2));
     }
+  }
+  if (tm == 8) {
+    if (p.kv_on) return blockscale ? launch_w4<8, true, 0, true>(p, blocks, stream, "gemm_w4_qkv_block_256x192") : launch_w4<8, false, 0, true>(p, blocks, stream, "gemm_w4_qkv_row_256x192");
+    return blockscale ? launch_w4<8, true, 0>(p, blocks, stream, "gemm_w4_block_256x192") : launch_w4<8, false, 0>(p, blocks, stream, "gemm_w4_row_256x192");
   }
   if (p.kv_on) {
     if (tm == 4) return blockscale ? launch_w4<4, true, 0, true>(p, blocks, stream, "gemm_w4_qkv_block_128x256") : launch_w4<4, false, 0, true>(p, blocks, stream, "gemm_w4_qkv_row_128x256");

@@ -1,0 +1,54 @@
+"""The four-wave kernel's tiles of 256 rows x 192 columns: the sums are the per-tile kernel's, in its order, so its bits are the
+reference: waves whose 96 columns lie in one block of weight scales, in two of them, in the last one and past it; row tiles and
+column tiles of one row or column group; few and many tiles per block.  The fused QKV projection: exact cases."""
+import pytest
+import torch
+
+import modular_amd as mx
+from modular_amd import _lib, synth
+from test_gpu_qkv import run_case
+from test_gpu_qkv_four_wave import BLOCK, RAGGED, ROW
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 192, 512), (257, 200, 512), (65, 96, 768), (511, 104, 512), (300, 224, 1024), (161, 1544, 768),
+                                   (255, 384, 512), (4096, 2112, 1024), (2011, 6144, 512), (8192, 9000, 512)])
+@pytest.mark.parametrize("kind", ["block", "row"])
+def test_bits_of_the_per_tile_kernel(dev, tune, M, N, K, kind):
+    a, b = synth.random_fp8((M, K), M).to(dev), synth.random_fp8((N, K), N + 1).to(dev)
+    if kind == "block":
+        sa, sb = synth.random_scales((K // 128, M), 3).to(dev), synth.random_scales((-(-N // 128), K // 128), 4).to(dev)
+        gran, g, a_ld, b_ld = (_lib.GRAN_BLOCK, _lib.GRAN_BLOCK), (1, 128, 128), M, K // 128
+    else:
+        sa, sb = synth.random_scales((1, M), 3, lo=0.01, hi=0.1).to(dev), synth.random_scales((N, 1), 4, lo=0.001, hi=0.01).to(dev)
+        gran, g, a_ld, b_ld = (_lib.GRAN_COLWISE, _lib.GRAN_ROWWISE), (-1, -1, -1), M, 1
+    stream = torch.cuda.current_stream(dev).cuda_stream
+
+    def run(c):
+        assert 0 == _lib.lib().maxfp8_matmul_dynamic_scaled_fp8(
+            c.data_ptr(), a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), M, N, K, K, K, N, *gran, *g, a_ld, b_ld,
+            _lib.BF16, _lib.F32, _lib.ALGO_TILED, None, 0, stream), _lib.last_error()
+
+    tune(MAXFP8_TILE="1", MAXFP8_W4="8")
+    assert "256x192" in _lib.matmul_describe(M, N, K, kind == "block", False)
+    guard = torch.full((M + 2, N), -7.0, dtype=torch.bfloat16, device=dev)
+    again = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+    run(guard[1:M + 1])
+    run(again)
+    tune(MAXFP8_TILE="1", MAXFP8_W4=None, MAXFP8_PERSIST="0")
+    want = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+    run(want)
+    assert torch.equal(guard[1:M + 1].view(torch.int16), want.view(torch.int16))
+    assert torch.equal(again.view(torch.int16), want.view(torch.int16))
+    assert bool((guard[0] == -7.0).all()) and bool((guard[M + 1] == -7.0).all())
+
+
+# (Q, K and V meet inside a wave's columns; no Q at all; heads whose ends are tiles' ends)
+@pytest.mark.parametrize("heads", [dict(Hq=21, H=7, D=16), dict(Hq=0, H=21, D=16, k_only=True), dict(Hq=6, H=2, D=64), dict(Hq=3, H=1, D=128)])
+@pytest.mark.parametrize("mnk", [BLOCK, ROW])
+@pytest.mark.parametrize("prompt,cached,page", RAGGED)
+def test_fused_qkv_exact(dev, tune, heads, mnk, prompt, cached, page):
+    tune(MAXFP8_W4="8")
+    run_case(dev, prompt, cached, K=512, mnk=mnk, page=page, layers=2, layer=1, nblocks=40, seed=8, algo="tiled", exact=True,
+             bias="k_only" not in heads, **heads)
