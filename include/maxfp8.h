@@ -268,6 +268,8 @@ int maxfp8_batched_matmul_dynamic_scaled_fp8(
  */
 int maxfp8_matmul_describe(int64_t M, int64_t N, int64_t K, int block_scaling, int with_workspace,
                            char* buf, size_t len);
+/* 1: ahead of what maxfp8_matmul_describe says, a bf16 result whose operands suit the four-wave kernel runs in its tiles of 256 x 192. */
+int maxfp8_matmul_tall(int64_t M, int64_t N, int64_t K, int block_scaling, int with_workspace);
 
 /* Bytes of workspace that lets the tiled kernels use every plan for this shape. */
 size_t maxfp8_matmul_workspace_bytes(int64_t M, int64_t N, int64_t K);

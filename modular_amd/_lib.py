@@ -42,6 +42,7 @@ EXPORTS = (
     "maxfp8_linear_qkv_workspace_bytes",
     "maxfp8_linear_qkv_ragged_paged_scale",
     "maxfp8_matmul_describe",
+    "maxfp8_matmul_tall",
     "maxfp8_grouped_matmul_dynamic_scaled_fp8",
     "maxfp8_grouped_matmul_rowwise_dynamic_scaled_fp8",
     "maxfp8_fused_qkv_matmul_ragged_paged_scale",
@@ -106,6 +107,8 @@ def lib() -> ctypes.CDLL:
     L.maxfp8_matmul_noalloc_max_scratch_bytes.argtypes = []
     L.maxfp8_batched_matmul_dynamic_scaled_fp8.restype = ci
     L.maxfp8_batched_matmul_dynamic_scaled_fp8.argtypes = [vp] * 5 + [i64] * 17 + [ci, ci, ci, vp]
+    L.maxfp8_matmul_tall.restype = ci
+    L.maxfp8_matmul_tall.argtypes = [i64, i64, i64, ci, ci]
     L.maxfp8_matmul_describe.restype = ci
     L.maxfp8_matmul_describe.argtypes = [i64, i64, i64, ci, ci, ctypes.c_char_p, ctypes.c_size_t]
     L.maxfp8_matmul_workspace_bytes.restype = ctypes.c_size_t
@@ -225,3 +228,8 @@ def matmul_describe(M: int, N: int, K: int, block_scaling: bool = True, with_wor
     buf = ctypes.create_string_buffer(256)
     lib().maxfp8_matmul_describe(M, N, K, int(block_scaling), int(with_workspace), buf, 256)
     return buf.value.decode()
+
+
+def matmul_tall(M: int, N: int, K: int, block_scaling: bool = True, with_workspace: bool = True) -> bool:
+    """Whether, ahead of what matmul_describe says, a bf16 result runs in the four-wave kernel's tiles of 256 x 192 (diagnostic)."""
+    return bool(lib().maxfp8_matmul_tall(M, N, K, int(block_scaling), int(with_workspace)))

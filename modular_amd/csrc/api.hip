@@ -55,6 +55,7 @@ int gemm_tiled_dispatch(const GemmArgs&, bool, size_t, int64_t, hipStream_t);
 size_t gemm_tiled_workspace_bytes(int64_t, int64_t, int64_t);
 size_t gemm_tiled_plan_workspace_bytes(int64_t, int64_t, int64_t, bool);
 int gemm_tiled_describe(int64_t, int64_t, int64_t, bool, bool, char*, size_t);
+int gemm_tiled_tall(int64_t, int64_t, int64_t, bool, bool);
 int gemm_grouped_dispatch(const GemmArgs&, bool, int64_t, int64_t, hipStream_t);
 int gemm_skinny_dispatch(const GemmArgs&, bool, int64_t, hipStream_t);
 bool gemm_skinny_quant_ok(int64_t M, int64_t N, int64_t K, bool blockscale);
@@ -641,6 +642,11 @@ static int matmul_common(void* c, const void* a, const void* b, const void* a_sc
 }  // namespace maxfp8
 
 extern "C" {
+
+int maxfp8_matmul_tall(int64_t M, int64_t N, int64_t K, int block_scaling, int with_workspace) {
+  if (M <= 0 || N <= 0 || K <= 0 || choose_kernel(M, N, K, block_scaling != 0).algo != MAXFP8_ALGO_TILED) return 0;
+  return gemm_tiled_tall(M, N, K, block_scaling != 0, with_workspace != 0);
+}
 
 int maxfp8_matmul_describe(int64_t M, int64_t N, int64_t K, int block_scaling, int with_workspace, char* buf, size_t len) {
   if (!buf || len == 0) return 0;

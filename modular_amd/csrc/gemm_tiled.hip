@@ -1710,6 +1710,7 @@ static bool persist_ok(const GemmArgs& p, bool blockscale, dim3 grid) {
 
 // The four-wave kernel (gemm_w4.hip): 0 (no), or the sixteen-row groups per wave -- 5: tiles of 160 x 256, 6: 192 x 256.
 bool gemm_w4_ok(const GemmArgs& p, bool blockscale);
+bool gemm_w4_tall_ok(const GemmArgs& p, bool blockscale);
 bool gemm_w4_grouped_ok(const GemmArgs& p, bool blockscale);
 int gemm_w4_grouped_launch(const GemmArgs& p, bool blockscale, hipStream_t stream);
 bool gemm_grouped_skinny_ok(const GemmArgs& p);
@@ -1998,7 +1999,8 @@ static TwoRegionPlan pick_two_regions(int64_t M, int64_t N, int nslab, bool bloc
 
 // What a tiled matmul will launch: one shape (possibly with K split), two regions, or the four-wave kernel (w4: 0, or
 // its sixteen-row groups per wave).
-struct TiledPlan { int variant; int splits; TwoRegionPlan two; bool streamk; int w4; bool w4_split; };
+// tall: ahead of all of these, the four-wave kernel in tiles of 256 x 192, for calls whose operands it takes; the others run what the rest of the plan says.
+struct TiledPlan { int variant; int splits; TwoRegionPlan two; bool streamk; int w4; bool w4_split; bool tall; };
 
 // One persistent launch of `tiles` tiles on `slots` CUs, a tile taking t microseconds with the chip full: whole rounds
 // cost t each; a last round that fills only part of the chip is faster than a full one but not in proportion (fewer
@@ -2021,7 +2023,6 @@ static float w4_slab(bool blockscale, int tm) { return (blockscale ? kW4SlabBloc
 static float w4_tile(bool blockscale, int tm, int nslab) {
   return tm != 8 ? kW4Tile : !blockscale ? kW4TallTileRow : kW4TallTileBlock + (nslab > 64 ? (float)(nslab - 64) * kW4TallLateSlab : 0.f);
 }
-static const int kW4Heights[4] = {4, 5, 6, 8};
 static int64_t w4_tiles(int64_t M, int64_t N, int tm) { return ceil_div(M, 32 * tm) * ceil_div(N, tm == 8 ? 192 : 256); }
 // ... and of its cut tiles, with few blocks to share the memory with
 static const float kW4CutSlabBlock[3] = {0.646f, 0.71f, 0.84f}, kW4CutSlabRow[3] = {0.56f, 0.72f, 0.80f};
@@ -2068,15 +2069,19 @@ static float w4_plan_cost(int64_t M, int64_t N, int64_t K, bool blockscale, int 
 // against 42; 768 x 2048 x 8192, 16 slabs: 27 against 32), behind with shorter pieces (8 slabs: 25 against 22) and with
 // fewer blocks (128 x 4096 x 14336, 16 tiles in 64 pieces: 38 against 27; 512 x 2048 x 28672, 128 pieces: 64 against 51).
 // The height with the shortest pieces: 338 x 8192 x 28672 96 tiles of 128 rows in two pieces each 117 us, 64 of 192 rows in four 88.
-static int pick_w4(int64_t M, int64_t N, int64_t K, bool blockscale, float other_cost, bool other_splits, size_t workspace_bytes, bool kv_on, bool* split) {
+static int pick_w4(int64_t M, int64_t N, int64_t K, bool blockscale, float other_cost, bool other_splits, size_t workspace_bytes, bool kv_on, bool* split, bool* tall) {
   const int forced = tuning().w4, cut = tuning().w4_split;
-  *split = false;
+  *split = *tall = false;
   if (forced == 0 || !tuning().persist || !w4_shape(M, N, K)) return 0;
+  if (forced == 8) {
+    *tall = true;
+    return 0;
+  }
   const int nslab = (int)(K / 128), slots = compute_units();
   // every tile of height tm cut, where its pieces are worth it (see above; forced: wherever there is a cut)
   auto every_cut = [&](int tm) {
     const W4Split sp = gemm_w4_split(M, N, K, tm);
-    if (tm == 8 || cut == 0 || sp.unit <= 0 || sp.bytes > workspace_bytes || ceil_div(M, 32 * tm) * ceil_div(N, 256) * 2 > slots) return false;
+    if (cut == 0 || sp.unit <= 0 || sp.bytes > workspace_bytes || ceil_div(M, 32 * tm) * ceil_div(N, 256) * 2 > slots) return false;
     // (more than four pieces only where they are long: 128 x 8192 x 28672 in eight pieces of 28 slabs 59 against 64 us,
     // 512 x 2048 x 28672 46 against 52; in eight of 16 slabs 128 x 8192 x 16384 47 against 41.  And only where the rows
     // fill three quarters of the tiles: 48 ... 64 rows on 8192 x 28672 took 56 against 48 ... 51.)
@@ -2099,7 +2104,7 @@ static int pick_w4(int64_t M, int64_t N, int64_t K, bool blockscale, float other
   }
   int best = 0;
   float best_cost = forced > 0 ? 3.0e38f : 0.97f * other_cost;  // (a forced height is taken whatever it costs)
-  for (const int tm : kW4Heights) {
+  for (int tm = 4; tm <= 6; ++tm) {
     if (forced > 0 && tm != forced) continue;
     const int64_t tiles = w4_tiles(M, N, tm);
     // (half a round or less: more, smaller tiles and a K split are the better fit; a little more than half is not: 166 x 36864 x 7168 in
@@ -2122,13 +2127,6 @@ static int pick_w4(int64_t M, int64_t N, int64_t K, bool blockscale, float other
     // tiles 33 and 34; 937 x 8192 x 6144 in 256 of them 48 and 57, 51 and 69)
     const bool slow = kv_on && !blockscale && tm == 4 && tiles * 8 < slots * 7;
     const float whole = slow ? persistent_cost(tiles, slots, (float)nslab * 0.93f + kW4Tile) : w4_plan_cost(M, N, K, blockscale, tm, false);
-    if (tm == 8) {
-      // (no cut.  Against another height it has to be 2 per cent ahead, and against whole tiles of 128 rows with block scaling, which are quicker than
-      // priced where the weights are small, 7: 1024 x 24576 x 1536 47.2 us in 512 of these tiles, 46.0 in 768 of those, 4096 x 6144 x 1024 39.9 and 39.0)
-      const float ahead = !best || forced > 0 ? 1.f : (best == 4 && blockscale && !*split ? 0.93f : 0.98f);
-      if (whole < ahead * best_cost) { best = tm; best_cost = whole; *split = false; }
-      continue;
-    }
     if (whole < best_cost) { best = tm; best_cost = whole; *split = false; }
     const W4Split sp = gemm_w4_split(M, N, K, tm);
     if (cut != 0 && sp.unit > 0 && sp.bytes <= workspace_bytes) {
@@ -2136,6 +2134,15 @@ static int pick_w4(int64_t M, int64_t N, int64_t K, bool blockscale, float other
       if (cut == 1) with_cut *= 1.0e-3f;  // (switched on: wherever there is one)
       if (with_cut < best_cost) { best = tm; best_cost = with_cut; *split = true; }
     }
+  }
+  // Tiles of 256 x 192 (no cut).  Against another height they have to be 2 per cent ahead, and against whole tiles of 128 rows with block scaling, which are
+  // quicker than priced where the weights are small, 7: 1024 x 24576 x 1536 47.2 us in 512 of these tiles, 46.0 in 768 of those, 4096 x 6144 x 1024 39.9 and 39.0.
+  // (Ahead: 2048 x 6144 x 4096 54.5 us against 65.8 on 256 x 256 tiles, 4096 x 18432 x 7168 441 against 454 on 192 x 256 with a cut tail.)
+  if (forced < 0) {
+    const int64_t tiles = w4_tiles(M, N, 8);
+    const bool small = tiles * 2 <= slots || (kv_on && tiles * 4 < slots * 3 && (!blockscale || N * K < ((int64_t)3 << 24)));
+    const float ahead = !best ? 1.f : (best == 4 && blockscale && !*split ? 0.93f : 0.98f);
+    *tall = !small && w4_plan_cost(M, N, K, blockscale, 8, false) < ahead * best_cost;
   }
   return best;
 }
@@ -2151,7 +2158,7 @@ static bool streamk_shape(int64_t M, int64_t N, size_t workspace_bytes) {
 }
 static TiledPlan make_plan(int64_t M, int64_t N, int64_t K, bool blockscale, bool has_workspace, size_t workspace_bytes,
                            int64_t batch, bool kv_on) {
-  TiledPlan plan = {0, 1, {0, 0, 0, 0, 0.f}, false, 0, false};
+  TiledPlan plan = {0, 1, {0, 0, 0, 0, 0.f}, false, 0, false, false};
   const int nslab = (int)ceil_div(K, 128);
   plan.variant = tile_override();
   const bool free_choice = plan.variant == 0;
@@ -2196,9 +2203,9 @@ static TiledPlan make_plan(int64_t M, int64_t N, int64_t K, bool blockscale, boo
     if (kv_on && has_workspace && free_choice) {
       const TileShape& u = kShapes[pick_shape(M, N, nslab, blockscale, true) - 1];
       if (pick_splits(ceil_div(M, u.bm) * ceil_div(N, u.bn), u.slots, nslab) > 1)
-        plan.w4 = pick_w4(M, N, K, blockscale, other, true, workspace_bytes, kv_on, &plan.w4_split);
+        plan.w4 = pick_w4(M, N, K, blockscale, other, true, workspace_bytes, kv_on, &plan.w4_split, &plan.tall);
     }
-    if (!plan.w4) plan.w4 = pick_w4(M, N, K, blockscale, other, wants_split, has_workspace ? workspace_bytes : 0, kv_on, &plan.w4_split);
+    if (!plan.w4) plan.w4 = pick_w4(M, N, K, blockscale, other, wants_split, has_workspace ? workspace_bytes : 0, kv_on, &plan.w4_split, &plan.tall);
     if (plan.w4) plan.splits = 1;
   }
   return plan;
@@ -2274,10 +2281,11 @@ static float few_rows_cost(const TiledPlan& plan, int64_t M, int64_t N, int64_t 
 float gemm_tiled_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
   const TiledPlan plan = cached_plan(M, N, K, blockscale, true, ~(size_t)0, 1, false);
   const float slabs = (float)ceil_div(K, 128), stream = (float)N * (float)K / 6e6f;
-  if (M <= 64 && !plan.two.axis) {
+  if (M <= 64 && !plan.two.axis && !plan.tall) {
     const float few = few_rows_cost(plan, M, N, K, blockscale);
     if (few > 0.f) return few;
   }
+  if (plan.tall) return w4_plan_cost(M, N, K, blockscale, 8, false);
   if (plan.w4) return w4_plan_cost(M, N, K, blockscale, plan.w4, plan.w4_split);
   if (plan.two.axis) return plan.two.cost;
   if (plan.splits > 1)
@@ -2295,6 +2303,7 @@ float gemm_tiled_cost(int64_t M, int64_t N, int64_t K, bool blockscale) {
 // The same for a fused QKV matmul, of any plan (with the workspace it asks for, or without any)
 float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool has_workspace) {
   const TiledPlan plan = cached_plan(M, N, K, blockscale, has_workspace, has_workspace ? ~(size_t)0 : 0, 1, true);
+  if (plan.tall) return w4_plan_cost(M, N, K, blockscale, 8, false);
   if (plan.w4) return w4_plan_cost(M, N, K, blockscale, plan.w4, plan.w4_split);
   if (plan.variant == 4) return three_stage_cost(M, N, K, blockscale);
   return region_cost(M, N, (int)ceil_div(K, 128), kShapes[plan.variant - 1], blockscale, true);
@@ -2304,6 +2313,11 @@ float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool
 size_t gemm_tiled_qkv_workspace_bytes(int64_t M, int64_t N, int64_t K, bool blockscale) {
   const TiledPlan plan = cached_plan(M, N, K, blockscale, true, ~(size_t)0, 1, true);
   return plan.w4 && plan.w4_split ? gemm_w4_split(M, N, K, plan.w4).bytes : 0;
+}
+
+// Whether a bf16 result of this shape runs in tiles of 256 x 192 ahead of what gemm_tiled_describe says
+int gemm_tiled_tall(int64_t M, int64_t N, int64_t K, bool blockscale, bool has_workspace) {
+  return make_plan(M, N, K, blockscale, has_workspace, has_workspace ? gemm_tiled_workspace_bytes(M, N, K) : 0, 1, false).tall ? 1 : 0;
 }
 
 // "256x256 x896" / "256x256 x448, K split 2" / "256x256 x768 + columns from 24576: 256x128 x256"
@@ -2319,7 +2333,7 @@ int gemm_tiled_describe(int64_t M, int64_t N, int64_t K, bool blockscale, bool h
                     n_tiles * 2 <= compute_units() ? "every tile" : "tail", sp.unit);
   }
   if (plan.w4)
-    return snprintf(buf, len, "%dx%d x%lld persistent, four waves", 32 * plan.w4, plan.w4 == 8 ? 192 : 256, (long long)w4_tiles(M, N, plan.w4));
+    return snprintf(buf, len, "%dx256 x%lld persistent, four waves", 32 * plan.w4, (long long)w4_tiles(M, N, plan.w4));
   if (plan.two.axis && !plan.streamk) {
     const TileShape &a = kShapes[plan.two.v1 - 1], &b = kShapes[plan.two.v2 - 1];
     const bool cols = plan.two.axis == 1;
@@ -2356,6 +2370,10 @@ int gemm_tiled_dispatch(const GemmArgs& p_in, bool blockscale, size_t workspace_
     // (the plan knows the shape; whether this call's pointers and strides suit the persistent kernels is checked here)
     if (persist_ok(p, blockscale, dim3(1, 1, 1)))
       return blockscale ? launch_streamk<true>(p, stream, "gemm_streamk_block_256x256") : launch_streamk<false>(p, stream, "gemm_streamk_row_256x256");
+  }
+  if (plan.tall && gemm_w4_tall_ok(p, blockscale)) {
+    p.splits = 1;
+    return gemm_w4_launch(p, blockscale, 8, false, stream);
   }
   if (plan.w4) {
     p.splits = 1;

@@ -1078,7 +1078,8 @@ bool gemm_w4_ok(const GemmArgs& p, bool blockscale) {
   return true;
 }
 // ... and for tiles of 256 x 192, which reach up to 255 rows and 191 columns past the end
-static bool w4_tall_ok(const GemmArgs& p, bool blockscale) {
+bool gemm_w4_tall_ok(const GemmArgs& p, bool blockscale) {
+  if (!gemm_w4_ok(p, blockscale)) return false;
   const int64_t lim = 0x7ff00000ll, rows = (int64_t)p.M + 256;
   return rows * p.lda < lim && ((int64_t)p.N + 192) * p.ldb < lim && rows * p.ldc * 2 < lim && (!blockscale || (p.K / 128 * p.a_scales_ld + rows) * 4 < lim);
 }
@@ -1138,7 +1139,6 @@ W4Split gemm_w4_split(int64_t M, int64_t N, int64_t K, int tm) {
 // gemm_w4_split asks for; not with tm = 8)
 int gemm_w4_launch(const GemmArgs& p_in, bool blockscale, int tm, bool split, hipStream_t stream) {
   GemmArgs p = p_in;
-  if (tm == 8 && !w4_tall_ok(p, blockscale)) tm = 6;
   const int64_t tiles = ceil_div(p.M, 32 * tm) * ceil_div(p.N, tm == 8 ? 192 : 256);
   const int cus = compute_units();
   unsigned blocks = (unsigned)(tiles < cus ? tiles : cus);

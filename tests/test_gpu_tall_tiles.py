@@ -31,7 +31,7 @@ def test_bits_of_the_per_tile_kernel(dev, tune, M, N, K, kind):
             _lib.BF16, _lib.F32, _lib.ALGO_TILED, None, 0, stream), _lib.last_error()
 
     tune(MAXFP8_TILE="1", MAXFP8_W4="8")
-    assert "256x192" in _lib.matmul_describe(M, N, K, kind == "block", False)
+    assert _lib.matmul_tall(M, N, K, kind == "block", False)
     guard = torch.full((M + 2, N), -7.0, dtype=torch.bfloat16, device=dev)
     again = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
     run(guard[1:M + 1])
@@ -42,6 +42,12 @@ def test_bits_of_the_per_tile_kernel(dev, tune, M, N, K, kind):
     assert torch.equal(guard[1:M + 1].view(torch.int16), want.view(torch.int16))
     assert torch.equal(again.view(torch.int16), want.view(torch.int16))
     assert bool((guard[0] == -7.0).all()) and bool((guard[M + 1] == -7.0).all())
+
+
+def test_where_they_are_taken():
+    assert _lib.matmul_tall(2011, 6144, 4096) and _lib.matmul_tall(2048, 24576, 7168, False)
+    # (as many tiles of 192 x 256 and a long K; half a round; row tiles mostly padding; K not an even number of slabs)
+    assert not any(_lib.matmul_tall(*s) for s in ((16384, 8192, 28672), (2048, 2112, 4096), (260, 24576, 4096), (2011, 6144, 4096 + 128)))
 
 
 # (Q, K and V meet inside a wave's columns; no Q at all; heads whose ends are tiles' ends)
