@@ -30,14 +30,7 @@
 // Promotion: the MFMA of (16-row group mt, fragment nt) writes a fresh product, and the four FMAs that fold it into the
 // accumulators are issued LAG MFMAs later, when the product has left the matrix pipe.
 //
-// Tile shapes: 128, 160 or 192 rows by 256 columns (a wave: 64, 80 or 96 x 128), and 256 x 192 (128 x 96), for the same
-// matrix work as 192 x 256 and other remainders: 8 row tiles where 192 rows make 11, a whole number of columns where
-// N = 6144.  A wave's 96 columns may lie in two blocks of weight scales: the product of the two scales is formed per
-// pair of fragments, 24 multiplications a slab instead of 8.  Measured with the quantiser in front: 2011 x 6144 x 4096
-// 67.6 us on 256 x 256 tiles in three quarters of a round, 54.6 in one whole round of these (row scales 57.1, 46.7);
-// 1024 x 12288 x 6144 89.4 and 71.0; 2048 x 24576 x 7168 306 and 289.
-//
-// Edges: any M and any N that is a multiple of 8 (rows of either operand past the end read as zero through the buffer
+// Tiles: any M and any N that is a multiple of 8 (rows of either operand past the end read as zero through the buffer
 // descriptors, stores of rows past M fall outside C's descriptor, lanes whose columns lie past N store nothing), K an
 // even number (at least four) of whole 128-byte slabs (the two sets of fragment registers alternate).
 // Sums are formed in the same order as by the eight-wave kernels (one product per slab, promoted in slab order):
@@ -138,6 +131,7 @@ constexpr int kW4GroupedTableBytes = (16 + 4 * kW4GroupedSlots + 8) * 4 + 4 * 96
 // Bound like the plain kernel, by the matrix pipe; the projection ran on the one-tile-per-block kernels before (quantiser
 // included, block scaling): 777 x 10240 x 8192 102.7 -> 72.5 us, 2011 x 10240 x 8192 207 -> 157, 3000 x 6144 x 4096 101 -> 80,
 // 4096 x 10240 x 8192 381 -> 299, 200 x 10240 x 8192 (every tile cut) 66 -> 38; the plain linear of those sizes: 64, 149, 72, 287, 35.
+constexpr int kW4LaneSequences = 63;  // sequences whose starts, and the last one's end, fit a wave's lanes
 template <int TN>
 __host__ __device__ constexpr int w4_side_bytes() { return TN == 6 ? 16 * 208 : 2048; }
 template <int TM, int TN, bool BLOCKSCALE, int PROBE, int GROUPED = 0, bool KV = false>
@@ -513,12 +507,48 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
         if (j * 64 + l < WM) row_tab[j * 64 + l] = off[j];
     }
   };
+  // KV, the first tile: the starts of up to 63 sequences and their cached lengths are one load each, issued in front of the first slabs' copies; the
+  // searches then run on the lanes' values and the pages are looked up while those copies are on their way.  (Behind the copies' wait, with the
+  // searches and lengths a chain of loads, the look-up cost 2 us: with the stores below, 2011 x 6144 x 4096 of five prompts 61.5 -> 58.6, 1024 42.6 -> 41.0.)
+  [[maybe_unused]] uint32_t seq_first = 0u, seq_cached = 0u;
+  [[maybe_unused]] auto load_sequences = [&]() {
+    const int l = lane_here();
+    if (l <= p.kv.batch) seq_first = p.kv.row_offsets[l];
+    if (l < p.kv.batch) seq_cached = p.kv.cache_lengths[l];
+  };
+  [[maybe_unused]] auto look_up_first_rows = [&](int row0) {
+    const KvStore& kv = p.kv;
+    constexpr int R = (WM + 63) / 64;
+    const int l = lane_here();
+    const int steps = kv.batch > 1 ? 32 - __builtin_clz((unsigned)(kv.batch - 1)) : 0;
+    uint32_t blk[R], slot_r[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int m = row0 + j * 64 + l;
+      int low = 0, high = kv.batch;  // (the last sequence whose first row is <= m)
+      for (int s = 0; s < steps; ++s) {
+        const int mid = (low + high) >> 1;
+        if ((int64_t)m >= (int64_t)(uint32_t)__shfl((int)seq_first, mid, 64)) low = mid; else high = mid;
+      }
+      const uint32_t token = (uint32_t)m - (uint32_t)__shfl((int)seq_first, low, 64) + (uint32_t)__shfl((int)seq_cached, low, 64);
+      const uint32_t page = token / (uint32_t)kv.page_size;
+      slot_r[j] = token - page * (uint32_t)kv.page_size;
+      blk[j] = j * 64 + l < WM && m < p.M && (int64_t)page < kv.lut_ld ? kv.lookup_table[(int64_t)low * kv.lut_ld + page] : 0xffffffffu;
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+      if (j * 64 + l < WM) row_tab[j * 64 + l] = (int64_t)blk[j] < kv.num_blocks ? (int64_t)blk[j] * kv.block_stride + (int64_t)slot_r[j] * kv.row_elems : -1;
+  };
   // ---- prologue: slabs 0 and 1 of the first tile
   int tm, tn, slot;
   locate(job.tile, tm, tn, slot);
   if constexpr (PROBE != 0) tm = tn = 0;
   TileAt cur_at = tile_at(tm, tn, slot);
   dma_idx(cur_at.row0);
+  [[maybe_unused]] const bool rows_now = KV && p.kv.batch <= kW4LaneSequences && tn * BN + wn * WN + WN > p.kv.q_dim && tn * BN + wn * WN < p.N;
+  if constexpr (KV) {
+    if (rows_now) load_sequences();
+  }
   {
     const SlabAt s0 = slab_at(cur_at, job.s0, 0u), s1 = slab_at(cur_at, job.s0 + 1, 0u), s2 = slab_at(cur_at, job.s0 + 2, 0u);
 #pragma unroll
@@ -531,6 +561,9 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
     for (int idx = 0; idx < PER_B; ++idx) dma_b(s1, 1, idx);
 #pragma unroll
     for (int idx = 0; idx < PER_B; ++idx) dma_b(s2, 2, idx);
+  }
+  if constexpr (KV) {
+    if (rows_now) look_up_first_rows(cur_at.row0 + wm * WM);
   }
   if constexpr (PROBE == 2) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -612,7 +645,7 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
     [[maybe_unused]] const uint32_t next_hi = TWO ? bs_hi_step(tn2) : 0u;
     [[maybe_unused]] const int from = TWO ? hi_from(tn) : 0;
     if constexpr (KV) {
-      if (tn * BN + wn * WN + WN > p.kv.q_dim && tn * BN + wn * WN < p.N) look_up_rows(cur_at.row0 + wm * WM);
+      if (!(k == 0 && rows_now) && tn * BN + wn * WN + WN > p.kv.q_dim && tn * BN + wn * WN < p.N) look_up_rows(cur_at.row0 + wm * WM);
     }
 
     v4f acc[TM][TN];
@@ -922,21 +955,36 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
         rd[i] = (uint32_t)(row_at[i] * PITCH + (chunk - row_at[i] * 12) * 16);
         dst[i] = col_at[i] < (KV ? p.kv.q_dim : p.N) ? (uint32_t)row_at[i] * c_row_bytes + (uint32_t)(chunk - row_at[i] * 12) * 16u : 0x80000000u;
       }
+      // (the columns of K and V: where they begin in the cache, without the row's offset)
+      [[maybe_unused]] uint16_t* kv_col[3];
+      [[maybe_unused]] bool kv_live[3];
+      if constexpr (KV) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          kv_live[i] = col_at[i] >= p.kv.q_dim && col_at[i] < p.N;
+          kv_col[i] = kv_dst(p.kv, nullptr, 0, 0, 0, max(col_at[i], p.kv.q_dim));
+        }
+      }
+      const bool has_kv = KV && tn * BN + wn * WN + WN > p.kv.q_dim;
       stage(0);
       static_for<TM>([&](auto S) {
         constexpr int mt = decltype(S)::value;
         v4u_t v[3];
+        [[maybe_unused]] int64_t off[3];
 #pragma unroll
         for (int i = 0; i < 3; ++i) v[i] = *reinterpret_cast<const v4u_t*>(wbuf + rd[i]);
+        // (a step's row offsets with its results: read store by store they were a chain of LDS round trips, a third of the 3 us that the cache's stores took)
+        if constexpr (KV) {
+#pragma unroll
+          for (int i = 0; i < 3; ++i) off[i] = row_tab[mt * 16 + row_at[i]];
+        }
         if constexpr (mt + 1 < TM) stage(mt + 1);
 #pragma unroll
         for (int i = 0; i < 3; ++i) buffer_store_b128_guarded<2>(v[i], c_rsrc, dst[i], c_tile + (uint32_t)(mt * 16) * c_row_bytes);
-        if constexpr (KV) if (tn * BN + wn * WN + WN > p.kv.q_dim) {
+        if constexpr (KV) if (has_kv) {
 #pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            const int64_t off = row_tab[mt * 16 + row_at[i]];
-            if (col_at[i] >= p.kv.q_dim && col_at[i] < p.N && off >= 0) *reinterpret_cast<v4u_t*>(kv_dst(p.kv, nullptr, 0, 0, off, col_at[i])) = v[i];
-          }
+          for (int i = 0; i < 3; ++i)
+            if (kv_live[i] && off[i] >= 0) *reinterpret_cast<v4u_t*>(kv_col[i] + off[i]) = v[i];
         }
       });
     } else {
@@ -977,6 +1025,11 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
     const __amdgpu_buffer_rsrc_t c_rsrc_tile =
         GROUPED ? t2_rsrc(p.c, t2_clamp_u32(((int64_t)(cur_at.row_end - 1) * p.ldc + p.N) * 2)) : c_rsrc;
     auto store_step = [&](const v4u_t (&v)[2], const uint32_t (&dst)[2], int mt, int h) {
+      [[maybe_unused]] int64_t off[2];
+      if constexpr (KV) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) off[i] = row_tab[mt * 16 + i * 8 + rr];
+      }
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         if constexpr (SCATTER)
@@ -988,10 +1041,8 @@ __device__ __forceinline__ void w4_body(const GemmArgs& p, uint8_t* smem) {
         if (tn * BN + wn * WN + h * 64 + 64 > p.kv.q_dim) {
           const int n = tn * BN + wn * WN + h * 64 + cc * 8;
 #pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            const int64_t off = row_tab[mt * 16 + i * 8 + rr];
-            if (n >= p.kv.q_dim && n < p.N && off >= 0) *reinterpret_cast<v4u_t*>(kv_dst(p.kv, nullptr, 0, 0, off, n)) = v[i];
-          }
+          for (int i = 0; i < 2; ++i)
+            if (n >= p.kv.q_dim && n < p.N && off[i] >= 0) *reinterpret_cast<v4u_t*>(kv_dst(p.kv, nullptr, 0, 0, off[i], n)) = v[i];
         }
       }
     };

@@ -58,3 +58,13 @@ def test_fused_qkv_exact(dev, tune, heads, mnk, prompt, cached, page):
     tune(MAXFP8_W4="8")
     run_case(dev, prompt, cached, K=512, mnk=mnk, page=page, layers=2, layer=1, nblocks=40, seed=8, algo="tiled", exact=True,
              bias="k_only" not in heads, **heads)
+
+
+# (the first tile's rows: the starts of up to 63 sequences sit in a wave's lanes, those of more are searched in memory; empty ones among them)
+@pytest.mark.parametrize("batch", [1, 2, 62, 63, 64, 130])
+@pytest.mark.parametrize("tm", ["4", "8"])
+def test_fused_qkv_sequences(dev, tune, tm, batch):
+    tune(MAXFP8_W4=tm)
+    prompt, cached = [(5 * i + 3) % 8 * (40 if batch < 3 else 1) for i in range(batch)], [(7 * i) % 50 for i in range(batch)]
+    run_case(dev, prompt, cached, Hq=6, H=2, D=64, K=512, mnk=ROW, page=16, layers=1, layer=0, nblocks=1100, seed=batch,
+             algo="tiled", exact=True)
