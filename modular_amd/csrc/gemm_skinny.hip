@@ -742,8 +742,15 @@ static int launch_grouped_skinny(const GemmArgs& p, int64_t most_tiles, hipStrea
 // experts of 7168 x 2048, 8 per token, 1 / 8 / 32 / 48 / 64 / 128 tokens 137 / 213 / 395 / 408 / 453 / 565 and 71 / 173 / 323 / 401 / 469 / 713; 128 of 4096 x 1536,
 // 8 per token, 1 / 16 / 64 / 80 tokens 95 / 146 / 251 / 254 and 45 / 116 / 240 / 274; 64 of 2048 x 1408, 6 per token, 1 / 16 / 80 / 96 tokens 70 / 88 / 121 /
 // 121 and 32 / 52 / 115 / 126.  Level at 400, 576 and 510 rows: what turns it is the slots of more than 32 rows, whose weights are read more than once.
-bool gemm_grouped_skinny_ok(const GemmArgs& p) {
-  return p.M <= tuning().grouped_decode && p.num_active <= GroupedSkinnyCfg<2, true>::MAX_SLOTS;
+// So few slots turn it at fewer rows: one matmul of 7168 x 2048, 2 slots with 64 / 128 / 256 rows in all 42 / 28 / 29 us and 17 / 30 / 57, 4 slots with 128 / 256
+// 44 / 29 and 27 / 50, 8 with 256 / 448 41 / 40 and 31 / 57; 4096 x 7168, 4 slots with 128 / 256 / 448 123 / 64 / 70 and 41 / 79 / 143.  And one large slot among many: 16 slots,
+// half of 256 / 448 rows in one of them (136 / 238), 4096 x 7168 107 / 116 and 116 / 158, 7168 x 2048 54 / 60 and 56 / 72.
+// max_rows: the caller's bound on a slot's rows; all rows there are stands for one that does not know.
+bool gemm_grouped_skinny_ok(const GemmArgs& p, int64_t max_rows) {
+  if (p.num_active > GroupedSkinnyCfg<2, true>::MAX_SLOTS) return false;
+  const int forced = tuning().grouped_decode;
+  if (forced >= 0) return p.M <= forced;
+  return p.M <= 448 && p.M <= 64 + 20 * p.num_active && (max_rows <= 128 || max_rows >= p.M);
 }
 int gemm_grouped_skinny_dispatch(const GemmArgs& p, bool blockscale, hipStream_t stream) {
   const int64_t slots = p.M < p.num_active ? p.M : p.num_active, wide = slots * ceil_div(p.N, 32);

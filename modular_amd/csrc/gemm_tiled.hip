@@ -1713,7 +1713,7 @@ bool gemm_w4_ok(const GemmArgs& p, bool blockscale);
 bool gemm_w4_tall_ok(const GemmArgs& p, bool blockscale);
 bool gemm_w4_grouped_ok(const GemmArgs& p, bool blockscale);
 int gemm_w4_grouped_launch(const GemmArgs& p, bool blockscale, hipStream_t stream);
-bool gemm_grouped_skinny_ok(const GemmArgs& p);
+bool gemm_grouped_skinny_ok(const GemmArgs& p, int64_t max_rows);
 int gemm_grouped_skinny_dispatch(const GemmArgs& p, bool blockscale, hipStream_t stream);
 int gemm_w4_launch(const GemmArgs& p, bool blockscale, int tm, bool split, hipStream_t stream);
 W4Split gemm_w4_split(int64_t M, int64_t N, int64_t K, int tm);
@@ -2490,7 +2490,7 @@ int gemm_grouped_dispatch(const GemmArgs& p_in, bool blockscale, int64_t T, int6
   // One persistent launch that shares the chip out between its four kinds of tiles (the tuning switch
   // `grouped_persist` = 0 goes back to the two launches below).
   if (tuning().grouped_persist && !big && p.num_active <= kGroupedMaxSlots) {
-    if (tune == 0 && gemm_grouped_skinny_ok(p)) return gemm_grouped_skinny_dispatch(p, blockscale, stream);
+    if (tune == 0 && gemm_grouped_skinny_ok(p, max_tokens)) return gemm_grouped_skinny_dispatch(p, blockscale, stream);
     p.share_bias = tuning().grouped_share * 2.0f;
     // A slot of more than 128 rows possible, and enough rows for it to matter: every slot's full 192-row
     // tiles, and a rest of more than 128 rows, go to the four-wave kernel (a quarter faster per row than the L tiles

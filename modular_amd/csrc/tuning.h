@@ -15,7 +15,7 @@
 //   MAXFP8_BIG_ROWS=n          grouped: slots with at least n rows use the large-tile launch (1024)
 //   MAXFP8_GROUPED_PERSIST=0   grouped: two launches (large tiles / the rest) instead of the one persistent launch
 //   MAXFP8_GROUPED_OVERLAP=0   grouped, two launches: in line on the caller's stream
-//   MAXFP8_GROUPED_DECODE=n    grouped: matmuls of at most n rows in all on the decode kernel's grouped form (0: none)
+//   MAXFP8_GROUPED_DECODE=n    grouped: matmuls of at most n rows in all on the decode kernel's grouped form (0: none; unset: by rows and slots)
 //   MAXFP8_GROUPED_SHARE=x     grouped: scales the estimate of how much of the chip the small tiles need (0.5)
 //   MAXFP8_SKINNY_ALDS=0       decode kernel: activations loaded per slab even where a wave's share of them fits LDS
 //   MAXFP8_SKINNY_QUANT=0      linears: always the quantiser's launch in front of the decode kernel
@@ -37,7 +37,7 @@ struct Tuning {
   int streamk = 1;
   int big_rows = 1024;
   bool grouped_persist = true;
-  int grouped_decode = 448;
+  int grouped_decode = -1;
   bool grouped_overlap = true;
   float grouped_share = 0.5f;
   // The grouped matmul's full 192-row tiles on the four-wave kernel, beside the persistent launch of the rest (block

@@ -27,9 +27,9 @@ def exact(counts, ids, N, K, kind, dev, spare=3):
     return ints(T, K), ints(E, N, K), *scales, off.to(torch.uint32).to(dev), torch.tensor(list(ids) + [-1] * (E - len(ids)), dtype=torch.int32).to(dev)
 
 
-def run(case, kind, out, active, row_index=None):
+def run(case, kind, out, active, row_index=None, most=None):
     a, b, sa, sb, off, ids = case
-    stats = torch.tensor([a.shape[0], active], dtype=torch.int64).to(torch.uint32)
+    stats = torch.tensor([most or a.shape[0], active], dtype=torch.int64).to(torch.uint32)
     if kind == "row":
         return mx.grouped_matmul_rowwise_dynamic_scaled_fp8(a, b, sa, sb, off, ids, stats, out_type=out)
     return mx.grouped_dynamic_scaled_fp8_matmul(a, b, sa, sb, off, ids, stats, BLK.input_scale, BLK.weight_scale, out_type=out,
@@ -78,12 +78,16 @@ def test_row_index_many_slots_and_stale_offsets(dev, tune):
     assert torch.equal(run((a, b, sa, sb, stale, ids), "block", torch.bfloat16, 2), want)
 
 
-def test_up_to_how_many_rows(dev):
+# rows in all, slots, the caller's bound on a slot's rows (None: the rows in all)
+@pytest.mark.parametrize("rows, slots, most, decode", [(448, 20, None, True), (449, 20, None, False), (84, 1, None, True), (85, 1, None, False), (104, 2, None, True),
+                                                       (105, 2, None, False), (440, 20, 128, True), (440, 20, 129, False), (512, 300, 2, False)])
+def test_up_to_how_many_rows(dev, rows, slots, most, decode):
     from torch.profiler import ProfilerActivity, profile
 
-    for rows, name in ((448, "gemm_grouped_skinny_kernel"), (449, "gemm_grouped_persist_kernel")):
-        operands = exact([rows - 1, 1], [0, 1], 32, 128, "block", dev, spare=0)
-        with profile(activities=[ProfilerActivity.CUDA]) as seen:
-            run(operands, "block", torch.bfloat16, 2)
-            torch.cuda.synchronize()
-        assert any(name in e.name for e in seen.events()), rows
+    even = rows // slots
+    operands = exact([rows - even * (slots - 1)] + [even] * (slots - 1), list(range(slots)), 32, 128, "block", dev, spare=0)
+    with profile(activities=[ProfilerActivity.CUDA]) as seen:
+        run(operands, "block", torch.bfloat16, slots, most=most)
+        torch.cuda.synchronize()
+    names = [e.name for e in seen.events()]
+    assert any("gemm_grouped_skinny_kernel" in n for n in names) == decode and any("gemm_grouped_persist_kernel" in n for n in names) != decode
