@@ -262,13 +262,14 @@ int maxfp8_batched_matmul_dynamic_scaled_fp8(
 
 /*
  * Diagnostic: which launches MAXFP8_ALGO_AUTO makes for a fast-layout M x N x K matmul, as text
- * ("256x256 x768 + columns from 24576: 256x128 x256", "256x128 x112, K split 4", "64x48 x86, 1 per CU, K split over the block's waves"
- * -- the small tiles of gemm_mid_kernel, blocks per CU --, "skinny" -- the decode kernel, as MAXFP8_ALGO_SKINNY).
+ * ("256x256 x768 + columns from 24576: 256x128 x256", "256x128 x112, K split 4", "256x192 x256 persistent, four waves",
+ * "64x48 x86, 1 per CU, K split over the block's waves" -- the small tiles of gemm_mid_kernel, blocks per CU --, "skinny" -- the decode kernel,
+ * as MAXFP8_ALGO_SKINNY).  Of a bf16 result with 16-byte aligned rows: another runs the plan next to it where the kernel named takes no such result.
  * Returns the length snprintf would have written.  No counterpart in the reference.
  */
 int maxfp8_matmul_describe(int64_t M, int64_t N, int64_t K, int block_scaling, int with_workspace,
                            char* buf, size_t len);
-/* 1: ahead of what maxfp8_matmul_describe says, a bf16 result whose operands suit the four-wave kernel runs in its tiles of 256 x 192. */
+/* 1: the plan described is the four-wave kernel's in tiles of 256 x 192. */
 int maxfp8_matmul_tall(int64_t M, int64_t N, int64_t K, int block_scaling, int with_workspace);
 
 /* Bytes of workspace that lets the tiled kernels use every plan for this shape. */

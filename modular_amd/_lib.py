@@ -231,5 +231,5 @@ def matmul_describe(M: int, N: int, K: int, block_scaling: bool = True, with_wor
 
 
 def matmul_tall(M: int, N: int, K: int, block_scaling: bool = True, with_workspace: bool = True) -> bool:
-    """Whether, ahead of what matmul_describe says, a bf16 result runs in the four-wave kernel's tiles of 256 x 192 (diagnostic)."""
+    """Whether the plan that matmul_describe names is the four-wave kernel's in tiles of 256 x 192 (diagnostic)."""
     return bool(lib().maxfp8_matmul_tall(M, N, K, int(block_scaling), int(with_workspace)))

@@ -2315,7 +2315,7 @@ size_t gemm_tiled_qkv_workspace_bytes(int64_t M, int64_t N, int64_t K, bool bloc
   return plan.w4 && plan.w4_split ? gemm_w4_split(M, N, K, plan.w4).bytes : 0;
 }
 
-// Whether a bf16 result of this shape runs in tiles of 256 x 192 ahead of what gemm_tiled_describe says
+// Whether a bf16 result of this shape runs in tiles of 256 x 192 ahead of the rest of its plan
 int gemm_tiled_tall(int64_t M, int64_t N, int64_t K, bool blockscale, bool has_workspace) {
   return make_plan(M, N, K, blockscale, has_workspace, has_workspace ? gemm_tiled_workspace_bytes(M, N, K) : 0, 1, false).tall ? 1 : 0;
 }
@@ -2326,6 +2326,7 @@ int gemm_tiled_describe(int64_t M, int64_t N, int64_t K, bool blockscale, bool h
   auto count = [](int64_t m, int64_t n, const TileShape& t) { return (long long)(ceil_div(m, t.bm) * ceil_div(n, t.bn)); };
   // (what a bf16 result with 16-byte aligned rows gets)
   auto how = [](int64_t m, int64_t n, int variant) { return persist_shape(m, n, variant) ? " persistent" : (variant == 4 ? " three-stage" : ""); };
+  if (plan.tall && !plan.streamk) return snprintf(buf, len, "256x192 x%lld persistent, four waves", (long long)w4_tiles(M, N, 8));
   if (plan.w4 && plan.w4_split) {
     const long long n_tiles = (long long)(ceil_div(M, 32 * plan.w4) * ceil_div(N, 256));
     const W4Split sp = gemm_w4_split(M, N, K, plan.w4);

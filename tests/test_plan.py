@@ -3,6 +3,7 @@ a K split when the caller brings a workspace, or two regions when the last round
 main shape would leave most of the chip idle."""
 import re
 
+import bench
 from modular_amd import _lib
 
 
@@ -12,8 +13,8 @@ def parse(text):
 
 
 def test_single_shapes_and_k_split():
-    assert _lib.matmul_describe(2048, 6144, 4096) == "256x256 x192 persistent"
-    assert _lib.matmul_describe(2040, 6144, 4096) == "256x256 x192"
+    assert _lib.matmul_describe(2048, 6144, 4096 + 128) == "256x256 x192 persistent"
+    assert _lib.matmul_describe(2040, 6144, 4096 + 128) == "256x256 x192"
     assert _lib.matmul_describe(8, 4096, 4096) == "skinny"
     assert "block's waves" in _lib.matmul_describe(32, 28672, 4096)
     # 33 to 64 rows: the tiles whose blocks split K among their waves, or the 128-row tiles: wide matrices of short K, and narrow ones
@@ -70,8 +71,20 @@ def test_four_wave_kernel_where_its_tile_count_fits_the_chip(tune):
     assert "four waves" not in _lib.matmul_describe(4096, 7164, 16384)
     assert "four waves" not in _lib.matmul_describe(4096, 7168, 16384 + 128)
     assert "four waves" not in _lib.matmul_describe(128, 28672, 4096, False)
+    # tiles of 256 x 192, named wherever they are what runs
+    assert _lib.matmul_describe(2048, 6144, 4096) == _lib.matmul_describe(2040, 6144, 4096) == "256x192 x256 persistent, four waves"
+    for M, N, K, block in ((4096, 57344, 8192, True), (4096, 18432, 7168, True), (512, 24576, 1536, True), (1024, 24576, 1536, False), (1216, 28672, 4096, True),
+                           (1024, 24576, 1536, True), (16384, 8192, 28672, True), (2048, 2112, 4096, True), (2040, 6144, 4096 + 128, True), (117, 6144, 4096, True)):
+        for workspace in (True, False):
+            text = _lib.matmul_describe(M, N, K, block, workspace)
+            assert _lib.matmul_tall(M, N, K, block, workspace) == text.startswith("256x192 "), (M, N, K, text)
+            if text.startswith("256x192 "):
+                assert text == f"256x192 x{-(-M // 256) * -(-N // 192)} persistent, four waves"
+                assert bench.kernels_launched("block", M, K, N) == ("gemm_w4_kernel", text) or not block
     tune(MAXFP8_W4="0")
     assert "four waves" not in _lib.matmul_describe(4096, 7168, 16384)
+    tune(MAXFP8_W4="8")
+    assert _lib.matmul_describe(4096, 7168, 16384) == "256x192 x608 persistent, four waves"
     tune(MAXFP8_W4="6", MAXFP8_W4_SPLIT="0")
     assert _lib.matmul_describe(4096, 7168, 16384) == "192x256 x616 persistent, four waves"
     # the cut wants a last round of at most half the CUs' number of tiles (216 of 160 x 256 are too many), slabs in fours
