@@ -190,7 +190,10 @@ __global__ __launch_bounds__((BLOCKS == 1 ? 512 : 256) + (KV ? 64 : 0)) __attrib
     v4f part[LAG + 1];
     auto promote = [&](auto j_c) {
       constexpr int j = decltype(j_c)::value, mt = j / NT, nt = j % NT;
-      acc[mt][nt] += part[j % (LAG + 1)] * (as[mt] * (NT == 3 && nt >= nt_hi ? b1 : b0));
+      // (fused by name: the loop's copies of this have parts in common, and a product and a sum the compiler would merge one by one, each rounded)
+      const float scale = as[mt] * (NT == 3 && nt >= nt_hi ? b1 : b0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[mt][nt][i] = fmaf(part[j % (LAG + 1)][i], scale, acc[mt][nt][i]);
     };
     static_for<NM>([&](auto i_c) {
       constexpr int i = decltype(i_c)::value, mt = i / NT, nt = i % NT, c0 = i * PER / NM, c1 = (i + 1) * PER / NM;
