@@ -644,23 +644,24 @@ int gemm_skinny_quant_dispatch(const GemmArgs& p, bool blockscale, hipStream_t s
 // the offsets which slots are in use (a list in LDS, once), then takes every gridDim.x-th tile: no claims, and four blocks per CU, so that one
 // block's start and end hide behind the others' streams.  The persistent launch of gemm_tiled.hip, made for mixed sizes, gives
 // a CU tiles of 512 weight rows that its block claims from counters in memory: a tile is 21 us and more for one CU however few there are.
-// A slot of more than 32 rows is computed 32 rows at a time, its weights read again for each.  (Four groups of 16 rows per pass take 168 registers,
+// A slot of more than 32 rows is computed 32 rows at a time, its weights read again for each, and each 32 rows are tiles of their own: one slot of most
+// of the rows is spread over the chip like many.  (Four groups of 16 rows per pass take 168 registers,
 // three blocks per CU and spills: one token of 8 experts 7168 x 2048 70 -> 93 us, 64 tokens 467 -> 560.)
 template <int NTW, bool BLOCKSCALE>
 struct GroupedSkinnyCfg {
   static constexpr int WAVES = 4, RING_KB = NTW == 1 ? 6 : 8, THREADS = 64 * WAVES;
   using One = SkinnyCfg<NTW, 1, BLOCKSCALE, RING_KB, WAVES>;
   using Two = SkinnyCfg<NTW, 2, BLOCKSCALE, RING_KB, WAVES>;
-  static constexpr int LIST = One::SMEM > Two::SMEM ? One::SMEM : Two::SMEM;  // the slots in use, 16 bits each, behind the rings and sums
-  static constexpr int MAX_SLOTS = 512, SMEM = LIST + MAX_SLOTS * 2 + 2 * WAVES * 4;
+  static constexpr int LIST = One::SMEM > Two::SMEM ? One::SMEM : Two::SMEM;  // the units of work, behind the rings and sums
+  static constexpr int MAX_SLOTS = 512, MAX_ROWS = 16384, MAX_UNITS = MAX_SLOTS + MAX_ROWS / 32, SMEM = LIST + MAX_UNITS * 4 + 2 * WAVES * 4;
 };
 template <int NTW, bool BLOCKSCALE>
 __global__ __launch_bounds__(256, 4) void gemm_grouped_skinny_kernel(GemmArgs g, int ncol) {
   using Cfg = GroupedSkinnyCfg<NTW, BLOCKSCALE>;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  uint16_t* const list = reinterpret_cast<uint16_t*>(smem + Cfg::LIST);
-  int* const counts = reinterpret_cast<int*>(list + Cfg::MAX_SLOTS);
+  uint32_t* const list = reinterpret_cast<uint32_t*>(smem + Cfg::LIST);  // slot, and which 32 of its rows << 16
+  int* const counts = reinterpret_cast<int*>(list + Cfg::MAX_UNITS);
   // (rows held inside [0, M): a stale routing tensor must not turn into accesses outside the operands)
   auto rows_of = [&](int z, int64_t& begin) {
     const int64_t M = g.M, b = g.offsets[z], e = g.offsets[z + 1];
@@ -668,30 +669,39 @@ __global__ __launch_bounds__(256, 4) void gemm_grouped_skinny_kernel(GemmArgs g,
     const int64_t end = e < M ? e : M;
     return (int)(end > begin ? end - begin : 0);
   };
-  int used = 0;
+  int units = 0;
 #pragma unroll
   for (int half = 0; half < Cfg::MAX_SLOTS / Cfg::THREADS; ++half) {
     const int z = half * Cfg::THREADS + tid;
     int64_t begin;
-    const bool in_use = z < g.num_active && rows_of(z, begin) > 0;
-    const uint64_t with = __ballot(in_use);
-    if (lane == 0) counts[half * Cfg::WAVES + wave] = __popcll(with);
+    const int mine = z < g.num_active ? (rows_of(z, begin) + 31) >> 5 : 0;
+    // (the sums over the lanes bit by bit: mostly there is one)
+    int in_front = 0, of_wave = 0;
+    for (int bit = 0; __ballot(mine >> bit) != 0; ++bit) {
+      const uint64_t with = __ballot(mine >> bit & 1);
+      in_front += __popcll(with & (((uint64_t)1 << lane) - 1)) << bit;
+      of_wave += __popcll(with) << bit;
+    }
+    if (lane == 0) counts[half * Cfg::WAVES + wave] = of_wave;
     __syncthreads();
-    int before = used;
+    int at = units + in_front;
     for (int w = 0; w < Cfg::WAVES; ++w) {
       const int c = counts[half * Cfg::WAVES + w];
-      if (w < wave) before += c;
-      used += c;
+      if (w < wave) at += c;
+      units += c;
     }
-    if (in_use) list[before + __popcll(with & (((uint64_t)1 << lane) - 1))] = (uint16_t)z;
+    // (more than fit only with stale offsets that overlap)
+    for (int i = 0; i < mine && at + i < Cfg::MAX_UNITS; ++i) list[at + i] = (uint32_t)z | (uint32_t)i << 16;
   }
-  used = __builtin_amdgcn_readfirstlane(used);
-  for (int t = (int)blockIdx.x; t < used * ncol; t += (int)gridDim.x) {
+  units = __builtin_amdgcn_readfirstlane(units < Cfg::MAX_UNITS ? units : Cfg::MAX_UNITS);
+  for (int t = (int)blockIdx.x; t < units * ncol; t += (int)gridDim.x) {
     __syncthreads();  // the list is there; the last tile's sums have been read
     const int j = t / ncol, n0 = (t - j * ncol) * 16 * NTW;
-    const int slot = __builtin_amdgcn_readfirstlane((int)list[j]);
+    const uint32_t unit = __builtin_amdgcn_readfirstlane(list[j]);
+    const int slot = (int)(unit & 0xffffu), r0 = (int)(unit >> 16) * 32;
     int64_t begin;
-    const int rows = rows_of(slot, begin);
+    const int all = rows_of(slot, begin), rows = all - r0 < 32 ? all - r0 : 32;
+    begin += r0;
     const int e = g.expert_ids[slot];
     const int64_t esize = g.c_dtype == MAXFP8_BF16 ? 2 : 4;
     if (e < 0) {
@@ -707,17 +717,13 @@ __global__ __launch_bounds__(256, 4) void gemm_grouped_skinny_kernel(GemmArgs g,
     MatmulArgs p = g;
     p.b = g.b + (int64_t)e * g.b_expert_stride;
     p.b_scales = g.b_scales + (int64_t)e * g.bs_expert_stride;
-    for (int r0 = 0; r0 < rows; r0 += 32) {
-      if (r0 > 0) __syncthreads();
-      const int64_t row = begin + r0;
-      p.M = rows - r0 < 32 ? rows - r0 : 32;
-      p.a = g.a + row * g.lda;
-      p.a_scales = g.a_scales + (BLOCKSCALE ? row : row * g.a_scale_stride);
-      const uint32_t* c_rows = g.c_row_index ? g.c_row_index + row : nullptr;
-      p.c = g.c_row_index ? g.c : reinterpret_cast<uint8_t*>(g.c) + row * g.ldc * esize;
-      if (p.M <= 16) skinny_body<NTW, 1, BLOCKSCALE, Cfg::RING_KB, Cfg::WAVES, kActsPerSlab, false, true>(p, smem, n0, c_rows);
-      else skinny_body<NTW, 2, BLOCKSCALE, Cfg::RING_KB, Cfg::WAVES, kActsPerSlab, false, true>(p, smem, n0, c_rows);
-    }
+    p.M = rows;
+    p.a = g.a + begin * g.lda;
+    p.a_scales = g.a_scales + (BLOCKSCALE ? begin : begin * g.a_scale_stride);
+    const uint32_t* c_rows = g.c_row_index ? g.c_row_index + begin : nullptr;
+    p.c = g.c_row_index ? g.c : reinterpret_cast<uint8_t*>(g.c) + begin * g.ldc * esize;
+    if (rows <= 16) skinny_body<NTW, 1, BLOCKSCALE, Cfg::RING_KB, Cfg::WAVES, kActsPerSlab, false, true>(p, smem, n0, c_rows);
+    else skinny_body<NTW, 2, BLOCKSCALE, Cfg::RING_KB, Cfg::WAVES, kActsPerSlab, false, true>(p, smem, n0, c_rows);
   }
 }
 
@@ -743,20 +749,25 @@ static int launch_grouped_skinny(const GemmArgs& p, int64_t most_tiles, hipStrea
 // 8 per token, 1 / 16 / 64 / 80 tokens 95 / 146 / 251 / 254 and 45 / 116 / 240 / 274; 64 of 2048 x 1408, 6 per token, 1 / 16 / 80 / 96 tokens 70 / 88 / 121 /
 // 121 and 32 / 52 / 115 / 126.  Level at 400, 576 and 510 rows: what turns it is the slots of more than 32 rows, whose weights are read more than once.
 // So few slots turn it at fewer rows: one matmul of 7168 x 2048, 2 slots with 64 / 128 / 256 rows in all 42 / 28 / 29 us and 17 / 30 / 57, 4 slots with 128 / 256
-// 44 / 29 and 27 / 50, 8 with 256 / 448 41 / 40 and 31 / 57; 4096 x 7168, 4 slots with 128 / 256 / 448 123 / 64 / 70 and 41 / 79 / 143.  And one large slot among many: 16 slots,
-// half of 256 / 448 rows in one of them (136 / 238), 4096 x 7168 107 / 116 and 116 / 158, 7168 x 2048 54 / 60 and 56 / 72.
+// 44 / 29 and 27 / 50, 8 with 256 / 448 41 / 40 and 31 / 57; 4096 x 7168, 4 slots with 128 / 256 / 448 123 / 64 / 70 and 41 / 79 / 143.  (Those were measured with a slot's
+// 32-row parts one after the other in a block.)  Skewed routings, whose host knows no better, one matmul, weights from memory, persistent launch, this one, and with the parts
+// one after the other: 448 rows all in one of 64 slots, 3072 x 4096 70 / 40 / 94 us, 4096 x 7168 115 / 81 / 160, 7168 x 2048 43 / 49 / 58; half of them in one of 20 slots 74 / 65 / 88,
+// 125 / 140 / 166, 85 / 83 / 85; half of 300 in one of 64 155 / 134 / 149, 349 / 300 / 320, 165 / 170 / 169.  Over 440 routings of 64 to 448 rows the worst is 14 per cent behind, at 448 rows (40 before).
 // max_rows: the caller's bound on a slot's rows; all rows there are stands for one that does not know.
 bool gemm_grouped_skinny_ok(const GemmArgs& p, int64_t max_rows) {
-  if (p.num_active > GroupedSkinnyCfg<2, true>::MAX_SLOTS) return false;
+  if (p.num_active > GroupedSkinnyCfg<2, true>::MAX_SLOTS || p.M > GroupedSkinnyCfg<2, true>::MAX_ROWS) return false;
+  if (((int64_t)p.num_active + p.M / 32) * ceil_div(p.N, 16) >= (int64_t)1 << 30) return false;  // (the tiles' numbers)
   const int forced = tuning().grouped_decode;
   if (forced >= 0) return p.M <= forced;
   return p.M <= 448 && p.M <= 64 + 20 * p.num_active && (max_rows <= 128 || max_rows >= p.M);
 }
 int gemm_grouped_skinny_dispatch(const GemmArgs& p, bool blockscale, hipStream_t stream) {
-  const int64_t slots = p.M < p.num_active ? p.M : p.num_active, wide = slots * ceil_div(p.N, 32);
-  if (wide >= 4 * (int64_t)compute_units())
+  const int64_t slots = p.M < p.num_active ? p.M : p.num_active, units = slots + p.M / 32;  // (at most)
+  if (slots * ceil_div(p.N, 32) >= 4 * (int64_t)compute_units()) {
+    const int64_t wide = units * ceil_div(p.N, 32);
     return blockscale ? launch_grouped_skinny<2, true>(p, wide, stream) : launch_grouped_skinny<2, false>(p, wide, stream);
-  const int64_t narrow = slots * ceil_div(p.N, 16);
+  }
+  const int64_t narrow = units * ceil_div(p.N, 16);
   return blockscale ? launch_grouped_skinny<1, true>(p, narrow, stream) : launch_grouped_skinny<1, false>(p, narrow, stream);
 }
 
