@@ -46,6 +46,7 @@
 #include "common.h"
 #include "gemm_args.h"
 #include "gemm_device.h"
+#include "scale_rows.h"
 #include "tuning.h"
 
 namespace maxfp8 {
@@ -259,7 +260,7 @@ __device__ __forceinline__ void tile_body(const GemmArgs& p, uint8_t* smem, cons
     mt_live = left <= 0 ? 0 : ((left + 15) >> 4 < TM ? (left + 15) >> 4 : TM);
   }
   const float* bs_row = nullptr;
-  if constexpr (BLOCKSCALE) bs_row = bs_ptr + (int64_t)((n0 + wn * WN) / 128) * p.b_scales_ld;
+  if constexpr (BLOCKSCALE) bs_row = bs_ptr + (int64_t)weight_scale_row(n0 + wn * WN, p.N) * p.b_scales_ld;
   const uint32_t s_rd = (uint32_t)((BM + BN) * 128) + scale_read_offset<TM>(wm * WM, lm);
 
   // NS LDS stages, one barrier per slab, DMA issued NS-1 slabs ahead.  At the top of slab j a
