@@ -1896,14 +1896,17 @@ static float tile_overhead(int64_t M, int64_t N, int i, int splits, bool kv_on =
 
 // cost of a shape (microseconds) = rounds of resident blocks * time of one tile
 static int pick_shape(int64_t M, int64_t N, int nslab, bool blockscale, bool can_split, int64_t batch = 1, bool kv_on = false) {
-  // A batch of one slab of K (what gemm_one_slab_kernel does not take: other result types, ragged columns) is starts, ends and stores: 128 x 128 tiles, whose stores overlap the start of the CU's other block, but where
-  // 256 x 256 tiles are little more than whole rounds of the CUs and the small ones more than one.  Fitted to 27 batches (16, 64, 128 heads,
-  // 48 to 1024 tokens, N = 512, from the cache; us, 256 x 256 and 128 x 128): 16 heads of 256 / 1024 tokens 7.5 / 9.8 and 5.0 / 7.9, 64 of 256 / 512 9.7 / 13.5 and
-  // 8.4 / 14.7, 128 of 200 / 256 / 777 10.5 / 13.3 / 38.7 and 14.1 / 16.0 / 31.8.
+  // A batch of one slab of K is starts, ends and stores.  What of these comes here -- gemm_one_slab_kernel takes bf16 results of whole 32-column groups at K = 128 --
+  // has float32 results, ragged columns or a shorter K: 128 x 128 tiles, whose stores overlap the start of the CU's other block, but where 256 x 256 tiles are little
+  // more than whole rounds of the CUs and the small ones more than one.  Measured on 481 such batches (2 to 128 matrices, 70 to 1024 tokens, N = 100 to 1536; K = 128 with
+  // float32 results, with bf16 of ragged columns, K = 64 and 96 with either): 0.4 per cent behind the best of the four shapes on average, 17 at most (64 x 200 x 500 x 128,
+  // bf16, 24.8 us, on 256 x 128 21.2); the estimate below 7.5 and 115 (2 x 256 x 1536 x 128, float32, 13.6 us on 256 x 256, 6.3 on 128 x 128), small tiles alone 0.7 and 27.
+  // us on 256 x 256 and 128 x 128: float32, 128 x 200 / 777 x 512 16.5 / 64.0 and 21.0 / 60.3, 64 x 256 x 512 15.2 and 13.1; bf16, 128 x 300 x 500 77 and 49.
+  // (The constants were fitted to both tiles' times for bf16 results of N = 512.)
   if (batch > 1 && nslab == 1 && !kv_on) {
     const float large = (float)(ceil_div(M, 256) * ceil_div(N, 256) * batch), small = (float)(ceil_div(M, 128) * ceil_div(N, 128) * batch);
     const float fill = 0.5f + 0.5f * (float)M / (float)(ceil_div(M, 128) * 128);
-    return 5.5f + 0.0331f * large < 4.0f + 0.0094f * small * fill + (small > 512.f ? 1.5f : 0.f) ? 1 : 3;
+    return 5.5f + 0.0331f * large < 4.0f + 0.0094f * small * fill + (small > (float)kShapes[2].slots ? 1.5f : 0.f) ? 1 : 3;
   }
   int best = 0;
   float best_cost = 0.f;
