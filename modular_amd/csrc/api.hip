@@ -54,6 +54,7 @@ int naive_grouped_dispatch(void*, const void*, const void*, const void*, const v
 int gemm_tiled_dispatch(const GemmArgs&, bool, size_t, int64_t, hipStream_t);
 size_t gemm_tiled_workspace_bytes(int64_t, int64_t, int64_t);
 size_t gemm_tiled_plan_workspace_bytes(int64_t, int64_t, int64_t, bool);
+bool gemm_tiled_needs_no_workspace(int64_t, int64_t, int64_t, bool);
 int gemm_tiled_describe(int64_t, int64_t, int64_t, bool, bool, char*, size_t);
 int gemm_tiled_tall(int64_t, int64_t, int64_t, bool, bool);
 int gemm_grouped_dispatch(const GemmArgs&, bool, int64_t, int64_t, hipStream_t);
@@ -284,9 +285,10 @@ static Choice choose_kernel(int64_t M, int64_t N, int64_t K, bool block) {
   if (M > 2048) return {MAXFP8_ALGO_TILED, 0};
   return choose(Asked::kMatmul, M, N, K, block);
 }
-// the workspace MAXFP8_ALGO_AUTO uses with this scaling
+// the workspace MAXFP8_ALGO_AUTO uses with this scaling (up to 64 rows the choice of kernel asks whether the plan's is there)
 static size_t auto_workspace(int64_t M, int64_t N, int64_t K, bool block) {
-  return choose_kernel(M, N, K, block).algo == MAXFP8_ALGO_TILED ? gemm_tiled_workspace_bytes(M, N, K) : 0;
+  if (choose_kernel(M, N, K, block).algo != MAXFP8_ALGO_TILED) return 0;
+  return M > gemm_skinny_max_m() && gemm_tiled_needs_no_workspace(M, N, K, block) ? 0 : gemm_tiled_workspace_bytes(M, N, K);
 }
 
 // The same for the fused QKV matmul: decode kernel (at most 16 rows, and up to 32 where it is ahead -- more often than of a plain matmul, since the small tiles' store

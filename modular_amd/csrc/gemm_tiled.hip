@@ -2231,6 +2231,18 @@ size_t gemm_tiled_plan_workspace_bytes(int64_t M, int64_t N, int64_t K, bool blo
   return plan.splits > 1 ? (size_t)plan.splits * (size_t)M * (size_t)N * 4 : 0;
 }
 
+// Whether no call of this shape makes use of a workspace, although its plan has a use for one: it runs in tiles of 256 x 192, with the workspace and without, which
+// need none, and a result that those do not take runs the same whole tiles either way (a tail that the four-wave kernel would cut is of no use to
+// it: that kernel takes the same results).  4096 x 18432 x 7168: 48 MB that a linear held for nothing.
+static bool tall_without_workspace(int64_t M, int64_t N, int64_t K, bool blockscale, bool kv_on) {
+  const TiledPlan with = cached_plan(M, N, K, blockscale, true, ~(size_t)0, 1, kv_on);
+  if (!with.tall || with.streamk || with.splits != 1) return false;
+  const TiledPlan none = cached_plan(M, N, K, blockscale, false, 0, 1, kv_on);
+  return none.tall && none.splits == 1 && none.variant == with.variant && none.two.axis == with.two.axis && none.two.cut == with.two.cut &&
+         none.two.v1 == with.two.v1 && none.two.v2 == with.two.v2;
+}
+bool gemm_tiled_needs_no_workspace(int64_t M, int64_t N, int64_t K, bool blockscale) { return tall_without_workspace(M, N, K, blockscale, false); }
+
 // make_plan tries every cut of every pair of shapes: microseconds of host time, as much as a small matmul
 // takes on the GPU.  Plans are kept in a small table, keyed by everything make_plan reads (the generation
 // of the tuning switches included, since tests and tuning runs reload them between calls).
@@ -2316,6 +2328,7 @@ float gemm_tiled_qkv_cost(int64_t M, int64_t N, int64_t K, bool blockscale, bool
 // The workspace of a fused QKV matmul's plan (its cut tiles' sums; 0: none are cut)
 size_t gemm_tiled_qkv_workspace_bytes(int64_t M, int64_t N, int64_t K, bool blockscale) {
   const TiledPlan plan = cached_plan(M, N, K, blockscale, true, ~(size_t)0, 1, true);
+  if (tall_without_workspace(M, N, K, blockscale, true)) return 0;
   return plan.w4 && plan.w4_split ? gemm_w4_split(M, N, K, plan.w4).bytes : 0;
 }
 

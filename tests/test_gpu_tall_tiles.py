@@ -68,3 +68,29 @@ def test_fused_qkv_sequences(dev, tune, tm, batch):
     prompt, cached = [(5 * i + 3) % 8 * (40 if batch < 3 else 1) for i in range(batch)], [(7 * i) % 50 for i in range(batch)]
     run_case(dev, prompt, cached, Hq=6, H=2, D=64, K=512, mnk=ROW, page=16, layers=1, layer=0, nblocks=1100, seed=batch,
              algo="tiled", exact=True)
+
+
+@pytest.mark.parametrize("kind", ["block", "row"])
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
+def test_the_same_without_the_workspace_that_is_not_asked_for(dev, kind, out):
+    """A plan that cuts a tail, behind tiles of 256 x 192: whatever the result's type, a workspace changes nothing."""
+    M, N, K = 1216, 28672, 4096
+    L = _lib.lib()
+    need = L.maxfp8_matmul_workspace_bytes(M, N, K)
+    assert L.maxfp8_matmul_auto_workspace_bytes(M, N, K) == 0 < need
+    a, b = synth.random_fp8((M, K), 1).to(dev), synth.random_fp8((N, K), 2).to(dev)
+    if kind == "block":
+        sa, sb = synth.random_scales((K // 128, M), 3).to(dev), synth.random_scales((N // 128, K // 128), 4).to(dev)
+        how = (_lib.GRAN_BLOCK, _lib.GRAN_BLOCK, 1, 128, 128, M, K // 128)
+    else:
+        sa, sb = synth.random_scales((1, M), 3, lo=0.01, hi=0.1).to(dev), synth.random_scales((N, 1), 4, lo=0.001, hi=0.01).to(dev)
+        how = (_lib.GRAN_COLWISE, _lib.GRAN_ROWWISE, -1, -1, -1, M, 1)
+    workspace = torch.empty(need, dtype=torch.uint8, device=dev)
+    results = []
+    for ws, size in ((workspace.data_ptr(), need), (None, 0)):
+        c = torch.full((M, N), float("nan"), dtype=out, device=dev)
+        assert 0 == L.maxfp8_matmul_dynamic_scaled_fp8(c.data_ptr(), a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), M, N, K, K, K, N, *how,
+                                                       _lib.BF16 if out == torch.bfloat16 else _lib.F32, _lib.F32, _lib.ALGO_AUTO, ws, size,
+                                                       torch.cuda.current_stream(dev).cuda_stream), _lib.last_error()
+        results.append(c)
+    assert bool(torch.isfinite(results[0].float()).all()) and torch.equal(*results)

@@ -148,3 +148,16 @@ def test_rows_quantised_inside_the_decode_kernel():
     for M, N, inside in ((1, 28672, True), (2, 24576, True), (2, 28672, False), (3, 16384, True), (3, 24576, False), (4, 16384, True), (5, 4096, False)):
         assert (need(M, N, 4096, _lib.GRAN_ROWWISE) == 0) == inside, (M, N)
     assert need(4, 28672, 4096, _lib.GRAN_BLOCK) == 0 < need(5, 28672, 4096, _lib.GRAN_BLOCK)
+
+
+def test_no_workspace_for_a_plan_that_does_not_run():
+    """Where tiles of 256 x 192, which need none, are ahead of a plan that cuts a tail, a linear's workspace is its quantised rows and their scales."""
+    L = _lib.lib()
+    for M, N, K in ((4096, 18432, 7168), (1216, 28672, 4096), (4096, 24576, 7168)):
+        for granularity, scales in ((_lib.GRAN_BLOCK, K // 128 * M * 4), (_lib.GRAN_ROWWISE, M * 4), (_lib.GRAN_TENSOR, 256)):
+            assert _lib.matmul_tall(M, N, K, granularity == _lib.GRAN_BLOCK)
+            assert L.maxfp8_linear_workspace_bytes(M, N, K, granularity) == M * K + -(-scales // 256) * 256
+        assert L.maxfp8_matmul_auto_workspace_bytes(M, N, K) == 0 < L.maxfp8_matmul_workspace_bytes(M, N, K)
+    # (tall with block scales only; a cut that does run)
+    assert L.maxfp8_linear_workspace_bytes(4096, 57344, 8192, _lib.GRAN_ROWWISE) > 48 << 20 > L.maxfp8_linear_workspace_bytes(4096, 57344, 8192, _lib.GRAN_BLOCK)
+    assert L.maxfp8_linear_workspace_bytes(4096, 7168, 16384, _lib.GRAN_BLOCK) > 4096 * 16384 + (48 << 20)
