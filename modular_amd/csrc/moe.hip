@@ -424,8 +424,8 @@ __device__ __forceinline__ uint2 pack_e4m3fn8(const float (&q)[8]) {
 // DPP, 8-byte packed fp8 store.  A group's scales leave as ROWS consecutive floats: with 32 rows a whole line, which no other XCD's L2
 // holds a part of (32768 x 2048: 16 groups of a row per block, every scale alone, 73 us; 4 rows 113; 16 rows 68; 32 rows 62).
 // Bound by the bytes (5 per output where the result is quantised) and, as close, by the arithmetic: 30 instructions per output, two of
-// them four times as long.  Graph timing, operands cold, before this form and now: 2048 x 14336 rounding twice and quantising 45 -> 32 us
-// (147 MB: 4.6 TB/s), 32768 x 2048 rounding once 82 -> 65, 512 x 14336 13 -> 10, 16 x 14336 3.6 -> 2.7.
+// them four times as long.  Graph timing, operands from memory, before this form and now: 2048 x 14336 rounding twice and quantising 38.6 -> 29.9 us
+// (147 MB: 4.9 TB/s), 32768 x 2048 rounding once 82 -> 65, 512 x 14336 rounding twice 13.7 -> 10.8, 16 x 14336 4.6 -> 3.6 (from the cache 3.8 -> 2.8).
 template <SiluOut OUT, bool ROUND_ACT, int ROWS, int U>
 __global__ __launch_bounds__(16 * ROWS) void fused_silu_bf16_kernel(void* __restrict__ out, float* __restrict__ scales,
                                                               const uint16_t* __restrict__ in,
@@ -571,8 +571,8 @@ int fused_silu_dispatch(void* out, float* scales, const void* in, const uint32_t
     return launch_status("fused_silu_quantized (row)");
   }
   // The number of rows in use is only known on the device: the grid is sized for max_rows and walks the tiles in strides.  Tiles of
-  // 32 rows x 2 groups, or of 16 x 1 where those would leave half of the CUs without one (16 x 14336 3.2 and 2.7 us, 333 x 1408 3.3 and
-  // 2.7, 128 x 14336 3.7 and 5.0).
+  // 32 rows x 2 groups, or of 16 x 1 where those would leave half of the CUs without one (rounding twice, from memory, us: 16 x 14336 3.7 and 3.6, 333 x 1408 4.4 and
+  // 3.7, 128 x 14336 5.2 and 6.1, 512 x 14336 10.8 and 14.5; from the cache 3.3 and 2.8, 4.0 and 3.4, 5.2 and 6.1).
   const int64_t large = ceil_div(max_rows, 32) * ceil_div(inter / 128, 2);
   auto launch = [&](auto kern, int rows, int64_t tiles) {
     hipLaunchKernelGGL(kern, dim3((unsigned)(tiles < 16384 ? tiles : 16384)), dim3(16 * rows), 0, stream, out, scales, (const uint16_t*)in, row_offsets,
