@@ -84,18 +84,36 @@ __global__ __launch_bounds__(256) void gemm_short_k_kernel(MatmulArgs p_in) {
 //
 // Bound: the bytes, of which the bf16 results are most, and a start of three microseconds.  The tiles of gemm_tiled.hip stage 128 or 256 rows, whole or not,
 // and their results again, and store in bursts; with all operands in a wave's registers, as below, an L1 delivers the tokens once per 32 columns.
-// Graph timing, from the cache, 128 heads of 128 -> 512, those registers for 1 / 16 / 32 tokens 3.6 / 4.3 / 5.1 us, here 3.2 / 3.5 / 3.9; tiles for 48 / 128 / 256 /
-// 1024 tokens 6.1 / 8.4 / 13.3 / 40, here 4.3 / 7.7 / 12.8 / 34 (bytes at 6 TB/s 2.6 / 4.5 / 7.7 / 27; behind where a last chunk is mostly empty: 200 tokens 10.7 and
-// 11.9); 16 heads of 256 / 1024 tokens 5.0 / 7.9 and 3.9 / 7.4.
-template <int MT>
-__global__ __launch_bounds__(256) void gemm_one_slab_kernel(MatmulArgs p_in) {
+//   * The column blocks of a matrix's rows sit on one XCD, one behind the other (blocks go to the XCDs round-robin): its L2 reads the tokens once and holds whole
+//     rows of the result, where four of them each wrote every fourth 256 bytes.  128 heads of 1000 tokens, 128 -> 512, results from the cache 39.0 -> 26.3 us.
+//   * Stores pass the L2 (device scope) without staying in it: 48.6 -> 30.3 us with the results going to memory, and 26.3 -> 28.3 from the cache; non-temporal alone 41 and 40,
+//     device scope alone 58 and 26.  112 tokens 9.2 -> 7.7 and 7.4 -> 6.1.  Non-temporal alone where four blocks per CU and more take two chunks at most (of more than 16 tokens): all of their
+//     stores come at once, and 100 tokens of 128 -> 1024 are 13.1 and 9.0 us with it, 14.4 and 8.2 at device scope, 13.1 and 10.1 with neither.
+//   * Two blocks per CU walk the chunks of more: the weights are read once per block, and a mostly empty last chunk costs little.  80 tokens 7.4 -> 5.5 and 6.0 -> 4.9.
+// Graph timing, 128 heads of 128 -> 512, results to memory (four sets of operands in turn) / from the cache (one), the tiles and this kernel: 48 tokens 6.9 / 6.2 and 4.6 / 4.2,
+// 80 8.1 / 6.9 and 5.5 / 4.9, 200 12.6 / 11.0 and 8.1 / 7.4, 400 21.3 / 20.3 and 13.1 / 12.4, 1000 42.3 / 38.5 and 27.8 / 27.3, 1500 59.5 / 50.5 and 45.6 / 44.5 (bytes at
+// 6 TB/s: 2.6, 3.7, 7.1, 13, 28, 41).  Before the three: 5.5 / 4.9, 9.5 / 8.1, 14.5 / 11.9, 23.1 / 17.5, 51.5 / 38.7, 78.1 / 51.3.
+constexpr int kNonTemporal = 2, kPastL2 = 18;  // (device scope and non-temporal)
+// grid: (XCDs, 128-column blocks, the walkers of all matrices over the XCDs)
+template <int MT, int STORE_POLICY>
+__global__ __launch_bounds__(256) void gemm_one_slab_kernel(MatmulArgs p_in, int walkers, int batch) {
   constexpr int CHUNK = 16 * MT, A_BYTES = MT * 2048, COPIES = 2 * MT;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[16384 + 2 * (A_BYTES + 256)];
-  const MatmulArgs p = batch_view(p_in, blockIdx.z);
+  // (all arguments at once: behind the branches their loads would begin when those of the two counts are back, 0.1 us of the shortest launches)
+  asm volatile("" ::"s"(p_in.a), "s"(p_in.b), "s"(p_in.c), "s"(p_in.a_scales), "s"(p_in.b_scales), "s"(p_in.M), "s"(p_in.N), "s"(p_in.K), "s"(p_in.lda), "s"(p_in.ldb),
+               "s"(p_in.ldc), "s"(p_in.b_scales_ld), "s"(p_in.a_batch), "s"(p_in.b_batch), "s"(p_in.c_batch), "s"(p_in.a_scales_batch), "s"(p_in.b_scales_batch), "s"(walkers), "s"(batch));
+  const int walker = (int)blockIdx.z * 8 + (int)blockIdx.x;
+  int matrix = walker, first = 0;
+  if (walkers > 1) {
+    matrix = walker / walkers;
+    first = walker - matrix * walkers;
+  }
+  if (matrix >= batch) return;
+  const MatmulArgs p = batch_view(p_in, matrix);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lm = lane & 15, lq = lane >> 4, cr = lane >> 3, cp = lane & 7;
-  const int n0 = ((int)blockIdx.x * 4 + wave) * 32;
+  const int n0 = ((int)blockIdx.y * 4 + wave) * 32;
   const int chunks = (p.M + CHUNK - 1) / CHUNK;
 
   // rows past M, columns past N (whole waves: N is a multiple of 32) and scales past M read as zero through the descriptors
@@ -118,7 +136,7 @@ __global__ __launch_bounds__(256) void gemm_one_slab_kernel(MatmulArgs p_in) {
     const uint32_t chunk = (uint32_t)(cp ^ (((i & 1) << 2) | (cr & 3)));
     __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, (lds_ptr_t)(w_lds + i * 1024), 16, (uint32_t)cr * (uint32_t)p.ldb + chunk * 16u, (uint32_t)(i * 8) * (uint32_t)p.ldb, 0, 0);
   }
-  int chunk = (int)blockIdx.y;
+  int chunk = first;
   send(chunk, 0);
   const float bs = n0 < p.N ? p.b_scales[(int64_t)(n0 / 128) * p.b_scales_ld] : 0.f;
 
@@ -132,11 +150,11 @@ __global__ __launch_bounds__(256) void gemm_one_slab_kernel(MatmulArgs p_in) {
   const uint32_t c_voff = ((uint32_t)lm * (uint32_t)p.ldc + (uint32_t)(n0 + lq * 8)) * 2u | (n0 < p.N ? 0u : 0x80000000u);
   for (int buf = 0;; buf ^= 1) {
     // this wave's copies of the chunk have landed (behind them only the MT stores of the chunk before), then everyone's
-    if (chunk == (int)blockIdx.y) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (chunk == first) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(MT) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (chunk == (int)blockIdx.y) {
+    if (chunk == first) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) w[h] = frag(w_lds + (wrow + 4 * h) * 128, lq ^ wsw, (lq + 4) ^ wsw);
     }
@@ -147,7 +165,7 @@ __global__ __launch_bounds__(256) void gemm_one_slab_kernel(MatmulArgs p_in) {
       a[t] = frag(a_lds(buf) + (t * 16 + lm) * 128, lq ^ (lm & 7), (lq + 4) ^ (lm & 7));
       as[t] = *reinterpret_cast<const float*>(a_lds(buf) + A_BYTES + (t * 16 + lm) * 4);
     }
-    const int next = chunk + (int)gridDim.y;
+    const int next = chunk + walkers;
     // (the other buffer: every wave has read it before this chunk's barrier)
     if (next < chunks) send(next, buf ^ 1);
     __builtin_amdgcn_sched_barrier(0);
@@ -164,7 +182,7 @@ __global__ __launch_bounds__(256) void gemm_one_slab_kernel(MatmulArgs p_in) {
       }
       const uint32_t m = (uint32_t)(chunk * CHUNK + t * 16);
       const uint32_t at = (c_voff + m * (uint32_t)p.ldc * 2u) | (m + (uint32_t)lm < (uint32_t)p.M ? 0u : 0x80000000u);
-      __builtin_amdgcn_raw_buffer_store_b128(v4u_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])}, c_rsrc, at, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(v4u_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])}, c_rsrc, at, 0, STORE_POLICY);
     }
     if (next >= chunks) break;
     chunk = next;
@@ -176,15 +194,16 @@ int compute_units();
 // Batches of one slab of K and whole 32-column groups, bf16 results with 16-byte rows, offsets of 31 bits
 bool gemm_one_slab_ok(const GemmArgs& p, bool blockscale, int64_t batch) {
   const int64_t rows = (int64_t)p.M + 64, lim = (int64_t)1 << 31;
-  return blockscale && tuning().short_k && batch > 1 && !p.kv_on && p.K == 128 && p.N % 32 == 0 && p.c_dtype == MAXFP8_BF16 && p.c_vec8_ok &&
+  return blockscale && tuning().short_k && batch > 1 && !p.kv_on && p.K == 128 && p.N % 32 == 0 && p.N <= 128 * 65535 && p.c_dtype == MAXFP8_BF16 && p.c_vec8_ok &&
          rows * p.lda < lim && 32 * p.ldb < lim && rows * p.ldc * 2 < lim;
 }
 template <int MT>
 static int launch_one_slab(const GemmArgs& p, int64_t batch, hipStream_t stream) {
-  // a chunk per block up to four blocks per CU, which is what fits; beyond, as many as fit walk the chunks, the same number each
-  const int64_t columns = ceil_div(p.N, 128) * batch, chunks = ceil_div(p.M, 16 * MT), fit = 4 * (int64_t)compute_units() / columns;
-  const int64_t walk = ceil_div(chunks, fit > 1 ? fit : 1);
-  hipLaunchKernelGGL(gemm_one_slab_kernel<MT>, dim3((unsigned)ceil_div(p.N, 128), (unsigned)ceil_div(chunks, walk), (unsigned)batch), dim3(256), 0, stream, static_cast<const MatmulArgs&>(p));
+  // a walker per chunk up to two blocks per CU; beyond, so many walk the chunks, the same number each (see above)
+  const int64_t columns = ceil_div(p.N, 128), chunks = ceil_div(p.M, 16 * MT), fit = 2 * (int64_t)compute_units() / (columns * batch);
+  const int64_t walkers = ceil_div(chunks, ceil_div(chunks, fit > 1 ? fit : 1));
+  const bool at_once = columns * batch >= 4 * (int64_t)compute_units() && chunks <= 2 && p.M > 16;
+  hipLaunchKernelGGL((at_once ? gemm_one_slab_kernel<MT, kNonTemporal> : gemm_one_slab_kernel<MT, kPastL2>), dim3(8, (unsigned)columns, (unsigned)ceil_div(walkers * batch, 8)), dim3(256), 0, stream, static_cast<const MatmulArgs&>(p), (int)walkers, (int)batch);
   return launch_status("gemm_one_slab");
 }
 int gemm_one_slab_dispatch(const GemmArgs& p, int64_t batch, hipStream_t stream) {
