@@ -447,7 +447,7 @@ __global__ __launch_bounds__(16 * ROWS) void fused_silu_bf16_kernel(void* __rest
     uint4 gate[U], up[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      gate[u] = up[u] = make_uint4(0, 0, 0, 0);
+      gate[u] = up[u] = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);  // (no value: ones, as in the quantiser)
       if (row_ok && g0 + u < groups) {
         gate[u] = *reinterpret_cast<const uint4*>(src + u * 128);
         up[u] = *reinterpret_cast<const uint4*>(src + u * 128 + inter);

@@ -44,9 +44,12 @@ __device__ __forceinline__ uint4 load_input(const uint4* p) {
 }
 
 // ---------------------------------------------------------------------------
-// ROWS: a thread's U items are rows of one group instead of groups of one row, for rows of fewer than U groups, which left most of a
-// block without work and made it store a fraction of a line of scales (latent attention, 128 heads of K = 128 read from [token, head, channel]: 1024 / 256 / 48
-// tokens 16.4 / 6.0 / 3.4 -> 9.7 / 4.0 / 3.2 us; bytes at 6 TB/s 8.4 / 2.1 / 0.4).
+// What the lanes of rows and groups that a block has too many of compute with: ones.  (Zeros would take the branch of dynamic_scale_f32 that they all wait
+// for: 1 row of 512 3.2 us, 3.1 with ones.)
+constexpr uint32_t kNoValue = 0x3f803f80u;
+
+// ROWS: a thread's U items are rows of one group instead of groups of one row, for many rows of fewer than U groups, which left most of a
+// block without work and made it store a fraction of a line of scales (see the launch).
 template <int U, bool STREAM, bool ROWS>
 __global__ __launch_bounds__(256) void quant_g128_bf16_kernel(
     uint8_t* __restrict__ out, float* __restrict__ scales, const uint16_t* __restrict__ in,
@@ -72,7 +75,7 @@ __global__ __launch_bounds__(256) void quant_g128_bf16_kernel(
     if (live(u))
       v[u] = load_input<STREAM>(reinterpret_cast<const uint4*>(in + (ROWS ? source(row_of(u)) : src_row) * in_stride + (int64_t)group_of(u) * 128 + sl * 8));
     else
-      v[u] = make_uint4(0, 0, 0, 0);
+      v[u] = make_uint4(kNoValue, kNoValue, kNoValue, kNoValue);
   }
 
   float my_scale = 0.0f;
@@ -128,7 +131,7 @@ __global__ __launch_bounds__(256) void quant_g128_bf16_scatter_kernel(
     if (row_ok && g < ngroups)
       v[u] = *reinterpret_cast<const uint4*>(in + (int64_t)row * in_stride + (int64_t)g * 128 + sl * 8);
     else
-      v[u] = make_uint4(0, 0, 0, 0);
+      v[u] = make_uint4(kNoValue, kNoValue, kNoValue, kNoValue);
   }
   float my_scale = 0.0f;
   uint2 code[U];
@@ -549,6 +552,7 @@ __global__ __launch_bounds__(256) void copy_bytes_kernel(uint4* __restrict__ dst
 // ---------------------------------------------------------------------------
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+int compute_units();
 int quantize_dispatch(void* out_fp8, void* out_scales, const void* in, int64_t M, int64_t K,
                       int64_t in_row_stride, int64_t out_row_stride, int64_t G, int64_t scales_ld,
                       int in_dtype, int scales_dtype, float scale_ub, int64_t batch, int64_t in_batch_stride,
@@ -566,7 +570,11 @@ int quantize_dispatch(void* out_fp8, void* out_scales, const void* in, int64_t M
                       (out_row_stride % 8 == 0) && (in_batch_stride % 8 == 0) && (out_batch_stride % 8 == 0);
   if (fast_types && vec_ok && G == 128) {
     constexpr int U = 4;
-    const bool rows = ngroups < U;
+    // The rows form where it is the quicker one: rows of one or two groups, and enough of them that a quarter of the blocks fills the chip.  Strided heads, us, groups form and
+    // rows form, one group: 64 heads of 64 / 100 / 200 / 1000 rows 3.0 / 3.3 / 3.9 / 8.8 and 3.3 / 3.4 / 3.6 / 7.1; two groups: 16 heads of 256 / 513 / 1024 rows 3.2 / 4.0 / 5.0 and 3.4 /
+    // 3.8 / 4.7, 128 of 200, a fifth of whose blocks of 64 rows is empty, 6.3 and 6.9, of 513 11.7 and 11.0; three groups: 16 of 1024 6.0 and 6.2, 64 of 1000 15.8 and 15.7.
+    const bool many = ceil_div(M, 16) * (int64_t)nb > 2 * (int64_t)compute_units(), full = ceil_div(M, 16 * U) * (16 * U) - M <= M / 8;
+    const bool rows = many && (ngroups == 1 || (ngroups == 2 && full));
     const int64_t nxb = rows ? ngroups : ceil_div(ngroups, U);
     const int64_t blocks = ceil_div(M, rows ? 16 * U : 16) * nxb;
     if (blocks < (int64_t)1 << 31) {

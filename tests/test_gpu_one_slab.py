@@ -80,3 +80,22 @@ def test_no_slower_than_the_tiles(dev, B, M, N):
         return min(times)
 
     assert milliseconds("auto") < milliseconds("tiled")
+
+
+# (rows form: a few rows of many matrices, a last block of few rows, two groups in blocks that are nearly full; groups form: blocks a fifth empty, three groups)
+@pytest.mark.parametrize("B,M,K,rows", [(200, 50, 128, True), (3, 2753, 128, True), (5, 2001, 256, True), (130, 65, 256, False), (129, 66, 384, False), (16, 200, 128, False), (1, 1, 128, False)])
+def test_quantiser_of_many_short_rows(dev, B, M, K, rows):
+    from torch.profiler import ProfilerActivity, profile
+
+    x = torch.randn((M, B, K + 64), generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+    x[M // 2, :, :K] = 0
+    on = x.to(dev)[:, :, :K].transpose(0, 1)
+    with profile(activities=[ProfilerActivity.CUDA]) as seen:
+        q, s = mx.batched_quantize_dynamic_scaled_fp8(on, 128)
+        torch.cuda.synchronize()
+    names = [e.name for e in seen.events() if "quant_g128_bf16_kernel<" in e.name]
+    assert [", true>" in n for n in names] == [rows], names
+    for h in {0, B // 2, B - 1}:
+        bits = x[:, h, :K].contiguous().view(torch.int16).numpy().view(np.uint16)
+        want_q, want_s = oracle.quantize_dynamic_scaled_fp8(bits, 128)
+        assert np.array_equal(q[h].cpu().view(torch.uint8).numpy(), want_q) and np.array_equal(s[h].cpu().numpy()[:, :M], want_s)
