@@ -200,9 +200,9 @@ bool gemm_one_slab_ok(const GemmArgs& p, bool blockscale, int64_t batch) {
 template <int MT>
 static int launch_one_slab(const GemmArgs& p, int64_t batch, hipStream_t stream) {
   // a walker per chunk up to two blocks per CU; beyond, so many walk the chunks, the same number each (see above)
-  const int64_t columns = ceil_div(p.N, 128), chunks = ceil_div(p.M, 16 * MT), fit = 2 * (int64_t)compute_units() / (columns * batch);
+  const int64_t cus = compute_units(), columns = ceil_div(p.N, 128), chunks = ceil_div(p.M, 16 * MT), fit = 2 * cus / (columns * batch);
   const int64_t walkers = ceil_div(chunks, ceil_div(chunks, fit > 1 ? fit : 1));
-  const bool at_once = columns * batch >= 4 * (int64_t)compute_units() && chunks <= 2 && p.M > 16;
+  const bool at_once = columns * batch >= 4 * cus && chunks <= 2 && p.M > 16;
   hipLaunchKernelGGL((at_once ? gemm_one_slab_kernel<MT, kNonTemporal> : gemm_one_slab_kernel<MT, kPastL2>), dim3(8, (unsigned)columns, (unsigned)ceil_div(walkers * batch, 8)), dim3(256), 0, stream, static_cast<const MatmulArgs&>(p), (int)walkers, (int)batch);
   return launch_status("gemm_one_slab");
 }

@@ -1721,8 +1721,10 @@ W4Split gemm_w4_split(int64_t M, int64_t N, int64_t K, int tm);
 
 int compute_units() {
   static int cached[64] = {0};
+  // (where there is one device it is the current one: the question is 0.05 us, and launches of 2 us ask it)
+  static const bool only = [] { int n = 0; return hipGetDeviceCount(&n) == hipSuccess && n == 1; }();
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (!only && (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)) return 256;
   if (!cached[dev]) {
     int n = 0;
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;

@@ -573,8 +573,8 @@ int quantize_dispatch(void* out_fp8, void* out_scales, const void* in, int64_t M
     // The rows form where it is the quicker one: rows of one or two groups, and enough of them that a quarter of the blocks fills the chip.  Strided heads, us, groups form and
     // rows form, one group: 64 heads of 64 / 100 / 200 / 1000 rows 3.0 / 3.3 / 3.9 / 8.8 and 3.3 / 3.4 / 3.6 / 7.1; two groups: 16 heads of 256 / 513 / 1024 rows 3.2 / 4.0 / 5.0 and 3.4 /
     // 3.8 / 4.7, 128 of 200, a fifth of whose blocks of 64 rows is empty, 6.3 and 6.9, of 513 11.7 and 11.0; three groups: 16 of 1024 6.0 and 6.2, 64 of 1000 15.8 and 15.7.
-    const bool many = ceil_div(M, 16) * (int64_t)nb > 2 * (int64_t)compute_units(), full = ceil_div(M, 16 * U) * (16 * U) - M <= M / 8;
-    const bool rows = many && (ngroups == 1 || (ngroups == 2 && full));
+    const bool full = ceil_div(M, 16 * U) * (16 * U) - M <= M / 8;
+    const bool rows = (ngroups == 1 || (ngroups == 2 && full)) && ceil_div(M, 16) * (int64_t)nb > 2 * (int64_t)compute_units();
     const int64_t nxb = rows ? ngroups : ceil_div(ngroups, U);
     const int64_t blocks = ceil_div(M, rows ? 16 * U : 16) * nxb;
     if (blocks < (int64_t)1 << 31) {
